@@ -257,6 +257,14 @@ int wh_modwt_fwd_many(const void* x, void* xmod, int64_t n, int64_t count, int n
                       int filter, int dtype, void* stream);
 int wh_modwt_inv_many(const void* xmod, void* x, int64_t n, int64_t count, int nlevels,
                       int filter, int dtype, const wh_thresh* thr, void* stream);
+/* The DWT of `count` signals of n samples at once (1 <= count <= 65535),
+   signals and coefficients n apart; same arithmetic per signal as
+   wh_dwt_fwd / wh_dwt_inv (reference src/la8.cpp:10-115), one launch per
+   pass for all signals.  The output may be the input. */
+int wh_dwt_fwd_many(const void* x, void* y, int64_t n, int64_t count, int nlevels, int filter,
+                    int dtype, void* stream);
+int wh_dwt_inv_many(const void* y, void* x, int64_t n, int64_t count, int nlevels, int filter,
+                    int dtype, const wh_thresh* thr, void* stream);
 /* wh_modwt_inv_many without any device allocation.  No counterpart in the
    reference; it is for callers that cannot allocate (code under HIP graph
    capture, tight serving loops, harnesses that forbid hipMalloc).  The

@@ -78,6 +78,8 @@ SIGNATURES = {
     "wh_coeff_labels": (_I, [_I64, _I, _I, _I, _VP, _VP, _VP, _VP]),
     "wh_modwt_fwd_many": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
     "wh_modwt_inv_many": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, C.POINTER(wh_thresh), _VP]),
+    "wh_dwt_fwd_many": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
+    "wh_dwt_inv_many": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, C.POINTER(wh_thresh), _VP]),
     "wh_modwt_fwd_adj": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
     "wh_modwt_inv_adj": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
     "wh_dwt_fwd_adj": (_I, [_VP, _VP, _I64, _I, _I, _I, _VP]),

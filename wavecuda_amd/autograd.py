@@ -5,6 +5,7 @@ Every backward is a hand-written adjoint kernel of libwavehip:
   modwt(x)            forward MODWT        backward: wh_modwt_fwd_adj
   imodwt(w, n)        inverse MODWT        backward: wh_modwt_inv_adj
   dwt(x), idwt(y)     DWT / inverse        backward: the orthogonal transpose
+                      (wh_dwt_fwd_many / wh_dwt_inv_many, all rows at once)
   threshold(c, lam)   per-level hard/soft  backward: wh_thresh_grad (c and lam)
 
 x may be one signal (n,) or a batch (B, n) of equal-length signals; the
@@ -78,41 +79,50 @@ class ImodwtFn(torch.autograd.Function):
         return (gw[0] if squeeze else gw), None, None, None
 
 
-def _dwt_rows(fn, name, x, J, filt):
+_MAX_ROWS = 65535  # signals of one launch
+
+
+def _dwt_rows(inverse, x, J, filt):
+    """The DWT (or its inverse) of every row of x, all rows in one launch per
+    pass."""
     x2, squeeze = _rows(x.contiguous())
+    B, n = x2.shape
     out = torch.empty_like(x2)
-    for b in range(x2.shape[0]):
-        W.check(fn(_vp(x2[b]), _vp(out[b]), x2.shape[1], J, filt, _dtype(x2), _stream()), name)
+    for b in range(0, B, _MAX_ROWS):
+        rows = min(_MAX_ROWS, B - b)
+        if inverse:
+            W.check(W.lib().wh_dwt_inv_many(_vp(x2[b]), _vp(out[b]), n, rows, J, filt, _dtype(x2),
+                                            None, _stream()), "wh_dwt_inv_many")
+        else:
+            W.check(W.lib().wh_dwt_fwd_many(_vp(x2[b]), _vp(out[b]), n, rows, J, filt, _dtype(x2),
+                                            _stream()), "wh_dwt_fwd_many")
     return out[0] if squeeze else out
 
+
+# the DWT is orthogonal: each direction's adjoint is the other direction
 
 class DwtFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, J, filt):
         ctx.meta = (J, filt)
-        return _dwt_rows(W.lib().wh_dwt_fwd, "wh_dwt_fwd", x, J, filt)
+        return _dwt_rows(False, x, J, filt)
 
     @staticmethod
     def backward(ctx, g):
         J, filt = ctx.meta
-        return _dwt_rows(W.lib().wh_dwt_fwd_adj, "wh_dwt_fwd_adj", g, J, filt), None, None
+        return _dwt_rows(True, g, J, filt), None, None
 
 
 class IdwtFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, y, J, filt):
         ctx.meta = (J, filt)
-        x2, squeeze = _rows(y.contiguous())
-        out = torch.empty_like(x2)
-        for b in range(x2.shape[0]):
-            W.check(W.lib().wh_dwt_inv(_vp(x2[b]), _vp(out[b]), x2.shape[1], J, filt, _dtype(x2),
-                                       None, _stream()), "wh_dwt_inv")
-        return out[0] if squeeze else out
+        return _dwt_rows(True, y, J, filt)
 
     @staticmethod
     def backward(ctx, g):
         J, filt = ctx.meta
-        return _dwt_rows(W.lib().wh_dwt_inv_adj, "wh_dwt_inv_adj", g, J, filt), None, None
+        return _dwt_rows(False, g, J, filt), None, None
 
 
 class ThresholdFn(torch.autograd.Function):

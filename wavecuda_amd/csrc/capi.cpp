@@ -204,7 +204,7 @@ int wh_dwt_fwd(const void* x, void* y, int64_t n, int nlevels, int filter, int d
                void* stream) {
   int J, rc = check_common(x, y, n, nlevels, filter, dtype, &J);
   if (rc) return rc;
-  return dwt_forward(x, y, n, J, filter, dtype, static_cast<hipStream_t>(stream));
+  return dwt_forward(x, y, n, 1, J, filter, dtype, static_cast<hipStream_t>(stream));
 }
 
 int wh_dwt_inv(const void* y, void* x, int64_t n, int nlevels, int filter, int dtype,
@@ -212,7 +212,7 @@ int wh_dwt_inv(const void* y, void* x, int64_t n, int nlevels, int filter, int d
   int J, rc = check_common(y, x, n, nlevels, filter, dtype, &J);
   if (rc) return rc;
   if ((rc = check_thresh(thr, J))) return rc;
-  return dwt_inverse(y, x, n, J, filter, dtype, thr, static_cast<hipStream_t>(stream));
+  return dwt_inverse(y, x, n, 1, J, filter, dtype, thr, static_cast<hipStream_t>(stream));
 }
 
 int wh_threshold(void* coeffs, int64_t n, int nlevels, int ttype, int filter, int dtype,
@@ -240,6 +240,21 @@ int wh_modwt_inv_many(const void* xmod, void* x, int64_t n, int64_t count, int n
   return modwt_inverse(xmod, x, n, count, J, filter, dtype, thr, static_cast<hipStream_t>(stream));
 }
 
+int wh_dwt_fwd_many(const void* x, void* y, int64_t n, int64_t count, int nlevels, int filter,
+                    int dtype, void* stream) {
+  int J, rc = check_common(x, y, n, nlevels, filter, dtype, &J);
+  if (rc || (rc = check_count(count))) return rc;
+  return dwt_forward(x, y, n, count, J, filter, dtype, static_cast<hipStream_t>(stream));
+}
+
+int wh_dwt_inv_many(const void* y, void* x, int64_t n, int64_t count, int nlevels, int filter,
+                    int dtype, const wh_thresh* thr, void* stream) {
+  int J, rc = check_common(y, x, n, nlevels, filter, dtype, &J);
+  if (rc || (rc = check_count(count))) return rc;
+  if ((rc = check_thresh(thr, J))) return rc;
+  return dwt_inverse(y, x, n, count, J, filter, dtype, thr, static_cast<hipStream_t>(stream));
+}
+
 int wh_modwt_fwd_adj(const void* gxmod, void* gx, int64_t n, int64_t count, int nlevels,
                      int filter, int dtype, void* stream) {
   int J, rc = check_common(gxmod, gx, n, nlevels, filter, dtype, &J);
@@ -260,14 +275,14 @@ int wh_dwt_fwd_adj(const void* gy, void* gx, int64_t n, int nlevels, int filter,
                    void* stream) {
   int J, rc = check_common(gy, gx, n, nlevels, filter, dtype, &J);
   if (rc) return rc;
-  return dwt_inverse(gy, gx, n, J, filter, dtype, nullptr, static_cast<hipStream_t>(stream));
+  return dwt_inverse(gy, gx, n, 1, J, filter, dtype, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int wh_dwt_inv_adj(const void* gx, void* gy, int64_t n, int nlevels, int filter, int dtype,
                    void* stream) {
   int J, rc = check_common(gx, gy, n, nlevels, filter, dtype, &J);
   if (rc) return rc;
-  return dwt_forward(gx, gy, n, J, filter, dtype, static_cast<hipStream_t>(stream));
+  return dwt_forward(gx, gy, n, 1, J, filter, dtype, static_cast<hipStream_t>(stream));
 }
 
 int wh_threshold_many(void* coeffs, int64_t n, int64_t count, int nlevels, int ttype, int filter,

@@ -18,9 +18,14 @@
 // s on as a compact array, so the next pass reads contiguous memory.  Once
 // the compact sequence fits one workgroup's LDS a single "whole" kernel
 // finishes every remaining level.  Thresholding is fused into the inverse
-// as the details are read.
+// as the details are read.  blockIdx.y selects the signal of a launch over
+// many equal-length signals: a row of 2^12 samples fills 8 of the 256 CUs,
+// and a launch per row left the chip idle and the host busy (63 FP32 rows,
+// J = 6, forward + inverse and both adjoints: 504 launches, 1.5 ms of
+// kernels; one launch per pass for all rows: 8 launches).
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "dwt_dev.h"
@@ -90,6 +95,8 @@ struct TileArgs {
   int write_coarse;  // fwd: write y[q] with ctz >= g (first pass only)
   int src_shift;
   Thr thr;
+  // elements between the signals of a launch (blockIdx.y)
+  int64_t bs_src, bs_y, bs_dst;
 };
 
 // ------------------------------------------------------------ forward tile
@@ -116,8 +123,9 @@ __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
   const int tid = threadIdx.x;
   const int g = a.g;
   const int64_t N = a.N;
-  const T* __restrict__ src = static_cast<const T*>(a.src);
-  T* __restrict__ y = static_cast<T*>(a.y);
+  const int64_t sig = blockIdx.y;
+  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * a.bs_src;
+  T* __restrict__ y = static_cast<T*>(a.y) + sig * a.bs_y;
 
   const int64_t base = int64_t(blockIdx.x) * TILE;
   const int K0 = TILE + halo_fwd(g, L);
@@ -206,7 +214,7 @@ __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
     }
   }
   if (!a.final_pass) {
-    T* __restrict__ dst = static_cast<T*>(a.dst);
+    T* __restrict__ dst = static_cast<T*>(a.dst) + sig * a.bs_dst;
     const int own = TILE >> g;
     for (int i = tid; i < own; i += kNT) dst[(base >> g) + i] = cur[i];
   }
@@ -254,8 +262,9 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
   const int g = a.g, j0 = a.j0;
   const int64_t N = a.N;
   const int64_t base = int64_t(blockIdx.x) * TILE;
-  const T* __restrict__ src = static_cast<const T*>(a.src);
-  const T* __restrict__ y = static_cast<const T*>(a.y);
+  const int64_t sig = blockIdx.y;
+  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * a.bs_src;
+  const T* __restrict__ y = static_cast<const T*>(a.y) + sig * a.bs_y;
 
   auto evn = [](int l) { return inv_evn(l, L); };
   auto doff = [](int l) { return (TILE / 4 - (TILE >> (l - 1))) + PADS * (l - 3); };
@@ -496,7 +505,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
     const int npairs = TILE / 2;  // e_0 = 0
     const int off = evn(1);
     const T t = thr_level<T>(a.thr, j0);
-    T* __restrict__ dst = static_cast<T*>(a.dst);
+    T* __restrict__ dst = static_cast<T*>(a.dst) + sig * a.bs_dst;
     E2 res[kPairs];
 #pragma unroll
     for (int k = 0; k < kPairs; ++k) {
@@ -530,6 +539,7 @@ struct WholeArgs {
   int64_t N;        // compact length at level j0
   int j0, J;
   Thr thr;
+  int64_t bs_src, bs_y, bs_dst;  // as in TileArgs
 };
 
 template <typename T, int FILT>
@@ -539,8 +549,8 @@ __global__ __launch_bounds__(kNTW) void dwt_fwd_whole(WholeArgs a) {
   T* A = reinterpret_cast<T*>(smem_raw);
   T* B = A + a.N;
   const int tid = threadIdx.x;
-  const T* __restrict__ src = static_cast<const T*>(a.src);
-  T* __restrict__ y = static_cast<T*>(a.y);
+  const T* __restrict__ src = static_cast<const T*>(a.src) + int64_t(blockIdx.x) * a.bs_src;
+  T* __restrict__ y = static_cast<T*>(a.y) + int64_t(blockIdx.x) * a.bs_y;
   const int N = int(a.N);
   for (int i = tid; i < N; i += kNTW) A[i] = src[i];
   __syncthreads();
@@ -576,8 +586,8 @@ __global__ __launch_bounds__(kNTW) void dwt_inv_whole(WholeArgs a) {
   T* B = A + a.N;
   T* Cf = B + a.N / 2;  // the N coefficients of levels j0+1..J, thresholded
   const int tid = threadIdx.x;
-  const T* __restrict__ y = static_cast<const T*>(a.src);
-  T* __restrict__ dst = static_cast<T*>(a.dst);
+  const T* __restrict__ y = static_cast<const T*>(a.src) + int64_t(blockIdx.x) * a.bs_src;
+  T* __restrict__ dst = static_cast<T*>(a.dst) + int64_t(blockIdx.x) * a.bs_dst;
   const int N = int(a.N);
   const int j0 = a.j0, J = a.J;
   // The level-j0 sequence y[q 2^j0], q < N, holds every coefficient the
@@ -692,62 +702,88 @@ Thr thr_of(const wh_thresh* t) {
   return r;
 }
 
-template <typename T, int FILT>
-int dwt_fwd_f(const void* x, void* y, int64_t n, int J, hipStream_t st) {
-  auto ps = plan_passes<T>(n, J);
-  const T* src = static_cast<const T*>(x);
-  // in place: the first pass reads halos of neighbouring tiles, so stage x
-  if (x == y && !ps.front().whole) {
-    void* p = nullptr;
-    int rc = scratch2_get(size_t(n) * sizeof(T), &p);
+// Tile size of a pass over N values of each of `count` signals: by the
+// values of the whole launch, since it is the grid that must fill the chip.
+template <typename FN>
+int by_tile(int64_t N, int64_t count, FN fn) {
+  if (N * count >= kBigTileN) return fn(std::integral_constant<int, kTile>{});
+  if (N * count >= kSmallTileN) return fn(std::integral_constant<int, kTileSmall>{});
+  return fn(std::integral_constant<int, kTileTiny>{});
+}
+
+// Scratch of `count` signals: the compact sequences handed between passes
+// (two slots used alternately), and a copy of the input of an in-place call
+// whose first pass reads the halos of neighbouring tiles.
+template <typename T>
+int dwt_scratch(const void* in, const void* out, int64_t n, int64_t count,
+                const std::vector<Pass>& ps, hipStream_t st, const T** src, T** comp) {
+  *src = static_cast<const T*>(in);
+  *comp = nullptr;
+  void* p = nullptr;
+  if (in == out && !ps.front().whole) {
+    const size_t bytes = size_t(n) * size_t(count) * sizeof(T);
+    int rc = scratch2_get(bytes, &p);
     if (rc) return rc;
-    WH_HIP_CHECK(hipMemcpyAsync(p, x, size_t(n) * sizeof(T), hipMemcpyDeviceToDevice, st));
-    src = static_cast<const T*>(p);
+    WH_HIP_CHECK(hipMemcpyAsync(p, in, bytes, hipMemcpyDeviceToDevice, st));
+    *src = static_cast<const T*>(p);
   }
-  T* comp = nullptr;
   if (ps.size() > 1) {
-    void* p = nullptr;
-    int rc = scratch_get(size_t(n >> kGmax) * 2 * sizeof(T) + 64, &p);
+    int rc = scratch_get(size_t(n >> kGmax) * size_t(count) * 2 * sizeof(T) + 64, &p);
     if (rc) return rc;
-    comp = static_cast<T*>(p);
+    *comp = static_cast<T*>(p);
   }
+  return WH_OK;
+}
+
+template <typename T, int FILT>
+int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream_t st) {
+  auto ps = plan_passes<T>(n, J);
+  const T* src = nullptr;
+  T* comp = nullptr;
+  int rc = dwt_scratch<T>(x, y, n, count, ps, st, &src, &comp);
+  if (rc) return rc;
+  const int64_t bc = n >> kGmax;  // signals' distance in the compact scratch
+  int64_t bs_src = n;
   int slot = 0;
-  for (size_t pi = 0; pi < ps.size(); ++pi) {
-    const Pass& P = ps[pi];
+  for (const Pass& P : ps) {
     if (P.whole) {
       WholeArgs a{};
       a.src = src;
+      a.bs_src = bs_src;
       a.y = y;
+      a.bs_y = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.J = J;
       size_t lds = size_t(P.N + P.N / 2) * sizeof(T);
       allow_big_lds(dwt_fwd_whole<T, FILT>);
-      hipLaunchKernelGGL((dwt_fwd_whole<T, FILT>), dim3(1), dim3(kNTW), lds, st, a);
+      hipLaunchKernelGGL((dwt_fwd_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
       TileArgs a{};
       a.src = src;
+      a.bs_src = bs_src;
       a.y = y;
-      T* out = comp + slot * (n >> kGmax);
+      a.bs_y = n;
+      T* out = comp + slot * bc * count;
       a.dst = out;
+      a.bs_dst = bc;
       a.n = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.g = P.g;
       a.final_pass = (P.j0 + P.g == J);
       a.write_coarse = (P.j0 == 0);
-      if (P.N >= kBigTileN)
-        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, kTile>), dim3(unsigned(P.N / kTile)), dim3(kNT),
-                           0, st, a);
-      else if (P.N >= kSmallTileN)
-        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, kTileSmall>), dim3(unsigned(P.N / kTileSmall)),
-                           dim3(kNT), 0, st, a);
-      else
-        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, kTileTiny>), dim3(unsigned(P.N / kTileTiny)),
-                           dim3(kNT), 0, st, a);
-      WH_HIP_CHECK(hipGetLastError());
+      rc = by_tile(P.N, count, [&](auto tile) -> int {
+        constexpr int TILE = decltype(tile)::value;
+        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, TILE>),
+                           dim3(unsigned(P.N / TILE), unsigned(count)), dim3(kNT), 0, st, a);
+        WH_HIP_CHECK(hipGetLastError());
+        return WH_OK;
+      });
+      if (rc) return rc;
       src = out;
+      bs_src = bc;
       slot ^= 1;
     }
   }
@@ -755,64 +791,58 @@ int dwt_fwd_f(const void* x, void* y, int64_t n, int J, hipStream_t st) {
 }
 
 template <typename T, int FILT>
-int dwt_inv_f(const void* yin, void* x, int64_t n, int J, const wh_thresh* thr,
+int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const wh_thresh* thr,
               hipStream_t st) {
   auto ps = plan_passes<T>(n, J);
-  const T* y = static_cast<const T*>(yin);
-  if (yin == x && !ps.front().whole) {
-    void* p = nullptr;
-    int rc = scratch2_get(size_t(n) * sizeof(T), &p);
-    if (rc) return rc;
-    WH_HIP_CHECK(hipMemcpyAsync(p, yin, size_t(n) * sizeof(T), hipMemcpyDeviceToDevice, st));
-    y = static_cast<const T*>(p);
-  }
+  const T* y = nullptr;
   T* comp = nullptr;
-  if (ps.size() > 1) {
-    void* p = nullptr;
-    int rc = scratch_get(size_t(n >> kGmax) * 2 * sizeof(T) + 64, &p);
-    if (rc) return rc;
-    comp = static_cast<T*>(p);
-  }
+  int rc = dwt_scratch<T>(yin, x, n, count, ps, st, &y, &comp);
+  if (rc) return rc;
   const Thr th = thr_of(thr);
+  const int64_t bc = n >> kGmax;
   const T* src = nullptr;  // compact s handed down between passes
   int slot = 0;
   for (int pi = int(ps.size()) - 1; pi >= 0; --pi) {
     const Pass& P = ps[pi];
-    T* out = (P.j0 == 0) ? static_cast<T*>(x) : comp + slot * (n >> kGmax);
+    T* out = (P.j0 == 0) ? static_cast<T*>(x) : comp + slot * bc * count;
+    const int64_t bs_out = (P.j0 == 0) ? n : bc;
     if (P.whole) {
       WholeArgs a{};
       a.src = y;
+      a.bs_src = n;
       a.dst = out;
+      a.bs_dst = bs_out;
       a.N = P.N;
       a.j0 = P.j0;
       a.J = J;
       a.thr = th;
       size_t lds = size_t(2 * P.N + P.N / 2) * sizeof(T);
       allow_big_lds(dwt_inv_whole<T, FILT>);
-      hipLaunchKernelGGL((dwt_inv_whole<T, FILT>), dim3(1), dim3(kNTW), lds, st, a);
+      hipLaunchKernelGGL((dwt_inv_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
       TileArgs a{};
       const bool top = (P.j0 + P.g == J);
       a.src = top ? static_cast<const void*>(y) : static_cast<const void*>(src);
+      a.bs_src = top ? n : bc;
       a.src_shift = top ? J : 0;
       a.y = const_cast<T*>(y);
+      a.bs_y = n;
       a.dst = out;
+      a.bs_dst = bs_out;
       a.n = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.g = P.g;
       a.thr = th;
-      if (P.N >= kBigTileN)
-        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, kTile>), dim3(unsigned(P.N / kTile)), dim3(kNT),
-                           0, st, a);
-      else if (P.N >= kSmallTileN)
-        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, kTileSmall>), dim3(unsigned(P.N / kTileSmall)),
-                           dim3(kNT), 0, st, a);
-      else
-        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, kTileTiny>), dim3(unsigned(P.N / kTileTiny)),
-                           dim3(kNT), 0, st, a);
-      WH_HIP_CHECK(hipGetLastError());
+      rc = by_tile(P.N, count, [&](auto tile) -> int {
+        constexpr int TILE = decltype(tile)::value;
+        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, TILE>),
+                           dim3(unsigned(P.N / TILE), unsigned(count)), dim3(kNT), 0, st, a);
+        WH_HIP_CHECK(hipGetLastError());
+        return WH_OK;
+      });
+      if (rc) return rc;
     }
     src = out;
     slot ^= 1;
@@ -821,37 +851,38 @@ int dwt_inv_f(const void* yin, void* x, int64_t n, int J, const wh_thresh* thr,
 }
 
 template <typename T>
-int dwt_fwd_t(const void* x, void* y, int64_t n, int J, int filt, hipStream_t st) {
+int dwt_fwd_t(const void* x, void* y, int64_t n, int64_t count, int J, int filt, hipStream_t st) {
   switch (filt) {
-    case kHAAR: return dwt_fwd_f<T, kHAAR>(x, y, n, J, st);
-    case kD4: return dwt_fwd_f<T, kD4>(x, y, n, J, st);
-    case kC6: return dwt_fwd_f<T, kC6>(x, y, n, J, st);
-    default: return dwt_fwd_f<T, kLA8>(x, y, n, J, st);
+    case kHAAR: return dwt_fwd_f<T, kHAAR>(x, y, n, count, J, st);
+    case kD4: return dwt_fwd_f<T, kD4>(x, y, n, count, J, st);
+    case kC6: return dwt_fwd_f<T, kC6>(x, y, n, count, J, st);
+    default: return dwt_fwd_f<T, kLA8>(x, y, n, count, J, st);
   }
 }
 
 template <typename T>
-int dwt_inv_t(const void* y, void* x, int64_t n, int J, int filt, const wh_thresh* thr,
-              hipStream_t st) {
+int dwt_inv_t(const void* y, void* x, int64_t n, int64_t count, int J, int filt,
+              const wh_thresh* thr, hipStream_t st) {
   switch (filt) {
-    case kHAAR: return dwt_inv_f<T, kHAAR>(y, x, n, J, thr, st);
-    case kD4: return dwt_inv_f<T, kD4>(y, x, n, J, thr, st);
-    case kC6: return dwt_inv_f<T, kC6>(y, x, n, J, thr, st);
-    default: return dwt_inv_f<T, kLA8>(y, x, n, J, thr, st);
+    case kHAAR: return dwt_inv_f<T, kHAAR>(y, x, n, count, J, thr, st);
+    case kD4: return dwt_inv_f<T, kD4>(y, x, n, count, J, thr, st);
+    case kC6: return dwt_inv_f<T, kC6>(y, x, n, count, J, thr, st);
+    default: return dwt_inv_f<T, kLA8>(y, x, n, count, J, thr, st);
   }
 }
 
 }  // namespace
 
-int dwt_forward(const void* x, void* y, int64_t n, int J, int filt, int dtype, hipStream_t st) {
-  return dtype == WH_F32 ? dwt_fwd_t<float>(x, y, n, J, filt, st)
-                         : dwt_fwd_t<double>(x, y, n, J, filt, st);
+int dwt_forward(const void* x, void* y, int64_t n, int64_t count, int J, int filt, int dtype,
+                hipStream_t st) {
+  return dtype == WH_F32 ? dwt_fwd_t<float>(x, y, n, count, J, filt, st)
+                         : dwt_fwd_t<double>(x, y, n, count, J, filt, st);
 }
 
-int dwt_inverse(const void* y, void* x, int64_t n, int J, int filt, int dtype,
+int dwt_inverse(const void* y, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
                 const wh_thresh* thr, hipStream_t st) {
-  return dtype == WH_F32 ? dwt_inv_t<float>(y, x, n, J, filt, thr, st)
-                         : dwt_inv_t<double>(y, x, n, J, filt, thr, st);
+  return dtype == WH_F32 ? dwt_inv_t<float>(y, x, n, count, J, filt, thr, st)
+                         : dwt_inv_t<double>(y, x, n, count, J, filt, thr, st);
 }
 
 }  // namespace wh

@@ -45,16 +45,16 @@ int stats_buf(StatsBuf** out) {
 
 int64_t coeff_len(int ttype, int64_t n, int J) { return ttype == kDWT ? n : 2 * n * J; }
 
-int fwd(int ttype, const void* x, void* w, int64_t n, int J, int filt, int dtype,
+int fwd(int ttype, const void* x, void* w, int64_t n, int64_t count, int J, int filt, int dtype,
         hipStream_t st) {
-  return ttype == kDWT ? dwt_forward(x, w, n, J, filt, dtype, st)
-                       : modwt_forward(x, w, n, 1, J, filt, dtype, st);
+  return ttype == kDWT ? dwt_forward(x, w, n, count, J, filt, dtype, st)
+                       : modwt_forward(x, w, n, count, J, filt, dtype, st);
 }
 
-int inv(int ttype, const void* w, void* x, int64_t n, int J, int filt, int dtype,
+int inv(int ttype, const void* w, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
         const wh_thresh* thr, hipStream_t st) {
-  return ttype == kDWT ? dwt_inverse(w, x, n, J, filt, dtype, thr, st)
-                       : modwt_inverse(w, x, n, 1, J, filt, dtype, thr, st);
+  return ttype == kDWT ? dwt_inverse(w, x, n, count, J, filt, dtype, thr, st)
+                       : modwt_inverse(w, x, n, count, J, filt, dtype, thr, st);
 }
 
 // Candidates the search will certainly evaluate from state `cs` on (not
@@ -132,7 +132,7 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   if (threshtype == 0 || threshtype == 1) {  // MANUAL / UNIV
     void* w = nullptr;
     if ((rc = ws_get(size_t(coeff_len(ttype, n, J)) * esz, &w))) return rc;
-    if ((rc = fwd(ttype, x, w, n, J, filt, dtype, st))) return rc;
+    if ((rc = fwd(ttype, x, w, n, 1, J, filt, dtype, st))) return rc;
     wh_thresh t{};
     t.enabled = 1;
     t.hardness = hardness;
@@ -147,7 +147,7 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
       if ((rc = broadcast_threshold(sb->levels, &sb->vals[0], 1.0, J, st))) return rc;
       t.levels = sb->levels;
     }
-    if ((rc = inv(ttype, w, x, n, J, filt, dtype, &t, st))) return rc;
+    if ((rc = inv(ttype, w, x, n, 1, J, filt, dtype, &t, st))) return rc;
     if (threshtype == 1 && thresh) {
       if ((rc = d2h(thresh, &sb->vals[0], st))) return rc;
     } else {
@@ -182,17 +182,12 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   p += lenh * esz;
   void* yo = p;
 
-  if ((rc = fwd(ttype, x, W, n, J, filt, dtype, st))) return rc;
+  if ((rc = fwd(ttype, x, W, n, 1, J, filt, dtype, st))) return rc;
   if ((rc = univ_thresh_dev(W, n, J, ttype, dtype, minlevel, maxlevel, &sb->vals[0], st))) return rc;
   if ((rc = split_halves(x, xe, xo, n, dtype, st))) return rc;
-  // the two half-length MODWTs run as one two-signal launch (xe, xo and
+  // the two half-length transforms run as one two-signal launch (xe, xo and
   // We, Wo and ye, yo are adjacent): twice the workgroups, half the launches
-  if (ttype == kDWT) {
-    if ((rc = fwd(ttype, xe, We, lenh, Jh, filt, dtype, st))) return rc;
-    if ((rc = fwd(ttype, xo, Wo, lenh, Jh, filt, dtype, st))) return rc;
-  } else if ((rc = modwt_forward(xe, We, lenh, 2, Jh, filt, dtype, st))) {
-    return rc;
-  }
+  if ((rc = fwd(ttype, xe, We, lenh, 2, Jh, filt, dtype, st))) return rc;
 
   // one candidate: the halves thresholded at the point cv_advance last wrote
   wh_thresh th{};
@@ -207,13 +202,8 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   cva.J = Jh;
   cva.tol = tol;
   auto eval = [&]() -> int {
-    int r;
-    if (ttype == kDWT) {
-      if ((r = inv(ttype, We, ye, lenh, Jh, filt, dtype, &th, st))) return r;
-      if ((r = inv(ttype, Wo, yo, lenh, Jh, filt, dtype, &th, st))) return r;
-    } else if ((r = modwt_inverse(We, ye, lenh, 2, Jh, filt, dtype, &th, st))) {
-      return r;
-    }
+    const int r = inv(ttype, We, ye, lenh, 2, Jh, filt, dtype, &th, st);
+    if (r) return r;
     // the error reduction's last block also advances the search
     return interp_mse(x, ye, yo, n, dtype, sb->partial, &sb->vals[1], st, cva);
   };
@@ -236,7 +226,7 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   tf.minlevel = minlevel;
   tf.maxlevel = maxlevel;
   tf.value = t;
-  if ((rc = inv(ttype, W, x, n, J, filt, dtype, &tf, st))) return rc;
+  if ((rc = inv(ttype, W, x, n, 1, J, filt, dtype, &tf, st))) return rc;
   WH_HIP_CHECK(hipStreamSynchronize(st));
   if (thresh) *thresh = t;
   return WH_OK;

@@ -101,8 +101,10 @@ int wavethresh_pack(const void* c, void* out, int64_t n, int J, int ttype, int d
 int modwt_order(const void* in, void* out, int64_t n, int J, bool to_po, int dtype,
                 hipStream_t st);
 
-int dwt_forward(const void* x, void* y, int64_t n, int J, int filt, int dtype, hipStream_t st);
-int dwt_inverse(const void* y, void* x, int64_t n, int J, int filt, int dtype,
+// DWT of `count` signals of n samples, n apart in every array
+int dwt_forward(const void* x, void* y, int64_t n, int64_t count, int J, int filt, int dtype,
+                hipStream_t st);
+int dwt_inverse(const void* y, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
                 const wh_thresh* thr, hipStream_t st);
 
 int univ_thresh_dev(const void* c, int64_t n, int J, int ttype, int dtype, int minlevel,
