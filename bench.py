@@ -81,13 +81,18 @@ def plan_knobs(D, inverse: bool, n: int, J: int, filt: int) -> str | None:
 def plan_kernels(plan: str, inverse: bool) -> str:
     """The fused MODWT kernels a plan string launches, in launch order
     (LA8, FP64): modwt_fwd_k<T, filter, R, threads, levels, map, store> /
-    modwt_inv_k<T, filter, R, threads, levels, map>."""
+    modwt_inv_k<T, filter, R, threads, levels, map>, and for tiles
+    modwt_fwd_tile_k<T, filter, R, levels, threads, store> /
+    modwt_inv_tile_k<T, filter, R, levels, threads>."""
     import re
 
-    groups = re.findall(r"\{j0=(\d+) g=(\d+) R=(\d+) NT=(\d+)", plan)
+    groups = re.findall(r"\{j0=(\d+) g=(\d+) R=(\d+) NT=(\d+)[^}]*?( tile)?\}", plan)
     names = []
-    for _, g, r, nt in (reversed(groups) if inverse else groups):
-        if inverse:
+    for _, g, r, nt, tile in (reversed(groups) if inverse else groups):
+        if tile:
+            names.append(f"modwt_inv_tile_k<double, 4, {r}, {g}, {nt}>" if inverse
+                         else f"modwt_fwd_tile_k<double, 4, {r}, {g}, {nt}, 0>")
+        elif inverse:
             names.append(f"modwt_inv_k<double, 4, {r}, {nt}, {g}, {2 if r == '1' else 0}>")
         else:
             names.append(f"modwt_fwd_k<double, 4, {r}, {nt}, {g}, 0, 0>")

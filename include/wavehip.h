@@ -237,7 +237,8 @@ int wh_modwt_tune(int64_t n, int nlevels, int filter, int dtype, void* stream);
    "{j0= g= R= NT= M= nseg= P= warm= chunks= lds=} ...", into buf.
    wh_debug_modwt_set_plan sets the planner's choices for one shape as
    wh_modwt_tune would (deepest first group g1max, segments per CU of the
-   first and deeper groups, 512 or 256 threads in the first inverse group);
+   first and deeper groups, 512 or 256 threads in the first inverse group;
+   -512 or -256: tiles of that many threads and at most g1max = 3..6 levels);
    g1max <= 0 restores the default rules.  Results never depend on the
    plan; these let a caller run and check every plan the tuner can pick. */
 int wh_debug_modwt_plan(int inverse, int64_t n, int nlevels, int filter, int dtype, char* buf,

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "modwt_kern.h"
+#include "modwt_tile.h"
 #include "wh_common.h"
 #include "wh_internal.h"
 
@@ -18,6 +19,7 @@ namespace wh {
 
 namespace {
 
+static_assert(tile_r(false) <= 8 && tile_r(true) <= 8, "a tile group may start at level 3");
 constexpr int kNT1 = 512;   // threads, group starting at level 1 (R = 1)
 constexpr int kNTR = 256;   // threads, deeper groups (R = 32)
 constexpr int kRdeep = 32;
@@ -28,6 +30,7 @@ constexpr int kRdeep = 32;
 constexpr int kDeepSegPerCu = 4;
 
 struct Group {
+  bool tile = false;  // one tile per workgroup (modwt_tile.h) instead of a sliding window
   int j0, g, R, NT, M;
   int64_t P;
   int nseg, warm, nchunks;
@@ -40,7 +43,9 @@ struct PlanKnobs {
   int first_per_cu = 1;              // segments per CU of the first group
   int deep_per_cu = kDeepSegPerCu;   // segments per CU of deeper groups
   int first_nt = kNT1;               // threads of the first inverse group (512, or 256:
-                                     // two workgroups per CU in half the LDS)
+                                     // two workgroups per CU in half the LDS); negative: a
+                                     // plan of tiles of that many threads, at most g1max
+                                     // levels each
   bool operator<(const PlanKnobs& o) const {
     return std::tie(g1max, first_per_cu, deep_per_cu, first_nt) <
            std::tie(o.g1max, o.first_per_cu, o.deep_per_cu, o.first_nt);
@@ -51,39 +56,93 @@ using KnobKey = std::tuple<int, int64_t, int, int, int>;  // inverse, n, J, filt
 std::mutex g_knob_mu;
 std::map<KnobKey, PlanKnobs> g_knobs;
 
-// Default plan knobs, measured on MI355X (LA8, J = 10; forward and inverse
-// timed alternately, as in a pipeline):
-//  * an inverse launch of up to 2^18 samples (length times signals) has too
-//    few segments for the whole GPU with one 512-thread workgroup per CU: a
-//    256-thread first group (two segments per CU) of at most six levels
-//    (0.025 vs 0.028 ms at n = 2^16, 0.032 vs 0.035 at 2^17);
-//  * a single-signal FP32 inverse of more than 2^20 samples: a 256-thread
-//    first group of at most six levels, four segments per CU (half the FP64
-//    LDS, so several workgroups share a CU): n = 2^22 0.090 -> 0.083 ms,
-//    2^24 0.307 -> 0.258 ms (at 2^20 it measured 2-4 % slower).
-// Rules of the same kind for FP64 at 2^20-2^22 and for the forward, taken
-// from the tuner's isolated timings, were slower in the pipeline (there
-// the 2nJ coefficients fit the last-level cache, and what the other
-// transform leaves in it matters as much as the plan), so those keep the
-// plain defaults.
-PlanKnobs default_knobs(bool inverse, int64_t n, int64_t count, size_t esz) {
+std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz,
+                               const PlanKnobs& k, int64_t count = 1);
+
+// Default plan knobs, measured on MI355X (replayed graphs, three sets of
+// buffers in turn; us, sliding windows -> tiles, LA8 / Haar):
+//  * the inverse of a launch of up to 2^21 samples (length times signals)
+//    runs as tiles: n = 2^14, J = 8 FP64 21.0 -> 9.0 / 18.6 -> 7.2; 2^18,
+//    J = 10 36.4 -> 14.2 / 34.2 -> 11.3; 2^20, J = 10 57.2 -> 36.5 /
+//    41.0 -> 30.7; 2^21, J = 10 77.7 -> 66.5 / 64.3 -> 56.1 (FP32 49.0 ->
+//    46.0 / 36.1 -> 35.4); at 2^22 the two are level in FP64 and the sliding
+//    windows ahead in FP32 (82.6 against 87.7).  Tiles of 256 threads up to
+//    2^17 samples (2^17, J = 9: 10.8 against 11.5), 512 beyond (2^18, J = 10:
+//    14.2 against 15.7);
+//  * the forward of up to 2^18 samples as tiles of 512 threads (2^14, J = 8:
+//    18.4 -> 8.9 / 15.8 -> 7.0; 2^18, J = 10: 29.6 -> 16.5 / 26.5 -> 12.9),
+//    and of up to 2^19 where the sliding windows need more than one group
+//    (2^19, J = 10 FP32: 22.7 -> 16.2; Haar's one group 10.9 against 14.2).
+//    Beyond, it is bound by its stores, which the sliding windows make
+//    in longer runs (2^20, J = 8 FP32: 18.5 against 19.7);
+//  * a single-signal FP32 inverse beyond that: a 256-thread first group of
+//    at most six levels, four segments per CU (half the FP64 LDS, so
+//    several workgroups share a CU): n = 2^22 90 -> 83, 2^24 307 -> 258.
+// Rules for the FP64 sliding windows taken from the tuner's isolated
+// timings were slower in the pipeline (what the other transform leaves in
+// the last-level cache matters as much as the plan), so those keep the plain
+// defaults.
+PlanKnobs default_knobs(bool inverse, int64_t n, int64_t count, int J, int filt, size_t esz) {
   PlanKnobs k;
-  auto small_inverse = [&k](int per_cu) {
-    k.first_nt = kNT1 / 2;
-    k.first_per_cu = per_cu;
-    k.g1max = 6;
+  const int64_t total = n * count;
+  auto tiles = [&k](int threads) {
+    k.first_nt = -threads;
+    k.g1max = kTileGmax;
   };
-  if (inverse && n * count <= (int64_t(1) << 18))
-    small_inverse(2);
-  else if (inverse && count == 1 && esz == 4 && n > (int64_t(1) << 20))
-    small_inverse(4);
+  if (inverse && total <= (int64_t(1) << 21)) {
+    tiles(total <= (int64_t(1) << 17) ? kNT1 / 2 : kNT1);
+  } else if (inverse && count == 1 && esz == 4) {
+    k.first_nt = kNT1 / 2;
+    k.first_per_cu = 4;
+    k.g1max = 6;
+  } else if (!inverse && (total <= (int64_t(1) << 18) ||
+                          (total <= (int64_t(1) << 19) &&
+                           plan_groups(false, n, J, filter_length(filt), esz, k, count).size() > 1))) {
+    tiles(kNT1);
+  }
   return k;
 }
 
 PlanKnobs knobs_for(bool inverse, int64_t n, int J, int filt, size_t esz, int64_t count = 1) {
   std::lock_guard<std::mutex> lk(g_knob_mu);
   auto it = g_knobs.find(KnobKey{inverse ? 1 : 0, n, J, filt, int(esz)});
-  return it == g_knobs.end() ? default_knobs(inverse, n, count, esz) : it->second;
+  // tuned on one signal: tiles chosen there say nothing about a larger launch
+  const bool use = it != g_knobs.end() && (count == 1 || it->second.first_nt > 0);
+  return use ? it->second : default_knobs(inverse, n, count, J, filt, esz);
+}
+
+// Tile groups: levels 1..J in ceil(J / depth) groups of nearly equal depth.
+// A first of several groups has at least three levels, so that the next one's
+// 2^{j0} residues make whole blocks of tile_r.
+std::vector<Group> plan_tiles(bool inverse, int64_t n, int J, int L, size_t esz,
+                              const PlanKnobs& k) {
+  std::vector<Group> gs;
+  const int NT = -k.first_nt;
+  const int cap = std::min(k.g1max, kTileGmax);
+  const int deep = std::min(cap, kTileGmax - 1);
+  const int ng = J <= cap ? 1 : (J + deep - 1) / deep;
+  int j0 = 0;
+  for (int i = 0; i < ng; ++i) {
+    Group G{};
+    G.tile = true;
+    G.j0 = j0;
+    G.g = (J - j0 + (ng - i) - 1) / (ng - i);
+    if (i == 0 && ng > 1) G.g = std::max(G.g, 3);
+    G.R = j0 == 0 ? 1 : tile_r(inverse);
+    G.NT = NT;
+    G.M = 2 * NT / G.R;
+    G.P = G.M;
+    G.nseg = int(std::max<int64_t>(1, (n >> j0) / G.P));
+    G.warm = tile_halo(L, G.g);
+    G.nchunks = 1;
+    const size_t top = size_t(2 * NT + tile_halo(L, G.g) * G.R);
+    const size_t below = size_t(2 * NT + tile_halo(L, G.g - 1) * G.R);
+    G.lds = inverse ? 2 * (top + (G.g > 1 ? below : 0)) * esz
+                    : (top + size_t(2 * NT + (G.warm - tile_halo(L, 1)) * G.R)) * esz;
+    gs.push_back(G);
+    j0 += G.g;
+  }
+  return gs;
 }
 
 // LDS elements of one residue's buffers (the first inverse group keeps the
@@ -101,7 +160,8 @@ int64_t round_up64(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 // budget allows while its warm-up stays at most half a segment (one
 // segment per CU for the first group, kDeepSegPerCu for deeper ones).
 std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz,
-                               const PlanKnobs& k, int64_t count = 1) {
+                               const PlanKnobs& k, int64_t count) {
+  if (k.first_nt < 0) return plan_tiles(inverse, n, J, L, esz, k);
   const DeviceInfo& dev = device_info();
   const size_t budget = std::min<size_t>(dev.max_lds_per_block, 160 * 1024) - 1024;
   const int64_t cus = std::max(1, dev.num_cus);
@@ -174,6 +234,7 @@ int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t c
   // residue class for the inverse (L + 1 interleaved (S, D) reads instead of
   // 2L; it is LDS-bound)
   gl.map = inverse ? 2 : 0;
+  if (G.tile) return modwt_tile_launch<T>(inverse, filt, gl, a, st);
   if (gl.blocks > 0x7fffffff) return set_error(WH_ERR_ARG, "modwt: grid too large");
   if (inverse && G.R == 1 && (int64_t(1) << G.g) > G.M)
     return set_error(WH_ERR_UNSUPPORTED, "modwt: inverse group deeper than its chunk allows");
@@ -223,8 +284,9 @@ template <typename T>
 int modwt_fwd_t(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt, int sp,
                 hipStream_t st) {
   const int L = filter_length(filt);
-  auto groups = plan_groups(false, n, J, L, sizeof(T),
-                            knobs_for(false, n, J, filt, sizeof(T), count), count);
+  PlanKnobs k = knobs_for(false, n, J, filt, sizeof(T), count);
+  if (sp == kStoreAdjoint && k.first_nt < 0) k = PlanKnobs{};  // the tiles store a forward only
+  auto groups = plan_groups(false, n, J, L, sizeof(T), k, count);
   const int64_t per = 2 * n * J;
   for (const Group& G : groups) {
     ModwtArgs a = args_of(G, n);
@@ -309,6 +371,12 @@ int modwt_forward(const void* x, void* xmod, int64_t n, int64_t count, int J, in
                          : modwt_fwd_t<double>(x, xmod, n, count, J, filt, kStoreAll, st);
 }
 
+int modwt_forward_details(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
+                          int dtype, hipStream_t st) {
+  return dtype == WH_F32 ? modwt_fwd_t<float>(x, xmod, n, count, J, filt, kStoreSmooth, st)
+                         : modwt_fwd_t<double>(x, xmod, n, count, J, filt, kStoreSmooth, st);
+}
+
 int modwt_inverse(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
                   const wh_thresh* thr, hipStream_t st) {
   return dtype == WH_F32 ? modwt_inv_t<float>(xmod, x, n, count, J, filt, thr, st)
@@ -384,11 +452,13 @@ int tune_t(int64_t n, int J, int filt, hipStream_t st) {
   for (int inv = 0; inv < 2 && !rc; ++inv) {
     const bool inverse = inv == 1;
     std::map<std::string, PlanKnobs> cands;  // distinct plans only
-    for (int nt : {kNT1, kNT1 / 2}) {
-      if (nt != kNT1 && !inverse) continue;
-      for (int g1 = std::min(J, 5); g1 <= kGmax; ++g1)
+    for (int nt : {kNT1, kNT1 / 2, -kNT1, -kNT1 / 2}) {
+      if (nt == kNT1 / 2 && !inverse) continue;
+      const bool tile = nt < 0;  // only the depth matters
+      for (int g1 = tile ? 3 : std::min(J, 5); g1 <= (tile ? kTileGmax : kGmax); ++g1)
         for (int f : {1, 2, 4})
           for (int d : {1, 2, 4, 8}) {
+            if (tile && (f != 1 || d != 1)) continue;
             PlanKnobs k;
             k.g1max = g1;
             k.first_per_cu = f;
@@ -408,7 +478,7 @@ int tune_t(int64_t n, int J, int filt, hipStream_t st) {
     constexpr float kMargin = 0.98f;
     const char* env = std::getenv("WH_TUNE_LOG");  // candidate timings to stderr
     const bool log = env && env[0] == '1';
-    std::vector<PlanKnobs> order{default_knobs(inverse, n, 1, esz)};
+    std::vector<PlanKnobs> order{default_knobs(inverse, n, 1, J, filt, esz)};
     for (auto& c : cands) order.push_back(c.second);
     auto time_knobs = [&](const PlanKnobs& k, float* ms) -> int {
       {
@@ -472,7 +542,8 @@ int modwt_force_plan(bool inverse, int64_t n, int J, int filt, int dtype, int g1
     return WH_OK;
   }
   if (g1max > kGmax || first_per_cu < 1 || deep_per_cu < 1 ||
-      (first_nt != kNT1 && first_nt != kNT1 / 2) || (!inverse && first_nt != kNT1))
+      (std::abs(first_nt) != kNT1 && std::abs(first_nt) != kNT1 / 2) ||
+      (!inverse && first_nt == kNT1 / 2) || (first_nt < 0 && (g1max < 3 || g1max > kTileGmax)))
     return set_error(WH_ERR_ARG, "modwt plan: knobs out of range");
   PlanKnobs k;
   k.g1max = g1max;
@@ -492,8 +563,9 @@ std::string modwt_plan_string(bool inverse, int64_t n, int J, int filt, int dtyp
   for (auto& G : gs) {
     char buf[256];
     snprintf(buf, sizeof buf,
-             "{j0=%d g=%d R=%d NT=%d M=%d nseg=%d P=%lld warm=%d chunks=%d lds=%zu} ", G.j0,
-             G.g, G.R, G.NT, G.M, G.nseg, (long long)G.P, G.warm, G.nchunks, G.lds);
+             "{j0=%d g=%d R=%d NT=%d M=%d nseg=%d P=%lld warm=%d chunks=%d lds=%zu%s} ", G.j0,
+             G.g, G.R, G.NT, G.M, G.nseg, (long long)G.P, G.warm, G.nchunks, G.lds,
+             G.tile ? " tile" : "");
     s += buf;
   }
   return s;

@@ -48,7 +48,7 @@ int64_t coeff_len(int ttype, int64_t n, int J) { return ttype == kDWT ? n : 2 * 
 int fwd(int ttype, const void* x, void* w, int64_t n, int64_t count, int J, int filt, int dtype,
         hipStream_t st) {
   return ttype == kDWT ? dwt_forward(x, w, n, count, J, filt, dtype, st)
-                       : modwt_forward(x, w, n, count, J, filt, dtype, st);
+                       : modwt_forward_details(x, w, n, count, J, filt, dtype, st);
 }
 
 int inv(int ttype, const void* w, void* x, int64_t n, int64_t count, int J, int filt, int dtype,

@@ -61,6 +61,10 @@ void allow_dynamic_lds(const void* kern);
 // MODWT of `count` signals of n samples (x, out: n apart; xmod: 2nJ apart)
 int modwt_forward(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
                   int dtype, hipStream_t st);
+// the same for a caller that reads the details and S_J only: the other S
+// slots may be left unwritten
+int modwt_forward_details(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
+                          int dtype, hipStream_t st);
 int modwt_inverse(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
                   const wh_thresh* thr, hipStream_t st);
 // the same with the level hand-off in the caller's device workspace ws of

@@ -181,8 +181,8 @@ def modwt_set_plan(inverse: bool, n: int, nlevels: int, filter="LA8", dtype=torc
                    knobs=None) -> None:
     """Set the planner's choices for one shape as the tuner would: knobs =
     (deepest first group, segments per CU of the first group, of deeper
-    groups, threads of the first inverse group); None restores the default
-    rules."""
+    groups, threads of the first inverse group -- negative for a plan of
+    tiles of that many threads); None restores the default rules."""
     g1, f, d, nt = knobs if knobs is not None else (0, 1, 1, 512)
     W.check(W.lib().wh_debug_modwt_set_plan(1 if inverse else 0, n, nlevels, filter_code(filter),
                                             _DT[dtype], g1, f, d, nt), "wh_debug_modwt_set_plan")
@@ -192,20 +192,19 @@ def modwt_plan_candidates(inverse: bool, n: int, nlevels: int, filter="LA8",
                           dtype=torch.float64):
     """Every distinct plan the tuner times for this shape: {plan text: knobs}
     (the tuner's search space: deepest first group min(J, 5)..10, segments
-    per CU of the first group 1/2/4 and of deeper groups 1/2/4/8, and for
-    the inverse a 256-thread first group).  Leaves the default rules in
-    force."""
+    per CU of the first group 1/2/4 and of deeper groups 1/2/4/8, for the
+    inverse a 256-thread first group, and tiles of 512 or 256 threads and
+    3..6 levels).  Leaves the default rules in force."""
     f = filter_code(filter)
     J = resolve_levels(n, nlevels, f)
     out = {}
     try:
-        for nt in ((512, 256) if inverse else (512,)):
-            for g1 in range(min(J, 5), 11):
-                for fp in (1, 2, 4):
-                    for dp in (1, 2, 4, 8):
-                        k = (g1, fp, dp, nt)
-                        modwt_set_plan(inverse, n, J, f, dtype, k)
-                        out.setdefault(modwt_plan(inverse, n, J, f, dtype), k)
+        knobs = [(g1, fp, dp, nt) for nt in ((512, 256) if inverse else (512,))
+                 for g1 in range(min(J, 5), 11) for fp in (1, 2, 4) for dp in (1, 2, 4, 8)]
+        knobs += [(g1, 1, 1, -nt) for nt in (512, 256) for g1 in range(3, 7)]
+        for k in knobs:
+            modwt_set_plan(inverse, n, J, f, dtype, k)
+            out.setdefault(modwt_plan(inverse, n, J, f, dtype), k)
     finally:
         modwt_set_plan(inverse, n, J, f, dtype, None)
     return out
