@@ -329,7 +329,9 @@ int wh_median(const void* x, int64_t count, int dtype, double* out, void* stream
   s.base = x;
   s.mode = 0;
   s.count = count;
-  return select_median(s, dtype, false, st, 0.0, out, static_cast<hipStream_t>(stream));
+  SelOut o;
+  o.out = out;
+  return select_median(s, dtype, st, o, static_cast<hipStream_t>(stream));
 }
 
 int wh_mad(const void* x, int64_t count, int dtype, double* out, void* stream) {
@@ -342,7 +344,10 @@ int wh_mad(const void* x, int64_t count, int dtype, double* out, void* stream) {
   s.base = x;
   s.mode = 0;
   s.count = count;
-  return select_mad(s, dtype, st, 0.0, out, static_cast<hipStream_t>(stream));
+  SelOut o;
+  o.out = out;
+  o.mad = 1;
+  return select_median(s, dtype, st, o, static_cast<hipStream_t>(stream));
 }
 
 int wh_univ_thresh(const void* coeffs, int64_t n, int nlevels, int ttype, int filter, int dtype,
@@ -355,7 +360,11 @@ int wh_univ_thresh(const void* coeffs, int64_t n, int nlevels, int ttype, int fi
   if (ttype != kDWT && ttype != kMODWT) return set_error(WH_ERR_ARG, "ttype must be 0 or 1");
   if (minlevel < 0 || minlevel > maxlevel || maxlevel >= J)
     return set_error(WH_ERR_ARG, "levels must satisfy 0 <= minlevel <= maxlevel < nlevels");
-  return univ_thresh_dev(coeffs, n, J, ttype, dtype, minlevel, maxlevel, out,
+  SelState* st;
+  if ((rc = stats_state(&st))) return rc;
+  SelOut o;
+  o.out = out;
+  return univ_thresh_dev(coeffs, n, J, ttype, dtype, minlevel, maxlevel, st, o,
                          static_cast<hipStream_t>(stream));
 }
 

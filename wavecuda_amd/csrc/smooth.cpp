@@ -87,10 +87,7 @@ int d2h(double* host, const double* dev, hipStream_t st) {
 // src/thresh.cpp:170-201 (with the time-ordered MODWT gathering detail
 // blocks from level 0 whatever minlevel is, src/wavutils.cpp:711-717)
 int univ_thresh_dev(const void* c, int64_t n, int J, int ttype, int dtype, int minlevel,
-                    int maxlevel, double* out, hipStream_t st) {
-  StatsBuf* sb = nullptr;
-  int rc = stats_buf(&sb);
-  if (rc) return rc;
+                    int maxlevel, SelState* sel, SelOut o, hipStream_t st) {
   SelSrc s{};
   s.base = c;
   s.n = n;
@@ -115,7 +112,9 @@ int univ_thresh_dev(const void* c, int64_t n, int J, int ttype, int dtype, int m
     s.count = int64_t(maxlevel - minlevel + 1) * n;
     factor = std::sqrt(2. * std::log(double(n)));
   }
-  return select_mad(s, dtype, &sb->sel, factor, out, st);
+  o.mad = 1;
+  o.factor = factor;
+  return select_median(s, dtype, sel, o, st);
 }
 
 int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int threshtype,
@@ -143,8 +142,11 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
       t.value = *thresh;
     } else {
       // univ_thresh(w, 0, 0) (src/rfunctions.cu:82-87)
-      if ((rc = univ_thresh_dev(w, n, J, ttype, dtype, 0, 0, &sb->vals[0], st))) return rc;
-      if ((rc = broadcast_threshold(sb->levels, &sb->vals[0], 1.0, J, st))) return rc;
+      SelOut o;
+      o.out = &sb->vals[0];
+      o.levels = sb->levels;
+      o.J = J;
+      if ((rc = univ_thresh_dev(w, n, J, ttype, dtype, 0, 0, &sb->sel, o, st))) return rc;
       t.levels = sb->levels;
     }
     if ((rc = inv(ttype, w, x, n, 1, J, filt, dtype, &t, st))) return rc;
@@ -171,9 +173,7 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   void* W = p;
   p += cw * esz;
   void* We = p;
-  p += ch * esz;
-  void* Wo = p;
-  p += ch * esz;
+  p += 2 * ch * esz;  // and the odd half's
   void* xe = p;
   p += lenh * esz;
   void* xo = p;
@@ -183,7 +183,11 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   void* yo = p;
 
   if ((rc = fwd(ttype, x, W, n, 1, J, filt, dtype, st))) return rc;
-  if ((rc = univ_thresh_dev(W, n, J, ttype, dtype, minlevel, maxlevel, &sb->vals[0], st))) return rc;
+  SelOut o;
+  o.levels = sb->cvlev;
+  o.J = Jh;
+  o.cv = &sb->cv;
+  if ((rc = univ_thresh_dev(W, n, J, ttype, dtype, minlevel, maxlevel, &sb->sel, o, st))) return rc;
   if ((rc = split_halves(x, xe, xo, n, dtype, st))) return rc;
   // the two half-length transforms run as one two-signal launch (xe, xo and
   // We, Wo and ye, yo are adjacent): twice the workgroups, half the launches
@@ -207,7 +211,6 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
     // the error reduction's last block also advances the search
     return interp_mse(x, ye, yo, n, dtype, sb->partial, &sb->vals[1], st, cva);
   };
-  if ((rc = cv_init(&sb->cv, &sb->vals[0], sb->cvlev, Jh, st))) return rc;
   CvState cs{};
   for (int batch = 2;;) {  // t1 and t2 first
     for (int i = 0; i < batch; ++i)

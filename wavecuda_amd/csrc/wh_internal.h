@@ -111,8 +111,6 @@ int dwt_forward(const void* x, void* y, int64_t n, int64_t count, int J, int fil
 int dwt_inverse(const void* y, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
                 const wh_thresh* thr, hipStream_t st);
 
-int univ_thresh_dev(const void* c, int64_t n, int J, int ttype, int dtype, int minlevel,
-                    int maxlevel, double* out, hipStream_t st);
 int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int threshtype,
            double* thresh, int hardness, int minlevel, int maxlevel, double tol,
            hipStream_t st);

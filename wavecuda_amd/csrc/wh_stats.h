@@ -28,20 +28,25 @@ struct SelSrc {
   int64_t count;
   int64_t off;
   int lmin, lmax, J;
+  int lgn;  // log2 n (set by select_median)
 };
 
-// device-resident selection state
-constexpr int kSelCandCap = 16384;  // keys the finishing workgroup keeps in LDS
+// device-resident selection state (select.hip); [2]: values, deviations
+constexpr int kSelCandCap = 1 << 17;  // gathered keys it keeps
+constexpr int kSelSample = 512;
+constexpr int kSelEdges = 104;        // +- 4.6 standard deviations of the sample's middle
+constexpr int kSelReplicas = 8;       // copies of the counters
+constexpr int kSelPad = 16;           // a cache line of counters
+constexpr int kSelBuckets = 2 * kSelEdges + 1;
 
 struct SelState {
-  uint64_t prefix[2];
-  long long k[2];
   double med;
-  double mad;
-  unsigned long long ncand;  // keys appended to cand by the compaction pass
-  uint64_t cmin[2], cmax[2];  // smallest / largest key under each prefix
-  unsigned long long hist[2 * 2048];
-  uint64_t cand[kSelCandCap];
+  unsigned long long ncand[2][kSelReplicas * kSelPad];
+  unsigned long long bins[2][kSelReplicas * kSelBuckets];
+  unsigned long long hist[2][2048];
+  uint64_t edges[2][kSelEdges];
+  uint64_t sample[kSelSample];
+  uint64_t cand[2][kSelCandCap];
 };
 
 constexpr int kMaxPartials = 1024;
@@ -55,14 +60,45 @@ struct CvState {
   int iter, pending, nevals, stop;
 };
 
+// bracket [0, t3] and the first point t1 into levels[0..J) (one thread)
+__device__ inline void cv_start(CvState* cs, double t3, double* levels, int J) {
+#pragma clang fp contract(off)
+  const double C = 1. - 0.61803399;
+  const double tb = t3 / 2.;
+  cs->t0 = 0.;
+  cs->t2 = tb;
+  cs->t1 = tb - C * (tb - 0.);
+  cs->t3 = t3;
+  cs->m1 = cs->m2 = 0.;
+  cs->iter = 0;
+  cs->pending = 1;
+  cs->nevals = 0;
+  cs->stop = 0;
+  for (int l = 0; l < J; ++l) levels[l] = cs->t1;
+}
+
 // in-place threshold of `count` transformed signals (DWT: n apart, MODWT:
 // 2nJ apart)
 int threshold_inplace(void* c, int64_t n, int64_t count, int J, int ttype, int dtype,
                       const wh_thresh* thr, hipStream_t st);
-int select_median(const SelSrc& s, int dtype, bool deviation, SelState* st, double factor,
-                  double* out, hipStream_t stream);
-int select_mad(const SelSrc& s, int dtype, SelState* st, double factor, double* out,
-               hipStream_t stream);
+// Median of the selection, or with `mad` 1.4826 times the median of the
+// deviations from it, times `factor` when > 0; written to *out, and to
+// levels[0..J) or, with cv, as the bracket of a search whose first point
+// goes there (each where not null).
+struct SelOut {
+  double* out = nullptr;
+  int mad = 0;
+  double factor = 0.0;
+  double* levels = nullptr;
+  int J = 0;
+  CvState* cv = nullptr;
+};
+int select_median(const SelSrc& s, int dtype, SelState* st, const SelOut& o, hipStream_t stream);
+// Universal threshold (smooth.cpp): the MAD of the levels' details times the
+// reference's factor, whose sqrt(2 ln n) comes from the host's C library so
+// that it rounds like the reference
+int univ_thresh_dev(const void* c, int64_t n, int J, int ttype, int dtype, int minlevel,
+                    int maxlevel, SelState* sel, SelOut o, hipStream_t st);
 // search state the CV error reduction advances (cs == nullptr: none)
 struct CvArgs {
   CvState* cs = nullptr;
@@ -73,9 +109,5 @@ struct CvArgs {
 int interp_mse(const void* xn, const void* ye, const void* yo, int64_t len, int dtype,
                double* partial_buf, double* out, hipStream_t st, const CvArgs& cv = CvArgs{});
 int split_halves(const void* x, void* e, void* o, int64_t len, int dtype, hipStream_t st);
-int broadcast_threshold(double* dst, const double* src, double scale, int J, hipStream_t st);
-// bracket [0, *tc] and the first point t1 into levels[0..J)
-int cv_init(CvState* cs, const double* tc, double* levels, int J, hipStream_t st);
-
 
 }  // namespace wh
