@@ -76,7 +76,17 @@ struct Thr {
   int on, hardness, minlevel, maxlevel;
   double value;
   const double* levels;
+  // candidates of `of` inputs (of > 0), as ModwtArgs
+  int of;
+  int64_t th_stride;
 };
+
+// the input that signal y of an inverse reads, and its thresholds
+__device__ __forceinline__ int thr_input(Thr& t, int y) {
+  if (t.of <= 0) return y;
+  if (t.levels) t.levels += (y / t.of) * t.th_stride;
+  return y % t.of;
+}
 
 template <typename T>
 __device__ __forceinline__ T thr_level(const Thr& t, int lev0) {
@@ -94,6 +104,7 @@ struct TileArgs {
   int final_pass;    // fwd: s_{j0+g} = s_J goes to y
   int write_coarse;  // fwd: write y[q] with ctz >= g (first pass only)
   int src_shift;
+  int src_in;        // inv: src holds the inputs (the top pass), not one entry per signal
   Thr thr;
   // elements between the signals of a launch (blockIdx.y)
   int64_t bs_src, bs_y, bs_dst;
@@ -263,8 +274,10 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
   const int64_t N = a.N;
   const int64_t base = int64_t(blockIdx.x) * TILE;
   const int64_t sig = blockIdx.y;
-  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * a.bs_src;
-  const T* __restrict__ y = static_cast<const T*>(a.y) + sig * a.bs_y;
+  Thr thr = a.thr;
+  const int64_t inp = thr_input(thr, int(blockIdx.y));
+  const T* __restrict__ src = static_cast<const T*>(a.src) + (a.src_in ? inp : sig) * a.bs_src;
+  const T* __restrict__ y = static_cast<const T*>(a.y) + inp * a.bs_y;
 
   auto evn = [](int l) { return inv_evn(l, L); };
   auto doff = [](int l) { return (TILE / 4 - (TILE >> (l - 1))) + PADS * (l - 3); };
@@ -401,14 +414,14 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
     for (int l = 3; l <= kGmax; ++l) {
       if (l <= g) {
         const int cnt = (TILE >> l) + evn(l);
-        const T t = thr_level<T>(a.thr, j0 + l - 1);
+        const T t = thr_level<T>(thr, j0 + l - 1);
         T* dl = rest + doff(l);
 #pragma unroll
         for (int k = 0; k < ((TILE >> l) + L + kNT - 1) / kNT; ++k) {
           const int i = tid + k * kNT;
           if (i < cnt) {
             T d = ev[l - 1][k];
-            if (t >= T(0)) d = thresh_coef(d, t, a.thr.hardness);
+            if (t >= T(0)) d = thresh_coef(d, t, thr.hardness);
             dl[i] = d;
           }
         }
@@ -469,7 +482,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
     const int elm = evn(1);
     const int npairs = ((TILE >> 1) + elm) / 2;
     const int off = evn(2) - elm / 2;
-    const T t = thr_level<T>(a.thr, j0 + 1);
+    const T t = thr_level<T>(thr, j0 + 1);
     E2 res[kPairs];
 #pragma unroll
     for (int k = 0; k < kPairs; ++k) {
@@ -481,7 +494,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
           const uint32_t sl = uint32_t(4 * (off + p - q)) + c2;
           sv[q] = pool[sl & pmask];
           const T d = pool[(sl + 2) & pmask];
-          dv[q] = (t >= T(0)) ? thresh_coef(d, t, a.thr.hardness) : d;
+          dv[q] = (t >= T(0)) ? thresh_coef(d, t, thr.hardness) : d;
         }
         T e, o;
         inv_pair<T, FILT>(sv, dv, e, o);
@@ -504,7 +517,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
   {
     const int npairs = TILE / 2;  // e_0 = 0
     const int off = evn(1);
-    const T t = thr_level<T>(a.thr, j0);
+    const T t = thr_level<T>(thr, j0);
     T* __restrict__ dst = static_cast<T*>(a.dst) + sig * a.bs_dst;
     E2 res[kPairs];
 #pragma unroll
@@ -516,7 +529,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
         for (int q = 0; q < L / 2; ++q) {
           const E2 v = *reinterpret_cast<const E2*>(pool + ((uint32_t(2 * (off + p - q)) + c1) & pmask));
           sv[q] = v.x;
-          dv[q] = (t >= T(0)) ? thresh_coef(v.y, t, a.thr.hardness) : v.y;
+          dv[q] = (t >= T(0)) ? thresh_coef(v.y, t, thr.hardness) : v.y;
         }
         T e, o;
         inv_pair<T, FILT>(sv, dv, e, o);
@@ -586,7 +599,9 @@ __global__ __launch_bounds__(kNTW) void dwt_inv_whole(WholeArgs a) {
   T* B = A + a.N;
   T* Cf = B + a.N / 2;  // the N coefficients of levels j0+1..J, thresholded
   const int tid = threadIdx.x;
-  const T* __restrict__ y = static_cast<const T*>(a.src) + int64_t(blockIdx.x) * a.bs_src;
+  Thr thr = a.thr;
+  const int64_t inp = thr_input(thr, int(blockIdx.x));
+  const T* __restrict__ y = static_cast<const T*>(a.src) + inp * a.bs_src;
   T* __restrict__ dst = static_cast<T*>(a.dst) + int64_t(blockIdx.x) * a.bs_dst;
   const int N = int(a.N);
   const int j0 = a.j0, J = a.J;
@@ -608,8 +623,8 @@ __global__ __launch_bounds__(kNTW) void dwt_inv_whole(WholeArgs a) {
       const int z = (q == 0) ? 31 : __builtin_ctz(unsigned(q));
       T d = ld[k];
       if (z < J - j0) {
-        const T t = thr_level<T>(a.thr, j0 + z);
-        if (t >= T(0)) d = thresh_coef(d, t, a.thr.hardness);
+        const T t = thr_level<T>(thr, j0 + z);
+        if (t >= T(0)) d = thresh_coef(d, t, thr.hardness);
       }
       Cf[q] = d;
     }
@@ -792,13 +807,15 @@ int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream
 
 template <typename T, int FILT>
 int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const wh_thresh* thr,
-              hipStream_t st) {
+              hipStream_t st, const Candidates& c) {
   auto ps = plan_passes<T>(n, J);
   const T* y = nullptr;
   T* comp = nullptr;
   int rc = dwt_scratch<T>(yin, x, n, count, ps, st, &y, &comp);
   if (rc) return rc;
-  const Thr th = thr_of(thr);
+  Thr th = thr_of(thr);
+  th.of = c.of;
+  th.th_stride = c.th_stride;
   const int64_t bc = n >> kGmax;
   const T* src = nullptr;  // compact s handed down between passes
   int slot = 0;
@@ -825,6 +842,7 @@ int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const w
       const bool top = (P.j0 + P.g == J);
       a.src = top ? static_cast<const void*>(y) : static_cast<const void*>(src);
       a.bs_src = top ? n : bc;
+      a.src_in = top;
       a.src_shift = top ? J : 0;
       a.y = const_cast<T*>(y);
       a.bs_y = n;
@@ -862,12 +880,12 @@ int dwt_fwd_t(const void* x, void* y, int64_t n, int64_t count, int J, int filt,
 
 template <typename T>
 int dwt_inv_t(const void* y, void* x, int64_t n, int64_t count, int J, int filt,
-              const wh_thresh* thr, hipStream_t st) {
+              const wh_thresh* thr, hipStream_t st, const Candidates& c) {
   switch (filt) {
-    case kHAAR: return dwt_inv_f<T, kHAAR>(y, x, n, count, J, thr, st);
-    case kD4: return dwt_inv_f<T, kD4>(y, x, n, count, J, thr, st);
-    case kC6: return dwt_inv_f<T, kC6>(y, x, n, count, J, thr, st);
-    default: return dwt_inv_f<T, kLA8>(y, x, n, count, J, thr, st);
+    case kHAAR: return dwt_inv_f<T, kHAAR>(y, x, n, count, J, thr, st, c);
+    case kD4: return dwt_inv_f<T, kD4>(y, x, n, count, J, thr, st, c);
+    case kC6: return dwt_inv_f<T, kC6>(y, x, n, count, J, thr, st, c);
+    default: return dwt_inv_f<T, kLA8>(y, x, n, count, J, thr, st, c);
   }
 }
 
@@ -880,9 +898,9 @@ int dwt_forward(const void* x, void* y, int64_t n, int64_t count, int J, int fil
 }
 
 int dwt_inverse(const void* y, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
-                const wh_thresh* thr, hipStream_t st) {
-  return dtype == WH_F32 ? dwt_inv_t<float>(y, x, n, count, J, filt, thr, st)
-                         : dwt_inv_t<double>(y, x, n, count, J, filt, thr, st);
+                const wh_thresh* thr, hipStream_t st, const Candidates& c) {
+  return dtype == WH_F32 ? dwt_inv_t<float>(y, x, n, count, J, filt, thr, st, c)
+                         : dwt_inv_t<double>(y, x, n, count, J, filt, thr, st, c);
 }
 
 }  // namespace wh

@@ -314,7 +314,8 @@ int modwt_fwd_t(const void* x, void* xmod, int64_t n, int64_t count, int J, int 
 
 template <typename T>
 int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt,
-                const wh_thresh* thr, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0) {
+                const wh_thresh* thr, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0,
+                const Candidates& c = Candidates{}) {
   const int L = filter_length(filt);
   auto groups = plan_groups(true, n, J, L, sizeof(T), knobs_for(true, n, J, filt, sizeof(T), count),
                             count);
@@ -347,6 +348,9 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
     T* dst = (G.j0 == 0) ? static_cast<T*>(x) : scratch + (gi & 1) * n * count;
     a.out = dst;
     a.bs_out = n;
+    a.of = c.of;
+    a.stop_of = c.of > 0 && gi + 1 == int(groups.size());
+    a.th_stride = c.th_stride;
     if (thr && thr->enabled) {
       a.th_on = 1;
       a.hardness = thr->hardness;
@@ -378,9 +382,9 @@ int modwt_forward_details(const void* x, void* xmod, int64_t n, int64_t count, i
 }
 
 int modwt_inverse(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
-                  const wh_thresh* thr, hipStream_t st) {
-  return dtype == WH_F32 ? modwt_inv_t<float>(xmod, x, n, count, J, filt, thr, st)
-                         : modwt_inv_t<double>(xmod, x, n, count, J, filt, thr, st);
+                  const wh_thresh* thr, hipStream_t st, const Candidates& c) {
+  return dtype == WH_F32 ? modwt_inv_t<float>(xmod, x, n, count, J, filt, thr, st, nullptr, 0, c)
+                         : modwt_inv_t<double>(xmod, x, n, count, J, filt, thr, st, nullptr, 0, c);
 }
 
 int modwt_inverse_ws(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt,

@@ -7,12 +7,12 @@
 // validation follows the reference's CPU algorithm (src/thresh.cpp:203-342)
 // step for step: the universal threshold of the full transform brackets a
 // golden-section search over the threshold of the even/odd half-length
-// transforms, each candidate costing one fused threshold+inverse launch over
+// transforms, each round costing one fused threshold+inverse launch over
 // both halves and one interpolation-error reduction.  The search's scalar
 // steps run on the device with the reference's arithmetic (cv_advance), so
-// candidates follow one another without the host; the host reads the
-// search state back only to learn how many more candidates the loop is
-// certain to evaluate.
+// rounds follow one another without the host; the host reads the search
+// state back only to learn how many more evaluations the loop is certain to
+// make.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -26,12 +26,22 @@ namespace wh {
 
 namespace {
 
+// Longest signals whose search evaluates kCvCandidates points a round: the
+// extra candidates run in workgroups the chip has to spare, and a round of
+// two steps costs 33 us of kernels at n = 2^18 (LA8 MODWT, J = 10) where
+// two rounds of one took 40 and four more launches; at n = 2^16 (D4 DWT) 18
+// against 29.  A round of three needs half again the memory traffic of two
+// steps, so where the halves fill the chip (3 n samples of MODWT beyond the
+// tiles' best range) one point a round stays.
+constexpr int64_t kCvRoundMaxModwt = int64_t(1) << 18;
+constexpr int64_t kCvRoundMaxDwt = int64_t(1) << 20;
+
 struct StatsBuf {
   SelState sel;
-  double partial[kMaxPartials];
+  double partial[kCvCandidates * kMaxPartials];
   double vals[16];
   double levels[64];
-  double cvlev[64];  // the candidate threshold of every level
+  double cvlev[kCvCandidates * kCvLevels];  // a candidate's threshold of every level
   CvState cv;
 };
 
@@ -52,9 +62,9 @@ int fwd(int ttype, const void* x, void* w, int64_t n, int64_t count, int J, int 
 }
 
 int inv(int ttype, const void* w, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
-        const wh_thresh* thr, hipStream_t st) {
-  return ttype == kDWT ? dwt_inverse(w, x, n, count, J, filt, dtype, thr, st)
-                       : modwt_inverse(w, x, n, count, J, filt, dtype, thr, st);
+        const wh_thresh* thr, hipStream_t st, const Candidates& c = Candidates{}) {
+  return ttype == kDWT ? dwt_inverse(w, x, n, count, J, filt, dtype, thr, st, c)
+                       : modwt_inverse(w, x, n, count, J, filt, dtype, thr, st, c);
 }
 
 // Candidates the search will certainly evaluate from state `cs` on (not
@@ -167,7 +177,10 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   const int Jh = J - 1;
   const int64_t cw = coeff_len(ttype, n, J), ch = coeff_len(ttype, lenh, Jh);
   void* ws = nullptr;
-  const size_t bytes = size_t(cw + 2 * ch + 4 * lenh) * esz + 256;
+  // Candidates per round: a round of three (the pending point and the one
+  // that follows it either way) takes two steps of the search.
+  const int cand = n <= (ttype == kDWT ? kCvRoundMaxDwt : kCvRoundMaxModwt) ? kCvCandidates : 1;
+  const size_t bytes = size_t(cw + 2 * ch + (2 + 2 * cand) * lenh) * esz + 256;
   if ((rc = ws_get(bytes, &ws))) return rc;
   char* p = static_cast<char*>(ws);
   void* W = p;
@@ -193,7 +206,7 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   // We, Wo and ye, yo are adjacent): twice the workgroups, half the launches
   if ((rc = fwd(ttype, xe, We, lenh, 2, Jh, filt, dtype, st))) return rc;
 
-  // one candidate: the halves thresholded at the point cv_advance last wrote
+  // one round: the halves thresholded at every candidate cv_points wrote
   wh_thresh th{};
   th.enabled = 1;
   th.hardness = hardness;
@@ -205,20 +218,26 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   cva.levels = sb->cvlev;
   cva.J = Jh;
   cva.tol = tol;
+  cva.cand = cand;
+  Candidates halves;
+  halves.of = 2;
+  halves.th_stride = kCvLevels;
   auto eval = [&]() -> int {
-    const int r = inv(ttype, We, ye, lenh, 2, Jh, filt, dtype, &th, st);
+    const int r = inv(ttype, We, ye, lenh, 2 * cand, Jh, filt, dtype, &th, st, halves);
     if (r) return r;
     // the error reduction's last block also advances the search
-    return interp_mse(x, ye, yo, n, dtype, sb->partial, &sb->vals[1], st, cva);
+    return interp_mse(x, ye, yo, n, dtype, sb->partial, nullptr, st, cva);
   };
+  // the tests the first bracket [0, t3] is sure to pass do not depend on t3
   CvState cs{};
-  for (int batch = 2;;) {  // t1 and t2 first
-    for (int i = 0; i < batch; ++i)
+  cs.t3 = 1.;
+  for (;;) {
+    const int sure = cv_sure_evals(cs, tol);
+    for (int i = 0; i < sure; i += cand == 1 ? 1 : 2)
       if ((rc = eval())) return rc;
     WH_HIP_CHECK(hipMemcpyAsync(&cs, &sb->cv, sizeof(CvState), hipMemcpyDeviceToHost, st));
     WH_HIP_CHECK(hipStreamSynchronize(st));
     if (cs.stop) break;
-    batch = cv_sure_evals(cs, tol);
   }
   const double t1 = cs.t1, t2 = cs.t2, m1 = cs.m1, m2 = cs.m2;
   double t = m1 < m2 ? t1 : t2;

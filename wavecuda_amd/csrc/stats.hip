@@ -72,10 +72,8 @@ int threshold_inplace(void* c, int64_t n, int64_t count, int J, int ttype, int d
 // The scalar steps of the reference's golden-section loop
 // (src/thresh.cpp:296-330), with products and sums rounded separately as
 // in its host build, so the visited thresholds are the same doubles.  One
-// thread: take the error m of the pending point, advance the bracket and
-// write the next point into levels[0..J).
-__device__ __noinline__ void cv_advance(CvState* cs, double m, double* levels, int J,
-                                        double tol) {
+// thread: take the error m of the pending point and advance the bracket.
+__device__ __noinline__ void cv_advance(CvState* cs, double m, double tol) {
 #pragma clang fp contract(off)
   if (cs->stop) return;
   const double R = 0.61803399, C = 1. - R;
@@ -84,33 +82,38 @@ __device__ __noinline__ void cv_advance(CvState* cs, double m, double* levels, i
   else
     cs->m2 = m;
   const int ne = ++cs->nevals;
-  double next;
   if (ne == 1) {  // the first two evaluations: t1, then t2
     cs->pending = 2;
-    next = cs->t2;
-  } else {
-    if (ne > 2) cs->iter++;  // the loop body that ordered this evaluation ends
-    if (!(fabs(cs->t3 - cs->t0) > tol * (cs->t1 + cs->t2)) || cs->iter > 50) {
-      cs->stop = 1;
-      return;
-    }
-    if (cs->m2 < cs->m1) {
-      cs->t0 = cs->t1;
-      cs->t1 = cs->t2;
-      cs->t2 = R * cs->t2 + C * cs->t3;
-      cs->m1 = cs->m2;
-      cs->pending = 2;
-      next = cs->t2;
-    } else {
-      cs->t3 = cs->t2;
-      cs->t2 = cs->t1;
-      cs->t1 = R * cs->t1 + C * cs->t0;
-      cs->m2 = cs->m1;
-      cs->pending = 1;
-      next = cs->t1;
-    }
+    return;
   }
-  for (int l = 0; l < J; ++l) levels[l] = next;
+  if (ne > 2) cs->iter++;  // the loop body that ordered this evaluation ends
+  if (!(fabs(cs->t3 - cs->t0) > tol * (cs->t1 + cs->t2)) || cs->iter > 50) {
+    cs->stop = 1;
+    return;
+  }
+  if (cs->m2 < cs->m1) {
+    cs->t0 = cs->t1;
+    cs->t1 = cs->t2;
+    cs->t2 = R * cs->t2 + C * cs->t3;
+    cs->m1 = cs->m2;
+    cs->pending = 2;
+  } else {
+    cs->t3 = cs->t2;
+    cs->t2 = cs->t1;
+    cs->t1 = R * cs->t1 + C * cs->t0;
+    cs->m2 = cs->m1;
+    cs->pending = 1;
+  }
+}
+
+// A round's errors m[0..cand): of the pending point, and with three
+// candidates of the point that follows it either way (cv_points), so the
+// search takes two steps.
+__device__ void cv_round(CvState* cs, const double* m, double* levels, int J, int cand,
+                         double tol) {
+  cv_advance(cs, m[0], tol);
+  if (cand == kCvCandidates && !cs->stop) cv_advance(cs, m[cs->pending == 2 ? 1 : 2], tol);
+  if (!cs->stop) cv_points(cs, levels, J);
 }
 
 // --------------------------------------------------------- interp_mse
@@ -121,6 +124,9 @@ __global__ __launch_bounds__(256) void interp_mse_partial(const T* __restrict__ 
                                                           int64_t per_block, double* partial) {
   __shared__ double red[256];
   const int64_t lenh = len / 2;
+  ye += int64_t(blockIdx.y) * len;  // a candidate's halves are adjacent
+  yo += int64_t(blockIdx.y) * len;
+  partial += int64_t(blockIdx.y) * kMaxPartials;
   const int64_t j0 = int64_t(blockIdx.x) * per_block;
   const int64_t j1 = std::min(lenh, j0 + per_block);
   double acc = 0.0;
@@ -149,21 +155,30 @@ __global__ __launch_bounds__(256) void interp_mse_partial(const T* __restrict__ 
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-__global__ __launch_bounds__(256) void sum_partials(const double* partial, int np, double scale,
-                                                    double* out, CvArgs cv) {
-  __shared__ double red[256];
+// 256 threads per candidate
+__global__ __launch_bounds__(256 * kCvCandidates) void sum_partials(const double* partial, int np,
+                                                                   double scale, double* out,
+                                                                   CvArgs cv) {
+  __shared__ double sums[kCvCandidates][256];
+  const int c = threadIdx.x >> 8, t = threadIdx.x & 255;
+  double* red = sums[c];
   double acc = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) acc += partial[i];
-  red[threadIdx.x] = acc;
+  for (int i = t; i < np; i += 256) acc += partial[c * kMaxPartials + i];
+  red[t] = acc;
   __syncthreads();
   for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+    if (t < off) red[t] += red[t + off];
     __syncthreads();
   }
+  if (t == 0) red[0] *= scale;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double v = red[0] * scale;
-    *out = v;
-    if (cv.cs) cv_advance(cv.cs, v, cv.levels, cv.J, cv.tol);
+    if (out) *out = sums[0][0];
+    if (cv.cs) {
+      double m[kCvCandidates];
+      for (int i = 0; i < cv.cand; ++i) m[i] = sums[i][0];
+      cv_round(cv.cs, m, cv.levels, cv.J, cv.cand, cv.tol);
+    }
   }
 }
 
@@ -173,15 +188,17 @@ int interp_mse(const void* xn, const void* ye, const void* yo, int64_t len, int 
   const int64_t per_block = 512;
   const int np = int(std::min<int64_t>((lenh + per_block - 1) / per_block, kMaxPartials));
   const int64_t pb = (lenh + np - 1) / np;
+  const dim3 grid{unsigned(np), unsigned(cv.cand)};
   if (dtype == WH_F32)
-    hipLaunchKernelGGL(interp_mse_partial<float>, dim3(np), dim3(256), 0, st,
+    hipLaunchKernelGGL(interp_mse_partial<float>, grid, dim3(256), 0, st,
                        static_cast<const float*>(xn), static_cast<const float*>(ye),
                        static_cast<const float*>(yo), len, pb, partial_buf);
   else
-    hipLaunchKernelGGL(interp_mse_partial<double>, dim3(np), dim3(256), 0, st,
+    hipLaunchKernelGGL(interp_mse_partial<double>, grid, dim3(256), 0, st,
                        static_cast<const double*>(xn), static_cast<const double*>(ye),
                        static_cast<const double*>(yo), len, pb, partial_buf);
-  hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, partial_buf, np, 0.5, out, cv);
+  hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256 * cv.cand), 0, st, partial_buf, np, 0.5, out,
+                     cv);
   WH_HIP_CHECK(hipGetLastError());
   return WH_OK;
 }

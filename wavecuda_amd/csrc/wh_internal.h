@@ -57,6 +57,14 @@ int noalloc_setup();
 // so it cannot surface in a later, unrelated call.
 void allow_dynamic_lds(const void* kern);
 
+// An inverse's `count` signals as count / of candidates of the same `of`
+// inputs (of > 0): signal y inverts input y % of with the per-level
+// thresholds levels + (y / of) th_stride.
+struct Candidates {
+  int of = 0;
+  int64_t th_stride = 0;
+};
+
 // transform back ends (device pointers)
 // MODWT of `count` signals of n samples (x, out: n apart; xmod: 2nJ apart)
 int modwt_forward(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
@@ -66,7 +74,7 @@ int modwt_forward(const void* x, void* xmod, int64_t n, int64_t count, int J, in
 int modwt_forward_details(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
                           int dtype, hipStream_t st);
 int modwt_inverse(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
-                  const wh_thresh* thr, hipStream_t st);
+                  const wh_thresh* thr, hipStream_t st, const Candidates& c = Candidates{});
 // the same with the level hand-off in the caller's device workspace ws of
 // ws_bytes (2 n count elements needed when the plan has several groups)
 int modwt_inverse_ws(const void* xmod, void* x, int64_t n, int64_t count, int J, int filt,
@@ -109,7 +117,7 @@ int modwt_order(const void* in, void* out, int64_t n, int J, bool to_po, int dty
 int dwt_forward(const void* x, void* y, int64_t n, int64_t count, int J, int filt, int dtype,
                 hipStream_t st);
 int dwt_inverse(const void* y, void* x, int64_t n, int64_t count, int J, int filt, int dtype,
-                const wh_thresh* thr, hipStream_t st);
+                const wh_thresh* thr, hipStream_t st, const Candidates& c = Candidates{});
 
 int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int threshtype,
            double* thresh, int hardness, int minlevel, int maxlevel, double tol,

@@ -49,18 +49,35 @@ struct SelState {
   uint64_t cand[2][kSelCandCap];
 };
 
-constexpr int kMaxPartials = 1024;
+constexpr int kMaxPartials = 1024;  // per candidate
 
 // Golden-section search of the cross-validated threshold, kept on the device
 // (reference src/thresh.cpp:296-330): the bracket t0 <= t1 <= t2 <= t3, the
 // errors m1, m2 at t1, t2, the loop count, which point the pending
 // evaluation is for (1: t1, 2: t2), evaluations consumed so far, and stop.
+constexpr int kCvCandidates = 3;  // points a round evaluates at once, at most
+constexpr int kCvLevels = 64;     // distance of the candidates' threshold arrays
 struct CvState {
   double t0, t1, t2, t3, m1, m2;
   int iter, pending, nevals, stop;
 };
 
-// bracket [0, t3] and the first point t1 into levels[0..J) (one thread)
+// The points of the next round into levels[c kCvLevels + 0..J): the pending
+// one, then the one the search visits after it -- t2 after the first t1;
+// else one for each outcome of the comparison, right (m2 < m1) and left.
+__device__ inline void cv_points(const CvState* cs, double* levels, int J) {
+#pragma clang fp contract(off)
+  const double R = 0.61803399, C = 1. - R;
+  double p[kCvCandidates] = {cs->pending == 2 ? cs->t2 : cs->t1, cs->t2, cs->t2};
+  if (cs->nevals > 0) {
+    p[1] = R * cs->t2 + C * cs->t3;
+    p[2] = R * cs->t1 + C * cs->t0;
+  }
+  for (int c = 0; c < kCvCandidates; ++c)
+    for (int l = 0; l < J; ++l) levels[c * kCvLevels + l] = p[c];
+}
+
+// bracket [0, t3] and the first round's points (one thread)
 __device__ inline void cv_start(CvState* cs, double t3, double* levels, int J) {
 #pragma clang fp contract(off)
   const double C = 1. - 0.61803399;
@@ -74,7 +91,7 @@ __device__ inline void cv_start(CvState* cs, double t3, double* levels, int J) {
   cs->pending = 1;
   cs->nevals = 0;
   cs->stop = 0;
-  for (int l = 0; l < J; ++l) levels[l] = cs->t1;
+  cv_points(cs, levels, J);
 }
 
 // in-place threshold of `count` transformed signals (DWT: n apart, MODWT:
@@ -105,7 +122,9 @@ struct CvArgs {
   double* levels = nullptr;
   int J = 0;
   double tol = 0.0;
+  int cand = 1;  // candidates (ye, yo: halves of candidate c at c len; 1 or kCvCandidates)
 };
+// partial_buf: kMaxPartials per candidate
 int interp_mse(const void* xn, const void* ye, const void* yo, int64_t len, int dtype,
                double* partial_buf, double* out, hipStream_t st, const CvArgs& cv = CvArgs{});
 int split_halves(const void* x, void* e, void* o, int64_t len, int dtype, hipStream_t st);
