@@ -71,9 +71,9 @@ int threshold_inplace(void* c, int64_t n, int64_t count, int J, int ttype, int d
 // ------------------------------------------------- cross-validation search
 // The scalar steps of the reference's golden-section loop
 // (src/thresh.cpp:296-330), with products and sums rounded separately as
-// in its host build, so the visited thresholds are the same doubles.  One
-// thread: take the error m of the pending point and advance the bracket.
-__device__ __noinline__ void cv_advance(CvState* cs, double m, double tol) {
+// in its host build, so the visited thresholds are the same doubles: take
+// the error m of the pending point and advance the bracket.
+__device__ __forceinline__ void cv_advance(CvState* cs, double m, double tol) {
 #pragma clang fp contract(off)
   if (cs->stop) return;
   const double R = 0.61803399, C = 1. - R;
@@ -104,16 +104,6 @@ __device__ __noinline__ void cv_advance(CvState* cs, double m, double tol) {
     cs->m2 = cs->m1;
     cs->pending = 1;
   }
-}
-
-// A round's errors m[0..cand): of the pending point, and with three
-// candidates of the point that follows it either way (cv_points), so the
-// search takes two steps.
-__device__ void cv_round(CvState* cs, const double* m, double* levels, int J, int cand,
-                         double tol) {
-  cv_advance(cs, m[0], tol);
-  if (cand == kCvCandidates && !cs->stop) cv_advance(cs, m[cs->pending == 2 ? 1 : 2], tol);
-  if (!cs->stop) cv_points(cs, levels, J);
 }
 
 // --------------------------------------------------------- interp_mse
@@ -155,13 +145,21 @@ __global__ __launch_bounds__(256) void interp_mse_partial(const T* __restrict__ 
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// 256 threads per candidate
+// The sums of every candidate's partials (256 threads each), then the
+// search's steps: the first candidate is the pending point, and with three
+// the others follow it either way (cv_points), so the search takes two.  The
+// state is fetched beside the partials and stepped in registers by one
+// thread; the points go out in parallel (4.8 -> 3.1 us against stepping it
+// in memory).
 __global__ __launch_bounds__(256 * kCvCandidates) void sum_partials(const double* partial, int np,
                                                                    double scale, double* out,
                                                                    CvArgs cv) {
   __shared__ double sums[kCvCandidates][256];
+  __shared__ double pts[kCvCandidates];
   const int c = threadIdx.x >> 8, t = threadIdx.x & 255;
   double* red = sums[c];
+  CvState cs{};
+  if (threadIdx.x == 0 && cv.cs) cs = *cv.cs;
   double acc = 0.0;
   for (int i = t; i < np; i += 256) acc += partial[c * kMaxPartials + i];
   red[t] = acc;
@@ -170,16 +168,20 @@ __global__ __launch_bounds__(256 * kCvCandidates) void sum_partials(const double
     if (t < off) red[t] += red[t + off];
     __syncthreads();
   }
-  if (t == 0) red[0] *= scale;
-  __syncthreads();
   if (threadIdx.x == 0) {
-    if (out) *out = sums[0][0];
+    if (out) *out = red[0] * scale;
     if (cv.cs) {
-      double m[kCvCandidates];
-      for (int i = 0; i < cv.cand; ++i) m[i] = sums[i][0];
-      cv_round(cv.cs, m, cv.levels, cv.J, cv.cand, cv.tol);
+      cv_advance(&cs, red[0] * scale, cv.tol);
+      if (cv.cand == kCvCandidates && !cs.stop)
+        cv_advance(&cs, sums[cs.pending == 2 ? 1 : 2][0] * scale, cv.tol);
+      *cv.cs = cs;
+      cv_points(cs, pts);
     }
   }
+  if (!cv.cs) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < cv.J * kCvCandidates; i += blockDim.x)
+    cv.levels[(i / cv.J) * kCvLevels + i % cv.J] = pts[i / cv.J];
 }
 
 int interp_mse(const void* xn, const void* ye, const void* yo, int64_t len, int dtype,

@@ -62,36 +62,33 @@ struct CvState {
   int iter, pending, nevals, stop;
 };
 
-// The points of the next round into levels[c kCvLevels + 0..J): the pending
-// one, then the one the search visits after it -- t2 after the first t1;
-// else one for each outcome of the comparison, right (m2 < m1) and left.
-__device__ inline void cv_points(const CvState* cs, double* levels, int J) {
+// The points of the next round: the pending one, then the one the search
+// visits after it -- t2 after the first t1; else one for each outcome of
+// the comparison, right (m2 < m1) and left.
+__device__ __forceinline__ void cv_points(const CvState& cs, double* p) {
 #pragma clang fp contract(off)
   const double R = 0.61803399, C = 1. - R;
-  double p[kCvCandidates] = {cs->pending == 2 ? cs->t2 : cs->t1, cs->t2, cs->t2};
-  if (cs->nevals > 0) {
-    p[1] = R * cs->t2 + C * cs->t3;
-    p[2] = R * cs->t1 + C * cs->t0;
-  }
-  for (int c = 0; c < kCvCandidates; ++c)
-    for (int l = 0; l < J; ++l) levels[c * kCvLevels + l] = p[c];
+  p[0] = cs.pending == 2 ? cs.t2 : cs.t1;
+  p[1] = cs.nevals > 0 ? R * cs.t2 + C * cs.t3 : cs.t2;
+  p[2] = cs.nevals > 0 ? R * cs.t1 + C * cs.t0 : cs.t2;
 }
 
 // bracket [0, t3] and the first round's points (one thread)
-__device__ inline void cv_start(CvState* cs, double t3, double* levels, int J) {
+__device__ inline void cv_start(CvState* out, double t3, double* levels, int J) {
 #pragma clang fp contract(off)
   const double C = 1. - 0.61803399;
   const double tb = t3 / 2.;
-  cs->t0 = 0.;
-  cs->t2 = tb;
-  cs->t1 = tb - C * (tb - 0.);
-  cs->t3 = t3;
-  cs->m1 = cs->m2 = 0.;
-  cs->iter = 0;
-  cs->pending = 1;
-  cs->nevals = 0;
-  cs->stop = 0;
-  cv_points(cs, levels, J);
+  CvState cs{};
+  cs.t2 = tb;
+  cs.t1 = tb - C * (tb - 0.);
+  cs.t3 = t3;
+  cs.pending = 1;
+  *out = cs;
+  double p[kCvCandidates];
+  cv_points(cs, p);
+#pragma unroll
+  for (int c = 0; c < kCvCandidates; ++c)
+    for (int l = 0; l < J; ++l) levels[c * kCvLevels + l] = p[c];
 }
 
 // in-place threshold of `count` transformed signals (DWT: n apart, MODWT:
