@@ -294,6 +294,26 @@ int wh_dwt_fwd_adj(const void* gy, void* gx, int64_t n, int nlevels, int filter,
                    void* stream);
 int wh_dwt_inv_adj(const void* gx, void* gy, int64_t n, int nlevels, int filter, int dtype,
                    void* stream);
+/* For pipelines that only read the details and S_J (smoothing layers):
+   wh_modwt_fwd_details is wh_modwt_fwd_many without the S_j slots, j < J
+   (their contents are undefined); wh_modwt_fwd_details_adj its adjoint, which
+   does not read them.  wh_modwt_thresh_inv_adj is the adjoint of
+   wh_modwt_inv_many with the threshold `thr` at the coefficients xmod:
+   gy (cotangent of the output) -> gxmod (cotangent of xmod, zero in the S_j
+   slots, j < J -- with details_only left as they are) and glam (DEVICE, dL/dt
+   of every level summed over signals, as wh_thresh_grad); either may be
+   NULL. */
+int wh_modwt_fwd_details(const void* x, void* xmod, int64_t n, int64_t count, int nlevels,
+                         int filter, int dtype, void* stream);
+int wh_modwt_fwd_details_adj(const void* gxmod, void* gx, int64_t n, int64_t count, int nlevels,
+                             int filter, int dtype, void* stream);
+int wh_modwt_thresh_inv_adj(const void* gy, const void* xmod, void* gxmod, int details_only,
+                            double* glam, int64_t n, int64_t count, int nlevels, int filter,
+                            int dtype, const wh_thresh* thr, void* stream);
+/* mean((y - ref)^2) of `total` values to the DEVICE double *out and its
+   gradient in y, 2 (y - ref) / total, to g (g may be y). */
+int wh_mse_grad(const void* y, const void* ref, void* g, int64_t total, int dtype, double* out,
+                void* stream);
 /* wh_threshold over `count` transformed signals (DWT n apart, MODWT 2nJ
    apart).  reference src/thresh.cpp:15-83, :142-157. */
 int wh_threshold_many(void* coeffs, int64_t n, int64_t count, int nlevels, int ttype, int filter,

@@ -84,6 +84,11 @@ SIGNATURES = {
     "wh_modwt_inv_adj": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
     "wh_dwt_fwd_adj": (_I, [_VP, _VP, _I64, _I, _I, _I, _VP]),
     "wh_dwt_inv_adj": (_I, [_VP, _VP, _I64, _I, _I, _I, _VP]),
+    "wh_modwt_fwd_details": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
+    "wh_modwt_fwd_details_adj": (_I, [_VP, _VP, _I64, _I64, _I, _I, _I, _VP]),
+    "wh_modwt_thresh_inv_adj": (_I, [_VP, _VP, _VP, _I, _VP, _I64, _I64, _I, _I, _I,
+                                     C.POINTER(wh_thresh), _VP]),
+    "wh_mse_grad": (_I, [_VP, _VP, _VP, _I64, _I, _VP, _VP]),
     "wh_threshold_many": (_I, [_VP, _I64, _I64, _I, _I, _I, _I, C.POINTER(wh_thresh), _VP]),
     "wh_thresh_grad": (_I, [_VP, _VP, _VP, _VP, _I64, _I64, _I, _I, _I, _I,
                             C.POINTER(wh_thresh), _VP]),

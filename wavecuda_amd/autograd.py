@@ -7,6 +7,8 @@ Every backward is a hand-written adjoint kernel of libwavehip:
   dwt(x), idwt(y)     DWT / inverse        backward: the orthogonal transpose
                       (wh_dwt_fwd_many / wh_dwt_inv_many, all rows at once)
   threshold(c, lam)   per-level hard/soft  backward: wh_thresh_grad (c and lam)
+  smooth_levels(x, lam)  MODWT, threshold, inverse  backward:
+                      wh_modwt_thresh_inv_adj, wh_modwt_fwd_details_adj
 
 x may be one signal (n,) or a batch (B, n) of equal-length signals; the
 MODWT coefficients of a batch are (B, 2 n J) in the reference's
@@ -210,6 +212,57 @@ class ThresholdInverseFn(torch.autograd.Function):
                 None)
 
 
+class SmoothLevelsFn(torch.autograd.Function):
+    """MODWT -> per-level threshold -> inverse as one function: the
+    coefficients in between need their details and S_J only, so the forward
+    leaves the other S_j slots unwritten (undefined in the saved tensor) and
+    neither adjoint touches them, and one kernel is the inverse's adjoint and
+    the threshold's gradient.  The same output and signal gradient as ModwtFn
+    followed by ThresholdInverseFn; the thresholds' sums in another order."""
+
+    @staticmethod
+    def forward(ctx, x, lam, J, filt, hardness):
+        x2, squeeze = _rows(x.contiguous())
+        B, n = x2.shape
+        w = torch.empty(B, 2 * n * J, dtype=x.dtype, device=x.device)
+        W.check(W.lib().wh_modwt_fwd_details(_vp(x2), _vp(w), n, B, J, filt, _dtype(x), _stream()),
+                "wh_modwt_fwd_details")
+        lam64 = lam.detach().to(device=x.device, dtype=torch.float64).contiguous()
+        if lam64.numel() != J:
+            raise W.WaveHipError("one threshold per level expected")
+        thr = W.make_thresh(True, hardness, 0, J - 1, 0.0, lam64.data_ptr())
+        y = torch.empty(B, n, dtype=x.dtype, device=x.device)
+        W.check(W.lib().wh_modwt_inv_many(_vp(w), _vp(y), n, B, J, filt, _dtype(x), C.byref(thr),
+                                          _stream()), "wh_modwt_inv_many")
+        ctx.save_for_backward(w, lam64)
+        ctx.meta = (n, J, filt, hardness, squeeze, lam.dtype)
+        return y[0] if squeeze else y
+
+    @staticmethod
+    def backward(ctx, g):
+        w, lam64 = ctx.saved_tensors
+        n, J, filt, hardness, squeeze, lam_dtype = ctx.meta
+        want_x, want_lam = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        if not (want_x or want_lam):
+            return None, None, None, None, None
+        B = w.shape[0]
+        g2 = g.contiguous().view(B, n)
+        gw = torch.empty_like(w) if want_x else None
+        glam = torch.empty(J, dtype=torch.float64, device=w.device) if want_lam else None
+        thr = W.make_thresh(True, hardness, 0, J - 1, 0.0, lam64.data_ptr())
+        W.check(W.lib().wh_modwt_thresh_inv_adj(
+            _vp(g2), _vp(w), None if gw is None else _vp(gw), 1,
+            None if glam is None else _vp(glam), n, B, J, filt, _dtype(g2), C.byref(thr),
+            _stream()), "wh_modwt_thresh_inv_adj")
+        gx = None
+        if want_x:
+            gx = torch.empty(B, n, dtype=w.dtype, device=w.device)
+            W.check(W.lib().wh_modwt_fwd_details_adj(_vp(gw), _vp(gx), n, B, J, filt, _dtype(w),
+                                                     _stream()), "wh_modwt_fwd_details_adj")
+            gx = gx[0] if squeeze else gx
+        return gx, None if glam is None else glam.to(lam_dtype), None, None, None
+
+
 def modwt(x, nlevels, filter="LA8"):
     f = filter_code(filter)
     n = x.shape[-1]
@@ -251,8 +304,7 @@ def smooth_levels(x, lam, nlevels, filter="LA8", ttype=W.MODWT, hardness=W.SOFT)
     n = x.shape[-1]
     J = resolve_levels(n, nlevels, f)
     if ttype == W.MODWT:
-        w = ModwtFn.apply(x, J, f)
-        return ThresholdInverseFn.apply(w, lam, n, J, f, hardness, 0, J - 1)
+        return SmoothLevelsFn.apply(x, lam, J, f, hardness)
     y = DwtFn.apply(x, J, f)
     return IdwtFn.apply(ThresholdFn.apply(y, lam, n, J, W.DWT, f, hardness, 0, J - 1), J, f)
 
@@ -275,26 +327,54 @@ def fit_level_thresholds(x, clean, nlevels, filter="LA8", lam0=None, steps=300, 
         w0 = D.modwt_fwd(x0.contiguous(), J, f) if ttype == W.MODWT else D.dwt_fwd(x0, J, f)
         t = D.univ_thresh(w0, n, J, ttype, f, 0, 0).item()
         lam0 = torch.full((J,), t, dtype=torch.float64)
-    lam = lam0.detach().to(device=x.device, dtype=torch.float64).clone().requires_grad_(True)
+    lam = lam0.detach().to(device=x.device, dtype=torch.float64).clone().contiguous()
+    lam.requires_grad_(True)
     opt = torch.optim.Adam([lam], lr=lr)
     xd = x.detach()
-    if ttype == W.MODWT:
-        # the signals do not change: transform them once, and let each step
-        # run the thresholding inverse and its adjoint only
-        w = ModwtFn.apply(xd, J, f)
+    if (ttype == W.MODWT and clean.shape == x.shape and clean.dtype == x.dtype
+            and clean.device == x.device and not clean.requires_grad and lam.numel() == J):
+        losses = _fit_modwt(xd, clean, lam, opt, J, f, steps)
+    else:  # shapes and types that torch broadcasts and promotes
+        losses = []  # kept on the device: no host round trip per step
+        for _ in range(steps):
+            opt.zero_grad(set_to_none=True)
+            loss = torch.mean((smooth_levels(xd, lam, J, f, ttype) - clean) ** 2)
+            loss.backward()
+            opt.step()
+            losses.append(loss.detach())
+        with torch.no_grad():
+            losses.append(torch.mean((smooth_levels(xd, lam, J, f, ttype) - clean) ** 2))
+        losses = torch.stack(losses)
+    return lam.detach(), losses.double().cpu().tolist()
 
-        def smooth(lv):
-            return ThresholdInverseFn.apply(w, lv, n, J, f, W.SOFT, 0, J - 1)
-    else:
-        def smooth(lv):
-            return smooth_levels(xd, lv, J, f, ttype)
-    losses = []  # kept on the device: no host round trip per step
-    for _ in range(steps):
-        opt.zero_grad(set_to_none=True)
-        loss = torch.mean((smooth(lam) - clean) ** 2)
-        loss.backward()
+
+def _fit_modwt(x, clean, lam, opt, J, filt, steps):
+    """The Adam steps of fit_level_thresholds for the MODWT.  The signals do
+    not change, so they are transformed once; a step is the thresholding
+    inverse, the error with its gradient in one pass, and the inverse's
+    adjoint, which sums the thresholds' gradients as it reads the
+    coefficients and writes no cotangent of them.  Returns the losses (device
+    tensor, in x's type as torch.mean would give them)."""
+    x2, _ = _rows(x.contiguous())
+    B, n = x2.shape
+    ref = clean.contiguous()
+    w = torch.empty(B, 2 * n * J, dtype=x.dtype, device=x.device)
+    y = torch.empty(B, n, dtype=x.dtype, device=x.device)
+    steps = max(steps, 0)
+    losses = torch.empty(steps + 1, dtype=torch.float64, device=x.device)
+    dt, L = _dtype(x), W.lib()
+    W.check(L.wh_modwt_fwd_details(_vp(x2), _vp(w), n, B, J, filt, dt, _stream()),
+            "wh_modwt_fwd_details")
+    lam.grad = torch.empty_like(lam)
+    thr = W.make_thresh(True, W.SOFT, 0, J - 1, 0.0, lam.data_ptr())
+    for i in range(steps + 1):
+        W.check(L.wh_modwt_inv_many(_vp(w), _vp(y), n, B, J, filt, dt, C.byref(thr), _stream()),
+                "wh_modwt_inv_many")
+        W.check(L.wh_mse_grad(_vp(y), _vp(ref), _vp(y), B * n, dt,
+                              C.c_void_p(losses.data_ptr() + 8 * i), _stream()), "wh_mse_grad")
+        if i == steps:
+            break
+        W.check(L.wh_modwt_thresh_inv_adj(_vp(y), _vp(w), None, 1, _vp(lam.grad), n, B, J, filt,
+                                          dt, C.byref(thr), _stream()), "wh_modwt_thresh_inv_adj")
         opt.step()
-        losses.append(loss.detach())
-    with torch.no_grad():
-        losses.append(torch.mean((smooth(lam) - clean) ** 2))
-    return lam.detach(), torch.stack(losses).double().cpu().tolist()
+    return losses.to(x.dtype)

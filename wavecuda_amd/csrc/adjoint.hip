@@ -1,16 +1,14 @@
-// adjoint.hip -- adjoints for differentiating through the transforms and
-// the soft threshold (gfx950).
+// adjoint.hip -- gradients of the soft threshold and of the mean squared
+// error (gfx950).  The transforms' adjoints: MODWT in modwt_tile.h and
+// modwt.hip; the DWT is orthogonal, so its forward and inverse are each
+// other's.
 //
 // MODWT forward F: x -> (S_1, D_1, ..., S_J, D_J) with
 //   S_j = H_j S_{j-1},  D_j = G_j S_{j-1},  (H_j u)[i] = sum_k C_k u[(i + k s) mod n]
 // (reference src/daub4.cpp:561-571, s = 2^{j-1}).  Its adjoint takes the
 // cotangents (Sb_j, Db_j) of every output back to x:
 //   u_J = Sb_J,  u_{j-1} = Sb_{j-1} + H_j^T u_j + G_j^T Db_j,  xb = u_0
-// with (H_j^T u)[p] = sum_k C_k u[(p - k s) mod n].  One kernel per level
-// reads u_j, Db_j and Sb_{j-1} and writes u_{j-1}; each of its L taps is a
-// shifted contiguous read, so the accesses are coalesced.  (The adjoint of
-// the inverse is the fused forward with exact 2^-j scalings, modwt.hip; the
-// DWT is orthogonal, so its forward and inverse are each other's adjoints.)
+// with (H_j^T u)[p] = sum_k C_k u[(p - k s) mod n].
 //
 // Soft threshold y = sign(c) max(|c| - t, 0) on the details of levels
 // [minlevel, maxlevel] (reference src/thresh.cpp:142-157): dy/dc = 1[|c| > t],
@@ -27,76 +25,6 @@
 namespace wh {
 
 namespace {
-
-template <typename T, int FILT>
-__global__ __launch_bounds__(256) void modwt_fwd_adj_level_k(const T* __restrict__ u0,
-                                                             int64_t bs_u,
-                                                             const T* __restrict__ gxm0,
-                                                             int64_t per, int j, T* __restrict__ out0,
-                                                             int64_t n) {
-  constexpr int L = Filter<FILT>::L;
-  const int64_t sig = blockIdx.y;
-  const T* __restrict__ u = u0 + sig * bs_u;
-  const T* __restrict__ db = gxm0 + sig * per + 2 * n * int64_t(j - 1) + n;
-  const T* __restrict__ sb = (j >= 2) ? gxm0 + sig * per + 2 * n * int64_t(j - 2) : nullptr;
-  T* __restrict__ out = out0 + sig * n;
-  const int64_t s = int64_t(1) << (j - 1);
-  const int64_t mask = n - 1;
-  for (int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; p < n;
-       p += int64_t(gridDim.x) * blockDim.x) {
-    T acc = sb ? sb[p] : T(0);
-#pragma unroll
-    for (int k = 0; k < L; ++k) {
-      const int64_t q = (p - k * s) & mask;
-      acc = fma(u[q], T(Filter<FILT>::c(k)), acc);
-      acc = fma(db[q], T(gcoef<FILT>(k)), acc);
-    }
-    out[p] = acc;
-  }
-}
-
-template <typename T>
-int fwd_adj_t(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
-              hipStream_t st) {
-  const int64_t per = 2 * n * J;
-  T* scratch = nullptr;
-  if (J > 1) {
-    void* p = nullptr;
-    int rc = scratch_get(2 * size_t(n) * size_t(count) * sizeof(T), &p);
-    if (rc) return rc;
-    scratch = static_cast<T*>(p);
-  }
-  const T* gxm = static_cast<const T*>(gxmod);
-  const T* u = gxm + 2 * n * int64_t(J - 1);  // u_J = Sb_J
-  int64_t bs_u = per;
-  const unsigned blocks = unsigned(std::min<int64_t>((n + 255) / 256, 2048));
-  const dim3 grid(blocks, unsigned(count));
-  for (int j = J; j >= 1; --j) {
-    T* dst = (j == 1) ? static_cast<T*>(gx) : scratch + int64_t(j & 1) * n * count;
-    switch (filt) {
-      case kHAAR:
-        hipLaunchKernelGGL((modwt_fwd_adj_level_k<T, kHAAR>), grid, dim3(256), 0, st, u, bs_u,
-                           gxm, per, j, dst, n);
-        break;
-      case kD4:
-        hipLaunchKernelGGL((modwt_fwd_adj_level_k<T, kD4>), grid, dim3(256), 0, st, u, bs_u, gxm,
-                           per, j, dst, n);
-        break;
-      case kC6:
-        hipLaunchKernelGGL((modwt_fwd_adj_level_k<T, kC6>), grid, dim3(256), 0, st, u, bs_u, gxm,
-                           per, j, dst, n);
-        break;
-      default:
-        hipLaunchKernelGGL((modwt_fwd_adj_level_k<T, kLA8>), grid, dim3(256), 0, st, u, bs_u,
-                           gxm, per, j, dst, n);
-        break;
-    }
-    WH_HIP_CHECK(hipGetLastError());
-    u = dst;
-    bs_u = n;
-  }
-  return WH_OK;
-}
 
 constexpr int kGradNT = 256;
 constexpr int kGradMinPer = 4096;         // elements per workgroup, at least
@@ -199,13 +127,6 @@ __global__ __launch_bounds__(kGradNT) void thresh_grad_reduce_k(const double* __
 
 }  // namespace
 
-int modwt_forward_adjoint(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
-                          int dtype, hipStream_t st) {
-  if (count < 1 || count > 65535) return set_error(WH_ERR_ARG, "adjoint: signal count out of range");
-  return dtype == WH_F32 ? fwd_adj_t<float>(gxmod, gx, n, count, J, filt, st)
-                         : fwd_adj_t<double>(gxmod, gx, n, count, J, filt, st);
-}
-
 int thresh_grad(const void* c, const void* gy, void* gc, double* glam, int64_t n, int64_t count,
                 int J, int ttype, int dtype, const wh_thresh* thr, hipStream_t st) {
   if (count < 1 || count > 65535) return set_error(WH_ERR_ARG, "threshold gradient: signal count out of range");
@@ -243,6 +164,68 @@ int thresh_grad(const void* c, const void* gy, void* gc, double* glam, int64_t n
                        glam, count, int(nchunk), thr->minlevel, thr->maxlevel);
     WH_HIP_CHECK(hipGetLastError());
   }
+  return WH_OK;
+}
+
+// ------------------------------------------------- mean squared error
+namespace {
+
+constexpr int kMsePer = 8;  // elements per thread, at least
+
+// g = 2 (y - ref) / total (the order of operations of torch's mean of a
+// square), and the workgroup's sum of (y - ref)^2 in 64 bits.  One read of
+// each array and one write: bound by HBM.
+template <typename T>
+__global__ __launch_bounds__(256) void mse_k(const T* y, const T* __restrict__ ref, T* g,
+                                             int64_t total, double* __restrict__ partial) {
+  const T inv = T(1) / T(total);
+  double acc = 0.0;
+  const int64_t stride = int64_t(gridDim.x) * 256;
+  for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < total; i += stride) {
+    const T d = y[i] - ref[i];
+    acc += double(d) * double(d);
+    g[i] = inv * (T(2) * d);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  __shared__ double red[4];
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+__global__ __launch_bounds__(256) void mse_sum_k(const double* __restrict__ partial, int np,
+                                                 int64_t total, double* out) {
+  __shared__ double red[256];
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < np; i += 256) acc += partial[i];
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = red[0] / double(total);
+}
+
+}  // namespace
+
+int mse_grad(const void* y, const void* ref, void* g, int64_t total, int dtype, double* out,
+             hipStream_t st) {
+  const unsigned np =
+      unsigned(std::max<int64_t>(1, std::min<int64_t>((total + 256 * kMsePer - 1) / (256 * kMsePer), 2048)));
+  void* p = nullptr;
+  int rc = stats_get(np * sizeof(double), &p);
+  if (rc) return rc;
+  double* partial = static_cast<double*>(p);
+  if (dtype == WH_F32)
+    hipLaunchKernelGGL(mse_k<float>, dim3(np), dim3(256), 0, st, static_cast<const float*>(y),
+                       static_cast<const float*>(ref), static_cast<float*>(g), total, partial);
+  else
+    hipLaunchKernelGGL(mse_k<double>, dim3(np), dim3(256), 0, st, static_cast<const double*>(y),
+                       static_cast<const double*>(ref), static_cast<double*>(g), total, partial);
+  hipLaunchKernelGGL(mse_sum_k, dim3(1), dim3(256), 0, st, partial, int(np), total, out);
+  WH_HIP_CHECK(hipGetLastError());
   return WH_OK;
 }
 

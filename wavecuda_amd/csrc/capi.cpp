@@ -259,8 +259,45 @@ int wh_modwt_fwd_adj(const void* gxmod, void* gx, int64_t n, int64_t count, int 
                      int filter, int dtype, void* stream) {
   int J, rc = check_common(gxmod, gx, n, nlevels, filter, dtype, &J);
   if (rc || (rc = check_count(count))) return rc;
-  return modwt_forward_adjoint(gxmod, gx, n, count, J, filter, dtype,
+  return modwt_forward_adjoint(gxmod, gx, n, count, J, filter, dtype, false,
                                static_cast<hipStream_t>(stream));
+}
+
+int wh_modwt_fwd_details(const void* x, void* xmod, int64_t n, int64_t count, int nlevels,
+                         int filter, int dtype, void* stream) {
+  int J, rc = check_common(x, xmod, n, nlevels, filter, dtype, &J);
+  if (rc || (rc = check_count(count))) return rc;
+  return modwt_forward_details(x, xmod, n, count, J, filter, dtype,
+                               static_cast<hipStream_t>(stream));
+}
+
+int wh_modwt_fwd_details_adj(const void* gxmod, void* gx, int64_t n, int64_t count, int nlevels,
+                             int filter, int dtype, void* stream) {
+  int J, rc = check_common(gxmod, gx, n, nlevels, filter, dtype, &J);
+  if (rc || (rc = check_count(count))) return rc;
+  return modwt_forward_adjoint(gxmod, gx, n, count, J, filter, dtype, true,
+                               static_cast<hipStream_t>(stream));
+}
+
+int wh_modwt_thresh_inv_adj(const void* gy, const void* xmod, void* gxmod, int details_only,
+                            double* glam, int64_t n, int64_t count, int nlevels, int filter,
+                            int dtype, const wh_thresh* thr, void* stream) {
+  int J, rc = check_common(gy, xmod, n, nlevels, filter, dtype, &J);
+  if (rc || (rc = check_count(count))) return rc;
+  if (!gxmod && !glam) return set_error(WH_ERR_ARG, "threshold gradient: gxmod and glam both NULL");
+  if (gxmod && (reinterpret_cast<uintptr_t>(gxmod) & (dtype == WH_F64 ? 15 : 7)))
+    return set_error(WH_ERR_ARG, "device buffers must be aligned to two elements (16 bytes FP64, 8 bytes FP32)");
+  if (!thr || !thr->enabled) return set_error(WH_ERR_ARG, "threshold gradient needs a threshold");
+  if ((rc = check_thresh(thr, J))) return rc;
+  return modwt_thresh_inverse_adjoint(gy, xmod, gxmod, details_only == 0, glam, n, count, J,
+                                      filter, dtype, thr, static_cast<hipStream_t>(stream));
+}
+
+int wh_mse_grad(const void* y, const void* ref, void* g, int64_t total, int dtype, double* out,
+                void* stream) {
+  if (!y || !ref || !g || !out || total <= 0) return set_error(WH_ERR_ARG, "null pointer or empty input");
+  if (!valid_dtype(dtype)) return set_error(WH_ERR_ARG, "bad dtype");
+  return mse_grad(y, ref, g, total, dtype, out, static_cast<hipStream_t>(stream));
 }
 
 int wh_modwt_inv_adj(const void* gx, void* gxmod, int64_t n, int64_t count, int nlevels,

@@ -234,7 +234,11 @@ int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t c
   // residue class for the inverse (L + 1 interleaved (S, D) reads instead of
   // 2L; it is LDS-bound)
   gl.map = inverse ? 2 : 0;
-  if (G.tile) return modwt_tile_launch<T>(inverse, filt, gl, a, st);
+  if (G.tile)
+    return modwt_tile_launch<T>(inverse ? TileOp::kInverse
+                                : sp == kStoreSmooth ? TileOp::kForwardDetails
+                                                     : TileOp::kForward,
+                                filt, gl, a, GradArgs{}, st);
   if (gl.blocks > 0x7fffffff) return set_error(WH_ERR_ARG, "modwt: grid too large");
   if (inverse && G.R == 1 && (int64_t(1) << G.g) > G.M)
     return set_error(WH_ERR_UNSUPPORTED, "modwt: inverse group deeper than its chunk allows");
@@ -367,6 +371,150 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
   return WH_OK;
 }
 
+// the tiles of the adjoint and gradient kernels
+std::vector<Group> adjoint_tiles(bool inverse, int64_t n, int J, int L, size_t esz) {
+  PlanKnobs k;
+  k.g1max = kTileGmax;
+  k.first_nt = -kTileAdjNT;
+  return plan_tiles(inverse, n, J, L, esz, k);
+}
+
+GroupLaunch launch_of(const Group& G, int64_t count) {
+  GroupLaunch gl{};
+  gl.R = G.R;
+  gl.NT = G.NT;
+  gl.G = G.g;
+  gl.count = count;
+  gl.blocks = ((int64_t(1) << G.j0) / G.R) * G.nseg;
+  return gl;
+}
+
+// adjoint of the forward: the level groups from the deepest up
+template <typename T>
+int fwd_adj_t(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
+              bool details, hipStream_t st) {
+  auto groups = adjoint_tiles(true, n, J, filter_length(filt), sizeof(T));
+  const int64_t per = 2 * n * J;
+  T* scratch = nullptr;
+  if (groups.size() > 1) {
+    void* p = nullptr;
+    int rc = scratch_get(2 * size_t(n) * size_t(count) * sizeof(T), &p);
+    if (rc) return rc;
+    scratch = static_cast<T*>(p);
+  }
+  const T* stop = static_cast<const T*>(gxmod) + 2 * n * int64_t(J - 1);
+  int64_t bs_stop = per;
+  for (int gi = int(groups.size()) - 1; gi >= 0; --gi) {
+    const Group& G = groups[gi];
+    ModwtArgs a = args_of(G, n);
+    a.xmod = const_cast<void*>(gxmod);
+    a.bs_xmod = per;
+    a.stop = stop;
+    a.bs_stop = bs_stop;
+    T* dst = (G.j0 == 0) ? static_cast<T*>(gx) : scratch + (gi & 1) * n * count;
+    a.out = dst;
+    a.bs_out = n;
+    int rc = modwt_tile_launch<T>(details ? TileOp::kAdjDetails : TileOp::kAdjFull, filt,
+                                  launch_of(G, count), a, GradArgs{}, st);
+    if (rc) return rc;
+    stop = dst;
+    bs_stop = n;
+  }
+  return WH_OK;
+}
+
+// workgroups per signal of the groups (partial sums of their levels)
+struct GradSums {
+  int ngroups;
+  int end[8];     // first level beyond the group
+  int64_t blocks[8];
+};
+
+// glam[l] = the sum of level l's partials over signals and workgroups, in a
+// fixed order; zero outside [minlevel, maxlevel]
+__global__ __launch_bounds__(256) void grad_sum_k(const double* __restrict__ partial,
+                                                  double* __restrict__ glam, int64_t count,
+                                                  int64_t per_signal, GradSums gs, int minlevel,
+                                                  int maxlevel) {
+  const int l = blockIdx.x;
+  __shared__ double red[256];
+  double acc = 0.0;
+  if (l >= minlevel && l <= maxlevel) {
+    int g = 0;
+    while (l >= gs.end[g]) ++g;
+    const int64_t nb = gs.blocks[g];
+    const double* p = partial + l * count * per_signal;
+    for (int64_t i = threadIdx.x; i < count * nb; i += 256) acc += p[(i / nb) * per_signal + i % nb];
+  }
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) glam[l] = red[0];
+}
+
+// adjoint of the thresholding inverse (thr null: of the plain inverse) over
+// the coefficients c
+template <typename T>
+int inv_grad_t(const void* gy, const void* c, void* gc, bool zero_s, double* glam, int64_t n,
+               int64_t count, int J, int filt, const wh_thresh* thr, hipStream_t st) {
+  auto groups = adjoint_tiles(false, n, J, filter_length(filt), sizeof(T));
+  if (groups.size() > 8) return set_error(WH_ERR_UNSUPPORTED, "adjoint: too many level groups");
+  GradArgs q{};
+  q.gc = gc;
+  q.zero_s = zero_s;
+  q.minlevel = 1;  // none
+  if (thr) {
+    q.hardness = thr->hardness;
+    q.minlevel = thr->minlevel;
+    q.maxlevel = thr->maxlevel;
+    q.value = thr->value;
+    q.levels = thr->levels;
+  }
+  GradSums gs{};
+  for (const Group& G : groups) {
+    gs.end[gs.ngroups] = G.j0 + G.g;
+    gs.blocks[gs.ngroups] = launch_of(G, count).blocks;
+    q.per_signal = std::max(q.per_signal, gs.blocks[gs.ngroups]);
+    ++gs.ngroups;
+  }
+  void* p = nullptr;
+  if (glam) {
+    int rc = stats_get(size_t(J) * size_t(count) * size_t(q.per_signal) * sizeof(double), &p);
+    if (rc) return rc;
+    q.partial = static_cast<double*>(p);
+  }
+  T* scratch = nullptr;
+  if (groups.size() > 1) {
+    int rc = scratch_get(2 * size_t(n) * size_t(count) * sizeof(T), &p);
+    if (rc) return rc;
+    scratch = static_cast<T*>(p);
+  }
+  const void* in = gy;
+  for (size_t gi = 0; gi < groups.size(); ++gi) {
+    const Group& G = groups[gi];
+    ModwtArgs a = args_of(G, n);
+    a.in = in;
+    a.bs_in = n;
+    a.xmod = const_cast<void*>(c ? c : gc);
+    a.bs_xmod = 2 * n * J;
+    a.out = scratch ? scratch + int64_t(gi & 1) * n * count : nullptr;
+    a.bs_out = n;
+    q.last = gi + 1 == groups.size();
+    int rc = modwt_tile_launch<T>(TileOp::kGrad, filt, launch_of(G, count), a, q, st);
+    if (rc) return rc;
+    in = a.out;
+  }
+  if (glam) {
+    hipLaunchKernelGGL(grad_sum_k, dim3(unsigned(J)), dim3(256), 0, st, q.partial, glam, count,
+                       q.per_signal, gs, q.minlevel, q.maxlevel);
+    WH_HIP_CHECK(hipGetLastError());
+  }
+  return WH_OK;
+}
+
 }  // namespace
 
 int modwt_forward(const void* x, void* xmod, int64_t n, int64_t count, int J, int filt,
@@ -396,8 +544,29 @@ int modwt_inverse_ws(const void* xmod, void* x, int64_t n, int64_t count, int J,
 
 int modwt_inverse_adjoint(const void* gx, void* gxmod, int64_t n, int64_t count, int J, int filt,
                           int dtype, hipStream_t st) {
+  // tiles where the forward runs as tiles (see default_knobs): the same
+  // stores bound both
+  if (n * count <= (int64_t(1) << 18))
+    return dtype == WH_F32
+               ? inv_grad_t<float>(gx, nullptr, gxmod, true, nullptr, n, count, J, filt, nullptr, st)
+               : inv_grad_t<double>(gx, nullptr, gxmod, true, nullptr, n, count, J, filt, nullptr,
+                                    st);
   return dtype == WH_F32 ? modwt_fwd_t<float>(gx, gxmod, n, count, J, filt, kStoreAdjoint, st)
                          : modwt_fwd_t<double>(gx, gxmod, n, count, J, filt, kStoreAdjoint, st);
+}
+
+int modwt_forward_adjoint(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
+                          int dtype, bool details, hipStream_t st) {
+  return dtype == WH_F32 ? fwd_adj_t<float>(gxmod, gx, n, count, J, filt, details, st)
+                         : fwd_adj_t<double>(gxmod, gx, n, count, J, filt, details, st);
+}
+
+int modwt_thresh_inverse_adjoint(const void* gy, const void* c, void* gc, bool zero_s,
+                                 double* glam, int64_t n, int64_t count, int J, int filt,
+                                 int dtype, const wh_thresh* thr, hipStream_t st) {
+  return dtype == WH_F32
+             ? inv_grad_t<float>(gy, c, gc, zero_s, glam, n, count, J, filt, thr, st)
+             : inv_grad_t<double>(gy, c, gc, zero_s, glam, n, count, J, filt, thr, st);
 }
 
 namespace {

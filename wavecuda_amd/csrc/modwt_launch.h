@@ -26,6 +26,10 @@ int modwt_launch_one(bool inverse, const GroupLaunch& gl, const ModwtArgs& a, hi
     auto kern = modwt_fwd_k<T, FILT, R, NT, G, 0, kStoreAdjoint>;
     modwt_allow_lds(kern);
     hipLaunchKernelGGL(kern, grid, dim3(NT), gl.lds, st, a);
+  } else if (gl.sp == kStoreSmooth) {
+    auto kern = modwt_fwd_k<T, FILT, R, NT, G, 0, kStoreSmooth>;
+    modwt_allow_lds(kern);
+    hipLaunchKernelGGL(kern, grid, dim3(NT), gl.lds, st, a);
   } else {
     auto kern = modwt_fwd_k<T, FILT, R, NT, G, 0, kStoreAll>;
     modwt_allow_lds(kern);

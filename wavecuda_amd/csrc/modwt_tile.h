@@ -33,6 +33,21 @@ constexpr int kTileGmax = 6;  // deepest tile group (5 beyond the first)
 // 11.9 -> 11.3 us from 4 to 8), the inverse the shorter halo.
 __host__ __device__ constexpr int tile_r(bool inverse) { return inverse ? 4 : 8; }
 
+constexpr int kTileAdjNT = 512;  // threads of the adjoint and gradient tiles
+
+// What the gradient tile needs beside ModwtArgs (in: the cotangent, xmod: the
+// coefficients before thresholding, out: the hand-off to the next group)
+struct GradArgs {
+  void* gc;         // cotangent of the coefficients, or null
+  int zero_s;       // also write zeros into its S_j slots, j < J
+  int last;         // this group ends at level J
+  double* partial;  // [level][signal][per_signal], or null
+  int64_t per_signal;
+  int hardness, minlevel, maxlevel;  // no level: minlevel > maxlevel
+  double value;
+  const double* levels;
+};
+
 __host__ __device__ constexpr int tile_halo(int L, int l) { return (L - 1) * ((1 << l) - 1); }
 
 // workgroup id -> (signal segment, residue block): workgroups are handed to
@@ -130,13 +145,166 @@ __global__ __launch_bounds__(NT) void modwt_fwd_tile_k(ModwtArgs args) {
   C::template levels<1>(lds, lds + C::N0, static_cast<T*>(a.xmod), a, r0 + (m0 << a.j0), Nm - m0);
 }
 
+// The adjoint of the thresholding inverse: the forward over the output's
+// cotangent, level l scaled by 2^-l, and at each detail the threshold's
+// gradient where the coefficient c passes it.  The coefficients are loaded
+// at the start; per-level sums of dL/dt stay in registers and leave as one
+// partial per workgroup, in an order that repeats.  With gc the cotangent of
+// the coefficients is stored (details, S_J, and zeros in the other S slots
+// if asked for); without it the kernel writes nothing but its hand-off and
+// partials: 512 x 2^14 FP32, J = 8, LA8 took a pass that stored the 2nJ
+// cotangents (102 us) and one that read them back beside c (108 us).
+template <typename T, int FILT, int R, int G, int NT>
+struct GradTile {
+  using F = FwdTile<T, FILT, R, G, NT, kStoreAll>;
+  static constexpr int L = F::L;
+  static constexpr int KO = F::PR / NT;  // owned outputs per thread
+  static constexpr int kWaves = NT / 64;
+  T c[G][KO];
+  double acc[G];
+
+  // c of level l and the threshold's gradient there; the owned outputs come
+  // first in every level's order, so output k < KO of a thread is owned
+  __device__ __forceinline__ T apply(const GradArgs& q, int l, int k, T g, T t, bool act) {
+    if (!act) return g;
+    const T v = c[l - 1][k], m = fabs(v);
+    if (q.hardness == kSOFT) {
+      const bool pass = m > t;
+      if (pass) acc[l - 1] += double(v < T(0) ? g : -g);
+      return pass ? g : T(0);
+    }
+    return m < t ? T(0) : g;
+  }
+
+  template <int l>
+  __device__ __forceinline__ void levels(T* b0, T* b1, const ModwtArgs& a, const GradArgs& q,
+                                         T* gc, int64_t base, int64_t qmax) {
+    if constexpr (l <= G) {
+      constexpr int s = 1 << (l - 1);
+      constexpr int cnt = F::PR + (F::WG - tile_halo(L, l)) * R;
+      constexpr T sc = T(1.0 / double(1 << l));
+      const T* in = (l & 1) ? b0 : b1;
+      T* nxt = (l & 1) ? b1 : b0;
+      const int lev = a.j0 + l - 1;
+      const bool act = lev >= q.minlevel && lev <= q.maxlevel;
+      const T t = !act ? T(0) : q.levels ? T(q.levels[lev]) : T(q.value);
+      T* oS = gc ? gc + 2 * a.n * int64_t(lev) : nullptr;
+      const bool top = l == G && q.last;  // S_J
+#pragma unroll
+      for (int k = 0; k < (cnt + NT - 1) / NT; ++k) {
+        const int o = int(threadIdx.x) + k * NT;
+        if (o < cnt) {
+          T w[L], S, D;
+#pragma unroll
+          for (int j = 0; j < L; ++j) w[j] = in[o + j * s * R];
+          analysis1<T, FILT>(w, S, D);
+          if constexpr (l < G) nxt[o] = S;
+          if (k < KO && o / R < qmax) {
+            const T g = apply(q, l, k < KO ? k : 0, D * sc, t, act);
+            const int64_t i = base + (o % R) + (int64_t(o / R) << a.j0);
+            if (oS) {
+              oS[a.n + i] = g;
+              if (top) oS[i] = S * sc;
+              else if (q.zero_s) oS[i] = T(0);
+            }
+            if (l == G && !q.last) static_cast<T*>(a.out)[i] = S * sc;
+          }
+        }
+      }
+      if constexpr (l < G) __syncthreads();
+      levels<l + 1>(b0, b1, a, q, gc, base, qmax);
+    }
+  }
+};
+
+template <typename T, int FILT, int R, int G, int NT>
+__global__ __launch_bounds__(NT) void modwt_grad_tile_k(ModwtArgs args, GradArgs q) {
+  using C = GradTile<T, FILT, R, G, NT>;
+  using F = typename C::F;
+  __shared__ __align__(16) T lds[F::kLdsElems];
+  __shared__ double red[G][C::kWaves];
+  const ModwtArgs a = batch_slice<T>(args);
+  constexpr int P = F::PR / R;
+  const int64_t Nm = a.n >> a.j0, nrb = (int64_t(1) << a.j0) / R;
+  const int64_t t = tile_index(blockIdx.x, gridDim.x);
+  const int64_t r0 = (t % nrb) * R, m0 = (t / nrb) * P;
+  const T* __restrict__ in = static_cast<const T*>(a.in);
+  const T* __restrict__ xm = static_cast<const T*>(a.xmod);
+  constexpr int K = (F::N0 + NT - 1) / NT;
+  C c;
+  T v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    const int ec = e < F::N0 ? e : F::N0 - 1;  // unconditional load, clamped
+    v[k] = in[r0 + (ec % R) + (((m0 + ec / R) & (Nm - 1)) << a.j0)];
+  }
+#pragma unroll
+  for (int l = 1; l <= G; ++l) {
+    c.acc[l - 1] = 0.0;
+#pragma unroll
+    for (int k = 0; k < C::KO; ++k) {
+      const int o = int(threadIdx.x) + k * NT, lev = a.j0 + l - 1;
+      const int64_t i = r0 + (o % R) + (((m0 + o / R) & (Nm - 1)) << a.j0);
+      c.c[l - 1][k] = lev >= q.minlevel && lev <= q.maxlevel
+                          ? xm[2 * a.n * int64_t(lev) + a.n + i]
+                          : T(0);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    if (e < F::N0) lds[e] = v[k];
+  }
+  __syncthreads();
+  T* gc = q.gc ? static_cast<T*>(q.gc) + int64_t(blockIdx.y) * a.bs_xmod : nullptr;
+  c.template levels<1>(lds, lds + F::N0, a, q, gc, r0 + (m0 << a.j0), Nm - m0);
+  if (!q.partial) return;
+#pragma unroll
+  for (int l = 0; l < G; ++l) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c.acc[l] += __shfl_xor(c.acc[l], o, 64);
+    if ((threadIdx.x & 63) == 0) red[l][threadIdx.x >> 6] = c.acc[l];
+  }
+  __syncthreads();
+  if (threadIdx.x < G) {
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < C::kWaves; ++w) sum += red[threadIdx.x][w];
+    q.partial[((a.j0 + int64_t(threadIdx.x)) * gridDim.y + blockIdx.y) * q.per_signal +
+              blockIdx.x] = sum;
+  }
+}
+
 // ---------------------------------------------------------------- inverse
 // Slot o of level l's buffer holds (S_l, D_l) at m = m0 - W_l + o / R.  The
 // details of every level are loaded to registers at the start; a level's
 // threads write the pair they own -- the S just computed and that level's
 // detail -- with one 16-byte store, into the buffer the level above it
 // (l + 1) did not read, so a level costs one barrier.
-template <typename T, int FILT, int R, int G, int NT>
+//
+// The same tile is the adjoint of the forward (Adj): u_{j-1} = Sb_{j-1} +
+// H_j^T u_j + G_j^T Db_j reads positions i - k s as the inverse does, without
+// the factor 1/2 and the threshold, and with each level's own S cotangent
+// Sb added (kAdjFull) or known to be zero (kAdjDetails).
+constexpr int kInverse = 0;
+constexpr int kAdjFull = 1;
+constexpr int kAdjDetails = 2;
+
+// one output of the adjoint: acc + sum_k C_k u[tap k] + g_k Db[tap k], k
+// ascending, tap k at w[L - 1 - k]
+template <typename T, int FILT>
+__device__ __forceinline__ T adjoint1(const T* wu, const T* wd, T acc) {
+  constexpr int L = Filter<FILT>::L;
+#pragma unroll
+  for (int k = 0; k < L; ++k) {
+    acc = fma(wu[L - 1 - k], T(Filter<FILT>::c(k)), acc);
+    acc = fma(wd[L - 1 - k], T(gcoef<FILT>(k)), acc);
+  }
+  return acc;
+}
+
+template <typename T, int FILT, int R, int G, int NT, int MODE>
 struct InvTile {
   using V = typename Vec2<T>::type;
   static constexpr int L = Filter<FILT>::L;
@@ -145,6 +313,7 @@ struct InvTile {
   static constexpr int K(int l) { return (cnt(l) + NT - 1) / NT; }
   static constexpr int kSlots = G > 1 ? cnt(G) + cnt(G - 1) : cnt(G);
   T d[G + 1][K(G)];  // details of levels 1..G-1 (and the group's top level)
+  T sb[MODE == kAdjFull ? G + 1 : 1][K(G)];  // Sb of the levels 0..G-1 of the group
 
   static __device__ __forceinline__ T thr(const ModwtArgs& a, int l) {
     const int lev = a.j0 + l - 1;
@@ -167,6 +336,17 @@ struct InvTile {
         const int e = int(threadIdx.x) + k * NT;
         d[l][k] = D[gidx<l>(a, r0, m0, Nm, e < cnt(l) ? e : cnt(l) - 1)];
       }
+      if constexpr (MODE == kAdjFull) {
+        // S_{j0 + l - 1}, this level's output slots; none below level 1
+        const bool have = a.j0 + l > 1;
+        const T* S = static_cast<const T*>(a.xmod) + 2 * a.n * int64_t(a.j0 + l - 2);
+#pragma unroll
+        for (int k = 0; k < K(l - 1); ++k) {
+          const int e = int(threadIdx.x) + k * NT;
+          sb[l - 1][k] =
+              have ? S[gidx<l - 1>(a, r0, m0, Nm, e < cnt(l - 1) ? e : cnt(l - 1) - 1)] : T(0);
+        }
+      }
       load<l - 1>(a, r0, m0, Nm);
     }
   }
@@ -176,7 +356,7 @@ struct InvTile {
     if constexpr (l >= 1) {
       constexpr int s = 1 << (l - 1);
       constexpr int no = cnt(l - 1);  // outputs of this level (cnt(0) = PR)
-      const T t = l > 1 ? thr(a, l - 1) : T(-1);
+      const T t = MODE == kInverse && l > 1 ? thr(a, l - 1) : T(-1);
 #pragma unroll
       for (int k = 0; k < (no + NT - 1) / NT; ++k) {
         const int o = int(threadIdx.x) + k * NT;
@@ -188,10 +368,12 @@ struct InvTile {
             ws[j] = v.x;
             wd[j] = v.y;
           }
-          const T e = synthesis<T, FILT>(ws, wd, L - 1);
+          T e;
+          if constexpr (MODE == kInverse) e = synthesis<T, FILT>(ws, wd, L - 1);
+          else e = adjoint1<T, FILT>(ws, wd, MODE == kAdjFull ? sb[l - 1][k] : T(0));
           if constexpr (l > 1) {
             T c = d[l - 1][k];
-            if (t >= T(0)) c = thresh_coef(c, t, a.hardness);
+            if (MODE == kInverse && t >= T(0)) c = thresh_coef(c, t, a.hardness);
             bb[o] = V{e, c};
           } else if (o / R < qmax) {
             out[base + (o % R) + (int64_t(o / R) << a.j0)] = e;
@@ -204,9 +386,9 @@ struct InvTile {
   }
 };
 
-template <typename T, int FILT, int R, int G, int NT>
+template <typename T, int FILT, int R, int G, int NT, int MODE>
 __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
-  using C = InvTile<T, FILT, R, G, NT>;
+  using C = InvTile<T, FILT, R, G, NT, MODE>;
   using V = typename Vec2<T>::type;
   __shared__ __align__(16) V lds[C::kSlots];
   const ModwtArgs a = batch_slice<T>(args);
@@ -223,7 +405,7 @@ __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
     sg[k] = S[C::template gidx<G>(a, r0, m0, Nm, e < C::cnt(G) ? e : C::cnt(G) - 1)];
   }
   c.template load<G>(a, r0, m0, Nm);
-  const T t = C::thr(a, G);
+  const T t = MODE == kInverse ? C::thr(a, G) : T(-1);
 #pragma unroll
   for (int k = 0; k < C::K(G); ++k) {
     const int e = int(threadIdx.x) + k * NT;
@@ -238,56 +420,74 @@ __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
                        Nm - m0);
 }
 
+// What a tile launch computes
+enum class TileOp { kForward, kForwardDetails, kInverse, kAdjFull, kAdjDetails, kGrad };
+
 // Launch of a tile group of (element type, filter); defined per element
 // type in modwt_tile_<type>.hip.
 template <typename T>
-int modwt_tile_launch(bool inverse, int filt, const GroupLaunch& gl, const ModwtArgs& a,
-                      hipStream_t st);
+int modwt_tile_launch(TileOp op, int filt, const GroupLaunch& gl, const ModwtArgs& a,
+                      const GradArgs& q, hipStream_t st);
 
 template <typename T, int FILT, bool INV, int R, int NT, int G>
-int tile_launch_g(const GroupLaunch& gl, const ModwtArgs& a, hipStream_t st) {
+int tile_launch_g(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const GradArgs& q,
+                  hipStream_t st) {
   if constexpr (G > kTileGmax || (R > 1 && G > kTileGmax - 1)) {
     return set_error(WH_ERR_UNSUPPORTED, "modwt: tile group depth out of range");
   } else {
-    if (gl.G != G) return tile_launch_g<T, FILT, INV, R, NT, G + 1>(gl, a, st);
+    if (gl.G != G) return tile_launch_g<T, FILT, INV, R, NT, G + 1>(op, gl, a, q, st);
     const dim3 grid(unsigned(gl.blocks), unsigned(gl.count));
-    if constexpr (INV)
-      hipLaunchKernelGGL((modwt_inv_tile_k<T, FILT, R, G, NT>), grid, dim3(NT), 0, st, a);
-    else if (gl.sp == kStoreSmooth)
-      hipLaunchKernelGGL((modwt_fwd_tile_k<T, FILT, R, G, NT, kStoreSmooth>), grid, dim3(NT), 0,
-                         st, a);
-    else
-      hipLaunchKernelGGL((modwt_fwd_tile_k<T, FILT, R, G, NT, kStoreAll>), grid, dim3(NT), 0, st,
-                         a);
+    if constexpr (INV) {
+      if (op == TileOp::kInverse)
+        hipLaunchKernelGGL((modwt_inv_tile_k<T, FILT, R, G, NT, kInverse>), grid, dim3(NT), 0, st,
+                           a);
+      else if constexpr (NT == kTileAdjNT)
+        hipLaunchKernelGGL((op == TileOp::kAdjFull
+                                ? modwt_inv_tile_k<T, FILT, R, G, NT, kAdjFull>
+                                : modwt_inv_tile_k<T, FILT, R, G, NT, kAdjDetails>),
+                           grid, dim3(NT), 0, st, a);
+    } else {
+      if (op == TileOp::kForward)
+        hipLaunchKernelGGL((modwt_fwd_tile_k<T, FILT, R, G, NT, kStoreAll>), grid, dim3(NT), 0,
+                           st, a);
+      else if (op == TileOp::kForwardDetails)
+        hipLaunchKernelGGL((modwt_fwd_tile_k<T, FILT, R, G, NT, kStoreSmooth>), grid, dim3(NT), 0,
+                           st, a);
+      else if constexpr (NT == kTileAdjNT)
+        hipLaunchKernelGGL((modwt_grad_tile_k<T, FILT, R, G, NT>), grid, dim3(NT), 0, st, a, q);
+    }
     WH_HIP_CHECK(hipGetLastError());
     return WH_OK;
   }
 }
 
 template <typename T, int FILT, bool INV>
-int tile_launch_f(const GroupLaunch& gl, const ModwtArgs& a, hipStream_t st) {
+int tile_launch_f(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const GradArgs& q,
+                  hipStream_t st) {
   constexpr int RD = tile_r(INV);
-  if (gl.R == 1 && gl.NT == 512) return tile_launch_g<T, FILT, INV, 1, 512, 1>(gl, a, st);
-  if (gl.R == 1 && gl.NT == 256) return tile_launch_g<T, FILT, INV, 1, 256, 1>(gl, a, st);
-  if (gl.R == RD && gl.NT == 512) return tile_launch_g<T, FILT, INV, RD, 512, 1>(gl, a, st);
-  if (gl.R == RD && gl.NT == 256) return tile_launch_g<T, FILT, INV, RD, 256, 1>(gl, a, st);
+  if (gl.R == 1 && gl.NT == 512) return tile_launch_g<T, FILT, INV, 1, 512, 1>(op, gl, a, q, st);
+  if (gl.R == 1 && gl.NT == 256) return tile_launch_g<T, FILT, INV, 1, 256, 1>(op, gl, a, q, st);
+  if (gl.R == RD && gl.NT == 512) return tile_launch_g<T, FILT, INV, RD, 512, 1>(op, gl, a, q, st);
+  if (gl.R == RD && gl.NT == 256) return tile_launch_g<T, FILT, INV, RD, 256, 1>(op, gl, a, q, st);
   return set_error(WH_ERR_UNSUPPORTED, "modwt: unsupported tile shape");
 }
 
 template <typename T, int FILT>
-int tile_launch(bool inverse, const GroupLaunch& gl, const ModwtArgs& a, hipStream_t st) {
-  return inverse ? tile_launch_f<T, FILT, true>(gl, a, st)
-                 : tile_launch_f<T, FILT, false>(gl, a, st);
+int tile_launch(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const GradArgs& q,
+                hipStream_t st) {
+  const bool inv = op == TileOp::kInverse || op == TileOp::kAdjFull || op == TileOp::kAdjDetails;
+  return inv ? tile_launch_f<T, FILT, true>(op, gl, a, q, st)
+             : tile_launch_f<T, FILT, false>(op, gl, a, q, st);
 }
 
 template <typename T>
-int modwt_tile_launch_impl(bool inverse, int filt, const GroupLaunch& gl, const ModwtArgs& a,
-                           hipStream_t st) {
+int modwt_tile_launch_impl(TileOp op, int filt, const GroupLaunch& gl, const ModwtArgs& a,
+                           const GradArgs& q, hipStream_t st) {
   switch (filt) {
-    case kHAAR: return tile_launch<T, kHAAR>(inverse, gl, a, st);
-    case kD4: return tile_launch<T, kD4>(inverse, gl, a, st);
-    case kC6: return tile_launch<T, kC6>(inverse, gl, a, st);
-    default: return tile_launch<T, kLA8>(inverse, gl, a, st);
+    case kHAAR: return tile_launch<T, kHAAR>(op, gl, a, q, st);
+    case kD4: return tile_launch<T, kD4>(op, gl, a, q, st);
+    case kC6: return tile_launch<T, kC6>(op, gl, a, q, st);
+    default: return tile_launch<T, kLA8>(op, gl, a, q, st);
   }
 }
 

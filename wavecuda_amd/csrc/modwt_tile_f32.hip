@@ -3,8 +3,8 @@
 
 namespace wh {
 template <>
-int modwt_tile_launch<float>(bool inverse, int filt, const GroupLaunch& gl, const ModwtArgs& a,
-                             hipStream_t st) {
-  return modwt_tile_launch_impl<float>(inverse, filt, gl, a, st);
+int modwt_tile_launch<float>(TileOp op, int filt, const GroupLaunch& gl, const ModwtArgs& a,
+                              const GradArgs& q, hipStream_t st) {
+  return modwt_tile_launch_impl<float>(op, filt, gl, a, q, st);
 }
 }  // namespace wh

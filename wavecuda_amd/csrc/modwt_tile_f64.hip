@@ -3,8 +3,8 @@
 
 namespace wh {
 template <>
-int modwt_tile_launch<double>(bool inverse, int filt, const GroupLaunch& gl, const ModwtArgs& a,
-                             hipStream_t st) {
-  return modwt_tile_launch_impl<double>(inverse, filt, gl, a, st);
+int modwt_tile_launch<double>(TileOp op, int filt, const GroupLaunch& gl, const ModwtArgs& a,
+                              const GradArgs& q, hipStream_t st) {
+  return modwt_tile_launch_impl<double>(op, filt, gl, a, q, st);
 }
 }  // namespace wh

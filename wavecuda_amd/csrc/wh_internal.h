@@ -83,8 +83,17 @@ int modwt_inverse_ws(const void* xmod, void* x, int64_t n, int64_t count, int J,
 // with exact 2^-j scalings) and of the forward (xmod-cotangent -> x-cotangent)
 int modwt_inverse_adjoint(const void* gx, void* gxmod, int64_t n, int64_t count, int J, int filt,
                           int dtype, hipStream_t st);
+// (details: the cotangents of the S_j, j < J, are taken as zero and not read)
 int modwt_forward_adjoint(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
-                          int dtype, hipStream_t st);
+                          int dtype, bool details, hipStream_t st);
+// of the thresholding inverse at the coefficients c: gy -> gc (may be null;
+// zeros in its S_j slots, j < J, if zero_s) and dL/dt per level (may be null)
+int modwt_thresh_inverse_adjoint(const void* gy, const void* c, void* gc, bool zero_s,
+                                 double* glam, int64_t n, int64_t count, int J, int filt,
+                                 int dtype, const wh_thresh* thr, hipStream_t st);
+// mean((y - ref)^2) to *out and its gradient in y to g (may be y)
+int mse_grad(const void* y, const void* ref, void* g, int64_t total, int dtype, double* out,
+             hipStream_t st);
 int thresh_grad(const void* c, const void* gy, void* gc, double* glam, int64_t n, int64_t count,
                 int J, int ttype, int dtype, const wh_thresh* thr, hipStream_t st);
 // the level groups a launch of `count` signals runs, as text
