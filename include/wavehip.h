@@ -238,7 +238,8 @@ int wh_modwt_tune(int64_t n, int nlevels, int filter, int dtype, void* stream);
    wh_debug_modwt_set_plan sets the planner's choices for one shape as
    wh_modwt_tune would (deepest first group g1max, segments per CU of the
    first and deeper groups, 512 or 256 threads in the first inverse group;
-   -512 or -256: tiles of that many threads and at most g1max = 3..6 levels);
+   -512 or -256: tiles of that many threads and at most g1max = 3..6 levels;
+   -256 with g1max 7 or 8: one wide tile, FP32 inverse, 3..8 levels, n >= 2048);
    g1max <= 0 restores the default rules.  Results never depend on the
    plan; these let a caller run and check every plan the tuner can pick. */
 int wh_debug_modwt_plan(int inverse, int64_t n, int nlevels, int filter, int dtype, char* buf,

@@ -20,7 +20,8 @@ from wavecuda_amd import device as D
 
 pytestmark = pytest.mark.gpu
 SHAPES = [(3, 16, 2, "D4"), (1, 1024, 6, "LA8"), (5, 256, 7, "Haar"), (2, 1 << 12, 8, "LA8"),
-          (3, 1 << 13, 10, "C6"), (2, 1 << 14, 13, "D4"), (70, 1 << 12, 8, "LA8")]
+          (3, 1 << 13, 10, "C6"), (2, 1 << 14, 13, "D4"), (70, 1 << 12, 8, "LA8"),
+          (130, 1 << 12, 8, "LA8"), (260, 1 << 12, 4, "Haar"), (520, 1 << 12, 6, "D4")]
 
 
 def _p(t):

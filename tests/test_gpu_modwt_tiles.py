@@ -64,3 +64,33 @@ def test_default_tiles_of_many_signals(n, count, J):
     for b in range(count):
         assert torch.equal(w[b], D.modwt_fwd(x[b], J, W.LA8))
         assert torch.equal(y[b], D.modwt_inv(w[b], n, J, W.LA8))
+
+
+WIDE = (8, 1, 1, -256)
+
+
+@pytest.mark.parametrize("filt,n,J", [("Haar", 2048, 3), ("D4", 4096, 5), ("C6", 2048, 6),
+                                      ("LA8", 2048, 8), ("LA8", 1 << 15, 7), ("Haar", 1 << 13, 8)])
+def test_wide_tiles_equal_sliding(filt, n, J):
+    """FP32 inverse as one wide tile: one tile per signal (the halo wraps) and
+    many, with and without thresholds."""
+    f, dtype = D.filter_code(filt), torch.float32
+    w = torch.randn(2 * n * J, dtype=dtype, device="cuda",
+                    generator=torch.Generator(device="cuda").manual_seed(n + J))
+    lam = torch.linspace(1.0, 0.1, J, dtype=torch.float64, device="cuda")
+    thrs = [None] + [dict(hardness=h, minlevel=lo, maxlevel=J - 1, levels=lam)
+                     for h, lo in ((W.SOFT, 0), (W.HARD, 1))]
+    try:
+        outs = []
+        for knobs in (SLIDING, WIDE):
+            D.modwt_set_plan(True, n, J, f, dtype, knobs)
+            outs.append([D.modwt_inv(w, n, J, f, t) for t in thrs])
+        plan = D.modwt_plan(True, n, J, f, dtype)
+        assert "tile" in plan and f" g={J} " in plan
+        for a, b in zip(*outs):
+            assert torch.equal(a, b)
+        with pytest.raises(W.WaveHipError):
+            D.modwt_set_plan(True, n, J, f, torch.float64, WIDE)
+    finally:
+        for dt in (torch.float32, torch.float64):
+            D.modwt_set_plan(True, n, J, f, dt, None)

@@ -31,6 +31,7 @@ constexpr int kDeepSegPerCu = 4;
 
 struct Group {
   bool tile = false;  // one tile per workgroup (modwt_tile.h) instead of a sliding window
+  bool wide = false;  // all levels in one wide tile
   int j0, g, R, NT, M;
   int64_t P;
   int nseg, warm, nchunks;
@@ -45,7 +46,7 @@ struct PlanKnobs {
   int first_nt = kNT1;               // threads of the first inverse group (512, or 256:
                                      // two workgroups per CU in half the LDS); negative: a
                                      // plan of tiles of that many threads, at most g1max
-                                     // levels each
+                                     // levels each (g1max 7 or 8: one wide tile)
   bool operator<(const PlanKnobs& o) const {
     return std::tie(g1max, first_per_cu, deep_per_cu, first_nt) <
            std::tie(o.g1max, o.first_per_cu, o.deep_per_cu, o.first_nt);
@@ -55,6 +56,12 @@ struct PlanKnobs {
 using KnobKey = std::tuple<int, int64_t, int, int, int>;  // inverse, n, J, filter, element size
 std::mutex g_knob_mu;
 std::map<KnobKey, PlanKnobs> g_knobs;
+
+// whether a launch's shape can be one wide tile: whole tiles of `per`
+// positions, FP32, 3..8 levels
+bool wide_fits(int per, int64_t n, int J, size_t esz) {
+  return esz == 4 && J >= kWideGmin && J <= kWideGmax && n >= per;
+}
 
 std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz,
                                const PlanKnobs& k, int64_t count = 1);
@@ -75,6 +82,13 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
 //    (2^19, J = 10 FP32: 22.7 -> 16.2; Haar's one group 10.9 against 14.2).
 //    Beyond, it is bound by its stores, which the sliding windows make
 //    in longer runs (2^20, J = 8 FP32: 18.5 against 19.7);
+//  * an FP32 inverse of at most 8 levels as one wide tile: with 7 or 8
+//    levels, which take two tile groups, from 2^19 samples (64 x 2^13, J = 8
+//    LA8 / Haar: 19.2 -> 14.9 / 16.4 -> 11.5; 32 x 2^14 level at 15.3) up to
+//    2^23 (512 x 2^14: sliding 152 -> 118 / 111 -> 64; one 2^24 signal 191
+//    against 195); with fewer, beyond the tiles' range and below 2^23 (2^22,
+//    J = 6 LA8 43.6 -> 39.3, J = 4 31.8 -> 28.9; 512 x 2^14, J = 6 75
+//    against 81);
 //  * a single-signal FP32 inverse beyond that: a 256-thread first group of
 //    at most six levels, four segments per CU (half the FP64 LDS, so
 //    several workgroups share a CU): n = 2^22 90 -> 83, 2^24 307 -> 258.
@@ -89,7 +103,13 @@ PlanKnobs default_knobs(bool inverse, int64_t n, int64_t count, int J, int filt,
     k.first_nt = -threads;
     k.g1max = kTileGmax;
   };
-  if (inverse && total <= (int64_t(1) << 21)) {
+  const bool deep = J > kTileGmax;  // two tile groups
+  if (inverse && wide_fits(kWideInvP, n, J, esz) &&
+      (deep ? total >= (int64_t(1) << 19) && total <= (int64_t(1) << 23)
+            : total > (int64_t(1) << 21) && total < (int64_t(1) << 23))) {
+    k.first_nt = -kWideInvNT;
+    k.g1max = kWideGmax;
+  } else if (inverse && total <= (int64_t(1) << 21)) {
     tiles(total <= (int64_t(1) << 17) ? kNT1 / 2 : kNT1);
   } else if (inverse && count == 1 && esz == 4) {
     k.first_nt = kNT1 / 2;
@@ -118,6 +138,21 @@ std::vector<Group> plan_tiles(bool inverse, int64_t n, int J, int L, size_t esz,
                               const PlanKnobs& k) {
   std::vector<Group> gs;
   const int NT = -k.first_nt;
+  if (k.g1max > kTileGmax) {
+    Group G{};
+    G.tile = G.wide = true;
+    G.g = J;
+    G.R = 1;
+    G.NT = NT;
+    G.P = inverse ? kWideInvP : kWideGradP;
+    G.M = int(G.P);
+    G.nseg = int(n / G.P);
+    G.warm = tile_halo(L, J);
+    G.nchunks = 1;
+    G.lds = size_t(G.P + G.warm) * (inverse ? 2 : 1) * esz;
+    gs.push_back(G);
+    return gs;
+  }
   const int cap = std::min(k.g1max, kTileGmax);
   const int deep = std::min(cap, kTileGmax - 1);
   const int ng = J <= cap ? 1 : (J + deep - 1) / deep;
@@ -224,6 +259,7 @@ int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t c
   gl.R = G.R;
   gl.NT = G.NT;
   gl.G = G.g;
+  gl.wide = G.wide;
   gl.sp = sp;
   gl.count = count;
   gl.blocks = ((int64_t(1) << G.j0) / G.R) * G.nseg;
@@ -371,11 +407,24 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
   return WH_OK;
 }
 
-// the tiles of the adjoint and gradient kernels
-std::vector<Group> adjoint_tiles(bool inverse, int64_t n, int J, int L, size_t esz) {
+// The tiles of the adjoint (of the details) and gradient kernels.  FP32
+// launches of at most 8 levels run as one wide tile: with 7 or 8 levels from
+// 2^19 samples (64 x 2^13, J = 8, LA8: adjoint 19.8 -> 14.0 us, gradient 24.0
+// -> 21.6; 512 x 2^14 140 -> 98 and 160 -> 105), with fewer the adjoint
+// beyond 2^21 (2^21, J = 6: 21.7 against 24.3; 512 x 2^14, J = 5 D4: 50 ->
+// 46) and the gradient from 2^20 (256 x 2^12, J = 6: 22.6 -> 18.5; 2^19: 15.5
+// against 17.4).
+std::vector<Group> adjoint_tiles(bool inverse, int64_t n, int64_t count, int J, int L,
+                                 size_t esz, bool can_wide) {
   PlanKnobs k;
-  k.g1max = kTileGmax;
-  k.first_nt = -kTileAdjNT;
+  const int64_t total = n * count;
+  const int64_t from = J > kTileGmax ? int64_t(1) << 19
+                       : inverse     ? (int64_t(1) << 21) + 1
+                                     : int64_t(1) << 20;
+  const bool wide =
+      can_wide && wide_fits(inverse ? kWideInvP : kWideGradP, n, J, esz) && total >= from;
+  k.g1max = wide ? kWideGmax : kTileGmax;
+  k.first_nt = wide ? -kWideInvNT : -kTileAdjNT;
   return plan_tiles(inverse, n, J, L, esz, k);
 }
 
@@ -384,6 +433,7 @@ GroupLaunch launch_of(const Group& G, int64_t count) {
   gl.R = G.R;
   gl.NT = G.NT;
   gl.G = G.g;
+  gl.wide = G.wide;
   gl.count = count;
   gl.blocks = ((int64_t(1) << G.j0) / G.R) * G.nseg;
   return gl;
@@ -393,7 +443,7 @@ GroupLaunch launch_of(const Group& G, int64_t count) {
 template <typename T>
 int fwd_adj_t(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
               bool details, hipStream_t st) {
-  auto groups = adjoint_tiles(true, n, J, filter_length(filt), sizeof(T));
+  auto groups = adjoint_tiles(true, n, count, J, filter_length(filt), sizeof(T), details);
   const int64_t per = 2 * n * J;
   T* scratch = nullptr;
   if (groups.size() > 1) {
@@ -460,7 +510,7 @@ __global__ __launch_bounds__(256) void grad_sum_k(const double* __restrict__ par
 template <typename T>
 int inv_grad_t(const void* gy, const void* c, void* gc, bool zero_s, double* glam, int64_t n,
                int64_t count, int J, int filt, const wh_thresh* thr, hipStream_t st) {
-  auto groups = adjoint_tiles(false, n, J, filter_length(filt), sizeof(T));
+  auto groups = adjoint_tiles(false, n, count, J, filter_length(filt), sizeof(T), true);
   if (groups.size() > 8) return set_error(WH_ERR_UNSUPPORTED, "adjoint: too many level groups");
   GradArgs q{};
   q.gc = gc;
@@ -708,7 +758,8 @@ int modwt_tune(int64_t n, int J, int filt, int dtype, hipStream_t st) {
 
 int modwt_force_plan(bool inverse, int64_t n, int J, int filt, int dtype, int g1max,
                      int first_per_cu, int deep_per_cu, int first_nt) {
-  const KnobKey key{inverse ? 1 : 0, n, J, filt, dtype == WH_F32 ? 4 : 8};
+  const size_t key_esz = dtype == WH_F32 ? 4 : 8;
+  const KnobKey key{inverse ? 1 : 0, n, J, filt, int(key_esz)};
   std::lock_guard<std::mutex> lk(g_knob_mu);
   if (g1max <= 0) {
     g_knobs.erase(key);
@@ -716,7 +767,9 @@ int modwt_force_plan(bool inverse, int64_t n, int J, int filt, int dtype, int g1
   }
   if (g1max > kGmax || first_per_cu < 1 || deep_per_cu < 1 ||
       (std::abs(first_nt) != kNT1 && std::abs(first_nt) != kNT1 / 2) ||
-      (!inverse && first_nt == kNT1 / 2) || (first_nt < 0 && (g1max < 3 || g1max > kTileGmax)))
+      (!inverse && first_nt == kNT1 / 2) || (first_nt < 0 && g1max < 3) ||
+      (first_nt < 0 && g1max > kTileGmax &&
+       !(inverse && first_nt == -kWideInvNT && wide_fits(kWideInvP, n, J, key_esz))))
     return set_error(WH_ERR_ARG, "modwt plan: knobs out of range");
   PlanKnobs k;
   k.g1max = g1max;

@@ -972,6 +972,7 @@ struct GroupLaunch {
   int R, NT, G;
   int map;  // R = 1 element mapping: 0 adjacent pairs, 1 two outputs of one residue class (set by the planner), 2 the same with linear buffers (inverse)
   int sp;   // forward store policy (kStoreAll, kStoreSmooth or kStoreAdjoint)
+  bool wide;  // modwt_tile.h's wide tiles
   int64_t blocks;
   int64_t count;  // signals (grid y)
   size_t lds;

@@ -154,6 +154,40 @@ __global__ __launch_bounds__(NT) void modwt_fwd_tile_k(ModwtArgs args) {
 // if asked for); without it the kernel writes nothing but its hand-off and
 // partials: 512 x 2^14 FP32, J = 8, LA8 took a pass that stored the 2nJ
 // cotangents (102 us) and one that read them back beside c (108 us).
+// the cotangent g of a detail through its threshold t (act: the level is
+// thresholded) at coefficient v, and dL/dt added to sum
+template <typename T>
+__device__ __forceinline__ T grad_cut(const GradArgs& q, T g, T v, T t, bool act, double& sum) {
+  if (!act) return g;
+  const T m = fabs(v);
+  if (q.hardness == kSOFT) {
+    const bool pass = m > t;
+    if (pass) sum += double(v < T(0) ? g : -g);
+    return pass ? g : T(0);
+  }
+  return m < t ? T(0) : g;
+}
+
+// the workgroup's sums of levels j0..j0+G-1 into its partials
+template <int G, int NT>
+__device__ __forceinline__ void grad_partials(double* acc, double (*red)[NT / 64], int j0,
+                                              const GradArgs& q) {
+#pragma unroll
+  for (int l = 0; l < G; ++l) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc[l] += __shfl_xor(acc[l], o, 64);
+    if ((threadIdx.x & 63) == 0) red[l][threadIdx.x >> 6] = acc[l];
+  }
+  __syncthreads();
+  if (threadIdx.x < G) {
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) sum += red[threadIdx.x][w];
+    q.partial[((j0 + int64_t(threadIdx.x)) * gridDim.y + blockIdx.y) * q.per_signal + blockIdx.x] =
+        sum;
+  }
+}
+
 template <typename T, int FILT, int R, int G, int NT>
 struct GradTile {
   using F = FwdTile<T, FILT, R, G, NT, kStoreAll>;
@@ -162,19 +196,6 @@ struct GradTile {
   static constexpr int kWaves = NT / 64;
   T c[G][KO];
   double acc[G];
-
-  // c of level l and the threshold's gradient there; the owned outputs come
-  // first in every level's order, so output k < KO of a thread is owned
-  __device__ __forceinline__ T apply(const GradArgs& q, int l, int k, T g, T t, bool act) {
-    if (!act) return g;
-    const T v = c[l - 1][k], m = fabs(v);
-    if (q.hardness == kSOFT) {
-      const bool pass = m > t;
-      if (pass) acc[l - 1] += double(v < T(0) ? g : -g);
-      return pass ? g : T(0);
-    }
-    return m < t ? T(0) : g;
-  }
 
   template <int l>
   __device__ __forceinline__ void levels(T* b0, T* b1, const ModwtArgs& a, const GradArgs& q,
@@ -199,8 +220,9 @@ struct GradTile {
           for (int j = 0; j < L; ++j) w[j] = in[o + j * s * R];
           analysis1<T, FILT>(w, S, D);
           if constexpr (l < G) nxt[o] = S;
+          // the owned outputs come first in every level's order
           if (k < KO && o / R < qmax) {
-            const T g = apply(q, l, k < KO ? k : 0, D * sc, t, act);
+            const T g = grad_cut(q, D * sc, c[l - 1][k < KO ? k : 0], t, act, acc[l - 1]);
             const int64_t i = base + (o % R) + (int64_t(o / R) << a.j0);
             if (oS) {
               oS[a.n + i] = g;
@@ -259,21 +281,7 @@ __global__ __launch_bounds__(NT) void modwt_grad_tile_k(ModwtArgs args, GradArgs
   __syncthreads();
   T* gc = q.gc ? static_cast<T*>(q.gc) + int64_t(blockIdx.y) * a.bs_xmod : nullptr;
   c.template levels<1>(lds, lds + F::N0, a, q, gc, r0 + (m0 << a.j0), Nm - m0);
-  if (!q.partial) return;
-#pragma unroll
-  for (int l = 0; l < G; ++l) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) c.acc[l] += __shfl_xor(c.acc[l], o, 64);
-    if ((threadIdx.x & 63) == 0) red[l][threadIdx.x >> 6] = c.acc[l];
-  }
-  __syncthreads();
-  if (threadIdx.x < G) {
-    double sum = 0.0;
-#pragma unroll
-    for (int w = 0; w < C::kWaves; ++w) sum += red[threadIdx.x][w];
-    q.partial[((a.j0 + int64_t(threadIdx.x)) * gridDim.y + blockIdx.y) * q.per_signal +
-              blockIdx.x] = sum;
-  }
+  if (q.partial) grad_partials<G, NT>(c.acc, red, a.j0, q);
 }
 
 // ---------------------------------------------------------------- inverse
@@ -420,6 +428,219 @@ __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
                        Nm - m0);
 }
 
+// ------------------------------------------------------------ wide tiles
+// FP32 launches that fill the chip many times over: all J <= 8 levels in one
+// group of one launch (no hand-off between groups, whole runs of one
+// position per lane), so the halo of the whole cascade -- 1785 positions for
+// LA8 at J = 8 -- is carried by tiles of 2048 (inverse) or 4096 (gradient)
+// positions.  One buffer serves every level: a level's outputs are held in
+// registers over a barrier and written back over its inputs, which leaves
+// LDS for several workgroups per CU, and only the next kWideAhead levels'
+// arrays are in flight, which leaves registers for them.  LA8, J = 8,
+// 512 x 2^14: inverse 147 us as one sliding group (one 80 KB workgroup per
+// CU) -> 92 (302 MB read; 256 threads x 8 outputs; 512 x 4 takes 100, 1024 x
+// 2 112); gradient in two tile groups 148 -> 85.  In FP64 the same kernels
+// need all 256 registers (252 us against 191 sliding), so they are not built.
+constexpr int kWideInvNT = 256, kWideInvPer = 8, kWideInvAhead = 3;
+constexpr int kWideGradNT = 512, kWideGradPer = 8, kWideGradAhead = 2;
+constexpr int kWideGmin = 3, kWideGmax = 8;
+constexpr int kWideInvP = kWideInvNT * kWideInvPer;     // positions per tile
+constexpr int kWideGradP = kWideGradNT * kWideGradPer;
+
+template <typename T, int FILT, int G, int MODE>
+struct InvWide {
+  using V = typename Vec2<T>::type;
+  static constexpr int L = Filter<FILT>::L, NT = kWideInvNT;
+  static constexpr int cnt(int l) { return kWideInvP + tile_halo(L, l); }  // slots of level l
+  static constexpr int K(int l) { return (cnt(l) + NT - 1) / NT; }
+  T d[G + 1][K(G)];
+
+  template <int l>
+  static __device__ __forceinline__ int64_t gidx(const ModwtArgs& a, int64_t m0, int k) {
+    const int e = int(threadIdx.x) + k * NT;
+    return (m0 - tile_halo(L, l) + (e < cnt(l) ? e : cnt(l) - 1)) & (a.n - 1);
+  }
+  template <int l>
+  __device__ __forceinline__ void load(const ModwtArgs& a, int64_t m0) {
+    if constexpr (l >= 1) {
+      const T* D = static_cast<const T*>(a.xmod) + 2 * a.n * int64_t(l - 1) + a.n;
+#pragma unroll
+      for (int k = 0; k < K(l); ++k) d[l][k] = __builtin_nontemporal_load(D + gidx<l>(a, m0, k));
+    }
+  }
+  template <int l, int left>
+  __device__ __forceinline__ void load_ahead(const ModwtArgs& a, int64_t m0) {
+    if constexpr (left > 0) {
+      load<l>(a, m0);
+      load_ahead<l - 1, left - 1>(a, m0);
+    }
+  }
+  template <int l>
+  __device__ __forceinline__ void levels(V* b, const ModwtArgs& a, int64_t m0) {
+    if constexpr (l >= 1) {
+      load<l - kWideInvAhead>(a, m0);
+      constexpr int s = 1 << (l - 1), no = cnt(l - 1), ko = K(l - 1);
+      T e[ko];
+#pragma unroll
+      for (int k = 0; k < ko; ++k) {
+        const int o = int(threadIdx.x) + k * NT;
+        if (o < no) {
+          T ws[L], wd[L];
+#pragma unroll
+          for (int j = 0; j < L; ++j) {
+            const V v = b[o + j * s];
+            ws[j] = v.x;
+            wd[j] = v.y;
+          }
+          if constexpr (MODE == kInverse) e[k] = synthesis<T, FILT>(ws, wd, L - 1);
+          else e[k] = adjoint1<T, FILT>(ws, wd, T(0));
+        }
+      }
+      if constexpr (l > 1) {
+        const T t = MODE == kInverse ? InvTile<T, FILT, 1, G, NT, MODE>::thr(a, l - 1) : T(-1);
+        __syncthreads();  // every tap of this level read before any is replaced
+#pragma unroll
+        for (int k = 0; k < ko; ++k) {
+          const int o = int(threadIdx.x) + k * NT;
+          T c = d[l - 1][k];
+          if (MODE == kInverse && t >= T(0)) c = thresh_coef(c, t, a.hardness);
+          if (o < no) b[o] = V{e[k], c};
+        }
+        __syncthreads();
+      } else {
+        T* out = static_cast<T*>(a.out);
+#pragma unroll
+        for (int k = 0; k < ko; ++k) out[m0 + threadIdx.x + k * NT] = e[k];
+      }
+      levels<l - 1>(b, a, m0);
+    }
+  }
+};
+
+// n is a multiple of kWideInvP
+template <typename T, int FILT, int G, int MODE>
+__global__ __launch_bounds__(kWideInvNT) void modwt_inv_wide_k(ModwtArgs args) {
+  using C = InvWide<T, FILT, G, MODE>;
+  using V = typename Vec2<T>::type;
+  __shared__ __align__(16) V lds[C::cnt(G)];
+  const ModwtArgs a = batch_slice<T>(args);
+  const int64_t m0 = tile_index(blockIdx.x, gridDim.x) * kWideInvP;
+  C c;
+  T sg[C::K(G)];
+#pragma unroll
+  for (int k = 0; k < C::K(G); ++k)
+    sg[k] = static_cast<const T*>(a.stop)[C::template gidx<G>(a, m0, k)];
+  c.template load_ahead<G, kWideInvAhead>(a, m0);
+  const T t = MODE == kInverse ? InvTile<T, FILT, 1, G, kWideInvNT, MODE>::thr(a, G) : T(-1);
+#pragma unroll
+  for (int k = 0; k < C::K(G); ++k) {
+    const int e = int(threadIdx.x) + k * kWideInvNT;
+    T d = c.d[G][k];
+    if (MODE == kInverse && t >= T(0)) d = thresh_coef(d, t, a.hardness);
+    if (e < C::cnt(G)) lds[e] = V{sg[k], d};
+  }
+  __syncthreads();
+  c.template levels<G>(lds, a, m0);
+}
+
+template <typename T, int FILT, int G>
+struct GradWide {
+  static constexpr int L = Filter<FILT>::L, NT = kWideGradNT, KO = kWideGradPer;
+  static constexpr int cnt(int l) { return kWideGradP + tile_halo(L, G) - tile_halo(L, l); }
+  T c[G + 1][KO];
+  double acc[G];
+
+  template <int l>
+  __device__ __forceinline__ void load(const ModwtArgs& a, const GradArgs& q, int64_t m0) {
+    if constexpr (l <= G) {
+      const T* D = static_cast<const T*>(a.xmod) + 2 * a.n * int64_t(l - 1) + a.n + m0;
+      const bool act = l - 1 >= q.minlevel && l - 1 <= q.maxlevel;
+#pragma unroll
+      for (int k = 0; k < KO; ++k)
+        c[l][k] = act ? __builtin_nontemporal_load(D + threadIdx.x + k * NT) : T(0);
+    }
+  }
+  template <int l, int left>
+  __device__ __forceinline__ void load_ahead(const ModwtArgs& a, const GradArgs& q, int64_t m0) {
+    if constexpr (left > 0) {
+      load<l>(a, q, m0);
+      load_ahead<l + 1, left - 1>(a, q, m0);
+    }
+  }
+  template <int l>
+  __device__ __forceinline__ void levels(T* b, const ModwtArgs& a, const GradArgs& q, T* gc,
+                                         int64_t m0) {
+    if constexpr (l <= G) {
+      load<l + kWideGradAhead>(a, q, m0);
+      constexpr int s = 1 << (l - 1), no = cnt(l), ko = (no + NT - 1) / NT;
+      constexpr T sc = T(1.0 / double(1 << l));
+      const bool act = l - 1 >= q.minlevel && l - 1 <= q.maxlevel;
+      const T t = !act ? T(0) : q.levels ? T(q.levels[l - 1]) : T(q.value);
+      T* oS = gc ? gc + 2 * a.n * int64_t(l - 1) + m0 : nullptr;
+      T S[ko];
+      double sum = 0.0;
+#pragma unroll
+      for (int k = 0; k < ko; ++k) {
+        const int o = int(threadIdx.x) + k * NT;
+        if (o < no) {
+          T w[L], D;
+#pragma unroll
+          for (int j = 0; j < L; ++j) w[j] = b[o + j * s];
+          analysis1<T, FILT>(w, S[k], D);
+          if (k < KO) {  // owned
+            const T g = grad_cut(q, D * sc, c[l][k < KO ? k : 0], t, act, sum);
+            if (oS) {
+              oS[a.n + o] = g;
+              if (l == G) oS[o] = S[k] * sc;
+              else if (q.zero_s) oS[o] = T(0);
+            }
+          }
+        }
+      }
+      acc[l - 1] = sum;
+      if constexpr (l < G) {
+        __syncthreads();  // every tap of this level read before any is replaced
+#pragma unroll
+        for (int k = 0; k < ko; ++k) {
+          const int o = int(threadIdx.x) + k * NT;
+          if (o < no) b[o] = S[k];
+        }
+        __syncthreads();
+      }
+      levels<l + 1>(b, a, q, gc, m0);
+    }
+  }
+};
+
+// n is a multiple of kWideGradP
+template <typename T, int FILT, int G>
+__global__ __launch_bounds__(kWideGradNT) void modwt_grad_wide_k(ModwtArgs args, GradArgs q) {
+  using C = GradWide<T, FILT, G>;
+  constexpr int NT = kWideGradNT, N0 = C::cnt(0), K = (N0 + NT - 1) / NT;
+  __shared__ __align__(16) T lds[N0];
+  __shared__ double red[G][NT / 64];
+  const ModwtArgs a = batch_slice<T>(args);
+  const int64_t m0 = tile_index(blockIdx.x, gridDim.x) * kWideGradP;
+  const T* __restrict__ in = static_cast<const T*>(a.in);
+  C c;
+  T v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    v[k] = in[(m0 + (e < N0 ? e : N0 - 1)) & (a.n - 1)];
+  }
+  c.template load_ahead<1, kWideGradAhead>(a, q, m0);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    if (e < N0) lds[e] = v[k];
+  }
+  __syncthreads();
+  T* gc = q.gc ? static_cast<T*>(q.gc) + int64_t(blockIdx.y) * a.bs_xmod : nullptr;
+  c.template levels<1>(lds, a, q, gc, m0);
+  if (q.partial) grad_partials<G, NT>(c.acc, red, 0, q);
+}
+
 // What a tile launch computes
 enum class TileOp { kForward, kForwardDetails, kInverse, kAdjFull, kAdjDetails, kGrad };
 
@@ -472,9 +693,35 @@ int tile_launch_f(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const Gr
   return set_error(WH_ERR_UNSUPPORTED, "modwt: unsupported tile shape");
 }
 
+template <typename T, int FILT, int G>
+int wide_launch_g(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const GradArgs& q,
+                  hipStream_t st) {
+  if constexpr (G > kWideGmax) {
+    return set_error(WH_ERR_UNSUPPORTED, "modwt: wide tile depth out of range");
+  } else {
+    if (gl.G != G) return wide_launch_g<T, FILT, G + 1>(op, gl, a, q, st);
+    const dim3 grid(unsigned(gl.blocks), unsigned(gl.count));
+    if (op == TileOp::kGrad)
+      hipLaunchKernelGGL((modwt_grad_wide_k<T, FILT, G>), grid, dim3(kWideGradNT), 0, st, a, q);
+    else if (op == TileOp::kInverse)
+      hipLaunchKernelGGL((modwt_inv_wide_k<T, FILT, G, kInverse>), grid, dim3(kWideInvNT), 0, st,
+                         a);
+    else if (op == TileOp::kAdjDetails)
+      hipLaunchKernelGGL((modwt_inv_wide_k<T, FILT, G, kAdjDetails>), grid, dim3(kWideInvNT), 0,
+                         st, a);
+    else
+      return set_error(WH_ERR_UNSUPPORTED, "modwt: no such wide tile");
+    WH_HIP_CHECK(hipGetLastError());
+    return WH_OK;
+  }
+}
+
 template <typename T, int FILT>
 int tile_launch(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const GradArgs& q,
                 hipStream_t st) {
+  if constexpr (sizeof(T) == 4) {
+    if (gl.wide) return wide_launch_g<T, FILT, kWideGmin>(op, gl, a, q, st);
+  }
   const bool inv = op == TileOp::kInverse || op == TileOp::kAdjFull || op == TileOp::kAdjDetails;
   return inv ? tile_launch_f<T, FILT, true>(op, gl, a, q, st)
              : tile_launch_f<T, FILT, false>(op, gl, a, q, st);

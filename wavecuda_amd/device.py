@@ -194,7 +194,8 @@ def modwt_plan_candidates(inverse: bool, n: int, nlevels: int, filter="LA8",
     (the tuner's search space: deepest first group min(J, 5)..10, segments
     per CU of the first group 1/2/4 and of deeper groups 1/2/4/8, for the
     inverse a 256-thread first group, and tiles of 512 or 256 threads and
-    3..6 levels).  Leaves the default rules in force."""
+    3..6 levels, and for FP32 inverses of 3..8 levels one wide tile).
+    Leaves the default rules in force."""
     f = filter_code(filter)
     J = resolve_levels(n, nlevels, f)
     out = {}
@@ -202,6 +203,8 @@ def modwt_plan_candidates(inverse: bool, n: int, nlevels: int, filter="LA8",
         knobs = [(g1, fp, dp, nt) for nt in ((512, 256) if inverse else (512,))
                  for g1 in range(min(J, 5), 11) for fp in (1, 2, 4) for dp in (1, 2, 4, 8)]
         knobs += [(g1, 1, 1, -nt) for nt in (512, 256) for g1 in range(3, 7)]
+        if inverse and dtype == torch.float32 and 3 <= J <= 8 and n >= 2048:
+            knobs.append((8, 1, 1, -256))
         for k in knobs:
             modwt_set_plan(inverse, n, J, f, dtype, k)
             out.setdefault(modwt_plan(inverse, n, J, f, dtype), k)
