@@ -20,6 +20,7 @@ import numpy as np
 import torch
 
 from . import _lib as W
+from .device import _stream
 
 
 def _dtype_code(dtype) -> int:
@@ -28,10 +29,6 @@ def _dtype_code(dtype) -> int:
     if dtype == torch.float32:
         return W.WH_F32
     raise W.WaveHipError(f"unsupported dtype {dtype}")
-
-
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def _ptr(t):

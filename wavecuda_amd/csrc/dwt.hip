@@ -26,7 +26,6 @@
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
-#include <vector>
 
 #include "dwt_dev.h"
 #include "wh_common.h"
@@ -668,31 +667,28 @@ struct Pass {
   int64_t N;
 };
 
-// Largest compact length finished by one workgroup: its LDS (2.5 N values
-// for the inverse) must fit the budget, and the one workgroup's serial walk
-// must stay short (kWholeWork, with kTile: a tile pass of one or two
-// workgroups is cheaper than one workgroup over more values).
+// Largest compact length finished by one workgroup: the one workgroup's
+// serial walk must stay short (a tile pass of one or two workgroups is cheaper
+// than one workgroup over more values).  Its LDS, 2.5 N values for the
+// inverse, is within what every launch may have.
+static_assert(kWholeWork >= kTile, "a tile pass covers at least two tiles");
+static_assert(kWholeWork * 5 / 2 * sizeof(double) <= 64 * 1024, "whole kernels' dynamic LDS");
 
-template <typename T>
-int64_t whole_max() {
-  const size_t budget = std::min<size_t>(device_info().max_lds_per_block, 160 * 1024);
-  int64_t m = 1;
-  while (m * 2 <= kWholeWork && size_t(5 * m) * sizeof(T) <= budget) m *= 2;
-  return m;
-}
+// the passes of a transform: at most one per level
+struct Passes {
+  Pass p[64];
+  int count = 0;
+  void push_back(const Pass& x) { p[count++] = x; }
+  const Pass* begin() const { return p; }
+  const Pass* end() const { return p + count; }
+};
 
-template <typename KERN>
-void allow_big_lds(KERN kern) {
-  allow_dynamic_lds(reinterpret_cast<const void*>(kern));
-}
-
-template <typename T>
-std::vector<Pass> plan_passes(int64_t n, int J) {
-  std::vector<Pass> ps;
+Passes plan_passes(int64_t n, int J) {
+  Passes ps;
   int j0 = 0;
   int64_t N = n;
   while (j0 < J) {
-    if (N <= whole_max<T>() || N < int64_t(kTile)) {
+    if (N <= kWholeWork) {
       ps.push_back({true, j0, J - j0, N});
       break;
     }
@@ -731,18 +727,18 @@ int by_tile(int64_t N, int64_t count, FN fn) {
 // whose first pass reads the halos of neighbouring tiles.
 template <typename T>
 int dwt_scratch(const void* in, const void* out, int64_t n, int64_t count,
-                const std::vector<Pass>& ps, hipStream_t st, const T** src, T** comp) {
+                const Passes& ps, hipStream_t st, const T** src, T** comp) {
   *src = static_cast<const T*>(in);
   *comp = nullptr;
   void* p = nullptr;
-  if (in == out && !ps.front().whole) {
+  if (in == out && !ps.p[0].whole) {
     const size_t bytes = size_t(n) * size_t(count) * sizeof(T);
     int rc = scratch2_get(bytes, &p);
     if (rc) return rc;
     WH_HIP_CHECK(hipMemcpyAsync(p, in, bytes, hipMemcpyDeviceToDevice, st));
     *src = static_cast<const T*>(p);
   }
-  if (ps.size() > 1) {
+  if (ps.count > 1) {
     int rc = scratch_get(size_t(n >> kGmax) * size_t(count) * 2 * sizeof(T) + 64, &p);
     if (rc) return rc;
     *comp = static_cast<T*>(p);
@@ -752,7 +748,7 @@ int dwt_scratch(const void* in, const void* out, int64_t n, int64_t count,
 
 template <typename T, int FILT>
 int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream_t st) {
-  auto ps = plan_passes<T>(n, J);
+  auto ps = plan_passes(n, J);
   const T* src = nullptr;
   T* comp = nullptr;
   int rc = dwt_scratch<T>(x, y, n, count, ps, st, &src, &comp);
@@ -771,7 +767,6 @@ int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream
       a.j0 = P.j0;
       a.J = J;
       size_t lds = size_t(P.N + P.N / 2) * sizeof(T);
-      allow_big_lds(dwt_fwd_whole<T, FILT>);
       hipLaunchKernelGGL((dwt_fwd_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
@@ -808,7 +803,7 @@ int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream
 template <typename T, int FILT>
 int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const wh_thresh* thr,
               hipStream_t st, const Candidates& c) {
-  auto ps = plan_passes<T>(n, J);
+  auto ps = plan_passes(n, J);
   const T* y = nullptr;
   T* comp = nullptr;
   int rc = dwt_scratch<T>(yin, x, n, count, ps, st, &y, &comp);
@@ -819,8 +814,8 @@ int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const w
   const int64_t bc = n >> kGmax;
   const T* src = nullptr;  // compact s handed down between passes
   int slot = 0;
-  for (int pi = int(ps.size()) - 1; pi >= 0; --pi) {
-    const Pass& P = ps[pi];
+  for (int pi = ps.count - 1; pi >= 0; --pi) {
+    const Pass& P = ps.p[pi];
     T* out = (P.j0 == 0) ? static_cast<T*>(x) : comp + slot * bc * count;
     const int64_t bs_out = (P.j0 == 0) ? n : bc;
     if (P.whole) {
@@ -834,7 +829,6 @@ int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const w
       a.J = J;
       a.thr = th;
       size_t lds = size_t(2 * P.N + P.N / 2) * sizeof(T);
-      allow_big_lds(dwt_inv_whole<T, FILT>);
       hipLaunchKernelGGL((dwt_inv_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
