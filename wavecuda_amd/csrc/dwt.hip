@@ -75,22 +75,27 @@ struct Thr {
   int on, hardness, minlevel, maxlevel;
   double value;
   const double* levels;
-  // candidates of `of` inputs (of > 0), as ModwtArgs
-  int of;
-  int64_t th_stride;
 };
-
-// the input that signal y of an inverse reads, and its thresholds
-__device__ __forceinline__ int thr_input(Thr& t, int y) {
-  if (t.of <= 0) return y;
-  if (t.levels) t.levels += (y / t.of) * t.th_stride;
-  return y % t.of;
-}
 
 template <typename T>
 __device__ __forceinline__ T thr_level(const Thr& t, int lev0) {
   if (!t.on || lev0 < t.minlevel || lev0 > t.maxlevel) return T(-1);
   return t.levels ? T(t.levels[lev0]) : T(t.value);
+}
+
+// The signals of a launch (blockIdx.y) lie n apart, their compact sequences
+// n >> kGmax apart; the candidates of an inverse (blockIdx.z: the same
+// signals at other thresholds, kCandLevels apart) follow one another.  The
+// tile kernels of one signal (MANY false) leave all of this out: the scalar
+// work before a workgroup's first load cost the 2^24-sample transform 1.5 %.
+__device__ __forceinline__ int64_t sig_dist(int64_t n, int j0) { return j0 == 0 ? n : n >> kGmax; }
+__device__ __forceinline__ int64_t sig_slot() {
+  return int64_t(blockIdx.z) * gridDim.y + blockIdx.y;
+}
+__device__ __forceinline__ Thr cand_thr(const Thr& t) {
+  Thr r = t;
+  if (r.levels) r.levels += blockIdx.z * kCandLevels;
+  return r;
 }
 
 struct TileArgs {
@@ -103,14 +108,11 @@ struct TileArgs {
   int final_pass;    // fwd: s_{j0+g} = s_J goes to y
   int write_coarse;  // fwd: write y[q] with ctz >= g (first pass only)
   int src_shift;
-  int src_in;        // inv: src holds the inputs (the top pass), not one entry per signal
   Thr thr;
-  // elements between the signals of a launch (blockIdx.y)
-  int64_t bs_src, bs_y, bs_dst;
 };
 
 // ------------------------------------------------------------ forward tile
-template <typename T, int FILT, int TILE>
+template <typename T, int FILT, int TILE, bool MANY>
 __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
   constexpr int L = Filter<FILT>::L;
   constexpr int HMAX = halo_fwd(kGmax, L);
@@ -133,9 +135,9 @@ __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
   const int tid = threadIdx.x;
   const int g = a.g;
   const int64_t N = a.N;
-  const int64_t sig = blockIdx.y;
-  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * a.bs_src;
-  T* __restrict__ y = static_cast<T*>(a.y) + sig * a.bs_y;
+  const int64_t sig = MANY ? blockIdx.y : 0;
+  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * sig_dist(a.n, a.j0);
+  T* __restrict__ y = static_cast<T*>(a.y) + sig * a.n;
 
   const int64_t base = int64_t(blockIdx.x) * TILE;
   const int K0 = TILE + halo_fwd(g, L);
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
     }
   }
   if (!a.final_pass) {
-    T* __restrict__ dst = static_cast<T*>(a.dst) + sig * a.bs_dst;
+    T* __restrict__ dst = static_cast<T*>(a.dst) + sig * (a.n >> kGmax);
     const int own = TILE >> g;
     for (int i = tid; i < own; i += kNT) dst[(base >> g) + i] = cur[i];
   }
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(kNT) void dwt_fwd_tile(TileArgs a) {
 //      barrier), level 1 too: s_1 and d_1 sit side by side there, one
 //      16-byte read a tap, and its outputs go straight to memory.
 // 25 KB of LDS in FP64 with LA8: six workgroups per CU.
-template <typename T, int FILT, int TILE>
+template <typename T, int FILT, int TILE, bool MANY>
 __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
   constexpr int L = Filter<FILT>::L;
   constexpr int PADS = 8;
@@ -272,11 +274,13 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
   const int g = a.g, j0 = a.j0;
   const int64_t N = a.N;
   const int64_t base = int64_t(blockIdx.x) * TILE;
-  const int64_t sig = blockIdx.y;
-  Thr thr = a.thr;
-  const int64_t inp = thr_input(thr, int(blockIdx.y));
-  const T* __restrict__ src = static_cast<const T*>(a.src) + (a.src_in ? inp : sig) * a.bs_src;
-  const T* __restrict__ y = static_cast<const T*>(a.y) + inp * a.bs_y;
+  const Thr thr = MANY ? cand_thr(a.thr) : a.thr;
+  const int64_t inp = MANY ? int64_t(blockIdx.y) * a.n : 0;
+  const int64_t slot = MANY ? sig_slot() : 0;
+  // the top pass reads s_J out of y, the others their own compact sequence
+  const T* __restrict__ src =
+      static_cast<const T*>(a.src) + (a.src_shift ? inp : slot * (a.n >> kGmax));
+  const T* __restrict__ y = static_cast<const T*>(a.y) + inp;
 
   auto evn = [](int l) { return inv_evn(l, L); };
   auto doff = [](int l) { return (TILE / 4 - (TILE >> (l - 1))) + PADS * (l - 3); };
@@ -517,7 +521,7 @@ __global__ __launch_bounds__(kNT) void dwt_inv_tile(TileArgs a) {
     const int npairs = TILE / 2;  // e_0 = 0
     const int off = evn(1);
     const T t = thr_level<T>(thr, j0);
-    T* __restrict__ dst = static_cast<T*>(a.dst) + sig * a.bs_dst;
+    T* __restrict__ dst = static_cast<T*>(a.dst) + slot * sig_dist(a.n, j0);
     E2 res[kPairs];
 #pragma unroll
     for (int k = 0; k < kPairs; ++k) {
@@ -551,7 +555,6 @@ struct WholeArgs {
   int64_t N;        // compact length at level j0
   int j0, J;
   Thr thr;
-  int64_t bs_src, bs_y, bs_dst;  // as in TileArgs
 };
 
 template <typename T, int FILT>
@@ -561,8 +564,9 @@ __global__ __launch_bounds__(kNTW) void dwt_fwd_whole(WholeArgs a) {
   T* A = reinterpret_cast<T*>(smem_raw);
   T* B = A + a.N;
   const int tid = threadIdx.x;
-  const T* __restrict__ src = static_cast<const T*>(a.src) + int64_t(blockIdx.x) * a.bs_src;
-  T* __restrict__ y = static_cast<T*>(a.y) + int64_t(blockIdx.x) * a.bs_y;
+  const int64_t n = a.N << a.j0, sig = blockIdx.y;
+  const T* __restrict__ src = static_cast<const T*>(a.src) + sig * sig_dist(n, a.j0);
+  T* __restrict__ y = static_cast<T*>(a.y) + sig * n;
   const int N = int(a.N);
   for (int i = tid; i < N; i += kNTW) A[i] = src[i];
   __syncthreads();
@@ -598,10 +602,10 @@ __global__ __launch_bounds__(kNTW) void dwt_inv_whole(WholeArgs a) {
   T* B = A + a.N;
   T* Cf = B + a.N / 2;  // the N coefficients of levels j0+1..J, thresholded
   const int tid = threadIdx.x;
-  Thr thr = a.thr;
-  const int64_t inp = thr_input(thr, int(blockIdx.x));
-  const T* __restrict__ y = static_cast<const T*>(a.src) + inp * a.bs_src;
-  T* __restrict__ dst = static_cast<T*>(a.dst) + int64_t(blockIdx.x) * a.bs_dst;
+  const Thr thr = cand_thr(a.thr);
+  const int64_t n = a.N << a.j0;
+  const T* __restrict__ y = static_cast<const T*>(a.src) + int64_t(blockIdx.y) * n;
+  T* __restrict__ dst = static_cast<T*>(a.dst) + sig_slot() * sig_dist(n, a.j0);
   const int N = int(a.N);
   const int j0 = a.j0, J = a.J;
   // The level-j0 sequence y[q 2^j0], q < N, holds every coefficient the
@@ -715,11 +719,15 @@ Thr thr_of(const wh_thresh* t) {
 
 // Tile size of a pass over N values of each of `count` signals: by the
 // values of the whole launch, since it is the grid that must fill the chip.
+// fn(tile size, whether there is more than one signal)
 template <typename FN>
 int by_tile(int64_t N, int64_t count, FN fn) {
-  if (N * count >= kBigTileN) return fn(std::integral_constant<int, kTile>{});
-  if (N * count >= kSmallTileN) return fn(std::integral_constant<int, kTileSmall>{});
-  return fn(std::integral_constant<int, kTileTiny>{});
+  auto many = [&](auto tile) {
+    return count > 1 ? fn(tile, std::true_type{}) : fn(tile, std::false_type{});
+  };
+  if (N * count >= kBigTileN) return many(std::integral_constant<int, kTile>{});
+  if (N * count >= kSmallTileN) return many(std::integral_constant<int, kTileSmall>{});
+  return many(std::integral_constant<int, kTileTiny>{});
 }
 
 // Scratch of `count` signals: the compact sequences handed between passes
@@ -754,46 +762,39 @@ int dwt_fwd_f(const void* x, void* y, int64_t n, int64_t count, int J, hipStream
   int rc = dwt_scratch<T>(x, y, n, count, ps, st, &src, &comp);
   if (rc) return rc;
   const int64_t bc = n >> kGmax;  // signals' distance in the compact scratch
-  int64_t bs_src = n;
   int slot = 0;
   for (const Pass& P : ps) {
     if (P.whole) {
       WholeArgs a{};
       a.src = src;
-      a.bs_src = bs_src;
       a.y = y;
-      a.bs_y = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.J = J;
       size_t lds = size_t(P.N + P.N / 2) * sizeof(T);
-      hipLaunchKernelGGL((dwt_fwd_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
+      hipLaunchKernelGGL((dwt_fwd_whole<T, FILT>), dim3(1, unsigned(count)), dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
       TileArgs a{};
       a.src = src;
-      a.bs_src = bs_src;
       a.y = y;
-      a.bs_y = n;
       T* out = comp + slot * bc * count;
       a.dst = out;
-      a.bs_dst = bc;
       a.n = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.g = P.g;
       a.final_pass = (P.j0 + P.g == J);
       a.write_coarse = (P.j0 == 0);
-      rc = by_tile(P.N, count, [&](auto tile) -> int {
+      rc = by_tile(P.N, count, [&](auto tile, auto many) -> int {
         constexpr int TILE = decltype(tile)::value;
-        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, TILE>),
+        hipLaunchKernelGGL((dwt_fwd_tile<T, FILT, TILE, decltype(many)::value>),
                            dim3(unsigned(P.N / TILE), unsigned(count)), dim3(kNT), 0, st, a);
         WH_HIP_CHECK(hipGetLastError());
         return WH_OK;
       });
       if (rc) return rc;
       src = out;
-      bs_src = bc;
       slot ^= 1;
     }
   }
@@ -806,51 +807,44 @@ int dwt_inv_f(const void* yin, void* x, int64_t n, int64_t count, int J, const w
   auto ps = plan_passes(n, J);
   const T* y = nullptr;
   T* comp = nullptr;
-  int rc = dwt_scratch<T>(yin, x, n, count, ps, st, &y, &comp);
+  int rc = dwt_scratch<T>(yin, x, n, count * c.count, ps, st, &y, &comp);
   if (rc) return rc;
-  Thr th = thr_of(thr);
-  th.of = c.of;
-  th.th_stride = c.th_stride;
+  const Thr th = thr_of(thr);
   const int64_t bc = n >> kGmax;
   const T* src = nullptr;  // compact s handed down between passes
   int slot = 0;
   for (int pi = ps.count - 1; pi >= 0; --pi) {
     const Pass& P = ps.p[pi];
-    T* out = (P.j0 == 0) ? static_cast<T*>(x) : comp + slot * bc * count;
-    const int64_t bs_out = (P.j0 == 0) ? n : bc;
+    T* out = (P.j0 == 0) ? static_cast<T*>(x) : comp + slot * bc * count * c.count;
     if (P.whole) {
       WholeArgs a{};
       a.src = y;
-      a.bs_src = n;
       a.dst = out;
-      a.bs_dst = bs_out;
       a.N = P.N;
       a.j0 = P.j0;
       a.J = J;
       a.thr = th;
       size_t lds = size_t(2 * P.N + P.N / 2) * sizeof(T);
-      hipLaunchKernelGGL((dwt_inv_whole<T, FILT>), dim3(unsigned(count)), dim3(kNTW), lds, st, a);
+      hipLaunchKernelGGL((dwt_inv_whole<T, FILT>), dim3(1, unsigned(count), unsigned(c.count)),
+                         dim3(kNTW), lds, st, a);
       WH_HIP_CHECK(hipGetLastError());
     } else {
       TileArgs a{};
       const bool top = (P.j0 + P.g == J);
       a.src = top ? static_cast<const void*>(y) : static_cast<const void*>(src);
-      a.bs_src = top ? n : bc;
-      a.src_in = top;
       a.src_shift = top ? J : 0;
       a.y = const_cast<T*>(y);
-      a.bs_y = n;
       a.dst = out;
-      a.bs_dst = bs_out;
       a.n = n;
       a.N = P.N;
       a.j0 = P.j0;
       a.g = P.g;
       a.thr = th;
-      rc = by_tile(P.N, count, [&](auto tile) -> int {
+      rc = by_tile(P.N, count * c.count, [&](auto tile, auto many) -> int {
         constexpr int TILE = decltype(tile)::value;
-        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, TILE>),
-                           dim3(unsigned(P.N / TILE), unsigned(count)), dim3(kNT), 0, st, a);
+        hipLaunchKernelGGL((dwt_inv_tile<T, FILT, TILE, decltype(many)::value>),
+                           dim3(unsigned(P.N / TILE), unsigned(count), unsigned(c.count)), dim3(kNT),
+                           0, st, a);
         WH_HIP_CHECK(hipGetLastError());
         return WH_OK;
       });

@@ -254,7 +254,7 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
 
 template <typename T>
 int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t count, int sp,
-           hipStream_t st) {
+           hipStream_t st, int cand = 1) {
   GroupLaunch gl;
   gl.R = G.R;
   gl.NT = G.NT;
@@ -262,6 +262,7 @@ int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t c
   gl.wide = G.wide;
   gl.sp = sp;
   gl.count = count;
+  gl.cand = unsigned(cand);
   gl.blocks = ((int64_t(1) << G.j0) / G.R) * G.nseg;
   gl.lds = G.lds;
   if (count < 1 || count > 65535) return set_error(WH_ERR_ARG, "modwt: signal count out of range");
@@ -357,8 +358,9 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
                 const wh_thresh* thr, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0,
                 const Candidates& c = Candidates{}) {
   const int L = filter_length(filt);
-  auto groups = plan_groups(true, n, J, L, sizeof(T), knobs_for(true, n, J, filt, sizeof(T), count),
-                            count);
+  const int64_t total = count * c.count;  // signals inverted
+  auto groups = plan_groups(true, n, J, L, sizeof(T), knobs_for(true, n, J, filt, sizeof(T), total),
+                            total);
   const int64_t per = 2 * n * J;
   // the S_{j0} handed between groups lives in library scratch, or in the
   // caller's workspace `ws` (2 n values per signal: two halves used
@@ -366,7 +368,7 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
   // reads it, so nothing needs clearing)
   T* scratch = nullptr;
   if (groups.size() > 1) {
-    const size_t need = 2 * size_t(n) * size_t(count) * sizeof(T);
+    const size_t need = 2 * size_t(n) * size_t(total) * sizeof(T);
     void* p = ws;
     if (ws) {
       if (need > ws_bytes) return set_error(WH_ERR_ARG, "modwt inverse: workspace too small");
@@ -377,7 +379,7 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
     scratch = static_cast<T*>(p);
   }
   const T* stop = static_cast<const T*>(xmod) + 2 * n * int64_t(J - 1);
-  int64_t bs_stop = per;
+  int64_t bs_stop = per, bs_stop_z = 0;
   for (int gi = int(groups.size()) - 1; gi >= 0; --gi) {
     const Group& G = groups[gi];
     ModwtArgs a = args_of(G, n);
@@ -385,12 +387,11 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
     a.bs_xmod = per;
     a.stop = stop;
     a.bs_stop = bs_stop;
-    T* dst = (G.j0 == 0) ? static_cast<T*>(x) : scratch + (gi & 1) * n * count;
+    T* dst = (G.j0 == 0) ? static_cast<T*>(x) : scratch + (gi & 1) * n * total;
     a.out = dst;
     a.bs_out = n;
-    a.of = c.of;
-    a.stop_of = c.of > 0 && gi + 1 == int(groups.size());
-    a.th_stride = c.th_stride;
+    a.bs_out_z = n * count;
+    a.bs_stop_z = bs_stop_z;
     if (thr && thr->enabled) {
       a.th_on = 1;
       a.hardness = thr->hardness;
@@ -399,10 +400,11 @@ int modwt_inv_t(const void* xmod, void* x, int64_t n, int64_t count, int J, int 
       a.th_value = thr->value;
       a.th_levels = thr->levels;
     }
-    int rc = launch<T>(true, filt, G, a, count, kStoreAll, st);
+    int rc = launch<T>(true, filt, G, a, count, kStoreAll, st, c.count);
     if (rc) return rc;
     stop = dst;
     bs_stop = n;
+    bs_stop_z = n * count;
   }
   return WH_OK;
 }

@@ -58,27 +58,21 @@ struct ModwtArgs {
   // signal batches: blockIdx.y selects the signal, offset by these strides
   // (elements) from in / xmod / stop / out
   int64_t bs_in, bs_xmod, bs_stop, bs_out;
-  // inverse of `of` inputs at several thresholds (of > 0): signal y reads
-  // input y % of and the thresholds th_levels + (y / of) th_stride;
-  // stop_of: the stop array holds the inputs, not one entry per signal
-  int of, stop_of;
-  int64_t th_stride;
+  // inverse at several thresholds: blockIdx.z selects the candidate, whose
+  // output and (between groups) stop are offset by these
+  int64_t bs_stop_z, bs_out_z;
 };
 
 // the arguments of the signal handled by this workgroup (blockIdx.y)
 template <typename T>
 __device__ __forceinline__ ModwtArgs batch_slice(const ModwtArgs& a) {
   ModwtArgs b = a;
-  const int64_t y = blockIdx.y;
-  int64_t yi = y;  // input
-  if (a.of > 0) {
-    yi = int(blockIdx.y) % a.of;
-    if (a.th_levels) b.th_levels = a.th_levels + (int(blockIdx.y) / a.of) * a.th_stride;
-  }
+  const int64_t y = blockIdx.y, z = blockIdx.z;
   b.in = static_cast<const T*>(a.in) + y * a.bs_in;
-  b.xmod = static_cast<T*>(a.xmod) + yi * a.bs_xmod;
-  b.stop = static_cast<const T*>(a.stop) + (a.stop_of ? yi : y) * a.bs_stop;
-  b.out = static_cast<T*>(a.out) + y * a.bs_out;
+  b.xmod = static_cast<T*>(a.xmod) + y * a.bs_xmod;
+  b.stop = static_cast<const T*>(a.stop) + y * a.bs_stop + z * a.bs_stop_z;
+  b.out = static_cast<T*>(a.out) + y * a.bs_out + z * a.bs_out_z;
+  if (a.th_levels) b.th_levels = a.th_levels + z * kCandLevels;
   return b;
 }
 
@@ -975,6 +969,7 @@ struct GroupLaunch {
   bool wide;  // modwt_tile.h's wide tiles
   int64_t blocks;
   int64_t count;  // signals (grid y)
+  unsigned cand = 1;  // candidates of each (grid z)
   size_t lds;
 };
 template <typename T, int FILT>

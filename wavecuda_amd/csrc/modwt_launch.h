@@ -16,7 +16,7 @@ inline void modwt_allow_lds(KERN kern) {
 
 template <typename T, int FILT, int R, int NT, int G>
 int modwt_launch_one(bool inverse, const GroupLaunch& gl, const ModwtArgs& a, hipStream_t st) {
-  const dim3 grid(unsigned(gl.blocks), unsigned(gl.count));
+  const dim3 grid(unsigned(gl.blocks), unsigned(gl.count), gl.cand);
   if (inverse) {
     constexpr int MAP = (R == 1) ? 2 : 0;
     auto kern = modwt_inv_k<T, FILT, R, NT, G, MAP>;
@@ -58,7 +58,7 @@ int modwt_launch_inv256(const GroupLaunch& gl, const ModwtArgs& a, hipStream_t s
     if (gl.G != G) return modwt_launch_inv256<T, FILT, G + 1>(gl, a, st);
     auto kern = modwt_inv_k<T, FILT, 1, 256, G, 2>;
     modwt_allow_lds(kern);
-    hipLaunchKernelGGL(kern, dim3(unsigned(gl.blocks), unsigned(gl.count)), dim3(256), gl.lds, st,
+    hipLaunchKernelGGL(kern, dim3(unsigned(gl.blocks), unsigned(gl.count), gl.cand), dim3(256), gl.lds, st,
                        a);
     WH_HIP_CHECK(hipGetLastError());
     return WH_OK;

@@ -657,7 +657,7 @@ int tile_launch_g(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const Gr
     return set_error(WH_ERR_UNSUPPORTED, "modwt: tile group depth out of range");
   } else {
     if (gl.G != G) return tile_launch_g<T, FILT, INV, R, NT, G + 1>(op, gl, a, q, st);
-    const dim3 grid(unsigned(gl.blocks), unsigned(gl.count));
+    const dim3 grid(unsigned(gl.blocks), unsigned(gl.count), gl.cand);
     if constexpr (INV) {
       if (op == TileOp::kInverse)
         hipLaunchKernelGGL((modwt_inv_tile_k<T, FILT, R, G, NT, kInverse>), grid, dim3(NT), 0, st,
@@ -700,7 +700,7 @@ int wide_launch_g(TileOp op, const GroupLaunch& gl, const ModwtArgs& a, const Gr
     return set_error(WH_ERR_UNSUPPORTED, "modwt: wide tile depth out of range");
   } else {
     if (gl.G != G) return wide_launch_g<T, FILT, G + 1>(op, gl, a, q, st);
-    const dim3 grid(unsigned(gl.blocks), unsigned(gl.count));
+    const dim3 grid(unsigned(gl.blocks), unsigned(gl.count), gl.cand);
     if (op == TileOp::kGrad)
       hipLaunchKernelGGL((modwt_grad_wide_k<T, FILT, G>), grid, dim3(kWideGradNT), 0, st, a, q);
     else if (op == TileOp::kInverse)

@@ -41,7 +41,7 @@ struct StatsBuf {
   double partial[kCvCandidates * kMaxPartials];
   double vals[16];
   double levels[64];
-  double cvlev[kCvCandidates * kCvLevels];  // a candidate's threshold of every level
+  double cvlev[kCvCandidates * kCandLevels];  // a candidate's threshold of every level
   CvState cv;
 };
 
@@ -219,11 +219,10 @@ int smooth(void* x, int64_t n, int J, int ttype, int filt, int dtype, int thresh
   cva.J = Jh;
   cva.tol = tol;
   cva.cand = cand;
-  Candidates halves;
-  halves.of = 2;
-  halves.th_stride = kCvLevels;
+  Candidates points;
+  points.count = cand;
   auto eval = [&]() -> int {
-    const int r = inv(ttype, We, ye, lenh, 2 * cand, Jh, filt, dtype, &th, st, halves);
+    const int r = inv(ttype, We, ye, lenh, 2, Jh, filt, dtype, &th, st, points);
     if (r) return r;
     // the error reduction's last block also advances the search
     return interp_mse(x, ye, yo, n, dtype, sb->partial, nullptr, st, cva);

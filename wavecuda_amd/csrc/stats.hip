@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256 * kCvCandidates) void sum_partials(const double
   if (!cv.cs) return;
   __syncthreads();
   for (int i = threadIdx.x; i < cv.J * kCvCandidates; i += blockDim.x)
-    cv.levels[(i / cv.J) * kCvLevels + i % cv.J] = pts[i / cv.J];
+    cv.levels[(i / cv.J) * kCandLevels + i % cv.J] = pts[i / cv.J];
 }
 
 int interp_mse(const void* xn, const void* ye, const void* yo, int64_t len, int dtype,

@@ -72,6 +72,9 @@ __host__ __device__ constexpr double gcoef(int k) {
   return (k & 1) ? -Filter<FILT>::c(Filter<FILT>::L - 1 - k) : Filter<FILT>::c(Filter<FILT>::L - 1 - k);
 }
 
+// distance of the per-level threshold arrays of an inverse's candidates
+constexpr int kCandLevels = 64;
+
 constexpr double kInvR2 = 0.70710678118654752440;
 constexpr double kHInvR2 = 0.35355339059327376220;
 

@@ -57,12 +57,11 @@ int noalloc_setup();
 // so it cannot surface in a later, unrelated call.
 void allow_dynamic_lds(const void* kern);
 
-// An inverse's `count` signals as count / of candidates of the same `of`
-// inputs (of > 0): signal y inverts input y % of with the per-level
-// thresholds levels + (y / of) th_stride.
+// An inverse of the same signals at `count` candidate thresholds: candidate
+// c uses the per-level thresholds levels + c kCandLevels, and its outputs
+// follow those of candidate c - 1.
 struct Candidates {
-  int of = 0;
-  int64_t th_stride = 0;
+  int count = 1;
 };
 
 // transform back ends (device pointers)

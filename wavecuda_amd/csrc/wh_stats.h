@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/wavehip.h"
+#include "wh_common.h"
 
 namespace wh {
 
@@ -56,7 +57,6 @@ constexpr int kMaxPartials = 1024;  // per candidate
 // errors m1, m2 at t1, t2, the loop count, which point the pending
 // evaluation is for (1: t1, 2: t2), evaluations consumed so far, and stop.
 constexpr int kCvCandidates = 3;  // points a round evaluates at once, at most
-constexpr int kCvLevels = 64;     // distance of the candidates' threshold arrays
 struct CvState {
   double t0, t1, t2, t3, m1, m2;
   int iter, pending, nevals, stop;
@@ -88,7 +88,7 @@ __device__ inline void cv_start(CvState* out, double t3, double* levels, int J) 
   cv_points(cs, p);
 #pragma unroll
   for (int c = 0; c < kCvCandidates; ++c)
-    for (int l = 0; l < J; ++l) levels[c * kCvLevels + l] = p[c];
+    for (int l = 0; l < J; ++l) levels[c * kCandLevels + l] = p[c];
 }
 
 // in-place threshold of `count` transformed signals (DWT: n apart, MODWT:
