@@ -360,8 +360,8 @@ int wh_smooth(void* x, int64_t n, int nlevels, int ttype, int filter, int dtype,
 
 /* ---- batched smoothing ------------------------------------------------ */
 
-/* Universal-threshold smoothing of many independent signals in one
-   persistent launch.  Replaces the reference's planned list API
+/* Universal-threshold smoothing of many independent signals in a fixed
+   sequence of launches.  Replaces the reference's planned list API
    RgpuTransformList (src/rfunctions.cu:139-154, a stub returning its first
    argument; R/rfunctions.R:614-643 commented GPUTransformList), and per
    signal computes exactly what the smoothing entry points do with threshtype
@@ -373,7 +373,7 @@ int wh_smooth(void* x, int64_t n, int nlevels, int ttype, int filter, int dtype,
    samples [off_i, off_i + lens[i]) with off_i = sum of the previous
    lengths.  Per signal: power-of-two length, filter 1..4, ttype 0 (DWT) or
    1 (MODWT), levels as RgpuSmooth's nlevels (0 = the reference's maximum;
-   the MODWT is fused in one group, so its depth must be <= 8).  hardness is
+   the MODWT runs as two groups of four levels, so its depth must be <= 8).  hardness is
    shared by the batch.  A plan owns its device tables, workspace and
    captured graph; calls on one plan must be ordered (one stream). */
 typedef struct wh_batch wh_batch;
@@ -398,9 +398,9 @@ int wh_batch_replay(wh_batch* plan, void* stream);
    tuning run (1) or the default rule (0). Any pointer may be NULL. */
 int wh_batch_info(const wh_batch* plan, int64_t* total, int* threads, int* workgroups,
                   int64_t* lds_bytes, int64_t* workspace_bytes, int* tuned);
-/* Diagnostics (no counterpart in the reference): set the plan's launch
-   shape as wh_batch_tune would -- threads per signal 128, 256 or 512 and
-   1..the resident maximum of workgroups -- growing the workspace if needed
+/* Diagnostics (no counterpart in the reference): set the shape of the
+   plan's persistent launch as wh_batch_tune would -- threads per signal 128,
+   256 or 512 and 1..the resident maximum of workgroups -- growing the workspace if needed
    and dropping a captured graph.  Results never depend on the shape; this
    lets a caller run and check every shape the tuner can pick. */
 int wh_debug_batch_set_shape(wh_batch* plan, int threads, int workgroups);

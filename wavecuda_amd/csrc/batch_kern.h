@@ -1,31 +1,28 @@
 // batch_kern.h -- device side of the batched smoothing pipeline.
 //
 // Thousands of independent signals of power-of-two lengths are smoothed
-// (forward transform -> hard/soft universal threshold -> inverse) by
-// persistent workgroups that take whole signals from a device work queue:
-// an atomic counter over an item list sorted longest-first, so the large
-// signals start first and the small ones fill the tail.  One launch serves
-// every transform, filter and length of the batch: each item dispatches to
-// a body specialised for its filter (and, for the MODWT, its depth, which is
-// the fused group depth), so the chunk geometry and tap arithmetic are
-// compile-time.  Every workgroup owns a slice of scratch for the
-// coefficients of the signal it is working on; nothing of the pipeline
-// returns to the host.
+// (forward transform -> hard/soft universal threshold -> inverse) by a fixed
+// sequence of launches, whatever their mix: the head tiles of every MODWT
+// signal (batch_tile.h), the persistent kernel below, and the MODWT's two
+// shrink passes.  The persistent workgroups take whole signals from a device
+// work queue: an atomic counter over an item list sorted longest-first, so
+// the large signals start first and the small ones fill the tail.
 //
-//   MODWT: the fused sliding-window forward (modwt_fwd_body) writes the J
-//   levels into scratch, block_mad takes the exact MAD of D_1 (the
-//   reference's univ_thresh(w, 0, 0): src/thresh.cpp:170-201,
-//   src/rfunctions.cu:82-87), and the fused inverse (modwt_inv_lin_body)
-//   thresholds every detail level as it reads it.
-//   DWT: levels run on compact sequences, through scratch while they are
-//   longer than the LDS tile and in LDS afterwards; the MAD is taken over
-//   the level-1 details (all of x[1..n-1] when J = 1, as in the reference)
-//   and the inverse thresholds the details as it reads them.
+//   MODWT: the item is the exact MAD of D_1 (the reference's univ_thresh(w,
+//   0, 0): src/thresh.cpp:170-201, src/rfunctions.cu:82-87), which the head
+//   left in the workspace.
+//   DWT: the whole smoothing.  Levels run on compact sequences, through the
+//   workgroup's slice of scratch while they are longer than the LDS tile and
+//   in LDS afterwards; the MAD is taken over the level-1 details (all of
+//   x[1..n-1] when J = 1, as in the reference) and the inverse thresholds
+//   the details as it reads them.
+//
+// Nothing of the pipeline returns to the host.
 #pragma once
 
+#include "batch_tile.h"
 #include "blocksel.h"
 #include "dwt_dev.h"
-#include "modwt_kern.h"
 
 namespace wh {
 
@@ -36,7 +33,7 @@ __host__ __device__ constexpr int kind_filter(int kind) { return kind & 7; }
 
 // One signal of the batch.
 struct BatchItem {
-  int64_t off;    // first sample in the packed signal buffers
+  int64_t off;    // first sample in the packed signal buffers (MODWT: D_1 in the tiles' workspace)
   double factor;  // sqrt(2 ln n) (sqrt(2 ln(n-1)) for a one-level DWT)
   int32_t n;      // length (power of two)
   int32_t J;      // levels
@@ -51,6 +48,8 @@ struct BatchArgs {
   const void* x;
   void* y;
   double* thresh_out;  // optional, one per signal
+  double* thresh;      // one per signal, for the shrink passes
+  const void* tiles;   // the MODWT tiles' workspace
   void* scratch;
   int64_t scratch_stride;  // elements per workgroup
   int hardness;
@@ -70,53 +69,6 @@ __device__ __forceinline__ int batch_next(int* counter, int* sh) {
 // write back and invalidate the L2 of the workgroup's XCD at every item.
 __device__ __forceinline__ void batch_phase() { __syncthreads(); }
 
-// MODWT item, forward: the fused forward of all J = G levels into scratch
-// (D_j and S_J).  Chunk width M = min(2 NT, n); the warm-up covers the
-// coarsest level's reach.
-template <typename T, int FILT, int NT, int G>
-__device__ __forceinline__ ModwtArgs batch_modwt_args(const BatchArgs& b, const BatchItem& I,
-                                                      T* scr) {
-  constexpr int L = Filter<FILT>::L;
-  const int64_t n = I.n;
-  ModwtArgs a{};
-  a.n = n;
-  a.P = n;
-  a.j0 = 0;
-  a.g = G;
-  a.M = int(n < 2 * NT ? n : 2 * NT);
-  const int64_t reach = int64_t(L - 1) * ((int64_t(1) << G) - 1);
-  a.warm = int((reach + a.M - 1) / a.M * a.M);
-  a.nchunks = int((n + a.warm) / a.M);
-  a.in = static_cast<const T*>(b.x) + I.off;
-  a.xmod = scr;
-  return a;
-}
-
-template <typename T, int FILT, int NT, int G>
-__device__ __forceinline__ void batch_modwt_fwd(const BatchArgs& b, const BatchItem& I, T* scr,
-                                                unsigned char* smem, unsigned* pre) {
-  const ModwtArgs a = batch_modwt_args<T, FILT, NT, G>(b, I, scr);
-  modwt_fwd_body<T, FILT, 1, NT, G, 0, kStoreSmoothHist>(a, 0, 0, smem, pre);
-}
-
-// MODWT item, inverse: the fused inverse into y, thresholding every detail
-// level at t as it reads it
-template <typename T, int FILT, int NT, int G>
-__device__ __forceinline__ void batch_modwt_inv(const BatchArgs& b, const BatchItem& I, T* scr,
-                                                unsigned char* smem, double t) {
-  ModwtArgs a = batch_modwt_args<T, FILT, NT, G>(b, I, scr);
-  const int64_t n = I.n;
-  a.stop = scr + 2 * n * (G - 1);
-  a.out = static_cast<T*>(b.y) + I.off;
-  a.th_on = 1;
-  a.hardness = b.hardness;
-  a.minlevel = 0;
-  a.maxlevel = G - 1;
-  a.th_value = t;
-  a.th_levels = nullptr;
-  modwt_inv_lin_body<T, FILT, NT, G>(a, 0, smem);
-}
-
 // LDS elements per ping-pong buffer of the DWT tail (64 KB in FP64, 32 KB
 // in FP32, so that several FP32 workgroups share a CU)
 template <typename T>
@@ -125,11 +77,10 @@ constexpr int batch_lds_elems() {
 }
 
 // FP64 512-thread workgroups keep a first-digit histogram of the median's
-// values (2048 counts) at this LDS offset, beyond the forward's rings (at
-// most 80 KB at J = 8), the DWT's LDS levels (64 KB) and the selection's
-// workspace; the plan sizes the launch's LDS to cover it.  Other shapes
+// values (2048 counts) at this LDS offset, beyond the DWT's LDS levels (64
+// KB) and the selection's workspace; the plan sizes the launch's LDS to cover it.  Other shapes
 // would need more LDS per workgroup than they have to spare.
-constexpr size_t kBatchPreOff = size_t(96) << 10;
+constexpr size_t kBatchPreOff = size_t(64) << 10;
 constexpr size_t kBatchPreEnd = kBatchPreOff + size_t(kSelBins) * 4;
 // LDS the histogram needs for NT threads and esz-byte elements (0: none)
 __host__ __device__ constexpr size_t batch_pre_lds(int NT, size_t esz) {
@@ -388,44 +339,6 @@ __device__ __forceinline__ void batch_dwt_inv(const BatchArgs& b, const BatchIte
   batch_phase();
 }
 
-template <typename T, int FILT, int NT>
-__device__ __forceinline__ void batch_fwd(const BatchArgs& b, const BatchItem& I, T* scr,
-                                          unsigned char* smem, unsigned* pre) {
-  if (kind_ttype(I.kind) == kDWT) {
-    batch_dwt_fwd<T, FILT, NT>(b, I, scr, smem, pre);
-    return;
-  }
-  switch (I.J) {
-    case 1: batch_modwt_fwd<T, FILT, NT, 1>(b, I, scr, smem, pre); break;
-    case 2: batch_modwt_fwd<T, FILT, NT, 2>(b, I, scr, smem, pre); break;
-    case 3: batch_modwt_fwd<T, FILT, NT, 3>(b, I, scr, smem, pre); break;
-    case 4: batch_modwt_fwd<T, FILT, NT, 4>(b, I, scr, smem, pre); break;
-    case 5: batch_modwt_fwd<T, FILT, NT, 5>(b, I, scr, smem, pre); break;
-    case 6: batch_modwt_fwd<T, FILT, NT, 6>(b, I, scr, smem, pre); break;
-    case 7: batch_modwt_fwd<T, FILT, NT, 7>(b, I, scr, smem, pre); break;
-    default: batch_modwt_fwd<T, FILT, NT, 8>(b, I, scr, smem, pre); break;
-  }
-}
-
-template <typename T, int FILT, int NT>
-__device__ __forceinline__ void batch_inv(const BatchArgs& b, const BatchItem& I, T* scr,
-                                          unsigned char* smem, double t) {
-  if (kind_ttype(I.kind) == kDWT) {
-    batch_dwt_inv<T, FILT, NT>(b, I, scr, smem, t);
-    return;
-  }
-  switch (I.J) {
-    case 1: batch_modwt_inv<T, FILT, NT, 1>(b, I, scr, smem, t); break;
-    case 2: batch_modwt_inv<T, FILT, NT, 2>(b, I, scr, smem, t); break;
-    case 3: batch_modwt_inv<T, FILT, NT, 3>(b, I, scr, smem, t); break;
-    case 4: batch_modwt_inv<T, FILT, NT, 4>(b, I, scr, smem, t); break;
-    case 5: batch_modwt_inv<T, FILT, NT, 5>(b, I, scr, smem, t); break;
-    case 6: batch_modwt_inv<T, FILT, NT, 6>(b, I, scr, smem, t); break;
-    case 7: batch_modwt_inv<T, FILT, NT, 7>(b, I, scr, smem, t); break;
-    default: batch_modwt_inv<T, FILT, NT, 8>(b, I, scr, smem, t); break;
-  }
-}
-
 // The persistent pipeline: every workgroup takes items until the queue is
 // empty; the last workgroup to leave rewinds the queue, so the launch can be
 // replayed (a captured graph) without a memset node.
@@ -446,32 +359,37 @@ __global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
     // selection leave free
     unsigned* pre = nullptr;
     if constexpr (batch_pre<T, NT>()) {
-      if (!(dwt && I.J == 1)) {
+      if (dwt && I.J != 1) {
         pre = reinterpret_cast<unsigned*>(smem + kBatchPreOff);
         for (int i = threadIdx.x; i < kSelBins; i += NT) pre[i] = 0;
         __syncthreads();
       }
     }
-    switch (kind_filter(I.kind)) {
-      case kHAAR: batch_fwd<T, kHAAR, NT>(b, I, scr, smem, pre); break;
-      case kD4: batch_fwd<T, kD4, NT>(b, I, scr, smem, pre); break;
-      case kC6: batch_fwd<T, kC6, NT>(b, I, scr, smem, pre); break;
-      default: batch_fwd<T, kLA8, NT>(b, I, scr, smem, pre); break;
+    if (dwt) {
+      switch (kind_filter(I.kind)) {
+        case kHAAR: batch_dwt_fwd<T, kHAAR, NT>(b, I, scr, smem, pre); break;
+        case kD4: batch_dwt_fwd<T, kD4, NT>(b, I, scr, smem, pre); break;
+        case kC6: batch_dwt_fwd<T, kC6, NT>(b, I, scr, smem, pre); break;
+        default: batch_dwt_fwd<T, kLA8, NT>(b, I, scr, smem, pre); break;
+      }
+      batch_phase();
     }
-    batch_phase();
     // the universal threshold from the level-1 details: one call site for
     // every kind of item, so the selection is inlined once (a called
     // function would keep its saved registers in scratch memory)
-    const int64_t moff = dwt ? 0 : n;
-    const int64_t mstride = 1;
+    const T* det = dwt ? scr : static_cast<const T*>(b.tiles) + I.off;
     const int64_t mcount = dwt ? (I.J == 1 ? n - 1 : n / 2) : n;
-    const double t = block_mad<T, NT>(scr, moff, mstride, mcount, smem, pre) * I.factor;
-    if (threadIdx.x == 0 && b.thresh_out) b.thresh_out[I.sig] = t;
+    const double t = block_mad<T, NT>(det, 0, 1, mcount, smem, pre) * I.factor;
+    if (threadIdx.x == 0) {
+      b.thresh[I.sig] = t;
+      if (b.thresh_out) b.thresh_out[I.sig] = t;
+    }
+    if (!dwt) continue;
     switch (kind_filter(I.kind)) {
-      case kHAAR: batch_inv<T, kHAAR, NT>(b, I, scr, smem, t); break;
-      case kD4: batch_inv<T, kD4, NT>(b, I, scr, smem, t); break;
-      case kC6: batch_inv<T, kC6, NT>(b, I, scr, smem, t); break;
-      default: batch_inv<T, kLA8, NT>(b, I, scr, smem, t); break;
+      case kHAAR: batch_dwt_inv<T, kHAAR, NT>(b, I, scr, smem, t); break;
+      case kD4: batch_dwt_inv<T, kD4, NT>(b, I, scr, smem, t); break;
+      case kC6: batch_dwt_inv<T, kC6, NT>(b, I, scr, smem, t); break;
+      default: batch_dwt_inv<T, kLA8, NT>(b, I, scr, smem, t); break;
     }
     batch_phase();
   }
@@ -484,15 +402,9 @@ __global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
   }
 }
 
-// largest MODWT depth of one batch item
-constexpr int kBatchMaxModwtJ = 8;
-
 // the first-digit histogram at kBatchPreOff stays clear of what an FP64
-// 512-thread item puts in LDS before its selection: the deepest forward's
-// rings (LA8, J = 8, chunks of 1024), the DWT's LDS levels and the
-// selection's workspace
-static_assert((kBatchMaxModwtJ * 1024 + fwd_win_sum(8, kBatchMaxModwtJ)) * 8 <= int(kBatchPreOff),
-              "forward rings overlap the first-digit histogram");
+// 512-thread item puts in LDS before its selection: the DWT's LDS levels and
+// the selection's workspace
 static_assert(2 * batch_lds_elems<double>() * 8 <= int(kBatchPreOff),
               "DWT LDS levels overlap the first-digit histogram");
 static_assert(block_sel_lds<512>() <= kBatchPreOff,

@@ -9,11 +9,21 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "batch_kern.h"
 #include "wh_common.h"
 #include "wh_internal.h"
+
+namespace wh {
+// Signals smoothed together: as many as the tiles' workspace holds.
+struct BatchChunk {
+  int item0 = 0, items = 0;  // of the persistent kernel
+  int64_t tile0 = 0;
+  unsigned tiles = 0, deep = 0;  // deep: leading tiles with levels beyond kBatchHead
+};
+}  // namespace wh
 
 struct wh_batch {
   int device = -1;
@@ -23,6 +33,11 @@ struct wh_batch {
   int64_t total = 0;
   std::string key;            // composition signature (tuning table key)
   wh::BatchItem* items = nullptr;
+  wh::BatchTile* tiles = nullptr;  // the MODWT signals' tiles
+  void* tscratch = nullptr;        // their workspace
+  size_t tile_bytes = 0;
+  double* thresh = nullptr;        // one per signal
+  std::vector<wh::BatchChunk> chunks;
   int* counter = nullptr;     // queue head, finished workgroups
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -45,21 +60,70 @@ std::map<std::string, std::pair<int, unsigned>> g_tune;  // key -> (NT, grid)
 
 int nt_index(int NT) { return NT == 512 ? 2 : (NT == 256 ? 1 : 0); }
 
+// The tiles' workspace is at most this large (a signal that needs more has a
+// chunk of its own): enough that the launches of a chunk fill the chip many
+// times over.
+constexpr int64_t kBatchTileBytes = int64_t(2) << 30;
+
 // dynamic LDS of one item for NT threads
-size_t item_lds(int ttype, int filt, int64_t n, int J, int NT, size_t esz) {
-  const int L = filter_length(filt);
+size_t item_lds(int ttype, int NT, size_t esz) {
   size_t b = (NT == 512) ? block_sel_lds<512>()
              : (NT == 256 ? block_sel_lds<256>() : block_sel_lds<128>());
+  if (ttype != kDWT) return b;
   b = std::max(b, batch_pre_lds(NT, esz));  // the forward's first-digit histogram
-  if (ttype == kDWT) {
-    const size_t tile = (esz == 8) ? size_t(batch_lds_elems<double>()) * 8
-                                   : size_t(batch_lds_elems<float>()) * 4;
-    return std::max(b, 2 * tile);
+  const size_t tile = (esz == 8) ? size_t(batch_lds_elems<double>()) * 8
+                                 : size_t(batch_lds_elems<float>()) * 4;
+  return std::max(b, 2 * tile);
+}
+
+// Chunks, tiles and workspace of a batch's items, longest first.  MODWT items
+// get their workspace offset and fill the chunks in order; the DWT's belong to
+// the first.  A chunk's deep tiles lead, and tiles of one kind are neighbours,
+// so that a CU's workgroups run the same code.
+void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
+                 std::vector<BatchChunk>& chunks, int64_t budget, int64_t* workspace) {
+  std::vector<std::vector<BatchItem>> by_chunk(1);
+  std::vector<std::vector<BatchTile>> heads(1);
+  int64_t used = 0;
+  *workspace = 0;
+  for (BatchItem I : items) {
+    if (kind_ttype(I.kind) == kDWT) {
+      by_chunk[0].push_back(I);
+      continue;
+    }
+    const int64_t need = 3 * batch_pad(I.n);
+    if (used && used + need > budget) {
+      by_chunk.emplace_back();
+      heads.emplace_back();
+      used = 0;
+    }
+    heads.back().push_back(BatchTile{I.off, used, I.n, 0, kind_filter(I.kind) | (I.J << 3), I.sig});
+    I.off = used;
+    by_chunk.back().push_back(I);
+    used += need;
+    *workspace = std::max(*workspace, used);
   }
-  const int M = int(std::min<int64_t>(2 * NT, n));
-  const size_t fwd = size_t(fwd_off(L, M, J)) * esz;
-  const size_t inv = size_t(2) * lin_off(L, M, J + 1) * esz;
-  return std::max(b, std::max(fwd, inv));
+  items.clear();
+  auto key = [](const BatchTile& t) {
+    const bool deep = (t.kind >> 3) > kBatchHead;
+    return std::make_tuple(!deep, t.kind, t.n < kBatchP);
+  };
+  for (size_t k = 0; k < by_chunk.size(); ++k) {
+    BatchChunk c;
+    c.item0 = int(items.size());
+    c.items = int(by_chunk[k].size());
+    c.tile0 = int64_t(tiles.size());
+    items.insert(items.end(), by_chunk[k].begin(), by_chunk[k].end());
+    std::stable_sort(heads[k].begin(), heads[k].end(),
+                     [&](const BatchTile& a, const BatchTile& b) { return key(a) < key(b); });
+    for (BatchTile t : heads[k]) {
+      const int nt = t.n > kBatchP ? t.n / kBatchP : 1;
+      for (t.tile = 0; t.tile < nt; ++t.tile) tiles.push_back(t);
+      if ((t.kind >> 3) > kBatchHead) c.deep = unsigned(int64_t(tiles.size()) - c.tile0);
+    }
+    c.tiles = unsigned(int64_t(tiles.size()) - c.tile0);
+    chunks.push_back(c);
+  }
 }
 
 int occupancy(int dtype, int NT, size_t lds, int* blocks) {
@@ -68,19 +132,20 @@ int occupancy(int dtype, int NT, size_t lds, int* blocks) {
 }
 
 // largest resident grid for NT threads
-int max_grid(const wh_batch* p, int NT, unsigned* grid) {
+int max_grid(const wh_batch* p, int NT, unsigned* grid, int64_t* resident = nullptr) {
   int occ = 0;
   int rc = occupancy(p->dtype, NT, p->lds[nt_index(NT)], &occ);
   if (rc) return rc;
   if (occ <= 0) return set_error(WH_ERR_UNSUPPORTED, "batch: kernel does not fit a CU");
   const int64_t g = int64_t(occ) * std::max(1, device_info().num_cus);
   *grid = unsigned(std::min<int64_t>(g, p->count));
+  if (resident) *resident = g;
   return WH_OK;
 }
 
 int ensure_scratch(wh_batch* p, unsigned grid) {
   const size_t esz = p->dtype == WH_F32 ? 4 : 8;
-  const size_t need = size_t(grid) * size_t(p->stride) * esz;
+  const size_t need = size_t(grid) * size_t(p->stride) * esz;  // 0: no DWT
   if (need <= p->scratch_bytes) return WH_OK;
   if (p->scratch) {
     WH_HIP_CHECK(hipDeviceSynchronize());
@@ -96,20 +161,48 @@ int ensure_scratch(wh_batch* p, unsigned grid) {
   return WH_OK;
 }
 
+int tile_pass(const wh_batch* p, BatchPass pass, unsigned count, const BatchTileArgs& a,
+              hipStream_t st) {
+  return p->dtype == WH_F32 ? batch_tile_launch<float>(pass, count, a, st)
+                            : batch_tile_launch<double>(pass, count, a, st);
+}
+
 int run(wh_batch* p, int NT, unsigned grid, const void* x, void* y, double* thresh_out,
         hipStream_t st) {
-  BatchArgs a{};
-  a.items = p->items;
-  a.count = p->count;
-  a.counter = p->counter;
-  a.x = x;
-  a.y = y;
-  a.thresh_out = thresh_out;
-  a.scratch = p->scratch;
-  a.scratch_stride = p->stride;
-  a.hardness = p->hardness;
-  BatchLaunch bl{NT, grid, p->lds[nt_index(NT)]};
-  return p->dtype == WH_F32 ? batch_launch<float>(bl, a, st) : batch_launch<double>(bl, a, st);
+  const size_t esz = p->dtype == WH_F32 ? 4 : 8;
+  const char *x0 = static_cast<const char*>(x), *y0 = static_cast<const char*>(y);
+  const int64_t bytes = p->total * int64_t(esz);
+  BatchTileArgs t{};
+  t.x = x;
+  t.y = y;
+  t.scratch = p->tscratch;
+  t.thresh = p->thresh;
+  // a tile reads beyond what it writes: overlapping buffers go through a copy
+  t.in_place = x0 < y0 + bytes && y0 < x0 + bytes;
+  t.hardness = p->hardness;
+  for (const BatchChunk& c : p->chunks) {
+    t.tiles = p->tiles + c.tile0;
+    if (int rc = tile_pass(p, BatchPass::kHead, c.tiles, t, st)) return rc;
+    BatchArgs a{};
+    a.items = p->items + c.item0;
+    a.count = c.items;
+    a.counter = p->counter;
+    a.x = x;
+    a.y = y;
+    a.thresh_out = thresh_out;
+    a.thresh = p->thresh;
+    a.tiles = p->tscratch;
+    a.scratch = p->scratch;
+    a.scratch_stride = p->stride;
+    a.hardness = p->hardness;
+    BatchLaunch bl{NT, std::min(grid, unsigned(c.items)), p->lds[nt_index(NT)]};
+    if (int rc = p->dtype == WH_F32 ? batch_launch<float>(bl, a, st)
+                                    : batch_launch<double>(bl, a, st))
+      return rc;
+    if (int rc = tile_pass(p, BatchPass::kSecond, c.deep, t, st)) return rc;
+    if (int rc = tile_pass(p, BatchPass::kFirst, c.tiles, t, st)) return rc;
+  }
+  return WH_OK;
 }
 
 void drop_graph(wh_batch* p) {
@@ -165,27 +258,33 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     const double nn = (tt == kDWT && J == 1) ? double(n - 1) : double(n);
     I.factor = std::sqrt(2.0 * std::log(nn));
     off += n;
-    stride = std::max<int64_t>(stride, tt == kDWT ? 2 * n : 2 * n * J);
-    for (int k = 0; k < 3; ++k)
-      lds[k] = std::max(lds[k], item_lds(tt, filt, n, J, kNTs[k], esz));
+    if (tt == kDWT) stride = std::max<int64_t>(stride, 2 * n);
+    for (int k = 0; k < 3; ++k) lds[k] = std::max(lds[k], item_lds(tt, kNTs[k], esz));
     int lg = 0;
     while ((int64_t(1) << lg) < n) ++lg;
     comp[(int64_t(I.kind) << 16) | (lg << 8) | J] += 1;
   }
-  // longest work first: MODWT moves about 2J + 4 words per sample, the DWT
-  // about 6 plus its level-serial latency
-  std::stable_sort(items.begin(), items.end(), [](const BatchItem& a, const BatchItem& b) {
-    auto cost = [](const BatchItem& I) {
-      return kind_ttype(I.kind) == kMODWT ? int64_t(I.n) * (2 * I.J + 4) : int64_t(I.n) * 6 + 256 * I.J;
-    };
-    return cost(a) > cost(b);
-  });
+  // longest work first within a chunk: a MODWT's item is the selection from
+  // D_1, the DWT moves about 6 words per sample plus its level-serial latency
+  auto cost = [](const BatchItem& I) {
+    return kind_ttype(I.kind) == kMODWT ? int64_t(I.n) * 2 : int64_t(I.n) * 6 + 256 * I.J;
+  };
+  std::stable_sort(items.begin(), items.end(),
+                   [&](const BatchItem& a, const BatchItem& b) { return cost(a) > cost(b); });
+  const double max_cost = double(cost(items[0]));
+  double sum_cost = 0.0;
+  for (const BatchItem& I : items) sum_cost += double(cost(I));
+  std::vector<BatchTile> tiles;
+  std::vector<BatchChunk> chunks;
+  int64_t tscr = 0;  // elements of the tiles' workspace
+  plan_chunks(items, tiles, chunks, int64_t(kBatchTileBytes / int64_t(esz)), &tscr);
 
   wh_batch* p = new wh_batch();
   p->device = dev;
   p->dtype = dtype;
   p->hardness = hardness;
   p->count = count;
+  p->chunks = std::move(chunks);
   p->total = off;
   p->stride = (stride + 63) / 64 * 64;
   for (int k = 0; k < 3; ++k) p->lds[k] = lds[k];
@@ -205,13 +304,32 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     p->counter = nullptr;
     return fail(set_error(WH_ERR_NOMEM, "batch: queue allocation failed"));
   }
+  if (hipMalloc(reinterpret_cast<void**>(&p->thresh), sizeof(double) * size_t(count)) !=
+      hipSuccess) {
+    p->thresh = nullptr;
+    return fail(set_error(WH_ERR_NOMEM, "batch: threshold allocation failed"));
+  }
+  p->tile_bytes = size_t(tscr) * esz;
+  if (!tiles.empty()) {
+    if (hipMalloc(reinterpret_cast<void**>(&p->tiles), sizeof(BatchTile) * tiles.size()) !=
+        hipSuccess) {
+      p->tiles = nullptr;
+      return fail(set_error(WH_ERR_NOMEM, "batch: tile table allocation failed"));
+    }
+    if (hipMalloc(&p->tscratch, p->tile_bytes) != hipSuccess) {
+      p->tscratch = nullptr;
+      return fail(set_error(WH_ERR_NOMEM, "batch: workspace allocation failed"));
+    }
+    if (hipMemcpy(p->tiles, tiles.data(), sizeof(BatchTile) * tiles.size(),
+                  hipMemcpyHostToDevice) != hipSuccess)
+      return fail(set_hip_error(hipGetLastError(), "batch: table upload"));
+  }
   if (hipMemcpy(p->items, items.data(), sizeof(BatchItem) * size_t(count),
                 hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(p->counter, 0, 2 * sizeof(int)) != hipSuccess)
     return fail(set_hip_error(hipGetLastError(), "batch: table upload"));
 
-  // launch shape: a tuned one for this composition, else 256 threads and
-  // every workgroup that fits
+  // the persistent kernel's shape: a tuned one for this composition, or
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(p->key);
@@ -222,13 +340,20 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     }
   }
   if (!p->tuned) {
-    // untuned: the shape the tuner picks for mixed batches on MI355X (one
-    // 512-thread workgroup per CU in FP64; in FP32 128 threads and every
-    // workgroup that fits); wh_batch_tune times the others
-    const int NT = dtype == WH_F32 ? 128 : 512;
-    int rc = max_grid(p, NT, &p->grid);
-    if (rc) return fail(rc);
-    p->NT = NT;
+    // untuned: 256 threads and every workgroup that fits, unless the longest
+    // item would still run when the others are done: then 512 threads, which
+    // take it in about two thirds of the time.  Mixed batches, us with 256 /
+    // 512 threads: 8192 signals to 2^16 samples FP64 2651 / 2843, FP32 1487 /
+    // 1770; 2000 to 2^16 FP64 737 / 738; 1200 to 2^16 (ratio 0.35 of the
+    // line's 0.4) FP64 508 / 441, FP32 354 / 287; 300 to 2^16 FP64 289 / 242.
+    // wh_batch_tune times the shapes.
+    int64_t resident = 0;
+    p->NT = 256;
+    if (int rc = max_grid(p, p->NT, &p->grid, &resident)) return fail(rc);
+    if (sum_cost < 0.4 * max_cost * double(resident)) {
+      p->NT = 512;
+      if (int rc = max_grid(p, p->NT, &p->grid)) return fail(rc);
+    }
   }
   if (int rc = ensure_scratch(p, p->grid)) return fail(rc);
   *out = p;
@@ -241,6 +366,9 @@ void wh_batch_destroy(wh_batch* p) {
   drop_graph(p);
   if (p->items) (void)hipFree(p->items);
   if (p->counter) (void)hipFree(p->counter);
+  if (p->tiles) (void)hipFree(p->tiles);
+  if (p->tscratch) (void)hipFree(p->tscratch);
+  if (p->thresh) (void)hipFree(p->thresh);
   if (p->scratch) (void)hipFree(p->scratch);
   delete p;
 }
@@ -363,7 +491,7 @@ int wh_batch_info(const wh_batch* p, int64_t* total, int* threads, int* workgrou
   if (threads) *threads = p->NT;
   if (workgroups) *workgroups = int(p->grid);
   if (lds_bytes) *lds_bytes = int64_t(p->lds[nt_index(p->NT)]);
-  if (workspace_bytes) *workspace_bytes = int64_t(p->scratch_bytes);
+  if (workspace_bytes) *workspace_bytes = int64_t(p->scratch_bytes + p->tile_bytes);
   if (tuned) *tuned = p->tuned;
   return WH_OK;
 }
