@@ -20,8 +20,8 @@ namespace wh {
 // Signals smoothed together: as many as the tiles' workspace holds.
 struct BatchChunk {
   int item0 = 0, items = 0;  // of the persistent kernel
-  int64_t tile0 = 0;
-  unsigned tiles = 0, deep = 0;  // deep: leading tiles with levels beyond kBatchHead
+  int64_t tile0[3] = {0, 0, 0};  // per pass
+  unsigned tiles[3] = {0, 0, 0};
 };
 }  // namespace wh
 
@@ -76,10 +76,40 @@ size_t item_lds(int ttype, int NT, size_t esz) {
   return std::max(b, 2 * tile);
 }
 
+// The tiles of one signal in a pass; t.kind holds filter and depth.
+void add_tiles(std::vector<BatchTile>& tiles, BatchTile t, BatchPass pass) {
+  const int J = tile_levels(t.kind), kind = t.kind;
+  if (pass == BatchPass::kHead) {
+    for (t.m0 = 0; t.m0 < t.n; t.m0 += kBatchP) tiles.push_back(t);
+    return;
+  }
+  const bool second = pass == BatchPass::kSecond;
+  if (second && J <= kBatchHead) return;
+  const int N = second ? t.n / kBatchRes : t.n, nseq = second ? kBatchRes : 1;
+  const int G = second ? J - kBatchHead : std::min(J, kBatchHead);
+  const int slots = shrink_slots(second);
+  if (N <= slots) {
+    const int per = slots / std::max(N, 1 << (G + 1));  // sequences of a tile
+    for (int q = 0; q < nseq; q += per) {
+      t.kind = kind | q << 8;
+      tiles.push_back(t);
+    }
+    return;
+  }
+  const int step = slots - 2 * tile_halo(filter_length(kind_filter(kind)), G);
+  for (int q = 0; q < nseq; ++q) {
+    t.kind = kind | q << 8;
+    for (int64_t m = 0; m < N; m += step) {
+      t.m0 = int32_t(m);
+      tiles.push_back(t);
+    }
+  }
+}
+
 // Chunks, tiles and workspace of a batch's items, longest first.  MODWT items
 // get their workspace offset and fill the chunks in order; the DWT's belong to
-// the first.  A chunk's deep tiles lead, and tiles of one kind are neighbours,
-// so that a CU's workgroups run the same code.
+// the first.  Tiles of one filter and depth are neighbours, so that a CU's
+// workgroups run the same code.
 void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
                  std::vector<BatchChunk>& chunks, int64_t budget, int64_t* workspace) {
   std::vector<std::vector<BatchItem>> by_chunk(1);
@@ -104,24 +134,18 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
     *workspace = std::max(*workspace, used);
   }
   items.clear();
-  auto key = [](const BatchTile& t) {
-    const bool deep = (t.kind >> 3) > kBatchHead;
-    return std::make_tuple(!deep, t.kind, t.n < kBatchP);
-  };
   for (size_t k = 0; k < by_chunk.size(); ++k) {
     BatchChunk c;
     c.item0 = int(items.size());
     c.items = int(by_chunk[k].size());
-    c.tile0 = int64_t(tiles.size());
     items.insert(items.end(), by_chunk[k].begin(), by_chunk[k].end());
     std::stable_sort(heads[k].begin(), heads[k].end(),
-                     [&](const BatchTile& a, const BatchTile& b) { return key(a) < key(b); });
-    for (BatchTile t : heads[k]) {
-      const int nt = t.n > kBatchP ? t.n / kBatchP : 1;
-      for (t.tile = 0; t.tile < nt; ++t.tile) tiles.push_back(t);
-      if ((t.kind >> 3) > kBatchHead) c.deep = unsigned(int64_t(tiles.size()) - c.tile0);
+                     [](const BatchTile& a, const BatchTile& b) { return a.kind > b.kind; });
+    for (int pass = 0; pass < 3; ++pass) {
+      c.tile0[pass] = int64_t(tiles.size());
+      for (const BatchTile& t : heads[k]) add_tiles(tiles, t, BatchPass(pass));
+      c.tiles[pass] = unsigned(int64_t(tiles.size()) - c.tile0[pass]);
     }
-    c.tiles = unsigned(int64_t(tiles.size()) - c.tile0);
     chunks.push_back(c);
   }
 }
@@ -161,8 +185,10 @@ int ensure_scratch(wh_batch* p, unsigned grid) {
   return WH_OK;
 }
 
-int tile_pass(const wh_batch* p, BatchPass pass, unsigned count, const BatchTileArgs& a,
+int tile_pass(const wh_batch* p, const BatchChunk& c, BatchPass pass, BatchTileArgs a,
               hipStream_t st) {
+  a.tiles = p->tiles + c.tile0[int(pass)];
+  const unsigned count = c.tiles[int(pass)];
   return p->dtype == WH_F32 ? batch_tile_launch<float>(pass, count, a, st)
                             : batch_tile_launch<double>(pass, count, a, st);
 }
@@ -181,8 +207,7 @@ int run(wh_batch* p, int NT, unsigned grid, const void* x, void* y, double* thre
   t.in_place = x0 < y0 + bytes && y0 < x0 + bytes;
   t.hardness = p->hardness;
   for (const BatchChunk& c : p->chunks) {
-    t.tiles = p->tiles + c.tile0;
-    if (int rc = tile_pass(p, BatchPass::kHead, c.tiles, t, st)) return rc;
+    if (int rc = tile_pass(p, c, BatchPass::kHead, t, st)) return rc;
     BatchArgs a{};
     a.items = p->items + c.item0;
     a.count = c.items;
@@ -199,8 +224,8 @@ int run(wh_batch* p, int NT, unsigned grid, const void* x, void* y, double* thre
     if (int rc = p->dtype == WH_F32 ? batch_launch<float>(bl, a, st)
                                     : batch_launch<double>(bl, a, st))
       return rc;
-    if (int rc = tile_pass(p, BatchPass::kSecond, c.deep, t, st)) return rc;
-    if (int rc = tile_pass(p, BatchPass::kFirst, c.tiles, t, st)) return rc;
+    if (int rc = tile_pass(p, c, BatchPass::kSecond, t, st)) return rc;
+    if (int rc = tile_pass(p, c, BatchPass::kFirst, t, st)) return rc;
   }
   return WH_OK;
 }

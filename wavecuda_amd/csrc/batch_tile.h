@@ -6,16 +6,15 @@
 // D_1 (batch_kern.h); then the levels beyond the fourth are computed,
 // thresholded and inverted in one pass over S_4 (giving S'_4), and the first
 // four in one pass over the signal and S'_4.  No detail level but the first
-// is ever stored: recomputing four levels costs 40 LDS-fed FMA pairs per
+// is ever stored: recomputing four levels costs 32 LDS-fed FMA pairs per
 // sample (LA8) where storing and reading their details costs 8 words, and
 // the deeper levels are computed once, in the pass that thresholds them.
 //
 // Beyond the fourth level a tap's distance is a multiple of 16, so S_4 is
 // kept residue by residue: 16 circular sequences of n / 16 contiguous values,
 // on which levels 5..8 are levels 1..4.  Every pass is therefore the same
-// tile: kBatchP consecutive values of a circular sequence, with the halo its
-// levels need on both sides (W = (L-1)(2^G - 1): 105 for LA8 and 4 levels, 10
-// % of a tile), or, where sequences are shorter than a tile, whole sequences
+// tile: consecutive values of a circular sequence, with the halo its levels
+// need (W = (L-1)(2^G - 1): 105 for LA8 and 4 levels), or, where sequences are shorter than a tile, whole sequences
 // without any.  All arithmetic is the single-signal path's, term by term.
 #pragma once
 
@@ -35,10 +34,13 @@ struct BatchTile {
   int64_t off;   // the signal's first sample
   int64_t scr;   // its workspace
   int32_t n;
-  int32_t tile;  // values kBatchP tile .. of each sequence array
-  int32_t kind;  // filter | J << 3
+  int32_t m0;    // first value stored, of its sequence
+  int32_t kind;  // filter | J << 3 | first sequence << 8
   int32_t sig;
 };
+
+__host__ __device__ constexpr int tile_levels(int kind) { return (kind >> 3) & 31; }
+__host__ __device__ constexpr int tile_seq(int kind) { return kind >> 8; }
 
 __host__ __device__ constexpr int64_t batch_pad(int64_t n) { return (n + 63) / 64 * 64; }
 
@@ -75,7 +77,7 @@ __device__ __forceinline__ void batch_head(const BatchTileArgs& a, const BatchTi
   constexpr int L = Filter<FILT>::L, NT = kBatchNT, W = tile_halo(L, G);
   constexpr int N0 = CIRC ? kBatchP : kBatchP + W, K = (N0 + NT - 1) / NT;
   constexpr int KO = kBatchP / NT;
-  const int64_t n = I.n, m0 = int64_t(I.tile) * kBatchP;
+  const int64_t n = I.n, m0 = I.m0;
   const int mask = int(n - 1), tid = threadIdx.x;
   const int cnt = CIRC ? int(n) : N0;  // a short signal is one tile
   const T* __restrict__ in = static_cast<const T*>(a.x) + I.off;
@@ -134,177 +136,281 @@ __device__ __forceinline__ void batch_head(const BatchTileArgs& a, const BatchTi
 // ------------------------------------------------------------------ shrink
 // G levels of a sequence array: forward, threshold, inverse.  The smooth of
 // the top level is the tile's own, or (COARSE) the already smoothed S'_4.
-// A thread keeps the details of its slots in registers; slot e of every level
-// is the value at m0 - W + e.
-template <typename T, int FILT, int G, bool CIRC, bool COARSE>
-__device__ __forceinline__ void batch_shrink(const T* __restrict__ in, T* __restrict__ out,
-                                             const T* __restrict__ coarse, int64_t N,
-                                             int64_t first, int cnt, T t, int hardness,
-                                             unsigned char* smem) {
-  using V = typename Vec2<T>::type;
-  constexpr int L = Filter<FILT>::L, NT = kBatchNT, W = CIRC ? 0 : tile_halo(L, G);
-  constexpr int N0 = kBatchP + 2 * W, K = (N0 + NT - 1) / NT;
-  T* b = reinterpret_cast<T*>(smem);
-  V* p = reinterpret_cast<V*>(smem);
-  const int tid = threadIdx.x, mask = int(N - 1);
-  // sequence and position of the tile (CIRC: whole sequences from `first`)
-  const int64_t seq = CIRC ? first : first & ~(N - 1), m0 = CIRC ? 0 : first & (N - 1);
-  auto pos = [&](int e) { return CIRC ? int64_t(e) : (m0 - W + e) & (N - 1); };
-  T S[K], d[G][K], top[COARSE ? K : 1];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int e = tid + k * NT;
-    const int ec = e < cnt ? e : cnt - 1;  // unconditional load, clamped
-    S[k] = in[seq + pos(ec)];
+//
+// The tile's slots hold shrink_slots values of one sequence, W of them halo
+// on either side (their results are wrong towards the ends and are not
+// stored), or whole sequences, on which taps wrap at `mask`; a sequence
+// shorter than a quad's reach, 2^(G+1), is repeated to that length.  LDS reads bound the
+// pass, so a thread computes four outputs a level's stride apart, which share
+// L + 3 taps (one by one they read 4 L), and keeps its details in registers.
+// With a fixed stride of 4 s slots between lanes those reads would fall on a
+// quarter of the banks: slot e of a buffer that is read at stride s lies at e ^
+// (row(e) s), the low two bits of its 128-byte row, which spreads them
+// over all.
+// 8192 mixed signals in FP64 / 3001 in FP32, us: one output at a time 521 /
+// 128 for levels 5..8 and 590 / 144 for levels 1..4, as quads 470 / 106 and 494
+// / 127 (vector instructions then busy 70 % of the time, LDS 60 %).  A tile of
+// 4096 slots holds a residue of 2^16 samples without halo; of the first
+// levels, which wait for more memory, four tiles of 2048 a CU overlap better
+// than two of 4096 (655 / 168).
+__host__ __device__ constexpr int shrink_nt(bool second) { return second ? 512 : 256; }
+__host__ __device__ constexpr int shrink_slots(bool second) { return 8 * shrink_nt(second); }
+
+template <typename T, int FILT, int G, bool COARSE, bool SECOND, bool HARD>
+struct Shrink {
+  static constexpr int L = Filter<FILT>::L, NT = shrink_nt(SECOND), P0 = shrink_slots(SECOND);
+  static constexpr int QN = P0 / 4 / NT, K = P0 / NT;
+  static constexpr int W = tile_halo(L, G);
+  static constexpr int kLog = sizeof(T) == 8 ? 3 : 2;
+  // log2 of a row in a buffer read at stride 2^ls: the 128 bytes of all banks,
+  // or a quad's block where that is longer
+  static constexpr int row(int ls) {
+    const int b = sizeof(T) == 8 ? 4 : 5;
+    return b > ls + 2 ? b : ls + 2;
   }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int e = tid + k * NT;
-    if (e < cnt) b[e] = S[k];
+  T S[QN][4], d[G][QN][4];
+  T *A, *B;
+  int mask, cnt;
+  T t;
+
+  // place of slot e in a buffer read at stride 2^ls
+  static __device__ __forceinline__ int place(int e, int ls) {
+    return e ^ (((e >> row(ls)) & 3) << ls);
   }
-  __syncthreads();
-  auto forward = [&](auto lc) {
-    constexpr int l = decltype(lc)::value, s = 1 << (l - 1);
-    if constexpr (l <= G) {
-      const int no = CIRC ? cnt : N0 - tile_halo(L, l);
+  // tap group jj of the quad whose block starts at b4 (offset o in it): its
+  // place and the exclusive-or of its four taps, in bytes
+  __device__ __forceinline__ int group(int b4, int o, int jj, int ls, int* x) const {
+    const int s4 = 4 << ls;
+    const int g = (b4 & ~mask) | ((b4 + jj * s4) & mask);
+    *x = ((g >> row(ls)) & 3) << (ls + kLog);
+    return (g + o) << kLog;
+  }
+  static __device__ __forceinline__ T at(const T* buf, int bytes) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(buf) + bytes);
+  }
+  // thresh_coef's values; soft in three operations, t = 0 where there is no
+  // threshold (a NaN), the maximum and minimum as instructions because the
+  // functions add one for signalling NaNs to each operand
+  __device__ __forceinline__ T cut(T c) const {
+    if constexpr (HARD) return fabs(c) < t ? T(0) : c;
+    T m;
+    batch_pin(c);  // rounded: no product of c's is fused into the difference
+    if constexpr (sizeof(T) == 8)
+      asm("v_max_f64 %0, %1, -%2\n\tv_min_f64 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
+    else
+      asm("v_max_f32 %0, %1, -%2\n\tv_min_f32 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
+    return c - m;
+  }
+
+  // levels l..last
+  template <int l, int last>
+  __device__ __forceinline__ void forward() {
+    if constexpr (l <= last) {
+      constexpr int ls = l - 1, s = 1 << ls;
+      const T* src = (l & 1) ? A : B;
+      T* dst = (l & 1) ? B : A;
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const int e = tid + k * NT;
-        d[l - 1][k] = T(0);
-        if (e < no) {
-          T w[L];
+      for (int q = 0; q < QN; ++q) {
+        const int u = int(threadIdx.x) + q * NT;
+        if (4 * u < cnt) {
+          const int b4 = (u >> ls) << (ls + 2), o = u & (s - 1);
+          T w[L + 3];
 #pragma unroll
-          for (int j = 0; j < L; ++j) w[j] = b[batch_slot<CIRC>(e, j * s, mask)];
-          T D;
-          analysis1<T, FILT>(w, S[k], D);
-          d[l - 1][k] = t >= T(0) ? thresh_coef(D, t, hardness) : D;
-          batch_pin(d[l - 1][k]);
-          if (l < G || !COARSE) batch_pin(S[k]);
+          for (int jj = 0; jj <= (L + 2) / 4; ++jj) {
+            int x;
+            const int g = group(b4, o, jj, ls, &x);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (4 * jj + i < L + 3) w[4 * jj + i] = at(src, g + ((i << (ls + kLog)) ^ x));
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            T D;
+            analysis1<T, FILT>(w + i, S[q][i], D);
+            d[l - 1][q][i] = cut(D);
+            batch_pin(d[l - 1][q][i]);
+            if (l < G || !COARSE) batch_pin(S[q][i]);
+          }
+          if constexpr (l < G) {  // to be read at stride 2 s
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const int p = place(b4 + o + 2 * c * s, l);
+              dst[p] = S[q][2 * c];
+              dst[p + s] = S[q][2 * c + 1];
+            }
+          }
         }
       }
-      __syncthreads();  // every tap of this level read before any is replaced
-      if constexpr (l < G) {
+      __syncthreads();
+      forward<l + 1, last>();
+    }
+  }
+  // v[q][i], the values of quads at stride 2^ls, into a buffer read at it
+  template <int ls>
+  __device__ __forceinline__ void park(T* buf, const T (*v)[4]) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const int e = tid + k * NT;
-          if (e < no) b[e] = S[k];
-        }
-        __syncthreads();
+    for (int q = 0; q < QN; ++q) {
+      const int u = int(threadIdx.x) + q * NT;
+      const int b4 = (u >> ls) << (ls + 2), o = u & ((1 << ls) - 1);
+      const int x = ((b4 >> row(ls)) & 3) << ls;
+      if (4 * u < cnt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) buf[b4 + o + ((i << ls) ^ x)] = v[q][i];
       }
     }
+  }
+  template <int l>
+  __device__ __forceinline__ void inverse() {
+    if constexpr (l >= 1) {
+      constexpr int ls = l - 1, s = 1 << ls, kBack = (L + 2) / 4;
+#pragma unroll
+      for (int q = 0; q < QN; ++q) {
+        const int u = int(threadIdx.x) + q * NT;
+        if (4 * u < cnt) {
+          const int b4 = (u >> ls) << (ls + 2), o = u & (s - 1);
+          T ws[L + 3], wd[L + 3];
+#pragma unroll
+          for (int jj = -kBack; jj <= 0; ++jj) {
+            int x;
+            const int g = group(b4, o, jj, ls, &x);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int j = 4 * jj + i + L - 1;
+              if (j >= 0) {
+                ws[j] = at(A, g + ((i << (ls + kLog)) ^ x));
+                wd[j] = at(B, g + ((i << (ls + kLog)) ^ x));
+              }
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            S[q][i] = synthesis<T, FILT>(ws, wd, L - 1 + i);
+            batch_pin(S[q][i]);
+          }
+        }
+      }
+      __syncthreads();
+      // to be read at stride s / 2 (the tile's output: in order)
+#pragma unroll
+      for (int q = 0; q < QN; ++q) {
+        const int u = int(threadIdx.x) + q * NT;
+        const int b4 = (u >> ls) << (ls + 2), o = u & (s - 1);
+        if (4 * u < cnt) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int e = b4 + o + i * s;
+            A[l > 1 ? place(e, l > 1 ? ls - 1 : 0) : e] = S[q][i];
+          }
+        }
+      }
+      if constexpr (l > 1) park<l - 2>(B, d[l - 2]);
+      __syncthreads();
+      inverse<l - 1>();
+    }
+  }
+};
+
+// nseq sequences of N values at `in`; the tile starts at value m0 of sequence
+// seq0
+template <typename T, int FILT, int G, bool COARSE, bool SECOND, bool HARD>
+__device__ __forceinline__ void batch_shrink(const T* __restrict__ in, T* __restrict__ out,
+                                             const T* __restrict__ coarse, int N, int nseq,
+                                             int seq0, int m0, T t, T* lds) {
+  using C = Shrink<T, FILT, G, COARSE, SECOND, HARD>;
+  constexpr int NT = C::NT, P0 = C::P0, K = C::K, W = C::W;
+  const bool circ = N <= P0;
+  const int lN = 31 - __builtin_clz(N);
+  const int lR = circ ? (lN > G + 1 ? lN : G + 1) : 31;  // slots per sequence
+  const int start = circ ? 0 : m0 - W;
+  const int64_t base = int64_t(seq0) << lN;
+  C c;
+  c.A = lds;
+  c.B = lds + P0;
+  c.t = HARD || t >= T(0) ? t : T(0);
+  c.mask = circ ? (1 << lR) - 1 : P0 - 1;
+  c.cnt = P0;
+  if (circ && (int64_t(nseq - seq0) << lR) < P0) c.cnt = (nseq - seq0) << lR;
+  auto index = [&](int e) {
+    return base + (int64_t(e >> lR) << lN) + ((start + e) & (N - 1));
   };
-  forward(std::integral_constant<int, 1>{});
-  forward(std::integral_constant<int, 2>{});
-  forward(std::integral_constant<int, 3>{});
-  forward(std::integral_constant<int, 4>{});
+  T v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    v[k] = in[index(e < c.cnt ? e : c.cnt - 1)];  // unconditional load, clamped
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = int(threadIdx.x) + k * NT;
+    c.A[C::place(e, 0)] = v[k];
+  }
+  __syncthreads();
+  c.template forward<1, G - 1>();
+  if constexpr (COARSE) {  // in flight during the last level
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int e = int(threadIdx.x) + k * NT;
+      const int i = int(index(e < c.cnt ? e : c.cnt - 1));
+      v[k] = coarse[int64_t(i & (kBatchRes - 1)) * (N / kBatchRes) + i / kBatchRes];
+    }
+  }
+  c.template forward<G, G>();
   if constexpr (COARSE) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const int e = tid + k * NT;
-      const int64_t i = pos(e < cnt ? e : cnt - 1);
-      top[k] = coarse[(i & (kBatchRes - 1)) * (N / kBatchRes) + i / kBatchRes];
+      const int e = int(threadIdx.x) + k * NT;
+      c.A[C::place(e, G - 1)] = v[k];
     }
+  } else {
+    c.template park<G - 1>(c.A, c.S);
   }
-  const int hi = CIRC ? cnt : W + kBatchP;
+  c.template park<G - 1>(c.B, c.d[G - 1]);
+  __syncthreads();
+  c.template inverse<G>();
+  // stored values: of HALO tiles those between the halos, of repeated
+  // sequences the first copy
+  const int lo = circ ? 0 : W, hi = circ ? c.cnt : (P0 - W < W + N - m0 ? P0 - W : W + N - m0);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int e = tid + k * NT;
-    if (e < hi) p[e] = V{COARSE ? top[COARSE ? k : 0] : S[k], d[G - 1][k]};
+    const int e = int(threadIdx.x) + k * NT;
+    if (e >= lo && e < hi && (!circ || (e & c.mask) < N)) out[index(e)] = c.A[e];
   }
-  __syncthreads();
-  auto inverse = [&](auto lc) {
-    constexpr int l = decltype(lc)::value, s = 1 << (l - 1);
-    if constexpr (l <= G) {
-      const int lo = CIRC ? 0 : W - tile_halo(L, l - 1);
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const int e = tid + k * NT;
-        if (e >= lo && e < hi) {
-          T ws[L], wd[L];
-#pragma unroll
-          for (int j = 0; j < L; ++j) {
-            const V v = p[batch_slot<CIRC>(e, (j - (L - 1)) * s, mask)];
-            ws[j] = v.x;
-            wd[j] = v.y;
-          }
-          S[k] = synthesis<T, FILT>(ws, wd, L - 1);
-          batch_pin(S[k]);
-          if constexpr (l == 1) out[seq + (CIRC ? e : m0 + e - W)] = S[k];
-        }
-      }
-      if constexpr (l > 1) {
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const int e = tid + k * NT;
-          if (e >= lo && e < hi) p[e] = V{S[k], d[l > 1 ? l - 2 : 0][k]};
-        }
-        __syncthreads();
-      }
-    }
-  };
-  inverse(std::integral_constant<int, 4>{});
-  inverse(std::integral_constant<int, 3>{});
-  inverse(std::integral_constant<int, 2>{});
-  inverse(std::integral_constant<int, 1>{});
-}
-
-template <typename T, int FILT, int G, bool COARSE>
-__device__ __forceinline__ void batch_shrink_len(const T* in, T* out, const T* coarse, int64_t N,
-                                                 int64_t total, int64_t first, T t, int hardness,
-                                                 unsigned char* smem) {
-  constexpr int W = tile_halo(Filter<FILT>::L, G);
-  if (N < kBatchP)
-    batch_shrink<T, FILT, G, true, COARSE>(in, out, coarse, N, first,
-                                           int(total < kBatchP ? total : kBatchP), t, hardness,
-                                           smem);
-  else
-    batch_shrink<T, FILT, G, false, COARSE>(in, out, coarse, N, first, kBatchP + 2 * W, t,
-                                            hardness, smem);
 }
 
 // SECOND: levels 5..J of S_4 into S'_4; else the first levels into y
-template <typename T, int FILT, bool SECOND>
+template <typename T, int FILT, bool SECOND, bool HARD>
 __device__ __forceinline__ void batch_shrink_f(const BatchTileArgs& a, const BatchTile& I,
-                                               unsigned char* smem) {
-  const int64_t n = I.n, first = int64_t(I.tile) * kBatchP;
-  const int J = I.kind >> 3, h = a.hardness;
+                                               T* lds) {
+  const int n = I.n, J = tile_levels(I.kind), seq = tile_seq(I.kind);
   T* scr = static_cast<T*>(a.scratch) + I.scr;
   const T* s4 = scr + batch_pad(n);
   const T t = T(a.thresh[I.sig]);
   if constexpr (SECOND) {
-    const int64_t N = n / kBatchRes;
+    const int N = n / kBatchRes, R = kBatchRes;
     switch (J - kBatchHead) {
-      case 1: batch_shrink_len<T, FILT, 1, false>(s4, scr, nullptr, N, n, first, t, h, smem); break;
-      case 2: batch_shrink_len<T, FILT, 2, false>(s4, scr, nullptr, N, n, first, t, h, smem); break;
-      case 3: batch_shrink_len<T, FILT, 3, false>(s4, scr, nullptr, N, n, first, t, h, smem); break;
-      default: batch_shrink_len<T, FILT, 4, false>(s4, scr, nullptr, N, n, first, t, h, smem);
+      case 1: batch_shrink<T, FILT, 1, false, SECOND, HARD>(s4, scr, nullptr, N, R, seq, I.m0, t, lds); break;
+      case 2: batch_shrink<T, FILT, 2, false, SECOND, HARD>(s4, scr, nullptr, N, R, seq, I.m0, t, lds); break;
+      case 3: batch_shrink<T, FILT, 3, false, SECOND, HARD>(s4, scr, nullptr, N, R, seq, I.m0, t, lds); break;
+      default: batch_shrink<T, FILT, 4, false, SECOND, HARD>(s4, scr, nullptr, N, R, seq, I.m0, t, lds);
     }
   } else {
     const T* x = a.in_place ? s4 + batch_pad(n) : static_cast<const T*>(a.x) + I.off;
     T* y = static_cast<T*>(a.y) + I.off;
     switch (J) {
-      case 1: batch_shrink_len<T, FILT, 1, false>(x, y, nullptr, n, n, first, t, h, smem); break;
-      case 2: batch_shrink_len<T, FILT, 2, false>(x, y, nullptr, n, n, first, t, h, smem); break;
-      case 3: batch_shrink_len<T, FILT, 3, false>(x, y, nullptr, n, n, first, t, h, smem); break;
-      case 4: batch_shrink_len<T, FILT, 4, false>(x, y, nullptr, n, n, first, t, h, smem); break;
-      default: batch_shrink_len<T, FILT, 4, true>(x, y, scr, n, n, first, t, h, smem);
+      case 1: batch_shrink<T, FILT, 1, false, SECOND, HARD>(x, y, nullptr, n, 1, 0, I.m0, t, lds); break;
+      case 2: batch_shrink<T, FILT, 2, false, SECOND, HARD>(x, y, nullptr, n, 1, 0, I.m0, t, lds); break;
+      case 3: batch_shrink<T, FILT, 3, false, SECOND, HARD>(x, y, nullptr, n, 1, 0, I.m0, t, lds); break;
+      case 4: batch_shrink<T, FILT, 4, false, SECOND, HARD>(x, y, nullptr, n, 1, 0, I.m0, t, lds); break;
+      default: batch_shrink<T, FILT, 4, true, SECOND, HARD>(x, y, scr, n, 1, 0, I.m0, t, lds);
     }
   }
-}
-
-// LDS of a tile: (S, D) pairs of a tile and its left halo, or the head's and
-// the forward's values with both halos
-template <typename T>
-constexpr int batch_tile_lds() {
-  return (kBatchP + tile_halo(8, kBatchHead)) * 2 * int(sizeof(T));
 }
 
 template <typename T>
 __global__ __launch_bounds__(kBatchNT) void batch_head_k(BatchTileArgs a) {
   __shared__ __align__(16) T b[kBatchP + tile_halo(8, kBatchHead)];
   const BatchTile I = a.tiles[blockIdx.x];
-  const bool deep = (I.kind >> 3) > kBatchHead, circ = I.n < kBatchP;
+  const bool deep = tile_levels(I.kind) > kBatchHead, circ = I.n < kBatchP;
 #define WH_HEAD(F)                                              \
   if (deep) {                                                   \
     if (circ) batch_head<T, F, kBatchHead, true>(a, I, b);      \
@@ -322,15 +428,15 @@ __global__ __launch_bounds__(kBatchNT) void batch_head_k(BatchTileArgs a) {
 #undef WH_HEAD
 }
 
-template <typename T, bool SECOND>
-__global__ __launch_bounds__(kBatchNT, 4) void batch_shrink_k(BatchTileArgs a) {
-  __shared__ __align__(16) unsigned char smem[batch_tile_lds<T>()];
+template <typename T, bool SECOND, bool HARD>
+__global__ __launch_bounds__(shrink_nt(SECOND), 4) void batch_shrink_k(BatchTileArgs a) {
+  __shared__ __align__(16) T lds[2 * shrink_slots(SECOND)];
   const BatchTile I = a.tiles[blockIdx.x];
   switch (I.kind & 7) {
-    case kHAAR: batch_shrink_f<T, kHAAR, SECOND>(a, I, smem); break;
-    case kD4: batch_shrink_f<T, kD4, SECOND>(a, I, smem); break;
-    case kC6: batch_shrink_f<T, kC6, SECOND>(a, I, smem); break;
-    default: batch_shrink_f<T, kLA8, SECOND>(a, I, smem); break;
+    case kHAAR: batch_shrink_f<T, kHAAR, SECOND, HARD>(a, I, lds); break;
+    case kD4: batch_shrink_f<T, kD4, SECOND, HARD>(a, I, lds); break;
+    case kC6: batch_shrink_f<T, kC6, SECOND, HARD>(a, I, lds); break;
+    default: batch_shrink_f<T, kLA8, SECOND, HARD>(a, I, lds); break;
   }
 }
 
@@ -343,14 +449,18 @@ template <typename T>
 int batch_tile_launch_impl(BatchPass pass, unsigned count, const BatchTileArgs& a,
                            hipStream_t st) {
   if (!count) return WH_OK;
-  const dim3 grid(count), nt(kBatchNT);
+  const dim3 grid(count), nt(pass == BatchPass::kHead ? kBatchNT : shrink_nt(pass == BatchPass::kSecond));
   switch (pass) {
     case BatchPass::kHead: hipLaunchKernelGGL((batch_head_k<T>), grid, nt, 0, st, a); break;
     case BatchPass::kSecond:
-      hipLaunchKernelGGL((batch_shrink_k<T, true>), grid, nt, 0, st, a);
+      hipLaunchKernelGGL((a.hardness == kHARD ? batch_shrink_k<T, true, true>
+                                              : batch_shrink_k<T, true, false>),
+                         grid, nt, 0, st, a);
       break;
     case BatchPass::kFirst:
-      hipLaunchKernelGGL((batch_shrink_k<T, false>), grid, nt, 0, st, a);
+      hipLaunchKernelGGL((a.hardness == kHARD ? batch_shrink_k<T, false, true>
+                                              : batch_shrink_k<T, false, false>),
+                         grid, nt, 0, st, a);
       break;
   }
   WH_HIP_CHECK(hipGetLastError());
