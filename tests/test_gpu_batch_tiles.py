@@ -1,4 +1,4 @@
-"""The batch's MODWT tiles against the single-signal path.
+"""The batch's tiles against the single-signal path.
 
 Every signal must equal wh_smooth's result bit for bit (the same terms in the
 same order, the same exact order statistics), whatever the tile does at its
@@ -53,6 +53,23 @@ def test_every_length_and_depth(filt, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("filt", [W.HAAR, W.D4, W.C6, W.LA8])
+def test_dwt_every_length(filt, dtype):
+    """Whole signals (up to 4096 samples, or up to four levels) and tiles."""
+    lens, levels = [], []
+    for k in range(1, 18):
+        n = 1 << k
+        if n < W.FILTER_LENGTHS[filt]:
+            continue
+        jmax = O.levels(n, 0, filt)
+        for J in sorted({1, 4, 5, 6, 9, jmax} & set(range(1, jmax + 1))):
+            lens.append(n)
+            levels.append(J)
+    count = len(lens)
+    check(lens, [filt] * count, [W.DWT] * count, levels, dtype, seed=10 + filt)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hardness", [W.SOFT, W.HARD])
 def test_in_place(hardness, dtype):
     rng = np.random.Generator(np.random.PCG64(4))
@@ -66,7 +83,7 @@ def test_in_place(hardness, dtype):
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_split_workspace(dtype):
     # each long signal needs more than half of the tiles' workspace
-    k = 26 if dtype == torch.float64 else 27
+    k = 27 if dtype == torch.float64 else 28
     lens = [1 << k, 1 << 12, 1 << k, 1 << 9]
     check(lens, [W.LA8, W.D4, W.HAAR, W.C6], [W.MODWT, W.DWT, W.MODWT, W.MODWT], [6, 0, 3, 5],
           dtype, seed=9)

@@ -2,16 +2,16 @@
 //
 // Thousands of independent signals of power-of-two lengths are smoothed
 // (forward transform -> hard/soft universal threshold -> inverse) by a fixed
-// sequence of launches, whatever their mix: the head tiles of every MODWT
-// signal (batch_tile.h), the persistent kernel below, and the MODWT's two
-// shrink passes.  The persistent workgroups take whole signals from a device
+// sequence of launches, whatever their mix: the head tiles of every signal
+// (batch_tile.h), the persistent kernel below, and the two shrink passes.  The persistent workgroups take whole signals from a device
 // work queue: an atomic counter over an item list sorted longest-first, so
 // the large signals start first and the small ones fill the tail.
 //
 //   MODWT: the item is the exact MAD of D_1 (the reference's univ_thresh(w,
 //   0, 0): src/thresh.cpp:170-201, src/rfunctions.cu:82-87), which the head
 //   left in the workspace.
-//   DWT: the whole smoothing.  Levels run on compact sequences, through the
+//   DWT: the same and the levels beyond the head's, or, of signals without
+//   tiles, the whole smoothing.  Levels run on compact sequences, through the
 //   workgroup's slice of scratch while they are longer than the LDS tile and
 //   in LDS afterwards; the MAD is taken over the level-1 details (all of
 //   x[1..n-1] when J = 1, as in the reference) and the inverse thresholds
@@ -33,7 +33,8 @@ __host__ __device__ constexpr int kind_filter(int kind) { return kind & 7; }
 
 // One signal of the batch.
 struct BatchItem {
-  int64_t off;    // first sample in the packed signal buffers (MODWT: D_1 in the tiles' workspace)
+  int64_t off;    // first sample in the packed signal buffers
+  int64_t scr;    // the tiles' workspace of the signal, or -1: no tiles
   double factor;  // sqrt(2 ln n) (sqrt(2 ln(n-1)) for a one-level DWT)
   int32_t n;      // length (power of two)
   int32_t J;      // levels
@@ -49,7 +50,7 @@ struct BatchArgs {
   void* y;
   double* thresh_out;  // optional, one per signal
   double* thresh;      // one per signal, for the shrink passes
-  const void* tiles;   // the MODWT tiles' workspace
+  void* tiles;         // the tiles' workspace
   void* scratch;
   int64_t scratch_stride;  // elements per workgroup
   int hardness;
@@ -76,21 +77,6 @@ constexpr int batch_lds_elems() {
   return 4096;
 }
 
-// FP64 512-thread workgroups keep a first-digit histogram of the median's
-// values (2048 counts) at this LDS offset, beyond the DWT's LDS levels (64
-// KB) and the selection's workspace; the plan sizes the launch's LDS to cover it.  Other shapes
-// would need more LDS per workgroup than they have to spare.
-constexpr size_t kBatchPreOff = size_t(64) << 10;
-constexpr size_t kBatchPreEnd = kBatchPreOff + size_t(kSelBins) * 4;
-// LDS the histogram needs for NT threads and esz-byte elements (0: none)
-__host__ __device__ constexpr size_t batch_pre_lds(int NT, size_t esz) {
-  return (esz == 8 && NT == 512) ? kBatchPreEnd : 0;
-}
-template <typename T, int NT>
-__host__ __device__ constexpr bool batch_pre() {
-  return batch_pre_lds(NT, sizeof(T)) != 0;
-}
-
 // DWT item coefficients in scratch C, level by level and each level
 // contiguous: d_j at C[n - n/2^{j-1} ..) (n/2^j values), then s_J; for
 // J = 1, s_1[0] goes last, so that C[0 .. n-1) holds d_1 and s_1[1..]: the
@@ -106,8 +92,8 @@ __device__ __forceinline__ int64_t batch_dwt_sidx(int64_t n, int J, int64_t m) {
 // longer than the LDS tile and in LDS afterwards; the coefficients end in
 // scratch C as above (n values, gA/gB n/2 each behind it).
 template <typename T, int FILT, int NT>
-__device__ __forceinline__ void batch_dwt_fwd(const BatchArgs& b, const BatchItem& I, T* C,
-                                              unsigned char* smem, unsigned* pre) {
+__device__ __forceinline__ void batch_dwt_fwd(const T* x, int64_t n, int J, T* C,
+                                              unsigned char* smem) {
   constexpr int L = Filter<FILT>::L;
   constexpr int kBatchLds = batch_lds_elems<T>();
   constexpr int kUp = 2;  // global-level output pairs of pairs per thread in flight
@@ -116,12 +102,8 @@ __device__ __forceinline__ void batch_dwt_fwd(const BatchArgs& b, const BatchIte
   T* lB = lA + kBatchLds;
   const int tid = threadIdx.x;
   {
-    const int64_t n = I.n;
-    const int J = I.J;
     T* gA = C + n;          // n/2
     T* gB = gA + n / 2;     // n/2
-    const T* x = static_cast<const T*>(b.x) + I.off;
-    T* y = static_cast<T*>(b.y) + I.off;
 
     // ---- forward: global levels while the input is longer than the tile
     const T* src = x;
@@ -159,10 +141,6 @@ __device__ __forceinline__ void batch_dwt_fwd(const BatchArgs& b, const BatchIte
             fwd_pair<T, FILT>(v[u] + 2, s1, d1);
             *reinterpret_cast<T2*>(dst + 2 * p) = T2{s0, s1};
             *reinterpret_cast<T2*>(dj + 2 * p) = T2{d0, d1};
-            if (pre && j == 1) {
-              atomicAdd(&pre[sel_digit0(d0)], 1u);
-              atomicAdd(&pre[sel_digit0(d1)], 1u);
-            }
           }
         }
       }
@@ -196,7 +174,6 @@ __device__ __forceinline__ void batch_dwt_fwd(const BatchArgs& b, const BatchIte
         fwd_pair<T, FILT>(v, s, d);
         nxt[m] = s;
         C[batch_dwt_doff(n, j) + m] = d;
-        if (pre && j == 1) atomicAdd(&pre[sel_digit0(d)], 1u);
       }
       __syncthreads();
       T* t = cur;
@@ -214,8 +191,8 @@ __device__ __forceinline__ void batch_dwt_fwd(const BatchArgs& b, const BatchIte
 // thresholding inverse into y (levels J.. in LDS while the output fits the
 // tile, the long levels through gA/gB)
 template <typename T, int FILT, int NT>
-__device__ __forceinline__ void batch_dwt_inv(const BatchArgs& b, const BatchItem& I, T* C,
-                                              unsigned char* smem, double t) {
+__device__ __forceinline__ void batch_dwt_inv(T* y, int64_t n, int J, T* C,
+                                              unsigned char* smem, double t, int hardness) {
   constexpr int L = Filter<FILT>::L;
   constexpr int kBatchLds = batch_lds_elems<T>();
   constexpr int kUp = 2;  // global-level output pairs of pairs per thread in flight
@@ -224,11 +201,8 @@ __device__ __forceinline__ void batch_dwt_inv(const BatchArgs& b, const BatchIte
   T* lB = lA + kBatchLds;
   const int tid = threadIdx.x;
   {
-    const int64_t n = I.n;
-    const int J = I.J;
     T* gA = C + n;          // n/2
     T* gB = gA + n / 2;     // n/2
-    T* y = static_cast<T*>(b.y) + I.off;
     const T tt = T(t);
     int64_t N;
     T* cur;
@@ -254,7 +228,7 @@ __device__ __forceinline__ void batch_dwt_inv(const BatchArgs& b, const BatchIte
         for (int q = 0; q < L / 2; ++q) {
           const int mm = (m - q) & int(N - 1);
           sv[q] = cur[mm];
-          dv[q] = thresh_coef(C[batch_dwt_doff(n, j) + mm], tt, b.hardness);
+          dv[q] = thresh_coef(C[batch_dwt_doff(n, j) + mm], tt, hardness);
         }
         T e, o;
         inv_pair<T, FILT>(sv, dv, e, o);
@@ -309,7 +283,7 @@ __device__ __forceinline__ void batch_dwt_inv(const BatchArgs& b, const BatchIte
             const int64_t p = p0 + int64_t(u) * NT;
             if (p < np) {
 #pragma unroll
-              for (int i = 0; i < 2 * K; ++i) wd[u][i] = thresh_coef(wd[u][i], tt, b.hardness);
+              for (int i = 0; i < 2 * K; ++i) wd[u][i] = thresh_coef(wd[u][i], tt, hardness);
               // output m = 2p + r reads s_j[m - q] = w[2K - 2 + r - q]
               T sv[H], dv[H], e0, o0, e1, o1;
 #pragma unroll
@@ -351,45 +325,39 @@ __global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
     const int it = batch_next(b.counter, &item_sh);
     if (it >= b.count) break;
     const BatchItem I = b.items[it];
-    const int64_t n = I.n;
-    const bool dwt = kind_ttype(I.kind) == kDWT;
-    // the forward counts the first radix digit of the values the median
-    // selects from (the level-1 details; not for a one-level DWT, whose
-    // selection also takes s_1[1..]) into LDS the forward and the
-    // selection leave free
-    unsigned* pre = nullptr;
-    if constexpr (batch_pre<T, NT>()) {
-      if (dwt && I.J != 1) {
-        pre = reinterpret_cast<unsigned*>(smem + kBatchPreOff);
-        for (int i = threadIdx.x; i < kSelBins; i += NT) pre[i] = 0;
-        __syncthreads();
-      }
-    }
+    const bool dwt = kind_ttype(I.kind) == kDWT, tiled = I.scr >= 0;
+    // a tiled signal's D_1 is in the tiles' workspace; the DWT's levels beyond
+    // the head's run here, from s_4 to s'_4
+    const int64_t n = dwt && tiled ? I.n >> kBatchHead : I.n;
+    const int J = dwt && tiled ? I.J - kBatchHead : I.J;
+    T* d1 = tiled ? static_cast<T*>(b.tiles) + I.scr : scr;
+    T* s4 = d1 + batch_pad(I.n);
+    const T* in = tiled ? s4 : static_cast<const T*>(b.x) + I.off;
+    T* out = tiled ? s4 + batch_pad(n) : static_cast<T*>(b.y) + I.off;
     if (dwt) {
       switch (kind_filter(I.kind)) {
-        case kHAAR: batch_dwt_fwd<T, kHAAR, NT>(b, I, scr, smem, pre); break;
-        case kD4: batch_dwt_fwd<T, kD4, NT>(b, I, scr, smem, pre); break;
-        case kC6: batch_dwt_fwd<T, kC6, NT>(b, I, scr, smem, pre); break;
-        default: batch_dwt_fwd<T, kLA8, NT>(b, I, scr, smem, pre); break;
+        case kHAAR: batch_dwt_fwd<T, kHAAR, NT>(in, n, J, scr, smem); break;
+        case kD4: batch_dwt_fwd<T, kD4, NT>(in, n, J, scr, smem); break;
+        case kC6: batch_dwt_fwd<T, kC6, NT>(in, n, J, scr, smem); break;
+        default: batch_dwt_fwd<T, kLA8, NT>(in, n, J, scr, smem); break;
       }
       batch_phase();
     }
     // the universal threshold from the level-1 details: one call site for
     // every kind of item, so the selection is inlined once (a called
     // function would keep its saved registers in scratch memory)
-    const T* det = dwt ? scr : static_cast<const T*>(b.tiles) + I.off;
-    const int64_t mcount = dwt ? (I.J == 1 ? n - 1 : n / 2) : n;
-    const double t = block_mad<T, NT>(det, 0, 1, mcount, smem, pre) * I.factor;
+    const int64_t mcount = !dwt ? n : tiled ? I.n / 2 : J == 1 ? n - 1 : n / 2;
+    const double t = block_mad<T, NT>(d1, 0, 1, mcount, smem) * I.factor;
     if (threadIdx.x == 0) {
       b.thresh[I.sig] = t;
       if (b.thresh_out) b.thresh_out[I.sig] = t;
     }
     if (!dwt) continue;
     switch (kind_filter(I.kind)) {
-      case kHAAR: batch_dwt_inv<T, kHAAR, NT>(b, I, scr, smem, t); break;
-      case kD4: batch_dwt_inv<T, kD4, NT>(b, I, scr, smem, t); break;
-      case kC6: batch_dwt_inv<T, kC6, NT>(b, I, scr, smem, t); break;
-      default: batch_dwt_inv<T, kLA8, NT>(b, I, scr, smem, t); break;
+      case kHAAR: batch_dwt_inv<T, kHAAR, NT>(out, n, J, scr, smem, t, b.hardness); break;
+      case kD4: batch_dwt_inv<T, kD4, NT>(out, n, J, scr, smem, t, b.hardness); break;
+      case kC6: batch_dwt_inv<T, kC6, NT>(out, n, J, scr, smem, t, b.hardness); break;
+      default: batch_dwt_inv<T, kLA8, NT>(out, n, J, scr, smem, t, b.hardness); break;
     }
     batch_phase();
   }
@@ -401,14 +369,6 @@ __global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
     }
   }
 }
-
-// the first-digit histogram at kBatchPreOff stays clear of what an FP64
-// 512-thread item puts in LDS before its selection: the DWT's LDS levels and
-// the selection's workspace
-static_assert(2 * batch_lds_elems<double>() * 8 <= int(kBatchPreOff),
-              "DWT LDS levels overlap the first-digit histogram");
-static_assert(block_sel_lds<512>() <= kBatchPreOff,
-              "selection workspace overlaps the first-digit histogram");
 
 struct BatchLaunch {
   int NT;

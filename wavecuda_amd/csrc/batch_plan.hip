@@ -20,8 +20,8 @@ namespace wh {
 // Signals smoothed together: as many as the tiles' workspace holds.
 struct BatchChunk {
   int item0 = 0, items = 0;  // of the persistent kernel
-  int64_t tile0[3] = {0, 0, 0};  // per pass
-  unsigned tiles[3] = {0, 0, 0};
+  int64_t tile0[kBatchPasses] = {};  // per pass
+  unsigned tiles[kBatchPasses] = {};
 };
 }  // namespace wh
 
@@ -63,23 +63,28 @@ int nt_index(int NT) { return NT == 512 ? 2 : (NT == 256 ? 1 : 0); }
 // The tiles' workspace is at most this large (a signal that needs more has a
 // chunk of its own): enough that the launches of a chunk fill the chip many
 // times over.
-constexpr int64_t kBatchTileBytes = int64_t(2) << 30;
+constexpr int64_t kBatchTileBytes = int64_t(4) << 30;
 
 // dynamic LDS of one item for NT threads
 size_t item_lds(int ttype, int NT, size_t esz) {
   size_t b = (NT == 512) ? block_sel_lds<512>()
              : (NT == 256 ? block_sel_lds<256>() : block_sel_lds<128>());
   if (ttype != kDWT) return b;
-  b = std::max(b, batch_pre_lds(NT, esz));  // the forward's first-digit histogram
   const size_t tile = (esz == 8) ? size_t(batch_lds_elems<double>()) * 8
                                  : size_t(batch_lds_elems<float>()) * 4;
   return std::max(b, 2 * tile);
 }
 
+// a DWT signal whose first levels run as tiles
+bool dwt_tiled(const BatchItem& I) { return I.n > kBatchDwtWhole && I.J > kBatchHead; }
+
 // The tiles of one signal in a pass; t.kind holds filter and depth.
 void add_tiles(std::vector<BatchTile>& tiles, BatchTile t, BatchPass pass) {
   const int J = tile_levels(t.kind), kind = t.kind;
-  if (pass == BatchPass::kHead) {
+  const bool dwt = kind & kTileDwt;
+  const bool last = pass == BatchPass::kDwtLast;
+  if (pass != BatchPass::kHead && dwt != last) return;
+  if (last || pass == BatchPass::kHead) {
     for (t.m0 = 0; t.m0 < t.n; t.m0 += kBatchP) tiles.push_back(t);
     return;
   }
@@ -106,9 +111,9 @@ void add_tiles(std::vector<BatchTile>& tiles, BatchTile t, BatchPass pass) {
   }
 }
 
-// Chunks, tiles and workspace of a batch's items, longest first.  MODWT items
-// get their workspace offset and fill the chunks in order; the DWT's belong to
-// the first.  Tiles of one filter and depth are neighbours, so that a CU's
+// Chunks, tiles and workspace of a batch's items, longest first.  Signals with
+// tiles get their workspace offset and fill the chunks in order; the others
+// belong to the first.  Tiles of one filter and depth are neighbours, so that a CU's
 // workgroups run the same code.
 void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
                  std::vector<BatchChunk>& chunks, int64_t budget, int64_t* workspace) {
@@ -117,7 +122,9 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
   int64_t used = 0;
   *workspace = 0;
   for (BatchItem I : items) {
-    if (kind_ttype(I.kind) == kDWT) {
+    I.scr = -1;
+    const bool dwt = kind_ttype(I.kind) == kDWT;
+    if (dwt && !dwt_tiled(I)) {
       by_chunk[0].push_back(I);
       continue;
     }
@@ -127,8 +134,9 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
       heads.emplace_back();
       used = 0;
     }
-    heads.back().push_back(BatchTile{I.off, used, I.n, 0, kind_filter(I.kind) | (I.J << 3), I.sig});
-    I.off = used;
+    heads.back().push_back(BatchTile{
+        I.off, used, I.n, 0, kind_filter(I.kind) | (I.J << 3) | (dwt ? kTileDwt : 0), I.sig});
+    I.scr = used;
     by_chunk.back().push_back(I);
     used += need;
     *workspace = std::max(*workspace, used);
@@ -141,7 +149,7 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
     items.insert(items.end(), by_chunk[k].begin(), by_chunk[k].end());
     std::stable_sort(heads[k].begin(), heads[k].end(),
                      [](const BatchTile& a, const BatchTile& b) { return a.kind > b.kind; });
-    for (int pass = 0; pass < 3; ++pass) {
+    for (int pass = 0; pass < kBatchPasses; ++pass) {
       c.tile0[pass] = int64_t(tiles.size());
       for (const BatchTile& t : heads[k]) add_tiles(tiles, t, BatchPass(pass));
       c.tiles[pass] = unsigned(int64_t(tiles.size()) - c.tile0[pass]);
@@ -226,6 +234,7 @@ int run(wh_batch* p, int NT, unsigned grid, const void* x, void* y, double* thre
       return rc;
     if (int rc = tile_pass(p, c, BatchPass::kSecond, t, st)) return rc;
     if (int rc = tile_pass(p, c, BatchPass::kFirst, t, st)) return rc;
+    if (int rc = tile_pass(p, c, BatchPass::kDwtLast, t, st)) return rc;
   }
   return WH_OK;
 }
@@ -283,16 +292,18 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     const double nn = (tt == kDWT && J == 1) ? double(n - 1) : double(n);
     I.factor = std::sqrt(2.0 * std::log(nn));
     off += n;
-    if (tt == kDWT) stride = std::max<int64_t>(stride, 2 * n);
+    if (tt == kDWT) stride = std::max<int64_t>(stride, 2 * (dwt_tiled(I) ? n >> kBatchHead : n));
     for (int k = 0; k < 3; ++k) lds[k] = std::max(lds[k], item_lds(tt, kNTs[k], esz));
     int lg = 0;
     while ((int64_t(1) << lg) < n) ++lg;
     comp[(int64_t(I.kind) << 16) | (lg << 8) | J] += 1;
   }
-  // longest work first within a chunk: a MODWT's item is the selection from
-  // D_1, the DWT moves about 6 words per sample plus its level-serial latency
+  // longest work first within a chunk: the selection passes over D_1, the
+  // DWT's levels move about 6 words per sample plus their serial latency
   auto cost = [](const BatchItem& I) {
-    return kind_ttype(I.kind) == kMODWT ? int64_t(I.n) * 2 : int64_t(I.n) * 6 + 256 * I.J;
+    if (kind_ttype(I.kind) == kMODWT) return int64_t(I.n) * 2;
+    if (dwt_tiled(I)) return int64_t(I.n) + (int64_t(I.n) >> kBatchHead) * 6 + 256 * I.J;
+    return int64_t(I.n) * 6 + 256 * I.J;
   };
   std::stable_sort(items.begin(), items.end(),
                    [&](const BatchItem& a, const BatchItem& b) { return cost(a) > cost(b); });

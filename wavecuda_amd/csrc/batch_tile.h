@@ -1,23 +1,27 @@
-// batch_tile.h -- tiles of the batched MODWT smoothing.
+// batch_tile.h -- tiles of the batched smoothing.
 //
 // A signal's universal threshold needs its level-1 details only, so a batch
 // is smoothed in passes over tiles of all signals at once: the head writes
 // D_1 and, for more than kBatchHead levels, S_4; the threshold follows from
-// D_1 (batch_kern.h); then the levels beyond the fourth are computed,
+// D_1 (batch_kern.h); then the MODWT's levels beyond the fourth are computed,
 // thresholded and inverted in one pass over S_4 (giving S'_4), and the first
-// four in one pass over the signal and S'_4.  No detail level but the first
-// is ever stored: recomputing four levels costs 32 LDS-fed FMA pairs per
+// four levels in one pass over the signal and S'_4.  No detail level but the
+// first is ever stored: recomputing four levels costs 32 LDS-fed FMA pairs per
 // sample (LA8) where storing and reading their details costs 8 words, and
 // the deeper levels are computed once, in the pass that thresholds them.
 //
-// Beyond the fourth level a tap's distance is a multiple of 16, so S_4 is
-// kept residue by residue: 16 circular sequences of n / 16 contiguous values,
-// on which levels 5..8 are levels 1..4.  Every pass is therefore the same
-// tile: consecutive values of a circular sequence, with the halo its levels
-// need (W = (L-1)(2^G - 1): 105 for LA8 and 4 levels), or, where sequences are shorter than a tile, whole sequences
-// without any.  All arithmetic is the single-signal path's, term by term.
+// MODWT: beyond the fourth level a tap's distance is a multiple of 16, so S_4
+// is kept residue by residue: 16 circular sequences of n / 16 contiguous
+// values, on which levels 5..8 are levels 1..4.  Every pass is therefore the
+// same tile: consecutive values of a circular sequence, with the halo its
+// levels need (W = (L-1)(2^G - 1): 105 for LA8 and 4 levels), or, where
+// sequences are shorter than a tile, whole sequences without any.
+// DWT (signals longer than kBatchDwtWhole): s_4 is a sixteenth of the signal,
+// and the levels beyond it run in the persistent kernel.
+// All arithmetic is the single-signal path's, term by term.
 #pragma once
 
+#include "dwt_dev.h"
 #include "modwt_tile.h"
 
 namespace wh {
@@ -28,19 +32,23 @@ constexpr int kBatchHead = 4;    // levels of the head group
 constexpr int kBatchMaxModwtJ = 2 * kBatchHead;  // deepest MODWT of a batch
 constexpr int kBatchRes = 1 << kBatchHead;       // residues of S_4
 
-// One tile of one signal.  The signal's workspace: D_1 (later S'_4), S_4 and
-// a copy of the signal (batches smoothed in place), batch_pad(n) values each.
+constexpr int kBatchDwtWhole = 4096;  // longest DWT signal that is no tiles
+
+// One tile of one signal.  The signal's workspace: D_1 (later S'_4), S_4 (the
+// DWT's s_4 and s'_4) and a copy of the signal (batches smoothed in place),
+// batch_pad(n) values each.
 struct BatchTile {
   int64_t off;   // the signal's first sample
   int64_t scr;   // its workspace
   int32_t n;
   int32_t m0;    // first value stored, of its sequence
-  int32_t kind;  // filter | J << 3 | first sequence << 8
+  int32_t kind;  // filter | J << 3 | first sequence << 8 | DWT << 16
   int32_t sig;
 };
 
 __host__ __device__ constexpr int tile_levels(int kind) { return (kind >> 3) & 31; }
-__host__ __device__ constexpr int tile_seq(int kind) { return kind >> 8; }
+__host__ __device__ constexpr int tile_seq(int kind) { return (kind >> 8) & 255; }
+constexpr int kTileDwt = 1 << 16;
 
 __host__ __device__ constexpr int64_t batch_pad(int64_t n) { return (n + 63) / 64 * 64; }
 
@@ -132,6 +140,177 @@ __device__ __forceinline__ void batch_head(const BatchTileArgs& a, const BatchTi
     level(std::integral_constant<int, 4>{});
   }
 }
+
+// -------------------------------------------------------------------- DWT
+// Tiles of kBatchP samples: level l owns kBatchP / 2^l values, computes R(l)
+// more to the right for the level above it and, in the last pass, E(l) to
+// the left, H(l) of which the inverse reads.  The head moves 1.6 words a
+// sample, the last pass 2.1.  One buffer serves every level, a level's outputs
+// waiting in registers until every tap has been read.
+// Threads of the last pass: it is bound by its short levels' instructions, so
+// fewer threads with more values each are faster (8192 mixed signals FP64:
+// 1024 threads 720 us, 512 413, 256 308, 128 281, 64 461, whose registers
+// leave one wave per SIMD).
+constexpr int kDwtLastNT = 128;
+
+template <typename T, int FILT, int NT>
+struct DwtTile {
+  typedef T T2 __attribute__((ext_vector_type(2)));
+  static constexpr int L = Filter<FILT>::L, A = kBatchHead;
+  static constexpr int R(int l) { return l == A ? 0 : 2 * R(l + 1) + L - 2; }
+  static constexpr int H(int l) { return l == 0 ? 0 : (H(l - 1) + 1) / 2 + L / 2 - 1; }
+  static constexpr int own(int l) { return kBatchP >> l; }
+  // values computed of level l, `left` of level 0 to the left of the tile's
+  static constexpr int cnt(int l, int left) { return own(l) + (left >> l) + R(l); }
+  static constexpr int kLeft = H(A) << A;
+  static constexpr int kElems = own(0) + kLeft + R(0);
+  static constexpr int per(int n) { return (n + NT - 1) / NT; }
+
+  // s_0 of the tile from x (and its copy to xc) into b
+  template <int left>
+  static __device__ __forceinline__ void load(const T* __restrict__ x, T* xc, int64_t n, int m0,
+                                              T* b) {
+    constexpr int np = cnt(0, left) / 2, K = per(np);
+    T2 v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int p = int(threadIdx.x) + k * NT;
+      const int pc = p < np ? p : np - 1;  // unconditional load, clamped
+      v[k] = *reinterpret_cast<const T2*>(x + ((m0 - left + 2 * pc) & (n - 1)));
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int p = int(threadIdx.x) + k * NT;
+      if (p < np) *reinterpret_cast<T2*>(b + 2 * p) = v[k];
+      if (xc && p < own(0) / 2) *reinterpret_cast<T2*>(xc + m0 + 2 * p) = v[k];
+    }
+    __syncthreads();
+  }
+  // level l of the buffer: f(slot, k, s, d); s_l replaces s_{l-1} unless l = A
+  template <int l, int left, typename F>
+  static __device__ __forceinline__ void level(T* b, F f) {
+    constexpr int no = cnt(l, left), K = per(no);
+    T s[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int m = int(threadIdx.x) + k * NT;
+      if (m < no) {
+        T v[L], d;
+#pragma unroll
+        for (int j = 0; j < L; j += 2) {
+          const T2 pr = *reinterpret_cast<const T2*>(b + 2 * m + j);
+          v[j] = pr.x;
+          v[j + 1] = pr.y;
+        }
+        fwd_pair<T, FILT>(v, s[k], d);
+        batch_pin(s[k]);
+        f(m, k, s[k], d);
+      }
+    }
+    __syncthreads();
+    if constexpr (l < A) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int m = int(threadIdx.x) + k * NT;
+        if (m < no) b[m] = s[k];
+      }
+      __syncthreads();
+    }
+  }
+
+  static __device__ __forceinline__ void head(const BatchTileArgs& a, const BatchTile& I, T* b) {
+    const int64_t n = I.n;
+    T* d1 = static_cast<T*>(a.scratch) + I.scr + I.m0 / 2;
+    T* s4 = static_cast<T*>(a.scratch) + I.scr + batch_pad(n) + (I.m0 >> A);
+    T* xc = static_cast<T*>(a.scratch) + I.scr + 2 * batch_pad(n);
+    load<0>(static_cast<const T*>(a.x) + I.off, a.in_place ? xc : nullptr, n, I.m0, b);
+    level<1, 0>(b, [&](int m, int, T, T d) {
+      if (m < own(1)) d1[m] = d;
+    });
+    level<2, 0>(b, [](int, int, T, T) {});
+    level<3, 0>(b, [](int, int, T, T) {});
+    level<A, 0>(b, [&](int m, int, T s, T) { s4[m] = s; });
+  }
+
+  // level l's (s', d) in S and D from slot of position own start - H(l) on:
+  // l - 1's, whose details are d[]
+  template <int l, int K>
+  static __device__ __forceinline__ void up(T* S, T* D, const T (&d)[K], T* y) {
+    constexpr int h = (H(l - 1) + 1) / 2, no = own(l) + h, KO = per(no), Q = L / 2;
+    T e[KO], o[KO];
+#pragma unroll
+    for (int k = 0; k < KO; ++k) {
+      const int m = int(threadIdx.x) + k * NT;
+      if (m < no) {
+        T sv[Q], dv[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          sv[q] = S[m + H(l) - h - q];
+          dv[q] = D[m + H(l) - h - q];
+        }
+        inv_pair<T, FILT>(sv, dv, e[k], o[k]);
+        batch_pin(e[k]);
+        batch_pin(o[k]);
+        if constexpr (l == 1) *reinterpret_cast<T2*>(y + 2 * m) = T2{e[k], o[k]};
+      }
+    }
+    if constexpr (l > 1) {
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < KO; ++k) {
+        const int m = int(threadIdx.x) + k * NT, j = 2 * (m - h) + H(l - 1);
+        if (m < no) {
+          if (j >= 0) S[j] = e[k];
+          S[j + 1] = o[k];
+        }
+      }
+      details<l - 1>(D, d);
+      __syncthreads();
+    }
+  }
+  template <int l, int K>
+  static __device__ __forceinline__ void details(T* D, const T (&d)[K]) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int j = int(threadIdx.x) + k * NT - ((kLeft >> l) - H(l));
+      if (j >= 0 && j < own(l) + H(l)) D[j] = d[k];
+    }
+  }
+
+  static __device__ __forceinline__ void last(const BatchTileArgs& a, const BatchTile& I, T* b) {
+    const int64_t n = I.n;
+    const T t = T(a.thresh[I.sig]);
+    const T* s4 = static_cast<const T*>(a.scratch) + I.scr + batch_pad(n) + batch_pad(n >> A);
+    const T* xc = static_cast<const T*>(a.scratch) + I.scr + 2 * batch_pad(n);
+    T* y = static_cast<T*>(a.y) + I.off + I.m0;
+    load<kLeft>(a.in_place ? xc : static_cast<const T*>(a.x) + I.off, nullptr, n, I.m0, b);
+    T d1[per(cnt(1, kLeft))], d2[per(cnt(2, kLeft))], d3[per(cnt(3, kLeft))],
+        d4[per(cnt(4, kLeft))];
+    const int hard = a.hardness;
+    auto cut = [&](T* d) {
+      return [=](int, int k, T, T v) {
+        d[k] = thresh_coef(v, t, hard);
+        batch_pin(d[k]);
+      };
+    };
+    level<1, kLeft>(b, cut(d1));
+    level<2, kLeft>(b, cut(d2));
+    level<3, kLeft>(b, cut(d3));
+    level<A, kLeft>(b, cut(d4));
+    T *S = b, *D = b + own(1) + H(1) + 1;
+#pragma unroll
+    for (int k = 0; k < per(own(A) + H(A)); ++k) {
+      const int c = int(threadIdx.x) + k * NT;
+      if (c < own(A) + H(A)) S[c] = s4[((I.m0 >> A) - H(A) + c) & ((n >> A) - 1)];
+    }
+    details<A>(D, d4);
+    __syncthreads();
+    up<4>(S, D, d3, y);
+    up<3>(S, D, d2, y);
+    up<2>(S, D, d1, y);
+    up<1>(S, D, d1, y);
+  }
+};
 
 // ------------------------------------------------------------------ shrink
 // G levels of a sequence array: forward, threshold, inverse.  The smooth of
@@ -410,6 +589,15 @@ template <typename T>
 __global__ __launch_bounds__(kBatchNT) void batch_head_k(BatchTileArgs a) {
   __shared__ __align__(16) T b[kBatchP + tile_halo(8, kBatchHead)];
   const BatchTile I = a.tiles[blockIdx.x];
+  if (I.kind & kTileDwt) {
+    switch (I.kind & 7) {
+      case kHAAR: DwtTile<T, kHAAR, kBatchNT>::head(a, I, b); break;
+      case kD4: DwtTile<T, kD4, kBatchNT>::head(a, I, b); break;
+      case kC6: DwtTile<T, kC6, kBatchNT>::head(a, I, b); break;
+      default: DwtTile<T, kLA8, kBatchNT>::head(a, I, b); break;
+    }
+    return;
+  }
   const bool deep = tile_levels(I.kind) > kBatchHead, circ = I.n < kBatchP;
 #define WH_HEAD(F)                                              \
   if (deep) {                                                   \
@@ -440,8 +628,23 @@ __global__ __launch_bounds__(shrink_nt(SECOND), 4) void batch_shrink_k(BatchTile
   }
 }
 
+// The DWT's last pass, apart from the MODWT's, whose registers and LDS would
+// halve the workgroups of a CU.
+template <typename T>
+__global__ __launch_bounds__(kDwtLastNT) void batch_dwt_last_k(BatchTileArgs a) {
+  __shared__ __align__(16) T lds[DwtTile<T, kLA8, kDwtLastNT>::kElems];
+  const BatchTile I = a.tiles[blockIdx.x];
+  switch (I.kind & 7) {
+    case kHAAR: DwtTile<T, kHAAR, kDwtLastNT>::last(a, I, lds); break;
+    case kD4: DwtTile<T, kD4, kDwtLastNT>::last(a, I, lds); break;
+    case kC6: DwtTile<T, kC6, kDwtLastNT>::last(a, I, lds); break;
+    default: DwtTile<T, kLA8, kDwtLastNT>::last(a, I, lds); break;
+  }
+}
+
 // launches over tiles [0, count); defined in batch_tile_<type>.hip
-enum class BatchPass { kHead, kSecond, kFirst };
+enum class BatchPass { kHead, kSecond, kFirst, kDwtLast };
+constexpr int kBatchPasses = 4;
 template <typename T>
 int batch_tile_launch(BatchPass pass, unsigned count, const BatchTileArgs& a, hipStream_t st);
 
@@ -449,9 +652,15 @@ template <typename T>
 int batch_tile_launch_impl(BatchPass pass, unsigned count, const BatchTileArgs& a,
                            hipStream_t st) {
   if (!count) return WH_OK;
-  const dim3 grid(count), nt(pass == BatchPass::kHead ? kBatchNT : shrink_nt(pass == BatchPass::kSecond));
+  const dim3 grid(count);
+  const bool shrink = pass == BatchPass::kFirst || pass == BatchPass::kSecond;
+  const dim3 nt(shrink ? shrink_nt(pass == BatchPass::kSecond)
+                       : pass == BatchPass::kHead ? kBatchNT : kDwtLastNT);
   switch (pass) {
     case BatchPass::kHead: hipLaunchKernelGGL((batch_head_k<T>), grid, nt, 0, st, a); break;
+    case BatchPass::kDwtLast:
+      hipLaunchKernelGGL((batch_dwt_last_k<T>), grid, nt, 0, st, a);
+      break;
     case BatchPass::kSecond:
       hipLaunchKernelGGL((a.hardness == kHARD ? batch_shrink_k<T, true, true>
                                               : batch_shrink_k<T, true, false>),
