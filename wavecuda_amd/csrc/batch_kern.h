@@ -70,8 +70,9 @@ __device__ __forceinline__ int batch_next(int* counter, int* sh) {
 // write back and invalidate the L2 of the workgroup's XCD at every item.
 __device__ __forceinline__ void batch_phase() { __syncthreads(); }
 
-// LDS elements per ping-pong buffer of the DWT tail (64 KB in FP64, 32 KB
-// in FP32, so that several FP32 workgroups share a CU)
+// Longest sequence in LDS.  A level's outputs (forward) or inputs (inverse) are
+// half of it, so the second buffer has half the size: 48 KB in FP64, three
+// workgroups a CU.
 template <typename T>
 constexpr int batch_lds_elems() {
   return 4096;
@@ -212,14 +213,17 @@ __device__ __forceinline__ void batch_dwt_inv(T* y, int64_t n, int J, T* C,
     // ---- inverse: levels J.. in LDS while the output fits the tile
     N = n >> J;  // length of s_J
     const bool lds_tail = (2 * N <= kBatchLds);
+    // levels that run in LDS: the last one's outputs need the whole buffer lA
+    int steps = 0;
+    while (steps < J && (N << steps) * 2 <= kBatchLds) ++steps;
+    cur = (steps & 1) ? lB : lA;
+    nxt = (steps & 1) ? lA : lB;
     if (lds_tail) {
-      for (int64_t m = tid; m < N; m += NT) lA[m] = C[batch_dwt_sidx(n, J, m)];
+      for (int64_t m = tid; m < N; m += NT) cur[m] = C[batch_dwt_sidx(n, J, m)];
     } else {
       for (int64_t m = tid; m < N; m += NT) gA[m] = C[batch_dwt_sidx(n, J, m)];
     }
     batch_phase();
-    cur = lA;
-    nxt = lB;
     j = J;
     while (j >= 1 && 2 * N <= kBatchLds) {
       for (int m = tid; m < int(N); m += NT) {
@@ -317,7 +321,7 @@ __device__ __forceinline__ void batch_dwt_inv(T* y, int64_t n, int J, T* C,
 // empty; the last workgroup to leave rewinds the queue, so the launch can be
 // replayed (a captured graph) without a memset node.
 template <typename T, int NT>
-__global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
+__global__ __launch_bounds__(NT, NT == 128 ? 2 : 3) void batch_smooth_k(BatchArgs b) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int item_sh;
   T* scr = static_cast<T*>(b.scratch) + int64_t(blockIdx.x) * b.scratch_stride;
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(NT) void batch_smooth_k(BatchArgs b) {
     // every kind of item, so the selection is inlined once (a called
     // function would keep its saved registers in scratch memory)
     const int64_t mcount = !dwt ? n : tiled ? I.n / 2 : J == 1 ? n - 1 : n / 2;
-    const double t = block_mad<T, NT>(d1, 0, 1, mcount, smem) * I.factor;
+    const double t = block_mad<T, NT>(d1, mcount, smem) * I.factor;
     if (threadIdx.x == 0) {
       b.thresh[I.sig] = t;
       if (b.thresh_out) b.thresh_out[I.sig] = t;

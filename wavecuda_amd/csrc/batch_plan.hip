@@ -69,10 +69,11 @@ constexpr int64_t kBatchTileBytes = int64_t(4) << 30;
 size_t item_lds(int ttype, int NT, size_t esz) {
   size_t b = (NT == 512) ? block_sel_lds<512>()
              : (NT == 256 ? block_sel_lds<256>() : block_sel_lds<128>());
+  b = std::max({b, sel_sampled_lds(NT, esz), sel_small_lds(esz)});
   if (ttype != kDWT) return b;
   const size_t tile = (esz == 8) ? size_t(batch_lds_elems<double>()) * 8
                                  : size_t(batch_lds_elems<float>()) * 4;
-  return std::max(b, 2 * tile);
+  return std::max(b, tile + tile / 2);
 }
 
 // a DWT signal whose first levels run as tiles
@@ -379,9 +380,9 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     // untuned: 256 threads and every workgroup that fits, unless the longest
     // item would still run when the others are done: then 512 threads, which
     // take it in about two thirds of the time.  Mixed batches, us with 256 /
-    // 512 threads: 8192 signals to 2^16 samples FP64 2651 / 2843, FP32 1487 /
-    // 1770; 2000 to 2^16 FP64 737 / 738; 1200 to 2^16 (ratio 0.35 of the
-    // line's 0.4) FP64 508 / 441, FP32 354 / 287; 300 to 2^16 FP64 289 / 242.
+    // 512 threads: 8192 signals to 2^16 samples FP64 2188 / 2453, FP32 1382 /
+    // 1637; 2000 to 2^16 FP64 629 / 620; 1200 to 2^16 (0.27 where the line is
+    // 0.4) FP64 445 / 376, FP32 296 / 257; 300 to 2^16 FP64 256 / 156.
     // wh_batch_tune times the shapes.
     int64_t resident = 0;
     p->NT = 256;

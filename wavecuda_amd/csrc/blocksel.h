@@ -17,12 +17,13 @@
 // within its bucket is counted directly, one pass and one barrier instead
 // of a radix digit's five barriers for each remaining digit.
 //
-// Two shortcuts, both exact: the first digit's counts of the median's values
-// may come precomputed (the batched forward counts them as it produces the
-// level-1 details), and the deviations |v - med|, whose keys crowd a few
+// Two shortcuts, both exact: the deviations |v - med|, whose keys crowd a few
 // exponents, are first counted into equal-width bins over [0, bound], the
-// bound following from the extreme first digits the values have.
+// bound following from the extreme first digits the values have; and long
+// inputs are read once per median, see block_median_sampled.
 #pragma once
+
+#include <type_traits>
 
 #include "wh_common.h"
 
@@ -103,18 +104,17 @@ __device__ __forceinline__ int* sel_range_slot(unsigned char* ws) {
                                 size_t(NT) * 4 + 96);
 }
 
-// f(key) for every value v[off + e * stride], e < count (|v - center| when
-// deviation).  Contiguous values (stride 1, v + off aligned to 16 bytes)
-// are read 16 bytes at a time (two FP64 or four FP32 values per load);
-// kSelUnroll loads in flight per thread either way.
+// f(key) for every value v[e], e < count (|v - center| when deviation).
+// Values aligned to 16 bytes are read 16 bytes at a time (two FP64 or four
+// FP32 values per load); kSelUnroll loads in flight per thread either way.
 template <typename T, int NT, typename F>
-__device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t off, int64_t stride,
-                                             int64_t count, bool deviation, T c, F f) {
+__device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t count,
+                                             bool deviation, T c, F f) {
   constexpr int kW = 16 / int(sizeof(T));
   typedef T TW __attribute__((ext_vector_type(kW)));
   auto key_of = [&](T y) { return sel_key(deviation ? T(fabs(y - c)) : y); };
-  if (stride == 1 && reinterpret_cast<uintptr_t>(v + off) % sizeof(TW) == 0) {
-    const TW* __restrict__ vw = reinterpret_cast<const TW*>(v + off);
+  if (reinterpret_cast<uintptr_t>(v) % sizeof(TW) == 0) {
+    const TW* __restrict__ vw = reinterpret_cast<const TW*>(v);
     const int64_t nv = count / kW;
     for (int64_t b = threadIdx.x; b < nv; b += int64_t(NT) * kSelUnroll) {
       TW x[kSelUnroll];
@@ -133,7 +133,7 @@ __device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t of
       }
     }
     const int64_t tail = nv * kW;
-    if (threadIdx.x < count - tail) f(key_of(v[off + tail + threadIdx.x]));
+    if (threadIdx.x < count - tail) f(key_of(v[tail + threadIdx.x]));
     return;
   }
   for (int64_t b = threadIdx.x; b < count; b += int64_t(NT) * kSelUnroll) {
@@ -141,7 +141,7 @@ __device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t of
 #pragma unroll
     for (int u = 0; u < kSelUnroll; ++u) {
       const int64_t e = b + int64_t(u) * NT;
-      x[u] = (e < count) ? v[off + e * stride] : T(0);
+      x[u] = (e < count) ? v[e] : T(0);
     }
 #pragma unroll
     for (int u = 0; u < kSelUnroll; ++u) {
@@ -151,20 +151,18 @@ __device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t of
   }
 }
 
-// Median of v[off + e * stride], e < count (|v - center| when deviation),
+// Median of v[e], e < count (|v - center| when deviation),
 // computed by all NT threads of the workgroup; returns the same value in
-// every thread.  ws: block_sel_lds<NT>() bytes of LDS.  pre: optional
-// counts of the values' first digits (sel_digit0), kSelBins of them, which
-// then replace the first counting pass.  bound > 0 (deviations only): every
-// value lies in [0, bound]; one pass then counts the values into kSelBins
+// every thread.  ws: block_sel_lds<NT>() bytes of LDS.  bound > 0
+// (deviations only): every value lies in [0, bound]; one pass then counts the values into kSelBins
 // equal-width bins, and when the middle ranks' bins hold at most
 // kSelDirect values they are copied to LDS and ranked directly (otherwise
-// the radix digits start from the top).  With kRange, the smallest and
-// largest first digit any value has are left at sel_range_slot(ws).
-template <typename T, int NT, bool kRange = false>
-__device__ double block_median(const T* __restrict__ v, int64_t off, int64_t stride, int64_t count,
-                               bool deviation, double center, unsigned char* ws,
-                               const unsigned* pre, double bound) {
+// the radix digits start from the top).  Of values, the smallest and largest
+// first digit any has are left at sel_range_slot(ws).
+template <typename T, int NT>
+__device__ __forceinline__ double block_median(const T* __restrict__ v, int64_t count,
+                                               bool deviation, double center,
+                                               unsigned char* ws, double bound) {
   uint64_t* cand = reinterpret_cast<uint64_t*>(ws);                     // [kSelCap]
   unsigned* hist = reinterpret_cast<unsigned*>(cand + kSelCap);        // [2][kSelBins]
   unsigned* part = hist + 2 * kSelBins;                                 // [NT]
@@ -191,7 +189,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
     const double scale = double(kSelBins) / bound;
     for (int i = tid; i < kSelBins; i += NT) hist[i] = 0;
     __syncthreads();
-    sel_for_each<T, NT>(v, off, stride, count, deviation, c, [&](uint64_t k) {
+    sel_for_each<T, NT>(v, count, deviation, c, [&](uint64_t k) {
       atomicAdd(&hist[sel_bin(sel_val(k, (T*)nullptr), scale)], 1u);
     });
     __syncthreads();
@@ -236,7 +234,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
     const long long total = cs[0] + (b1 != b0 ? cs[1] : 0);
     if (total <= kSelDirect) {
       const long long r0 = ks[0], r1 = (b1 != b0 ? cs[0] : 0) + ks[1];
-      sel_for_each<T, NT>(v, off, stride, count, deviation, c, [&](uint64_t k) {
+      sel_for_each<T, NT>(v, count, deviation, c, [&](uint64_t k) {
         const int q = sel_bin(sel_val(k, (T*)nullptr), scale);
         if (q >= b0 && q <= b1) cand[atomicAdd(ncand, 1)] = k;
       });
@@ -311,10 +309,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
       break;
     }
     const int lo = hi > kSelBits ? hi - kSelBits : 0;
-    const bool counted = pre && hi == kbits;  // the first digit's counts are given
-    if (!counted) {
-      for (int i = tid; i < 2 * kSelBins; i += NT) hist[i] = 0;
-    }
+    for (int i = tid; i < 2 * kSelBins; i += NT) hist[i] = 0;
     __syncthreads();
     const uint64_t p0 = st[0], p1 = st[1];
     const bool same = (p0 == p1);
@@ -325,12 +320,10 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
       if (top == p0) atomicAdd(&hist[d], 1u);
       if (!same && top == p1) atomicAdd(&hist[kSelBins + d], 1u);
     };
-    if (counted) {
-      // nothing to count
-    } else if (in_lds) {
+    if (in_lds) {
       for (int i = tid; i < nc; i += NT) count_key(cand[i]);
     } else {
-      sel_for_each<T, NT>(v, off, stride, count, deviation, c, count_key);
+      sel_for_each<T, NT>(v, count, deviation, c, count_key);
     }
     __syncthreads();
     // Both ranks' bucket counts packed in one word (rank 0 in the low 32
@@ -339,7 +332,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
     // `per` buckets, a wave scans by shuffles, then the wave totals.
     uint64_t* wsum = reinterpret_cast<uint64_t*>(part);  // [kWaves]
     const long long k0 = ks[0], k1 = ks[1];  // the finder below updates ks
-    const unsigned* h0 = counted ? pre : hist;
+    const unsigned* h0 = hist;
     const unsigned* h1 = same ? h0 : hist + kSelBins;
     uint64_t loc = 0;
 #pragma unroll
@@ -384,7 +377,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
     __syncthreads();
     // the first digit's counts cover every value: their extreme digits
     // bound the values (the copy area is free until a copy pass)
-    if (kRange && hi == kbits) {
+    if (!deviation && hi == kbits) {
       int dmin, dmax;
       sel_digit_range<NT>(h0, reinterpret_cast<int*>(cand), &dmin, &dmax);
       if (tid == 0) {
@@ -399,7 +392,7 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
       const long long total = cs[0] + (q0 != q1 ? cs[1] : 0);
       if (total <= kSelCap) {
         // one more pass keeps the keys under the selected prefixes in LDS
-        sel_for_each<T, NT>(v, off, stride, count, deviation, c, [&](uint64_t k) {
+        sel_for_each<T, NT>(v, count, deviation, c, [&](uint64_t k) {
           const uint64_t top = k >> hi;
           if (top == q0 || top == q1) cand[atomicAdd(ncand, 1)] = k;
         });
@@ -414,40 +407,365 @@ __device__ double block_median(const T* __restrict__ v, int64_t off, int64_t str
   return 0.5 * (a + b);
 }
 
-// 1.4826 median|v - median(v)|
-// pre: optional first-digit counts of the values (see block_median).  The
-// smallest and largest first digits present (from pre or from the median's
-// own first digit) bound the values, so the deviations' median can start
-// from equal-width bins.
+// ------------------------------------------------- selection from a sample
+// Long inputs are read once per median instead of twice (the persistent
+// kernel of 8192 mixed signals in FP64 697 -> 493 us, with 48 KB of LDS
+// instead of 64): a sample of
+// kSelSample values gives a bracket around the middle ranks, one pass counts
+// the values below it and keeps those inside (about a fifteenth) in LDS, and
+// the ranks are resolved there.  Exact: the counts tell whether the middle
+// ranks lie inside; if not, or if too many values do, block_median starts
+// over from the whole input.
+constexpr int kSelSample = 2048;   // values sampled, in runs of kSelRun
+constexpr int kSelRun = 8;
+constexpr int kSelMargin = 96;     // sample ranks on either side of the middle, at most
+// values kept: a 512-thread workgroup has its CU's LDS alone, of the others
+// three share it
+__host__ __device__ constexpr int sel_gather(int NT) { return NT == 512 ? 8192 : 4608; }
+// below, the passes saved are shorter than the sample's
+constexpr int64_t kSelSampledMin = 16384;
+constexpr int64_t kSelSampledMax = 1 << 16;  // beyond, the bracket holds too many
+
+// keys as wide as the values
+template <typename T>
+using SelKey = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
+
+__host__ __device__ constexpr size_t sel_sampled_lds(int NT, size_t esz) {
+  return size_t(sel_gather(NT) + kSelDirect) * esz + size_t(kSelBins) * 4 + 16 * 8 + 256;
+}
+
+// Bins of the ranks r0 <= r1 in h[0..kSelBins): the bin, the count before it
+// and its own, for each rank, in f[0..2], f[3..5].  Ends with a barrier.
+template <int NT>
+__device__ __forceinline__ void sel_find(const unsigned* h, int r0, int r1, int* wsum, int* f) {
+  constexpr int per = kSelBins / NT, kWaves = NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int loc = 0;
+#pragma unroll
+  for (int i = 0; i < per; ++i) loc += int(h[tid * per + i]);
+  int inc = loc;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += t;
+  }
+  if (lane == 63) wsum[wave] = inc;
+  __syncthreads();
+  int before = inc - loc;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+    if (w < wave) before += wsum[w];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int k = r ? r1 : r0;
+    if (before <= k && k < before + loc) {
+      int acc = before;
+      for (int i = 0; i < per; ++i) {
+        const int c = int(h[tid * per + i]);
+        if (acc + c > k) {
+          f[3 * r] = tid * per + i;
+          f[3 * r + 1] = acc;
+          f[3 * r + 2] = c;
+          break;
+        }
+        acc += c;
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// The median of v[0..count) (of |v - center| when deviation) into *res, the
+// same in every thread; false: not resolved.  ws: sel_sampled_lds bytes.
 template <typename T, int NT>
-__device__ double block_mad(const T* __restrict__ v, int64_t off, int64_t stride, int64_t count,
-                            unsigned char* ws, const unsigned* pre = nullptr) {
-  const bool binned = count > kSelDirect;
-  // without pre the median's first digit gives the range
-  const double med =
-      (binned && !pre) ? block_median<T, NT, true>(v, off, stride, count, false, 0.0, ws, pre, 0.0)
-                       : block_median<T, NT>(v, off, stride, count, false, 0.0, ws, pre, 0.0);
-  int dr[2];
-  if (binned && pre) {
-    sel_digit_range<NT>(pre, reinterpret_cast<int*>(ws), &dr[0], &dr[1]);
-  } else {
-    const int* slot = sel_range_slot<NT>(ws);  // written before block_median's last barrier
-    dr[0] = slot[0];
-    dr[1] = slot[1];
+__device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, int64_t count,
+                                                     bool deviation, double center,
+                                                     unsigned char* ws, double* res) {
+  constexpr int kWaves = NT / 64, K = kSelSample / NT, kGather = sel_gather(NT);
+  constexpr int kRuns = kSelSample / kSelRun;
+  using Key = SelKey<T>;
+  Key* cand = reinterpret_cast<Key*>(ws);
+  Key* top = cand + kGather;                                     // [kSelDirect]
+  unsigned* hist = reinterpret_cast<unsigned*>(top + kSelDirect);   // [kSelBins]
+  double* red = reinterpret_cast<double*>(hist + kSelBins);         // [2 kWaves]
+  int* wsum = reinterpret_cast<int*>(red + 16);                     // [kWaves]
+  int* f = wsum + 8;                                                // [6]
+  int* ngat = f + 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const T c = T(center);
+  double s[K], mn = 1.0e300, mx = -1.0e300;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + k * NT;
+    const int64_t run = int64_t(i / kSelRun) * count / kRuns;
+    const int64_t p = (run & ~int64_t(kSelRun - 1)) + i % kSelRun;
+    const T x = v[p];
+    s[k] = double(deviation ? T(fabs(x - c)) : x);
+    mn = fmin(mn, s[k]);
+    mx = fmax(mx, s[k]);
   }
-  double bound = 0.0;
-  if (binned && dr[0] <= dr[1]) {
-    // every value lies in [vlo, vhi], the ends of those digits' key
-    // ranges; |v - med| computed as the selection computes it (v - med
-    // rounds monotonically in v) is then at most max(vhi - med, med - vlo)
-    constexpr int sh = int(sizeof(T)) * 8 - kSelBits;
-    const T vlo = T(sel_val(uint64_t(dr[0]) << sh, (T*)nullptr));
-    const T vhi = T(sel_val((uint64_t(dr[1]) << sh) | ((uint64_t(1) << sh) - 1), (T*)nullptr));
-    const T cm = T(med);
-    const double b = double(fmax(vhi - cm, cm - vlo));
-    if (b > 0.0 && b <= 1.0e300 && double(kSelBins) / b < 1.0e300) bound = b;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    mn = fmin(mn, __shfl_xor(mn, o, 64));
+    mx = fmax(mx, __shfl_xor(mx, o, 64));
   }
-  return 1.4826 * block_median<T, NT>(v, off, stride, count, true, med, ws, nullptr, bound);
+  if (lane == 0) {
+    red[wave] = mn;
+    red[kWaves + wave] = mx;
+  }
+  for (int i = tid; i < kSelBins; i += NT) hist[i] = 0;
+  if (tid == 0) *ngat = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    mn = fmin(mn, red[w]);
+    mx = fmax(mx, red[kWaves + w]);
+  }
+  const double scale = double(kSelBins) / (mx - mn);
+  if (!(mx > mn && mx - mn < 1.0e300 && scale < 1.0e300)) return false;  // (uniform)
+#pragma unroll
+  for (int k = 0; k < K; ++k) atomicAdd(&hist[sel_bin(s[k] - mn, scale)], 1u);
+  __syncthreads();
+  // ranks to either side: four standard deviations of independent samples, or
+  // what leaves the kept values room
+  const int fit = int(0.8 * double(kGather) / double(count) * double(kSelSample / 2));
+  const int margin = fit < kSelMargin ? fit : kSelMargin;
+  sel_find<NT>(hist, kSelSample / 2 - margin, kSelSample / 2 + margin, wsum, f);
+  const int b0 = f[0], b1 = f[3], inside = f[4] + f[5] - f[1];
+  if (double(inside) * double(count) > 0.9 * double(kSelSample) * double(kGather)) return false;
+  const T lo = T(mn + double(b0) / scale), hi = T(mn + double(b1 + 1) / scale);
+  const Key klo = Key(sel_key(lo)), khi = Key(sel_key(hi));
+  for (int i = tid; i < kSelBins; i += NT) hist[i] = 0;
+
+  // one pass: count below, keep inside
+  constexpr int kW = 16 / int(sizeof(T)), kU = 16 / kW;
+  typedef T TW __attribute__((ext_vector_type(kW)));
+  const TW* __restrict__ vw = reinterpret_cast<const TW*>(v);
+  const int nv = int(count / kW);  // count is a multiple of 64
+  int below = 0;
+  for (int b = tid; b < nv; b += NT * kU) {
+    TW x[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int p = b + u * NT;
+      x[u] = vw[p < nv ? p : b];
+    }
+    unsigned in = 0;  // bit per value
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+#pragma unroll
+      for (int w = 0; w < kW; ++w) {
+        const T y = x[u][w];
+        const Key k = Key(sel_key(deviation ? T(fabs(y - c)) : y));
+        const bool have = b + u * NT < nv;
+        below += have && k < klo;
+        in |= unsigned(have && k >= klo && k <= khi) << (u * kW + w);
+      }
+    }
+    const int mine = __popc(in);
+    int inc = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += t;
+    }
+    int base = 0;
+    if (lane == 63) base = atomicAdd(ngat, inc);
+    int at = __shfl(base, 63, 64) + inc - mine;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+#pragma unroll
+      for (int w = 0; w < kW; ++w) {
+        if (in >> (u * kW + w) & 1) {
+          const T y = x[u][w];
+          if (at < kGather) cand[at] = Key(sel_key(deviation ? T(fabs(y - c)) : y));
+          ++at;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o, 64);
+  if (lane == 0) wsum[wave] = below;
+  __syncthreads();
+  below = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) below += wsum[w];
+  const int n = *ngat;
+  const int r0 = int((count - 1) / 2) - below, r1 = int(count / 2) - below;
+  const double width = double(hi) - double(lo), sc = double(kSelBins) / width;
+  if (r0 < 0 || r1 >= n || n > kGather || !(width > 0.0 && sc < 1.0e300)) return false;
+  __syncthreads();  // wsum and ngat have been read
+  if (tid == 0) *ngat = 0;
+  auto bin = [&](Key k) { return sel_bin(sel_val(k, (T*)nullptr) - double(lo), sc); };
+  for (int i = tid; i < n; i += NT) atomicAdd(&hist[bin(cand[i])], 1u);
+  __syncthreads();
+  sel_find<NT>(hist, r0, r1, wsum, f);
+  const int q0 = f[0], q1 = f[3], first = f[1], last = f[4] + f[5];
+  if (last - first > kSelDirect) return false;
+  for (int i = tid; i < n; i += NT) {
+    const Key k = cand[i];
+    const int q = bin(k);
+    if (q >= q0 && q <= q1) top[atomicAdd(ngat, 1)] = k;
+  }
+  __syncthreads();
+  const int m = last - first, k0 = r0 - first, k1 = r1 - first;
+  for (int i = tid; i < m; i += NT) {
+    const Key x = top[i];
+    int lt = 0, eq = 0;
+    for (int j = 0; j < m; ++j) {
+      lt += top[j] < x;
+      eq += top[j] == x;
+    }
+    if (lt <= k0 && k0 < lt + eq) red[0] = sel_val(x, (T*)nullptr);
+    if (lt <= k1 && k1 < lt + eq) red[1] = sel_val(x, (T*)nullptr);
+  }
+  __syncthreads();
+  *res = 0.5 * (red[0] + red[1]);
+  __syncthreads();  // the workspace is free again
+  return true;
+}
+
+// Short inputs stay in registers: equal-width bins between the extremes, the
+// middle ranks' bins ranked directly, seven barriers a median.  Reading them
+// once per digit cost 20 to 25 us of latency an item, which bounded batches of
+// short signals.
+constexpr int kSelSmallPer = 8;  // values a thread
+
+// LDS: kSelDirect keys, the bins and what sel_find needs
+__host__ __device__ constexpr size_t sel_small_lds(size_t esz) {
+  return size_t(kSelDirect) * esz + size_t(kSelBins) * 4 + 16 * 8 + 256;
+}
+
+// 1.4826 median|v - median(v)| of count <= kSelSmallPer NT values into *res, the
+// same in every thread; false: not resolved (NaN, infinities, a crowded bin)
+template <typename T, int NT>
+__device__ __forceinline__ bool block_mad_small(const T* __restrict__ v, int count,
+                                                unsigned char* ws, double* res) {
+  using Key = SelKey<T>;
+  constexpr int kWaves = NT / 64, K = kSelSmallPer;
+  Key* top = reinterpret_cast<Key*>(ws);                            // [kSelDirect]
+  unsigned* hist = reinterpret_cast<unsigned*>(top + kSelDirect);   // [kSelBins]
+  double* red = reinterpret_cast<double*>(hist + kSelBins);         // [2 kWaves]
+  int* wsum = reinterpret_cast<int*>(red + 16);                     // [kWaves]
+  int* f = wsum + 8;                                                // [6]
+  int* ngat = f + 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  T x[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = tid + k * NT;
+    x[k] = v[e < count ? e : count - 1];
+  }
+  double med = 0.0;
+#pragma unroll 1
+  for (int dev = 0; dev < 2; ++dev) {
+    double mn = 1.0e300, mx = -1.0e300;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (dev) x[k] = T(fabs(x[k] - T(med)));
+      mn = fmin(mn, double(x[k]));
+      mx = x[k] == x[k] ? fmax(mx, double(x[k])) : double(INFINITY);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      mn = fmin(mn, __shfl_xor(mn, o, 64));
+      mx = fmax(mx, __shfl_xor(mx, o, 64));
+    }
+    if (lane == 0) {
+      red[wave] = mn;
+      red[kWaves + wave] = mx;
+    }
+    for (int i = tid; i < kSelBins; i += NT) hist[i] = 0;
+    if (tid == 0) *ngat = 0;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      mn = fmin(mn, red[w]);
+      mx = fmax(mx, red[kWaves + w]);
+    }
+    if (!(mx < 1.0e300 && mn > -1.0e300)) return false;  // (uniform)
+    const double width = mx - mn, scale = double(kSelBins) / width;
+    if (width > 0.0 && !(scale < 1.0e300)) return false;
+    if (width == 0.0) {
+      med = mn;
+      __syncthreads();  // red and hist are written again
+      continue;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (tid + k * NT < count) atomicAdd(&hist[sel_bin(double(x[k]) - mn, scale)], 1u);
+    __syncthreads();
+    const int r0 = (count - 1) / 2, r1 = count / 2;
+    sel_find<NT>(hist, r0, r1, wsum, f);
+    const int q0 = f[0], q1 = f[3], first = f[1], m = f[4] + f[5] - first;
+    if (m > kSelDirect) return false;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (tid + k * NT < count) {
+        const int q = sel_bin(double(x[k]) - mn, scale);
+        if (q >= q0 && q <= q1) top[atomicAdd(ngat, 1)] = Key(sel_key(x[k]));
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < m; i += NT) {
+      const Key y = top[i];
+      int lt = 0, eq = 0;
+      for (int j = 0; j < m; ++j) {
+        lt += top[j] < y;
+        eq += top[j] == y;
+      }
+      if (lt <= r0 - first && r0 - first < lt + eq) red[0] = sel_val(y, (T*)nullptr);
+      if (lt <= r1 - first && r1 - first < lt + eq) red[1] = sel_val(y, (T*)nullptr);
+    }
+    __syncthreads();
+    med = 0.5 * (red[0] + red[1]);
+    __syncthreads();  // red, hist and top are written again
+  }
+  *res = 1.4826 * med;
+  return true;
+}
+
+// 1.4826 median|v - median(v)|, v 16-byte aligned where it is long enough
+// to be sampled.  The smallest and largest first digits present (from the
+// median's own first digit) bound the values, so the deviations' median can
+// start from equal-width bins.
+template <typename T, int NT>
+__device__ __forceinline__ double block_mad(const T* __restrict__ v, int64_t count,
+                                            unsigned char* ws) {
+  const bool sampled = count >= kSelSampledMin && count <= kSelSampledMax &&
+                       reinterpret_cast<uintptr_t>(v) % 16 == 0 && count % 64 == 0;
+  if (count <= kSelSmallPer * NT) {
+    double mad;
+    if (block_mad_small<T, NT>(v, int(count), ws, &mad)) return mad;
+    __syncthreads();
+  }
+  double med[2] = {0.0, 0.0}, bound = 0.0;  // of the values, of the deviations
+#pragma unroll 1
+  for (int dev = 0; dev < 2; ++dev) {
+    double m;
+    if (!sampled || !block_median_sampled<T, NT>(v, count, dev, med[0], ws, &m)) {
+      __syncthreads();
+      m = block_median<T, NT>(v, count, dev, med[0], ws, bound);
+      const int* slot = sel_range_slot<NT>(ws);  // written before block_median's last barrier
+      const int d0 = slot[0], d1 = slot[1];
+      if (count > kSelDirect && d0 <= d1) {
+        // every value lies in [vlo, vhi], the ends of those digits' key
+        // ranges; |v - med| computed as the selection computes it (v - med
+        // rounds monotonically in v) is then at most max(vhi - med, med - vlo)
+        constexpr int sh = int(sizeof(T)) * 8 - kSelBits;
+        const T vlo = T(sel_val(uint64_t(d0) << sh, (T*)nullptr));
+        const T vhi = T(sel_val((uint64_t(d1) << sh) | ((uint64_t(1) << sh) - 1), (T*)nullptr));
+        const T cm = T(m);
+        const double b = double(fmax(vhi - cm, cm - vlo));
+        if (b > 0.0 && b <= 1.0e300 && double(kSelBins) / b < 1.0e300) bound = b;
+      }
+      __syncthreads();
+    }
+    if (dev) med[1] = m;
+    else med[0] = m;
+  }
+  return 1.4826 * med[1];
 }
 
 }  // namespace wh
