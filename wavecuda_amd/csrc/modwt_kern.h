@@ -67,12 +67,16 @@ struct ModwtArgs {
 template <typename T>
 __device__ __forceinline__ ModwtArgs batch_slice(const ModwtArgs& a) {
   ModwtArgs b = a;
-  const int64_t y = blockIdx.y, z = blockIdx.z;
+  const int64_t y = blockIdx.y;
   b.in = static_cast<const T*>(a.in) + y * a.bs_in;
   b.xmod = static_cast<T*>(a.xmod) + y * a.bs_xmod;
-  b.stop = static_cast<const T*>(a.stop) + y * a.bs_stop + z * a.bs_stop_z;
-  b.out = static_cast<T*>(a.out) + y * a.bs_out + z * a.bs_out_z;
-  if (a.th_levels) b.th_levels = a.th_levels + z * kCandLevels;
+  b.stop = static_cast<const T*>(a.stop) + y * a.bs_stop;
+  b.out = static_cast<T*>(a.out) + y * a.bs_out;
+  if (const int64_t z = blockIdx.z) {
+    b.stop = static_cast<const T*>(b.stop) + z * a.bs_stop_z;
+    b.out = static_cast<T*>(b.out) + z * a.bs_out_z;
+    if (a.th_levels) b.th_levels = a.th_levels + z * kCandLevels;
+  }
   return b;
 }
 
