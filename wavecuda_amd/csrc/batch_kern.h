@@ -2,10 +2,11 @@
 //
 // Thousands of independent signals of power-of-two lengths are smoothed
 // (forward transform -> hard/soft universal threshold -> inverse) by a fixed
-// sequence of launches, whatever their mix: the head tiles of every signal
-// (batch_tile.h), the persistent kernel below, and the two shrink passes.  The persistent workgroups take whole signals from a device
-// work queue: an atomic counter over an item list sorted longest-first, so
-// the large signals start first and the small ones fill the tail.
+// sequence of launches, whatever their mix: the head tiles (batch_tile.h), the
+// persistent kernel below, and the last passes' tiles.  The persistent
+// workgroups take whole signals from a device work queue: an atomic counter
+// over an item list sorted longest-first, so the large signals start first and
+// the small ones fill the tail.
 //
 //   MODWT: the item is the exact MAD of D_1 (the reference's univ_thresh(w,
 //   0, 0): src/thresh.cpp:170-201, src/rfunctions.cu:82-87), which the head

@@ -69,14 +69,6 @@ __device__ __forceinline__ int batch_slot(int e, int o, int mask) {
   return CIRC ? ((e & ~mask) | ((e + o) & mask)) : e + o;
 }
 
-// Pins the computation of v here.  A slot's outputs are first used after the
-// barrier, so the compiler would sink their FMAs there and keep the taps of
-// all nine slots in registers instead (446 in FP64).
-template <typename T>
-__device__ __forceinline__ void batch_pin(T& v) {
-  asm volatile("" : "+v"(v));
-}
-
 // ------------------------------------------------------------------- head
 // G = 1: D_1.  G = kBatchHead: D_1 and S_G, one buffer for all levels (a
 // level's outputs wait in registers until every tap has been read).
@@ -115,7 +107,7 @@ __device__ __forceinline__ void batch_head(const BatchTileArgs& a, const BatchTi
 #pragma unroll
         for (int j = 0; j < L; ++j) w[j] = b[batch_slot<CIRC>(e, j * s, mask)];
         analysis1<T, FILT>(w, v[k], D);
-        if (l < G) batch_pin(v[k]);
+        if (l < G) tile_pin(v[k]);
         if (l == 1 && k < KO) d1[m0 + e] = D;
         if (l == kBatchHead && k < KO) {
           const int64_t i = m0 + e;
@@ -203,7 +195,7 @@ struct DwtTile {
           v[j + 1] = pr.y;
         }
         fwd_pair<T, FILT>(v, s[k], d);
-        batch_pin(s[k]);
+        tile_pin(s[k]);
         f(m, k, s[k], d);
       }
     }
@@ -249,8 +241,8 @@ struct DwtTile {
           dv[q] = D[m + H(l) - h - q];
         }
         inv_pair<T, FILT>(sv, dv, e[k], o[k]);
-        batch_pin(e[k]);
-        batch_pin(o[k]);
+        tile_pin(e[k]);
+        tile_pin(o[k]);
         if constexpr (l == 1) *reinterpret_cast<T2*>(y + 2 * m) = T2{e[k], o[k]};
       }
     }
@@ -290,7 +282,7 @@ struct DwtTile {
     auto cut = [&](T* d) {
       return [=](int, int k, T, T v) {
         d[k] = thresh_coef(v, t, hard);
-        batch_pin(d[k]);
+        tile_pin(d[k]);
       };
     };
     level<1, kLeft>(b, cut(d1));
@@ -322,10 +314,9 @@ struct DwtTile {
 // shorter than a quad's reach, 2^(G+1), is repeated to that length.  LDS reads bound the
 // pass, so a thread computes four outputs a level's stride apart, which share
 // L + 3 taps (one by one they read 4 L), and keeps its details in registers.
-// With a fixed stride of 4 s slots between lanes those reads would fall on a
-// quarter of the banks: slot e of a buffer that is read at stride s lies at e ^
-// (row(e) s), the low two bits of its 128-byte row, which spreads them
-// over all.
+// Lanes being 4 slots a stride apart, those reads would fall on a quarter of the
+// banks: slot e of a buffer that is read at stride s lies at e ^ (r s), r the low
+// two bits of its 128-byte row, which spreads them over all.
 // 8192 mixed signals in FP64 / 3001 in FP32, us: one output at a time 521 /
 // 128 for levels 5..8 and 590 / 144 for levels 1..4, as quads 470 / 106 and 494
 // / 127 (vector instructions then busy 70 % of the time, LDS 60 %).  A tile of
@@ -367,18 +358,11 @@ struct Shrink {
   static __device__ __forceinline__ T at(const T* buf, int bytes) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(buf) + bytes);
   }
-  // thresh_coef's values; soft in three operations, t = 0 where there is no
-  // threshold (a NaN), the maximum and minimum as instructions because the
-  // functions add one for signalling NaNs to each operand
+  // thresh_coef's values (t = 0 where there is no threshold, a NaN)
   __device__ __forceinline__ T cut(T c) const {
     if constexpr (HARD) return fabs(c) < t ? T(0) : c;
-    T m;
-    batch_pin(c);  // rounded: no product of c's is fused into the difference
-    if constexpr (sizeof(T) == 8)
-      asm("v_max_f64 %0, %1, -%2\n\tv_min_f64 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
-    else
-      asm("v_max_f32 %0, %1, -%2\n\tv_min_f32 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
-    return c - m;
+    tile_pin(c);  // rounded: no product of c's is fused into the difference
+    return soft_cut(c, t);
   }
 
   // levels l..last
@@ -407,8 +391,8 @@ struct Shrink {
             T D;
             analysis1<T, FILT>(w + i, S[q][i], D);
             d[l - 1][q][i] = cut(D);
-            batch_pin(d[l - 1][q][i]);
-            if (l < G || !COARSE) batch_pin(S[q][i]);
+            tile_pin(d[l - 1][q][i]);
+            if (l < G || !COARSE) tile_pin(S[q][i]);
           }
           if constexpr (l < G) {  // to be read at stride 2 s
 #pragma unroll
@@ -464,7 +448,7 @@ struct Shrink {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             S[q][i] = synthesis<T, FILT>(ws, wd, L - 1 + i);
-            batch_pin(S[q][i]);
+            tile_pin(S[q][i]);
           }
         }
       }

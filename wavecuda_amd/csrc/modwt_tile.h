@@ -58,6 +58,34 @@ __device__ __forceinline__ int64_t tile_index(int64_t id, int64_t blocks) {
   return (id & 7) * (blocks >> 3) + (id >> 3);
 }
 
+// Pins the computation of v here: the compiler would sink it beyond the next
+// barrier, where v is used, and keep its taps in registers instead.
+template <typename T>
+__device__ __forceinline__ void tile_pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// thresh_coef's soft values at t >= 0 in three operations (t = 0: c itself)
+// where it takes twelve in FP64;
+// maximum and minimum as instructions because the functions add one for
+// signalling NaNs to each operand
+template <typename T>
+__device__ __forceinline__ T soft_cut(T c, T t) {
+  T m;
+  if constexpr (sizeof(T) == 8)
+    asm("v_max_f64 %0, %1, -%2\n\tv_min_f64 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
+  else
+    asm("v_max_f32 %0, %1, -%2\n\tv_min_f32 %0, %0, %2" : "=&v"(m) : "v"(c), "v"(t));
+  return c - m;
+}
+
+// thresh_coef at a threshold t that is t >= 0 or none (negative, a NaN)
+template <typename T>
+__device__ __forceinline__ T tile_cut(T c, T t, bool soft) {
+  if (soft) return soft_cut(c, t >= T(0) ? t : T(0));
+  return fabs(c) < t ? T(0) : c;
+}
+
 // ---------------------------------------------------------------- forward
 // one output (S, D) of taps w[0..L-1] (the terms and order of analysis2)
 template <typename T, int FILT>
@@ -381,7 +409,7 @@ struct InvTile {
           else e = adjoint1<T, FILT>(ws, wd, MODE == kAdjFull ? sb[l - 1][k] : T(0));
           if constexpr (l > 1) {
             T c = d[l - 1][k];
-            if (MODE == kInverse && t >= T(0)) c = thresh_coef(c, t, a.hardness);
+            if (MODE == kInverse) c = tile_cut(c, t, a.hardness == kSOFT);
             bb[o] = V{e, c};
           } else if (o / R < qmax) {
             out[base + (o % R) + (int64_t(o / R) << a.j0)] = e;
@@ -419,7 +447,7 @@ __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
     const int e = int(threadIdx.x) + k * NT;
     if (e < C::cnt(G)) {
       T d = c.d[G][k];
-      if (t >= T(0)) d = thresh_coef(d, t, a.hardness);
+      if (MODE == kInverse) d = tile_cut(d, t, a.hardness == kSOFT);
       lds[e] = V{sg[k], d};
     }
   }
@@ -439,8 +467,11 @@ __global__ __launch_bounds__(NT) void modwt_inv_tile_k(ModwtArgs args) {
 // arrays are in flight, which leaves registers for them.  LA8, J = 8,
 // 512 x 2^14: inverse 147 us as one sliding group (one 80 KB workgroup per
 // CU) -> 92 (302 MB read; 256 threads x 8 outputs; 512 x 4 takes 100, 1024 x
-// 2 112); gradient in two tile groups 148 -> 85.  In FP64 the same kernels
-// need all 256 registers (252 us against 191 sliding), so they are not built.
+// 2 112) -> 84 with the short soft threshold; gradient in two tile groups 148
+// -> 85 -> 80.  Quads of outputs that share their taps read less LDS (thresholded
+// 87 us) but leave launches of few tiles slower (2^20 samples D4 16.4 us against
+// 15.6).  In FP64 the kernels need all 256 registers (252 us against 191
+// sliding), so they are not built.
 constexpr int kWideInvNT = 256, kWideInvPer = 8, kWideInvAhead = 3;
 constexpr int kWideGradNT = 512, kWideGradPer = 8, kWideGradAhead = 2;
 constexpr int kWideGmin = 3, kWideGmax = 8;
@@ -503,7 +534,7 @@ struct InvWide {
         for (int k = 0; k < ko; ++k) {
           const int o = int(threadIdx.x) + k * NT;
           T c = d[l - 1][k];
-          if (MODE == kInverse && t >= T(0)) c = thresh_coef(c, t, a.hardness);
+          if (MODE == kInverse) c = tile_cut(c, t, a.hardness == kSOFT);
           if (o < no) b[o] = V{e[k], c};
         }
         __syncthreads();
@@ -536,7 +567,7 @@ __global__ __launch_bounds__(kWideInvNT) void modwt_inv_wide_k(ModwtArgs args) {
   for (int k = 0; k < C::K(G); ++k) {
     const int e = int(threadIdx.x) + k * kWideInvNT;
     T d = c.d[G][k];
-    if (MODE == kInverse && t >= T(0)) d = thresh_coef(d, t, a.hardness);
+    if (MODE == kInverse) d = tile_cut(d, t, a.hardness == kSOFT);
     if (e < C::cnt(G)) lds[e] = V{sg[k], d};
   }
   __syncthreads();
@@ -587,6 +618,7 @@ struct GradWide {
 #pragma unroll
           for (int j = 0; j < L; ++j) w[j] = b[o + j * s];
           analysis1<T, FILT>(w, S[k], D);
+          tile_pin(S[k]);
           if (k < KO) {  // owned
             const T g = grad_cut(q, D * sc, c[l][k < KO ? k : 0], t, act, sum);
             if (oS) {
