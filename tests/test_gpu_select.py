@@ -83,3 +83,22 @@ def test_dwt_level_ranges(n, lo, hi):
     y = np.random.Generator(np.random.PCG64(n)).standard_normal(n)
     got = D.univ_thresh(torch.tensor(y, device="cuda"), n, J, 0, "Haar", lo, hi).item()
     assert got == O.univ_thresh(y, n, J, 0, lo, hi)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [ONE, 1 << 17])
+@pytest.mark.parametrize("which", [0, 1])
+def test_one_middle_rank_is_an_edge(which, n, dtype):
+    """A sampled value at one middle rank and a thousand values, the other
+    middle rank among them, to the next sampled one: more than are ranked by
+    counting."""
+    k = n // 2 - 1 + which
+    sampled = np.concatenate([np.linspace(10, k - 1000, 255), [k],
+                              np.linspace(k + 1000, n - 10, 256)]).astype(np.int64)
+    x = np.empty(n)
+    pos = sample_positions(n)
+    x[pos] = sampled
+    rest = np.setdiff1d(np.arange(n), pos)
+    x[rest] = np.random.Generator(np.random.PCG64(which)).permutation(
+        np.setdiff1d(np.arange(n), sampled))
+    check(x, dtype)

@@ -277,7 +277,7 @@ __device__ void block_pick(const B* bins, const uint64_t* edges, int64_t count, 
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const u64 K = u64(r == 0 ? (count - 1) / 2 : count / 2);
-    u64 below = incl - loc;
+    u64 below = incl - loc, in = 0;
     int hit = -1;
     if (below <= K && K < incl) {
 #pragma unroll
@@ -285,7 +285,7 @@ __device__ void block_pick(const B* bins, const uint64_t* edges, int64_t count, 
         if (hit >= 0) continue;
         if (K < below + cnt[i]) {
           hit = b0 + i;
-          p->inside = cnt[i];
+          in = cnt[i];
         } else {
           below += cnt[i];
         }
@@ -305,7 +305,8 @@ __device__ void block_pick(const B* bins, const uint64_t* edges, int64_t count, 
       const uint64_t hi = hit == nb ? 0ull : edges[i];      // exclusive; 0: none
       p->base = lo + 1;
       p->width = hi - lo - 1;
-      if (hit == nb) p->inside = u64(count) - below;
+      // of the open bucket alone: the other rank may sit in an equality one
+      p->inside = hit == nb ? u64(count) - below : in;
     }
   }
   __syncthreads();
