@@ -2,7 +2,7 @@
 
 Many signals of power-of-two lengths, mixed filters and mixed transforms
 are smoothed (forward -> MAD universal threshold -> hard/soft threshold ->
-inverse) by one persistent HIP launch fed by a device work queue.  Per
+inverse) by a fixed sequence of HIP launches, whatever their mix.  Per
 signal the result is what the single-signal smoothing computes with
 threshtype UNIV over the full level range (reference src/rfunctions.cu:82-87
 and src/thresh.cpp:170-201).
