@@ -543,6 +543,7 @@ __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, in
   const TW* __restrict__ vw = reinterpret_cast<const TW*>(v);
   const int nv = int(count / kW);  // count is a multiple of 64
   int below = 0;
+  T bad = T(0);  // NaN and infinities: block_median has the rule for them
   for (int b = tid; b < nv; b += NT * kU) {
     TW x[kU];
 #pragma unroll
@@ -550,6 +551,11 @@ __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, in
       const int p = b + u * NT;
       x[u] = vw[p < nv ? p : b];
     }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int w = 0; w < kW; ++w) bad = fma(x[u][w], T(0), bad);
+    asm volatile("" : "+v"(bad));  // here, not beyond the loop
     unsigned in = 0;  // bit per value
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
@@ -587,7 +593,7 @@ __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, in
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o, 64);
   if (lane == 0) wsum[wave] = below;
-  __syncthreads();
+  if (__syncthreads_or(!(bad == T(0)))) return false;
   below = 0;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) below += wsum[w];
