@@ -1,0 +1,49 @@
+"""The selection where its gathered bucket may outgrow the buffer (2^22 values
+and more): equal to sorting, and no input of plain noise falls to the last
+resort, one workgroup reading every value (3 ms a median at 2^24 values, where a
+call takes 0.2 ms)."""
+import pytest
+import torch
+
+from wavecuda_amd import device as D
+
+pytestmark = pytest.mark.gpu
+
+
+def noise(n, dtype, seed):
+    return torch.randn(n, dtype=dtype, device="cuda",
+                       generator=torch.Generator(device="cuda").manual_seed(seed))
+
+
+def middle(s):
+    n = s.numel()
+    return 0.5 * (s[(n - 1) // 2].double() + s[n // 2].double())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1 << 22, (1 << 22) + 1, 1 << 24])
+def test_equals_sorting(n, dtype):
+    for seed in range(4):
+        x = noise(n, dtype, seed)
+        m = middle(torch.sort(x)[0])
+        d = middle(torch.sort((x - m.to(dtype)).abs())[0])
+        assert D.median(x).item() == m.item()
+        assert D.mad(x).item() == 1.4826 * d.item()
+
+
+def test_every_call_takes_the_gather():
+    times = []
+    for seed in range(16):
+        x = noise(1 << 24, torch.float32, seed)
+        D.mad(x)
+        best = float("inf")
+        for _ in range(3):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            D.mad(x)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times.append(best)
+    print("ms:", [round(t, 3) for t in times], flush=True)
+    assert max(times) < 4 * min(times)

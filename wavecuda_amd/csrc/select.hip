@@ -44,7 +44,7 @@ constexpr int kNTB = 1024;  // threads of the one-workgroup steps
 constexpr int kFly = 4;     // loads in flight per thread of the passes
 constexpr int kHold = 8;    // values a thread of the one-workgroup kernel holds
 constexpr int kOneMax = kHold * kNTB;
-constexpr int64_t kRefineMin = int64_t(1) << 24;  // a third pass beyond: see sel_refine_k
+constexpr int64_t kRefineMin = int64_t(1) << 22;  // a third pass beyond, if need be: see sel_refine_k
 constexpr int kBits = 11;
 constexpr int kBins = 1 << kBits;
 constexpr int kDirect = 256;  // keys ranked by counting
@@ -577,9 +577,19 @@ __global__ __launch_bounds__(kNT) void sel_count_k(SelSrc s, SelState* st, int r
       atomicAdd(&st->bins[round][(blockIdx.x % kReplicas) * kSelBuckets + i], u64(bins[i]));
 }
 
-// Beyond kRefineMin values the open bucket (count / kSelSample values on
-// average) may outgrow the candidate buffer: one more pass counts the
-// leading 11 bits of its keys' offsets.
+// The open bucket that holds the middle ranks is 2 count / kSelSample values
+// on average (a rank falls in a bucket in proportion to its size) and x times
+// count / kSelSample with probability (1 + x) e^-x.  Up to kRefineMin values it
+// outgrows half of the candidate buffer (x = 16) in two of a million calls;
+// at 2^24 (x = 4) in one of eleven, and a workgroup alone then reads every value:
+// cross-validated smoothing of 2^21 FP32 samples, eight levels of details, 7.0
+// ms instead of 1.0.  So beyond kRefineMin, where the bucket is that full, one
+// more pass counts the leading 11 bits of its keys' offsets.  (Half of the
+// buffer, for the regions fill unevenly.)
+__device__ __forceinline__ bool sel_refines(int refine, const Pick& p) {
+  return refine && p.inside > u64(kSelCandCap) / 2;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kNT) void sel_refine_k(SelSrc s, SelState* st, int round) {
   __shared__ unsigned hist[kBins];
@@ -587,7 +597,7 @@ __global__ __launch_bounds__(kNT) void sel_refine_k(SelSrc s, SelState* st, int 
   __shared__ Pick p;
   const int tid = threadIdx.x;
   block_pick<kNT, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
-  if (p.found[0] && p.found[1]) return;
+  if ((p.found[0] && p.found[1]) || !sel_refines(1, p)) return;
   for (int i = tid; i < kBins; i += kNT) hist[i] = 0;
   __syncthreads();
   const T med = round ? T(st->med) : T(0);
@@ -617,7 +627,7 @@ __global__ __launch_bounds__(kNT) void sel_gather_k(SelSrc s, SelState* st, int 
   if (tid == 0) nlist = 0;
   block_pick<kNT, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
   if (p.found[0] && p.found[1]) return;
-  if (refine) (void)block_narrow<kNT>(st->hist[round], &p, wsum);
+  if (sel_refines(refine, p)) (void)block_narrow<kNT>(st->hist[round], &p, wsum);
   if (p.inside > u64(kSelCandCap)) return;  // the last step reads the values
   const T med = round ? T(st->med) : T(0);
   const uint64_t base = p.base, width = p.width;
@@ -657,7 +667,8 @@ __global__ __launch_bounds__(kNTB) void sel_finish_k(SelSrc s, SelState* st, int
   const int tid = threadIdx.x;
   if (next && tid < kSelSample) smp[tid] = st->sample[tid];
   block_pick<kNTB, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
-  if (refine && !(p.found[0] && p.found[1])) (void)block_narrow<kNTB>(st->hist[round], &p, wsum);
+  if (!(p.found[0] && p.found[1]) && sel_refines(refine, p))
+    (void)block_narrow<kNTB>(st->hist[round], &p, wsum);
   const T med = round ? T(st->med) : T(0);
   // gathered unless there were too many in all, or for one region
   unsigned nc[kReplicas];
