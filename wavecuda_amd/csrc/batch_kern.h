@@ -205,7 +205,7 @@ __device__ __forceinline__ void batch_dwt_inv(T* y, int64_t n, int J, T* C,
   {
     T* gA = C + n;          // n/2
     T* gB = gA + n / 2;     // n/2
-    const T tt = T(t);
+    const T tt = t >= 0.0 ? T(t) : T(0);  // a NaN is no threshold, as in dwt.hip
     int64_t N;
     T* cur;
     T* nxt;

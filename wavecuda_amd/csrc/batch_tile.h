@@ -271,7 +271,8 @@ struct DwtTile {
 
   static __device__ __forceinline__ void last(const BatchTileArgs& a, const BatchTile& I, T* b) {
     const int64_t n = I.n;
-    const T t = T(a.thresh[I.sig]);
+    const double t0 = a.thresh[I.sig];
+    const T t = t0 >= 0.0 ? T(t0) : T(0);  // a NaN is no threshold, as in dwt.hip
     const T* s4 = static_cast<const T*>(a.scratch) + I.scr + batch_pad(n) + batch_pad(n >> A);
     const T* xc = static_cast<const T*>(a.scratch) + I.scr + 2 * batch_pad(n);
     T* y = static_cast<T*>(a.y) + I.off + I.m0;
