@@ -46,10 +46,11 @@ __device__ __forceinline__ double sel_val(uint64_t k, float*) {
 }
 
 // bin of a value y in [0, hi] among kSelBins equal-width bins (scale =
-// kSelBins / hi); monotone non-decreasing in y, clamped to the last bin
+// kSelBins / hi); monotone non-decreasing in y's key, clamped to the last bin,
+// which also takes NaN: keys rank positive NaN above every number
 __device__ __forceinline__ int sel_bin(double y, double scale) {
   const double u = y * scale;
-  return u > 0.0 ? (u < double(kSelBins - 1) ? int(u) : kSelBins - 1) : 0;
+  return u < double(kSelBins - 1) ? (u > 0.0 ? int(u) : 0) : kSelBins - 1;
 }
 
 // smallest and largest digit with a non-zero count in h[0..kSelBins), by
@@ -154,8 +155,8 @@ __device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t co
 // Median of v[e], e < count (|v - center| when deviation),
 // computed by all NT threads of the workgroup; returns the same value in
 // every thread.  ws: block_sel_lds<NT>() bytes of LDS.  bound > 0
-// (deviations only): every value lies in [0, bound]; one pass then counts the values into kSelBins
-// equal-width bins, and when the middle ranks' bins hold at most
+// (deviations only): every finite value lies in [0, bound]; one pass then counts the values into
+// kSelBins equal-width bins (what lies beyond in the last), and when the middle ranks' bins hold at most
 // kSelDirect values they are copied to LDS and ranked directly (otherwise
 // the radix digits start from the top).  Of values, the smallest and largest
 // first digit any has are left at sel_range_slot(ws).
@@ -543,7 +544,7 @@ __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, in
   const TW* __restrict__ vw = reinterpret_cast<const TW*>(v);
   const int nv = int(count / kW);  // count is a multiple of 64
   int below = 0;
-  T bad = T(0);  // NaN and infinities: block_median has the rule for them
+  T bad = T(0);  // NaN and infinities: left to block_median
   for (int b = tid; b < nv; b += NT * kU) {
     TW x[kU];
 #pragma unroll
@@ -758,7 +759,9 @@ __device__ __forceinline__ double block_mad(const T* __restrict__ v, int64_t cou
       if (count > kSelDirect && d0 <= d1) {
         // every value lies in [vlo, vhi], the ends of those digits' key
         // ranges; |v - med| computed as the selection computes it (v - med
-        // rounds monotonically in v) is then at most max(vhi - med, med - vlo)
+        // rounds monotonically in v) is then at most max(vhi - med, med - vlo).
+        // An end that decodes to a NaN (infinities, NaN) is left out: what is
+        // beyond the bound shares the last bin
         constexpr int sh = int(sizeof(T)) * 8 - kSelBits;
         const T vlo = T(sel_val(uint64_t(d0) << sh, (T*)nullptr));
         const T vhi = T(sel_val((uint64_t(d1) << sh) | ((uint64_t(1) << sh) - 1), (T*)nullptr));
