@@ -63,11 +63,10 @@ struct ModwtArgs {
   int64_t bs_stop_z, bs_out_z;
 };
 
-// the arguments of the signal handled by this workgroup (blockIdx.y)
+// the arguments of signal y, the one this workgroup handles
 template <typename T>
-__device__ __forceinline__ ModwtArgs batch_slice(const ModwtArgs& a) {
+__device__ __forceinline__ ModwtArgs batch_slice(const ModwtArgs& a, int64_t y) {
   ModwtArgs b = a;
-  const int64_t y = blockIdx.y;
   b.in = static_cast<const T*>(a.in) + y * a.bs_in;
   b.xmod = static_cast<T*>(a.xmod) + y * a.bs_xmod;
   b.stop = static_cast<const T*>(a.stop) + y * a.bs_stop;
@@ -430,7 +429,7 @@ template <typename T, int FILT, int R, int NT, int G, int MAP, int SP>
 __global__ __launch_bounds__(NT) void modwt_fwd_k(ModwtArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int64_t nrb = (int64_t(1) << a.j0) / R;
-  const ModwtArgs b = batch_slice<T>(a);
+  const ModwtArgs b = batch_slice<T>(a, blockIdx.y);
   modwt_fwd_body<T, FILT, R, NT, G, MAP, SP>(b, int64_t(blockIdx.x) % nrb,
                                              int64_t(blockIdx.x) / nrb, smem_raw);
 }
@@ -940,7 +939,7 @@ template <typename T, int FILT, int R, int NT, int G, int MAP>
 __global__ __launch_bounds__(NT) void modwt_inv_k(ModwtArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int64_t nrb = (int64_t(1) << a.j0) / R;
-  const ModwtArgs b = batch_slice<T>(a);
+  const ModwtArgs b = batch_slice<T>(a, blockIdx.y);
   if constexpr (MAP == 2) {
     static_assert(R == 1, "linear buffers serve the first group");
     modwt_inv_lin_body<T, FILT, NT, G>(b, int64_t(blockIdx.x), smem_raw);
