@@ -65,6 +65,17 @@ bool wide_fits(int per, int64_t n, int J, size_t esz) {
 
 std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz,
                                const PlanKnobs& k, int64_t count = 1);
+std::vector<Group> plan_tiles(bool inverse, int64_t n, int J, int L, size_t esz,
+                              const PlanKnobs& k);
+
+// elements of a tile plan's largest launch, the padding of sequences that are
+// shorter than a tile among them
+int64_t padded_elems(const std::vector<Group>& tiles, int64_t count) {
+  int64_t m = 0;
+  for (const Group& G : tiles)
+    m = std::max(m, (int64_t(1) << G.j0) * G.nseg * G.M * count);
+  return m;
+}
 
 // Default plan knobs, measured on MI355X (replayed graphs, three sets of
 // buffers in turn; us, sliding windows -> tiles, LA8 / Haar):
@@ -76,12 +87,23 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
 //    windows ahead in FP32 (82.6 against 87.7).  Tiles of 256 threads up to
 //    2^17 samples (2^17, J = 9: 10.8 against 11.5), 512 beyond (2^18, J = 10:
 //    14.2 against 15.7);
+//  * not where a deeper group's sequences, n / 2^j0 long, leave most of a tile
+//    empty and the sliding windows need only one or two groups (Haar, calls back
+//    to back: 1024 x 2^8, J = 8 FP32, padding 16 to 1, 17.5 against 21.4; 256 x
+//    2^12, J = 12 FP64, 16 to 1, 55.5 against 84; 256 x 2^13, J = 12, 2^24 elements
+//    padded 8 to 1, 88 against 105; but 1024 x 2^10, J = 10 FP64, 8 to 1, 87.9 -> 52.6;
+//    64 x 2^12, J = 12, 16 to 1, five sliding groups, 34.4 -> 26.6);
 //  * the forward of up to 2^18 samples as tiles of 512 threads (2^14, J = 8:
-//    18.4 -> 8.9 / 15.8 -> 7.0; 2^18, J = 10: 29.6 -> 16.5 / 26.5 -> 12.9),
-//    and of up to 2^19 where the sliding windows need more than one group
-//    (2^19, J = 10 FP32: 22.7 -> 16.2; Haar's one group 10.9 against 14.2).
-//    Beyond, it is bound by its stores, which the sliding windows make
-//    in longer runs (2^20, J = 8 FP32: 18.5 against 19.7);
+//    18.4 -> 8.9 / 15.8 -> 7.0; 2^18, J = 10: 29.6 -> 16.5 / 26.5 -> 12.9)
+//    unless the sliding windows take fewer steps than two chunks a tile group:
+//    short signals whose levels all fit one group (n = 2^10, J = 7..10: Haar, two
+//    chunks, 4.9 against 6.8 and at 256 signals 7.5 against 10.4; LA8 J = 8, three
+//    chunks, 9.2 -> 7.8 and 10.4 -> 9.1);
+//  * of up to 2^19 where they take at least three (2^19, J = 10 FP32: 22.7 ->
+//    16.2; J = 8 level to 1.1 times ahead; 64 x 2^13, J = 12 Haar FP32, five for
+//    three tile groups, 17.0 against 20.3).  Beyond, it is bound by its stores,
+//    which the sliding windows make in longer runs (2^20, J = 8 FP32: 18.5 against
+//    19.7);
 //  * an FP32 inverse of at most 8 levels as one wide tile: with 7 or 8
 //    levels, which take two tile groups, from 2^19 samples (64 x 2^13, J = 8
 //    LA8 / Haar: 19.2 -> 14.9 / 16.4 -> 11.5; 32 x 2^14 level at 15.3) up to
@@ -89,38 +111,49 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
 //    against 195); with fewer, beyond the tiles' range and below 2^23 (2^22,
 //    J = 6 LA8 43.6 -> 39.3, J = 4 31.8 -> 28.9; 512 x 2^14, J = 6 75
 //    against 81);
-//  * a single-signal FP32 inverse beyond that: a 256-thread first group of
-//    at most six levels, four segments per CU (half the FP64 LDS, so
-//    several workgroups share a CU): n = 2^22 90 -> 83, 2^24 307 -> 258.
+//  * sliding inverses: of up to 2^18 samples a 256-thread first group of at most
+//    six levels, two segments per CU (one 512-thread workgroup per CU has too few:
+//    2^16 28 -> 25); of one FP32 signal beyond 2^20 the same with four (half the
+//    FP64 LDS, so several workgroups share a CU): n = 2^22 90 -> 83, 2^24 307 -> 258.
 // Rules for the FP64 sliding windows taken from the tuner's isolated
 // timings were slower in the pipeline (what the other transform leaves in
 // the last-level cache matters as much as the plan), so those keep the plain
 // defaults.
 PlanKnobs default_knobs(bool inverse, int64_t n, int64_t count, int J, int filt, size_t esz) {
-  PlanKnobs k;
   const int64_t total = n * count;
-  auto tiles = [&k](int threads) {
-    k.first_nt = -threads;
-    k.g1max = kTileGmax;
-  };
-  const bool deep = J > kTileGmax;  // two tile groups
+  const int L = filter_length(filt);
+  const bool deep = J > kTileGmax;  // two tile groups or more
+  PlanKnobs k;
   if (inverse && wide_fits(kWideInvP, n, J, esz) &&
       (deep ? total >= (int64_t(1) << 19) && total <= (int64_t(1) << 23)
             : total > (int64_t(1) << 21) && total < (int64_t(1) << 23))) {
     k.first_nt = -kWideInvNT;
     k.g1max = kWideGmax;
-  } else if (inverse && total <= (int64_t(1) << 21)) {
-    tiles(total <= (int64_t(1) << 17) ? kNT1 / 2 : kNT1);
-  } else if (inverse && count == 1 && esz == 4) {
-    k.first_nt = kNT1 / 2;
-    k.first_per_cu = 4;
-    k.g1max = 6;
-  } else if (!inverse && (total <= (int64_t(1) << 18) ||
-                          (total <= (int64_t(1) << 19) &&
-                           plan_groups(false, n, J, filter_length(filt), esz, k, count).size() > 1))) {
-    tiles(kNT1);
+    return k;
   }
-  return k;
+  if (inverse && (total <= (int64_t(1) << 18) ||
+                  (count == 1 && esz == 4 && n > (int64_t(1) << 20)))) {
+    k.first_nt = kNT1 / 2;
+    k.first_per_cu = total <= (int64_t(1) << 18) ? 2 : 4;
+    k.g1max = 6;
+  }
+  if (total > (int64_t(1) << (inverse ? 21 : 19))) return k;
+  PlanKnobs t;
+  t.first_nt = inverse && total <= (int64_t(1) << 17) ? -kNT1 / 2 : -kNT1;
+  t.g1max = kTileGmax;
+  if (!deep && (inverse || total <= (int64_t(1) << 18))) return t;
+  const auto sliding = plan_groups(inverse, n, J, L, esz, k, count);
+  if (!deep) return sliding.size() > 1 ? t : k;
+  const auto tiles = plan_tiles(inverse, n, J, L, esz, t);
+  if (inverse) {
+    const int64_t padded = padded_elems(tiles, count);
+    const bool full = padded <= 8 * total && padded <= (int64_t(1) << 23);
+    return full || sliding.size() > 2 ? t : k;
+  }
+  size_t chunks = 0;
+  for (const Group& G : sliding) chunks += size_t(G.nchunks);
+  const bool pays = total <= (int64_t(1) << 18) ? chunks > tiles.size() : chunks >= 3 * tiles.size();
+  return pays ? t : k;
 }
 
 PlanKnobs knobs_for(bool inverse, int64_t n, int J, int filt, size_t esz, int64_t count = 1) {
@@ -598,7 +631,8 @@ int modwt_inverse_adjoint(const void* gx, void* gxmod, int64_t n, int64_t count,
                           int dtype, hipStream_t st) {
   // tiles where the forward runs as tiles (see default_knobs): the same
   // stores bound both
-  if (n * count <= (int64_t(1) << 18))
+  if (n * count <= (int64_t(1) << 18) &&
+      default_knobs(false, n, count, J, filt, dtype == WH_F32 ? 4 : 8).first_nt < 0)
     return dtype == WH_F32
                ? inv_grad_t<float>(gx, nullptr, gxmod, true, nullptr, n, count, J, filt, nullptr, st)
                : inv_grad_t<double>(gx, nullptr, gxmod, true, nullptr, n, count, J, filt, nullptr,
