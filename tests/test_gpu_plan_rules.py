@@ -61,3 +61,21 @@ def test_values(inverse, n, J, filt, dtype, count, tiles):
         v *= torch.tensor([2.0 ** -l for l in range(1, J + 1)], dtype=dtype, device="cuda").view(J, 1, 1)
         v[:, : J - 1, 0] = 0
         assert torch.equal(w, out)
+
+
+@pytest.mark.parametrize("details", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,J,count", [(1 << 12, 12, 64), (1 << 8, 8, 1024), (1 << 10, 10, 1024)])
+def test_adjoint_by_level(n, J, count, dtype, details):
+    """The forward's adjoint whose deepest levels run one by one, against
+    launches of fewer signals, which run as tiles."""
+    code = W.WH_F64 if dtype == torch.float64 else W.WH_F32
+    g = torch.Generator(device="cuda").manual_seed(J)
+    w = torch.randn(count, 2 * n * J, dtype=dtype, device="cuda", generator=g)
+    out, one = (torch.empty(count, n, dtype=dtype, device="cuda") for _ in range(2))
+    call = W.lib().wh_modwt_fwd_details_adj if details else W.lib().wh_modwt_fwd_adj
+    W.check(call(C.c_void_p(w.data_ptr()), C.c_void_p(out.data_ptr()), n, count, J, W.HAAR, code, None))
+    for i in range(0, count, 16):
+        W.check(call(C.c_void_p(w[i].data_ptr()), C.c_void_p(one[i].data_ptr()), n, 16, J, W.HAAR,
+                     code, None))
+    assert torch.equal(out, one)

@@ -68,13 +68,10 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
 std::vector<Group> plan_tiles(bool inverse, int64_t n, int J, int L, size_t esz,
                               const PlanKnobs& k);
 
-// elements of a tile plan's largest launch, the padding of sequences that are
-// shorter than a tile among them
-int64_t padded_elems(const std::vector<Group>& tiles, int64_t count) {
-  int64_t m = 0;
-  for (const Group& G : tiles)
-    m = std::max(m, (int64_t(1) << G.j0) * G.nseg * G.M * count);
-  return m;
+// elements of a tile launch, the padding of sequences that are shorter than a
+// tile among them
+int64_t padded_elems(const Group& G, int64_t count) {
+  return (int64_t(1) << G.j0) * G.nseg * G.M * count;
 }
 
 // Default plan knobs, measured on MI355X (replayed graphs, three sets of
@@ -146,7 +143,8 @@ PlanKnobs default_knobs(bool inverse, int64_t n, int64_t count, int J, int filt,
   if (!deep) return sliding.size() > 1 ? t : k;
   const auto tiles = plan_tiles(inverse, n, J, L, esz, t);
   if (inverse) {
-    const int64_t padded = padded_elems(tiles, count);
+    int64_t padded = 0;
+    for (const Group& G : tiles) padded = std::max(padded, padded_elems(G, count));
     const bool full = padded <= 8 * total && padded <= (int64_t(1) << 23);
     return full || sliding.size() > 2 ? t : k;
   }
@@ -474,12 +472,65 @@ GroupLaunch launch_of(const Group& G, int64_t count) {
   return gl;
 }
 
+// One level of the forward's adjoint: out = Sb_{j-1} + H_j^T u + G_j^T Db_j, a
+// tap k 2^{j-1} positions back (the terms and order of adjoint1).  Every tap is a
+// shifted contiguous read.  Levels whose sequences are too short for tiles.
+template <typename T, int FILT>
+__global__ __launch_bounds__(256) void fwd_adj_level_k(const T* __restrict__ u0, int64_t bs_u,
+                                                       const T* __restrict__ gxm0, int64_t per,
+                                                       int j, int with_s, T* __restrict__ out0,
+                                                       int64_t n) {
+  constexpr int L = Filter<FILT>::L;
+  const int64_t sig = blockIdx.y;
+  const T* __restrict__ u = u0 + sig * bs_u;
+  const T* __restrict__ db = gxm0 + sig * per + 2 * n * int64_t(j - 1) + n;
+  const T* __restrict__ sb =
+      with_s && j >= 2 ? gxm0 + sig * per + 2 * n * int64_t(j - 2) : nullptr;
+  T* __restrict__ out = out0 + sig * n;
+  const int64_t s = int64_t(1) << (j - 1), mask = n - 1;
+  for (int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x; p < n; p += int64_t(gridDim.x) * 256) {
+    T acc = sb ? sb[p] : T(0);
+#pragma unroll
+    for (int k = 0; k < L; ++k) {
+      const int64_t q = (p - k * s) & mask;
+      acc = fma(u[q], T(Filter<FILT>::c(k)), acc);
+      acc = fma(db[q], T(gcoef<FILT>(k)), acc);
+    }
+    out[p] = acc;
+  }
+}
+
+template <typename T>
+int fwd_adj_level(const T* u, int64_t bs_u, const T* gxm, int64_t per, int j, bool with_s, T* out,
+                  int64_t n, int64_t count, int filt, hipStream_t st) {
+  const dim3 grid(unsigned(std::min<int64_t>((n + 255) / 256, 2048)), unsigned(count));
+  auto kern = filt == kHAAR ? fwd_adj_level_k<T, kHAAR>
+              : filt == kD4 ? fwd_adj_level_k<T, kD4>
+              : filt == kC6 ? fwd_adj_level_k<T, kC6>
+                            : fwd_adj_level_k<T, kLA8>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, u, bs_u, gxm, per, j, with_s ? 1 : 0, out, n);
+  WH_HIP_CHECK(hipGetLastError());
+  return WH_OK;
+}
+
+// Whether a group of the forward's adjoint runs level by level: its sequences
+// fill an eighth of a tile or less and the launch is large (Haar, whole call, us,
+// tiles -> levels: 1024 x 2^12, J = 12 FP64 585 -> 252; 256 x 2^12, J = 12 122 -> 60;
+// 1024 x 2^8, J = 8 33.5 -> 20.5; 1024 x 2^10, J = 10 FP32 56 -> 34; short of the line,
+// 64 x 2^13, J = 12 FP64, 44 as tiles against 55 with every level a launch).
+bool by_level(const Group& G, int64_t n, int64_t count) {
+  const int64_t padded = padded_elems(G, count), total = n * count;
+  return !G.wide && ((padded >= 16 * total && padded >= (int64_t(1) << 22)) ||
+                     (padded >= 8 * total && padded >= (int64_t(1) << 23)));
+}
+
 // adjoint of the forward: the level groups from the deepest up
 template <typename T>
 int fwd_adj_t(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int filt,
               bool details, hipStream_t st) {
   auto groups = adjoint_tiles(true, n, count, J, filter_length(filt), sizeof(T), details);
   const int64_t per = 2 * n * J;
+  const T* gxm = static_cast<const T*>(gxmod);
   T* scratch = nullptr;
   if (groups.size() > 1) {
     void* p = nullptr;
@@ -487,16 +538,32 @@ int fwd_adj_t(const void* gxmod, void* gx, int64_t n, int64_t count, int J, int 
     if (rc) return rc;
     scratch = static_cast<T*>(p);
   }
-  const T* stop = static_cast<const T*>(gxmod) + 2 * n * int64_t(J - 1);
+  const T* stop = gxm + 2 * n * int64_t(J - 1);
   int64_t bs_stop = per;
+  int half = 0;  // of the scratch, to be written next; the other holds stop
+  auto next = [&](bool last) {
+    T* dst = last ? static_cast<T*>(gx) : scratch + half * n * count;
+    half ^= 1;
+    return dst;
+  };
   for (int gi = int(groups.size()) - 1; gi >= 0; --gi) {
     const Group& G = groups[gi];
+    if (gi > 0 && by_level(G, n, count)) {
+      for (int j = G.j0 + G.g; j > G.j0; --j) {
+        T* dst = next(false);
+        int rc = fwd_adj_level<T>(stop, bs_stop, gxm, per, j, !details, dst, n, count, filt, st);
+        if (rc) return rc;
+        stop = dst;
+        bs_stop = n;
+      }
+      continue;
+    }
     ModwtArgs a = args_of(G, n);
     a.xmod = const_cast<void*>(gxmod);
     a.bs_xmod = per;
     a.stop = stop;
     a.bs_stop = bs_stop;
-    T* dst = (G.j0 == 0) ? static_cast<T*>(gx) : scratch + (gi & 1) * n * count;
+    T* dst = next(G.j0 == 0);
     a.out = dst;
     a.bs_out = n;
     int rc = modwt_tile_launch<T>(details ? TileOp::kAdjDetails : TileOp::kAdjFull, filt,
