@@ -18,8 +18,13 @@
  *    bytes for FP64, 8 for FP32; hipMalloc gives 256); WH_ERR_ARG otherwise.
  *
  *    Scratch: the library keeps per-device work buffers, grown on demand
- *    and held until exit (the MODWT inverse's level hand-off, DWT staging,
- *    the selection and cross-validation state, smoothing workspaces).
+ *    and held until exit: the level hand-off of the MODWT inverse, of
+ *    wh_modwt_fwd_adj, wh_modwt_fwd_details_adj and of wh_modwt_thresh_inv_adj
+ *    without gxmod or with details_only; DWT staging; the selection and
+ *    cross-validation state; the partial sums of wh_thresh_grad,
+ *    wh_modwt_thresh_inv_adj (with glam) and wh_mse_grad; smoothing workspaces.
+ *    wh_modwt_fwd, wh_modwt_fwd_many, wh_modwt_fwd_details and wh_modwt_inv_adj
+ *    use none.
  *    Calls on one device that use them must not overlap in time: issue
  *    them on one stream, or synchronize between streams.  Batch plans own
  *    their workspace.  Error messages are per thread.

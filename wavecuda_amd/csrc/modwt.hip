@@ -338,6 +338,16 @@ __global__ void zero_slot_k(T* __restrict__ p, int64_t n, int64_t stride) {
     q[i] = T(0);
 }
 
+// zeros into the S slot of level j (1-based) of every signal's coefficients
+template <typename T>
+int zero_slot(void* xmod, int j, int64_t n, int64_t count, int64_t per, hipStream_t st) {
+  T* slot = static_cast<T*>(xmod) + 2 * n * int64_t(j - 1);
+  const unsigned blocks = unsigned(std::min<int64_t>((n + 255) / 256, 1024));
+  hipLaunchKernelGGL(zero_slot_k<T>, dim3(blocks, unsigned(count)), dim3(256), 0, st, slot, n, per);
+  WH_HIP_CHECK(hipGetLastError());
+  return WH_OK;
+}
+
 // the tuner's test signal: values uniform in [-1, 1) from a hash of the
 // index (a zero signal runs at other speeds than real data does)
 template <typename T>
@@ -373,12 +383,8 @@ int modwt_fwd_t(const void* x, void* xmod, int64_t n, int64_t count, int J, int 
     // the S slots at group boundaries carried the next group's input; the
     // adjoint of the inverse is zero there
     for (size_t gi = 0; gi + 1 < groups.size(); ++gi) {
-      const int j = groups[gi].j0 + groups[gi].g;  // 1-based level of the slot
-      T* slot = static_cast<T*>(xmod) + 2 * n * int64_t(j - 1);
-      const unsigned blocks = unsigned(std::min<int64_t>((n + 255) / 256, 1024));
-      hipLaunchKernelGGL(zero_slot_k<T>, dim3(blocks, unsigned(count)), dim3(256), 0, st, slot,
-                         n, per);
-      WH_HIP_CHECK(hipGetLastError());
+      int rc = zero_slot<T>(xmod, groups[gi].j0 + groups[gi].g, n, count, per, st);
+      if (rc) return rc;
     }
   }
   return WH_OK;
@@ -638,26 +644,41 @@ int inv_grad_t(const void* gy, const void* c, void* gc, bool zero_s, double* gla
     if (rc) return rc;
     q.partial = static_cast<double*>(p);
   }
+  // The S between groups: through the cotangent's own slot of that level where
+  // zeros are to be left there afterwards, as the sliding form does, so that the
+  // plain adjoint uses no library scratch (callers may have several streams, or be
+  // capturing); through scratch where the slots are not to be written.
+  const bool slots = gc && zero_s;
   T* scratch = nullptr;
-  if (groups.size() > 1) {
+  if (groups.size() > 1 && !slots) {
     int rc = scratch_get(2 * size_t(n) * size_t(count) * sizeof(T), &p);
     if (rc) return rc;
     scratch = static_cast<T*>(p);
   }
+  const int64_t per = 2 * n * J;
   const void* in = gy;
+  int64_t bs_in = n;
   for (size_t gi = 0; gi < groups.size(); ++gi) {
     const Group& G = groups[gi];
     ModwtArgs a = args_of(G, n);
     a.in = in;
-    a.bs_in = n;
+    a.bs_in = bs_in;
     a.xmod = const_cast<void*>(c ? c : gc);
-    a.bs_xmod = 2 * n * J;
-    a.out = scratch ? scratch + int64_t(gi & 1) * n * count : nullptr;
-    a.bs_out = n;
+    a.bs_xmod = per;
     q.last = gi + 1 == groups.size();
+    if (!q.last) {
+      a.out = slots ? static_cast<T*>(gc) + 2 * n * int64_t(G.j0 + G.g - 1)
+                    : scratch + int64_t(gi & 1) * n * count;
+      a.bs_out = slots ? per : n;
+    }
     int rc = modwt_tile_launch<T>(TileOp::kGrad, filt, launch_of(G, count), a, q, st);
     if (rc) return rc;
     in = a.out;
+    bs_in = a.bs_out;
+  }
+  for (size_t gi = 0; slots && gi + 1 < groups.size(); ++gi) {
+    int rc = zero_slot<T>(gc, groups[gi].j0 + groups[gi].g, n, count, per, st);
+    if (rc) return rc;
   }
   if (glam) {
     hipLaunchKernelGGL(grad_sum_k, dim3(unsigned(J)), dim3(256), 0, st, q.partial, glam, count,

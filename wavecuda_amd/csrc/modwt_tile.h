@@ -39,7 +39,8 @@ constexpr int kTileAdjNT = 512;  // threads of the adjoint and gradient tiles
 // coefficients before thresholding, out: the hand-off to the next group)
 struct GradArgs {
   void* gc;         // cotangent of the coefficients, or null
-  int zero_s;       // also write zeros into its S_j slots, j < J
+  int zero_s;       // also write zeros into its S_j slots, j < J (the group's last
+                    // level apart: a slot that may hold the hand-off)
   int last;         // this group ends at level J
   double* partial;  // [level][signal][per_signal], or null
   int64_t per_signal;
@@ -273,7 +274,7 @@ struct GradTile {
             if (oS) {
               oS[a.n + i] = g;
               if (top) oS[i] = S * sc;
-              else if (q.zero_s) oS[i] = T(0);
+              else if (l < G && q.zero_s) oS[i] = T(0);
             }
             if (l == G && !q.last) static_cast<T*>(a.out)[i] = S * sc;
           }
