@@ -283,6 +283,22 @@ std::vector<Group> plan_groups(bool inverse, int64_t n, int J, int L, size_t esz
   return gs;
 }
 
+// the groups as text: what wh_debug_modwt_plan returns, and what tells one plan
+// from another (the kind of a launch among it: a tile and a sliding window may
+// agree in depth, segments and threads)
+std::string plan_text(const std::vector<Group>& gs) {
+  std::string s;
+  for (const Group& G : gs) {
+    char buf[256];
+    snprintf(buf, sizeof buf,
+             "{j0=%d g=%d R=%d NT=%d M=%d nseg=%d P=%lld warm=%d chunks=%d lds=%zu%s} ", G.j0,
+             G.g, G.R, G.NT, G.M, G.nseg, (long long)G.P, G.warm, G.nchunks, G.lds,
+             G.tile ? " tile" : "");
+    s += buf;
+  }
+  return s;
+}
+
 template <typename T>
 int launch(bool inverse, int filt, const Group& G, const ModwtArgs& a, int64_t count, int sp,
            hipStream_t st, int cand = 1) {
@@ -799,25 +815,23 @@ int tune_t(int64_t n, int J, int filt, hipStream_t st) {
   for (int inv = 0; inv < 2 && !rc; ++inv) {
     const bool inverse = inv == 1;
     std::map<std::string, PlanKnobs> cands;  // distinct plans only
-    for (int nt : {kNT1, kNT1 / 2, -kNT1, -kNT1 / 2}) {
+    auto add = [&](int g1, int f, int d, int nt) {
+      PlanKnobs k;
+      k.g1max = g1;
+      k.first_per_cu = f;
+      k.deep_per_cu = d;
+      k.first_nt = nt;
+      cands.emplace(plan_text(plan_groups(inverse, n, J, L, esz, k)), k);
+    };
+    for (int nt : {kNT1, kNT1 / 2}) {
       if (nt == kNT1 / 2 && !inverse) continue;
-      const bool tile = nt < 0;  // only the depth matters
-      for (int g1 = tile ? 3 : std::min(J, 5); g1 <= (tile ? kTileGmax : kGmax); ++g1)
+      for (int g1 = std::min(J, 5); g1 <= kGmax; ++g1)
         for (int f : {1, 2, 4})
-          for (int d : {1, 2, 4, 8}) {
-            if (tile && (f != 1 || d != 1)) continue;
-            PlanKnobs k;
-            k.g1max = g1;
-            k.first_per_cu = f;
-            k.deep_per_cu = d;
-            k.first_nt = nt;
-            std::string key;
-            for (const Group& G : plan_groups(inverse, n, J, L, esz, k))
-              key += std::to_string(G.g) + "/" + std::to_string(G.nseg) + "/" +
-                     std::to_string(G.NT) + ";";
-            cands.emplace(key, k);
-          }
+          for (int d : {1, 2, 4, 8}) add(g1, f, d, nt);
     }
+    for (int nt : {kNT1, kNT1 / 2})  // tiles: only the depth matters
+      for (int g1 = 3; g1 <= kTileGmax; ++g1) add(g1, 1, 1, -nt);
+    if (inverse && wide_fits(kWideInvP, n, J, esz)) add(kWideGmax, 1, 1, -kWideInvNT);
     // the default plan is timed first and another one is taken only when
     // it is faster by more than the run-to-run spread of these timings
     // (about 1%), so that noise cannot replace the default by a plan that is
@@ -908,17 +922,8 @@ std::string modwt_plan_string(bool inverse, int64_t n, int J, int filt, int dtyp
                               int64_t count) {
   const int L = filter_length(filt);
   size_t esz = dtype == WH_F32 ? 4 : 8;
-  auto gs = plan_groups(inverse, n, J, L, esz, knobs_for(inverse, n, J, filt, esz, count), count);
-  std::string s;
-  for (auto& G : gs) {
-    char buf[256];
-    snprintf(buf, sizeof buf,
-             "{j0=%d g=%d R=%d NT=%d M=%d nseg=%d P=%lld warm=%d chunks=%d lds=%zu%s} ", G.j0,
-             G.g, G.R, G.NT, G.M, G.nseg, (long long)G.P, G.warm, G.nchunks, G.lds,
-             G.tile ? " tile" : "");
-    s += buf;
-  }
-  return s;
+  return plan_text(
+      plan_groups(inverse, n, J, L, esz, knobs_for(inverse, n, J, filt, esz, count), count));
 }
 
 }  // namespace wh
