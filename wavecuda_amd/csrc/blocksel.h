@@ -427,6 +427,17 @@ __host__ __device__ constexpr int sel_gather(int NT) { return NT == 512 ? 8192 :
 constexpr int64_t kSelSampledMin = 16384;
 constexpr int64_t kSelSampledMax = 1 << 16;  // beyond, the bracket holds too many
 
+// Whether block_median_sampled takes `count` values: its loop asks lane 63 of a
+// wave for the wave's place, so a wave takes part with all its lanes or none (64
+// loads of 16 bytes).
+__host__ __device__ constexpr bool sel_sampled_takes(int64_t count, size_t esz) {
+  return count >= kSelSampledMin && count <= kSelSampledMax && count % int64_t(64 * (16 / esz)) == 0;
+}
+static_assert(sel_sampled_takes(1 << 14, 8) && sel_sampled_takes(1 << 14, 4) &&
+                  sel_sampled_takes((1 << 14) + 128, 8) && !sel_sampled_takes((1 << 14) + 64, 8) &&
+                  !sel_sampled_takes((1 << 14) + 128, 4),
+              "a wave of the sampled selection must be whole");
+
 // keys as wide as the values
 template <typename T>
 using SelKey = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
@@ -542,7 +553,7 @@ __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, in
   constexpr int kW = 16 / int(sizeof(T)), kU = 16 / kW;
   typedef T TW __attribute__((ext_vector_type(kW)));
   const TW* __restrict__ vw = reinterpret_cast<const TW*>(v);
-  const int nv = int(count / kW);  // count is a multiple of 64
+  const int nv = int(count / kW);  // whole waves: see sel_sampled_takes
   int below = 0;
   T bad = T(0);  // NaN and infinities: left to block_median
   for (int b = tid; b < nv; b += NT * kU) {
@@ -740,8 +751,8 @@ __device__ __forceinline__ bool block_mad_small(const T* __restrict__ v, int cou
 template <typename T, int NT>
 __device__ __forceinline__ double block_mad(const T* __restrict__ v, int64_t count,
                                             unsigned char* ws) {
-  const bool sampled = count >= kSelSampledMin && count <= kSelSampledMax &&
-                       reinterpret_cast<uintptr_t>(v) % 16 == 0 && count % 64 == 0;
+  const bool sampled =
+      sel_sampled_takes(count, sizeof(T)) && reinterpret_cast<uintptr_t>(v) % 16 == 0;
   if (count <= kSelSmallPer * NT) {
     double mad;
     if (block_mad_small<T, NT>(v, int(count), ws, &mad)) return mad;
