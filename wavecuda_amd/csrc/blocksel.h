@@ -45,12 +45,12 @@ __device__ __forceinline__ double sel_val(uint64_t k, float*) {
   return double(__uint_as_float(u));
 }
 
-// bin of a value y in [0, hi] among kSelBins equal-width bins (scale =
+// bin of a value y >= 0 among kSelBins equal-width bins over [0, hi] (scale =
 // kSelBins / hi); monotone non-decreasing in y's key, clamped to the last bin,
 // which also takes NaN: keys rank positive NaN above every number
 __device__ __forceinline__ int sel_bin(double y, double scale) {
   const double u = y * scale;
-  return u < double(kSelBins - 1) ? (u > 0.0 ? int(u) : 0) : kSelBins - 1;
+  return u < double(kSelBins - 1) ? int(u) : kSelBins - 1;
 }
 
 // smallest and largest digit with a non-zero count in h[0..kSelBins), by
