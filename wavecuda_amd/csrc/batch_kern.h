@@ -79,6 +79,19 @@ constexpr int batch_lds_elems() {
   return 4096;
 }
 
+// FP64 512-thread workgroups count the first radix digit of the level-1 details
+// as the forward makes them, where there are more than the selection samples:
+// kSelBins counts at this LDS offset, beyond the forward's levels and
+// block_median's workspace.  It saves the median's first pass over them (a DWT of
+// 2^20 samples, J = 3 LA8: 1990 -> 1826 us).
+constexpr size_t kBatchPreOff = size_t(48) << 10;
+__host__ __device__ constexpr size_t batch_pre_lds(int NT, size_t esz) {
+  return esz == 8 && NT == 512 ? kBatchPreOff + size_t(kSelBins) * 4 : 0;
+}
+static_assert(batch_lds_elems<double>() * 8 * 3 / 2 <= int(kBatchPreOff) &&
+                  block_sel_lds<512>() <= kBatchPreOff,
+              "the first-digit counts lie beyond the forward's and the selection's LDS");
+
 // DWT item coefficients in scratch C, level by level and each level
 // contiguous: d_j at C[n - n/2^{j-1} ..) (n/2^j values), then s_J; for
 // J = 1, s_1[0] goes last, so that C[0 .. n-1) holds d_1 and s_1[1..]: the
@@ -95,7 +108,7 @@ __device__ __forceinline__ int64_t batch_dwt_sidx(int64_t n, int J, int64_t m) {
 // scratch C as above (n values, gA/gB n/2 each behind it).
 template <typename T, int FILT, int NT>
 __device__ __forceinline__ void batch_dwt_fwd(const T* x, int64_t n, int J, T* C,
-                                              unsigned char* smem) {
+                                              unsigned char* smem, unsigned* pre) {
   constexpr int L = Filter<FILT>::L;
   constexpr int kBatchLds = batch_lds_elems<T>();
   constexpr int kUp = 2;  // global-level output pairs of pairs per thread in flight
@@ -143,6 +156,10 @@ __device__ __forceinline__ void batch_dwt_fwd(const T* x, int64_t n, int J, T* C
             fwd_pair<T, FILT>(v[u] + 2, s1, d1);
             *reinterpret_cast<T2*>(dst + 2 * p) = T2{s0, s1};
             *reinterpret_cast<T2*>(dj + 2 * p) = T2{d0, d1};
+            if (pre && j == 1) {
+              atomicAdd(&pre[sel_digit0(d0)], 1u);
+              atomicAdd(&pre[sel_digit0(d1)], 1u);
+            }
           }
         }
       }
@@ -339,12 +356,21 @@ __global__ __launch_bounds__(NT, NT == 128 ? 2 : 3) void batch_smooth_k(BatchArg
     T* s4 = d1 + batch_pad(I.n);
     const T* in = tiled ? s4 : static_cast<const T*>(b.x) + I.off;
     T* out = tiled ? s4 + batch_pad(n) : static_cast<T*>(b.y) + I.off;
+    unsigned* pre = nullptr;
+    if constexpr (batch_pre_lds(NT, sizeof(T)) > 0) {
+      // (not of a one-level DWT, whose selection takes s_1[1..] too)
+      if (dwt && !tiled && J > 1 && n / 2 > sel_sampled_max(NT, sizeof(T))) {
+        pre = reinterpret_cast<unsigned*>(smem + kBatchPreOff);
+        for (int i = threadIdx.x; i < kSelBins; i += NT) pre[i] = 0;
+        __syncthreads();
+      }
+    }
     if (dwt) {
       switch (kind_filter(I.kind)) {
-        case kHAAR: batch_dwt_fwd<T, kHAAR, NT>(in, n, J, scr, smem); break;
-        case kD4: batch_dwt_fwd<T, kD4, NT>(in, n, J, scr, smem); break;
-        case kC6: batch_dwt_fwd<T, kC6, NT>(in, n, J, scr, smem); break;
-        default: batch_dwt_fwd<T, kLA8, NT>(in, n, J, scr, smem); break;
+        case kHAAR: batch_dwt_fwd<T, kHAAR, NT>(in, n, J, scr, smem, pre); break;
+        case kD4: batch_dwt_fwd<T, kD4, NT>(in, n, J, scr, smem, pre); break;
+        case kC6: batch_dwt_fwd<T, kC6, NT>(in, n, J, scr, smem, pre); break;
+        default: batch_dwt_fwd<T, kLA8, NT>(in, n, J, scr, smem, pre); break;
       }
       batch_phase();
     }
@@ -352,7 +378,7 @@ __global__ __launch_bounds__(NT, NT == 128 ? 2 : 3) void batch_smooth_k(BatchArg
     // every kind of item, so the selection is inlined once (a called
     // function would keep its saved registers in scratch memory)
     const int64_t mcount = !dwt ? n : tiled ? I.n / 2 : J == 1 ? n - 1 : n / 2;
-    const double t = block_mad<T, NT>(d1, mcount, smem) * I.factor;
+    const double t = block_mad<T, NT>(d1, mcount, smem, pre) * I.factor;
     if (threadIdx.x == 0) {
       b.thresh[I.sig] = t;
       if (b.thresh_out) b.thresh_out[I.sig] = t;

@@ -69,12 +69,16 @@ constexpr int64_t kBatchTileBytes = int64_t(4) << 30;
 size_t item_lds(int ttype, int NT, size_t esz) {
   size_t b = (NT == 512) ? block_sel_lds<512>()
              : (NT == 256 ? block_sel_lds<256>() : block_sel_lds<128>());
-  b = std::max({b, sel_sampled_lds(NT, esz), sel_small_lds(esz)});
+  b = std::max({b, sel_sampled_lds(NT, esz), sel_small_lds(esz), batch_pre_lds(NT, esz)});
   if (ttype != kDWT) return b;
   const size_t tile = (esz == 8) ? size_t(batch_lds_elems<double>()) * 8
                                  : size_t(batch_lds_elems<float>()) * 4;
   return std::max(b, tile + tile / 2);
 }
+
+// shortest DWT signal without tiles that counts as a long walk (see the
+// untuned shape in wh_batch_create)
+constexpr int kBatchWalk = 1 << 16;
 
 // a DWT signal whose first levels run as tiles
 bool dwt_tiled(const BatchItem& I) { return I.n > kBatchDwtWhole && I.J > kBatchHead; }
@@ -309,8 +313,11 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
   std::stable_sort(items.begin(), items.end(),
                    [&](const BatchItem& a, const BatchItem& b) { return cost(a) > cost(b); });
   const double max_cost = double(cost(items[0]));
-  double sum_cost = 0.0;
-  for (const BatchItem& I : items) sum_cost += double(cost(I));
+  double sum_cost = 0.0, walk_cost = 0.0;  // walk: long DWT signals without tiles
+  for (const BatchItem& I : items) {
+    sum_cost += double(cost(I));
+    if (kind_ttype(I.kind) == kDWT && !dwt_tiled(I) && I.n >= kBatchWalk) walk_cost += double(cost(I));
+  }
   std::vector<BatchTile> tiles;
   std::vector<BatchChunk> chunks;
   int64_t tscr = 0;  // elements of the tiles' workspace
@@ -382,12 +389,15 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     // take it in about two thirds of the time.  Mixed batches, us with 256 /
     // 512 threads: 8192 signals to 2^16 samples FP64 2188 / 2453, FP32 1382 /
     // 1637; 2000 to 2^16 FP64 629 / 620; 1200 to 2^16 (0.27 where the line is
-    // 0.4) FP64 445 / 376, FP32 296 / 257; 300 to 2^16 FP64 256 / 156.
-    // wh_batch_tune times the shapes.
+    // 0.4) FP64 445 / 376, FP32 296 / 257; 300 to 2^16 FP64 256 / 156.  512
+    // threads also where most of the work is long DWT signals without tiles,
+    // whose walk through memory gains nothing from a third workgroup a CU (J = 3,
+    // 1024 x 2^17 FP64 1942 / 1789, FP32 1235 / 1081; 1024 x 2^16 976 / 880 and 629 /
+    // 494; of 2^14, 4096 825 / 902 and 487 / 654).  wh_batch_tune times the shapes.
     int64_t resident = 0;
     p->NT = 256;
     if (int rc = max_grid(p, p->NT, &p->grid, &resident)) return fail(rc);
-    if (sum_cost < 0.4 * max_cost * double(resident)) {
+    if (sum_cost < 0.4 * max_cost * double(resident) || walk_cost > 0.5 * sum_cost) {
       p->NT = 512;
       if (int rc = max_grid(p, p->NT, &p->grid)) return fail(rc);
     }

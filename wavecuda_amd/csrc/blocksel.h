@@ -45,6 +45,12 @@ __device__ __forceinline__ double sel_val(uint64_t k, float*) {
   return double(__uint_as_float(u));
 }
 
+// first radix digit of a value's key
+template <typename T>
+__device__ __forceinline__ unsigned sel_digit0(T v) {
+  return unsigned(sel_key(v) >> (sizeof(T) * 8 - kSelBits));
+}
+
 // bin of a value y >= 0 among kSelBins equal-width bins over [0, hi] (scale =
 // kSelBins / hi); monotone non-decreasing in y's key, clamped to the last bin,
 // which also takes NaN: keys rank positive NaN above every number
@@ -159,11 +165,13 @@ __device__ __forceinline__ void sel_for_each(const T* __restrict__ v, int64_t co
 // kSelBins equal-width bins (what lies beyond in the last), and when the middle ranks' bins hold at most
 // kSelDirect values they are copied to LDS and ranked directly (otherwise
 // the radix digits start from the top).  Of values, the smallest and largest
-// first digit any has are left at sel_range_slot(ws).
+// first digit any has are left at sel_range_slot(ws).  pre (or null): the
+// values' first digits, already counted.
 template <typename T, int NT>
 __device__ __forceinline__ double block_median(const T* __restrict__ v, int64_t count,
                                                bool deviation, double center,
-                                               unsigned char* ws, double bound) {
+                                               unsigned char* ws, double bound,
+                                               const unsigned* pre) {
   uint64_t* cand = reinterpret_cast<uint64_t*>(ws);                     // [kSelCap]
   unsigned* hist = reinterpret_cast<unsigned*>(cand + kSelCap);        // [2][kSelBins]
   unsigned* part = hist + 2 * kSelBins;                                 // [NT]
@@ -323,6 +331,8 @@ __device__ __forceinline__ double block_median(const T* __restrict__ v, int64_t 
     };
     if (in_lds) {
       for (int i = tid; i < nc; i += NT) count_key(cand[i]);
+    } else if (pre && !deviation && hi == kbits) {
+      for (int i = tid; i < kSelBins; i += NT) hist[i] = pre[i];
     } else {
       sel_for_each<T, NT>(v, count, deviation, c, count_key);
     }
@@ -422,20 +432,33 @@ constexpr int kSelRun = 8;
 constexpr int kSelMargin = 96;     // sample ranks on either side of the middle, at most
 // values kept: a 512-thread workgroup has its CU's LDS alone, of the others
 // three share it
-__host__ __device__ constexpr int sel_gather(int NT) { return NT == 512 ? 8192 : 4608; }
+__host__ __device__ constexpr int sel_gather(int NT, size_t esz) {
+  return NT == 512 ? (esz == 8 ? 16384 : 12288) : 4608;
+}
 // below, the passes saved are shorter than the sample's
 constexpr int64_t kSelSampledMin = 16384;
-constexpr int64_t kSelSampledMax = 1 << 16;  // beyond, the bracket holds too many
+// The longest input sampled, sixteen values a kept one: beyond, the bracket that
+// fits is narrower than 2.2 standard deviations of the sample's middle, the middle
+// ranks fall outside it too often, and then the pass was for nothing.  Batches of
+// MODWT signals, J = 4 (a D_1 as long as the signal), us, read in whole / sampled:
+// 512 threads FP64 2^17 one signal 238 / 119, 256 signals 671 / 531; 2^18 431 / 196
+// and 1384 / 1251; FP32 2^17 364 / 351 and beyond the line, 2^18, 722 / 789; 256
+// threads FP64 2^17 784 / 891.
+__host__ __device__ constexpr int64_t sel_sampled_max(int NT, size_t esz) {
+  return 16 * sel_gather(NT, esz);
+}
 
 // Whether block_median_sampled takes `count` values: its loop asks lane 63 of a
 // wave for the wave's place, so a wave takes part with all its lanes or none (64
 // loads of 16 bytes).
-__host__ __device__ constexpr bool sel_sampled_takes(int64_t count, size_t esz) {
-  return count >= kSelSampledMin && count <= kSelSampledMax && count % int64_t(64 * (16 / esz)) == 0;
+__host__ __device__ constexpr bool sel_sampled_takes(int NT, int64_t count, size_t esz) {
+  return count >= kSelSampledMin && count <= sel_sampled_max(NT, esz) &&
+         count % int64_t(64 * (16 / esz)) == 0;
 }
-static_assert(sel_sampled_takes(1 << 14, 8) && sel_sampled_takes(1 << 14, 4) &&
-                  sel_sampled_takes((1 << 14) + 128, 8) && !sel_sampled_takes((1 << 14) + 64, 8) &&
-                  !sel_sampled_takes((1 << 14) + 128, 4),
+static_assert(sel_sampled_takes(256, 1 << 14, 8) && sel_sampled_takes(256, 1 << 14, 4) &&
+                  sel_sampled_takes(256, (1 << 14) + 128, 8) &&
+                  !sel_sampled_takes(256, (1 << 14) + 64, 8) &&
+                  !sel_sampled_takes(256, (1 << 14) + 128, 4),
               "a wave of the sampled selection must be whole");
 
 // keys as wide as the values
@@ -443,7 +466,7 @@ template <typename T>
 using SelKey = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
 
 __host__ __device__ constexpr size_t sel_sampled_lds(int NT, size_t esz) {
-  return size_t(sel_gather(NT) + kSelDirect) * esz + size_t(kSelBins) * 4 + 16 * 8 + 256;
+  return size_t(sel_gather(NT, esz) + kSelDirect) * esz + size_t(kSelBins) * 4 + 16 * 8 + 256;
 }
 
 // Bins of the ranks r0 <= r1 in h[0..kSelBins): the bin, the count before it
@@ -493,7 +516,7 @@ template <typename T, int NT>
 __device__ __forceinline__ bool block_median_sampled(const T* __restrict__ v, int64_t count,
                                                      bool deviation, double center,
                                                      unsigned char* ws, double* res) {
-  constexpr int kWaves = NT / 64, K = kSelSample / NT, kGather = sel_gather(NT);
+  constexpr int kWaves = NT / 64, K = kSelSample / NT, kGather = sel_gather(NT, sizeof(T));
   constexpr int kRuns = kSelSample / kSelRun;
   using Key = SelKey<T>;
   Key* cand = reinterpret_cast<Key*>(ws);
@@ -747,12 +770,13 @@ __device__ __forceinline__ bool block_mad_small(const T* __restrict__ v, int cou
 // 1.4826 median|v - median(v)|, v 16-byte aligned where it is long enough
 // to be sampled.  The smallest and largest first digits present (from the
 // median's own first digit) bound the values, so the deviations' median can
-// start from equal-width bins.
+// start from equal-width bins.  pre: see block_median (beyond the sampled counts
+// only, whose workspace may overlap it).
 template <typename T, int NT>
 __device__ __forceinline__ double block_mad(const T* __restrict__ v, int64_t count,
-                                            unsigned char* ws) {
+                                            unsigned char* ws, const unsigned* pre) {
   const bool sampled =
-      sel_sampled_takes(count, sizeof(T)) && reinterpret_cast<uintptr_t>(v) % 16 == 0;
+      sel_sampled_takes(NT, count, sizeof(T)) && reinterpret_cast<uintptr_t>(v) % 16 == 0;
   if (count <= kSelSmallPer * NT) {
     double mad;
     if (block_mad_small<T, NT>(v, int(count), ws, &mad)) return mad;
@@ -764,7 +788,7 @@ __device__ __forceinline__ double block_mad(const T* __restrict__ v, int64_t cou
     double m;
     if (!sampled || !block_median_sampled<T, NT>(v, count, dev, med[0], ws, &m)) {
       __syncthreads();
-      m = block_median<T, NT>(v, count, dev, med[0], ws, bound);
+      m = block_median<T, NT>(v, count, dev, med[0], ws, bound, pre);
       const int* slot = sel_range_slot<NT>(ws);  // written before block_median's last barrier
       const int d0 = slot[0], d1 = slot[1];
       if (count > kSelDirect && d0 <= d1) {
