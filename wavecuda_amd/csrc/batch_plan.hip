@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <cmath>
 #include <cstdint>
 #include <map>
@@ -32,13 +33,14 @@ struct wh_batch {
   int count = 0;
   int64_t total = 0;
   std::string key;            // composition signature (tuning table key)
+  void* tables = nullptr;          // holds the next four
   wh::BatchItem* items = nullptr;
-  wh::BatchTile* tiles = nullptr;  // the MODWT signals' tiles
-  void* tscratch = nullptr;        // their workspace
-  size_t tile_bytes = 0;
+  wh::BatchTile* tiles = nullptr;  // of the signals that run as tiles
   double* thresh = nullptr;        // one per signal
+  int* counter = nullptr;          // queue head, finished workgroups
+  void* tscratch = nullptr;        // the tiles' workspace
+  size_t tile_bytes = 0;
   std::vector<wh::BatchChunk> chunks;
-  int* counter = nullptr;     // queue head, finished workgroups
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
   int64_t stride = 0;         // workspace elements per workgroup
@@ -125,6 +127,7 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
   std::vector<std::vector<BatchItem>> by_chunk(1);
   std::vector<std::vector<BatchTile>> heads(1);
   int64_t used = 0;
+  size_t expect = 0;  // tiles, about
   *workspace = 0;
   for (BatchItem I : items) {
     I.scr = -1;
@@ -143,10 +146,12 @@ void plan_chunks(std::vector<BatchItem>& items, std::vector<BatchTile>& tiles,
         I.off, used, I.n, 0, kind_filter(I.kind) | (I.J << 3) | (dwt ? kTileDwt : 0), I.sig});
     I.scr = used;
     by_chunk.back().push_back(I);
+    expect += size_t(3 + I.n / (kBatchP / 4));
     used += need;
     *workspace = std::max(*workspace, used);
   }
   items.clear();
+  tiles.reserve(expect);
   for (size_t k = 0; k < by_chunk.size(); ++k) {
     BatchChunk c;
     c.item0 = int(items.size());
@@ -339,39 +344,36 @@ int wh_batch_create(const int* lens, const int* filters, const int* ttypes, cons
     wh_batch_destroy(p);
     return rc;
   };
-  if (hipMalloc(reinterpret_cast<void**>(&p->items), sizeof(BatchItem) * size_t(count)) !=
-      hipSuccess) {
-    p->items = nullptr;
-    return fail(set_error(WH_ERR_NOMEM, "batch: item table allocation failed"));
+  // the device tables in one allocation: items, the queue's two zeros, room for the
+  // thresholds, tiles.  What is small goes up in one copy (an allocation or a copy
+  // costs a plan of a few short signals as much as the rest of its creation); the
+  // tiles of a large batch are not copied once more for it.
+  const size_t item_bytes = sizeof(BatchItem) * size_t(count), head_bytes = item_bytes + 8;
+  const size_t list_at = head_bytes + sizeof(double) * size_t(count);
+  const size_t list_bytes = sizeof(BatchTile) * tiles.size();
+  static_assert(sizeof(BatchItem) % 8 == 0 && 2 * sizeof(int) == 8, "tables stay aligned");
+  const bool one = list_at + list_bytes <= (size_t(1) << 16);
+  std::vector<unsigned char> up(one ? list_at + list_bytes : head_bytes);
+  std::memcpy(up.data(), items.data(), item_bytes);
+  if (one && list_bytes) std::memcpy(up.data() + list_at, tiles.data(), list_bytes);
+  if (hipMalloc(&p->tables, list_at + list_bytes) != hipSuccess) {
+    p->tables = nullptr;
+    return fail(set_error(WH_ERR_NOMEM, "batch: table allocation failed"));
   }
-  if (hipMalloc(reinterpret_cast<void**>(&p->counter), 2 * sizeof(int)) != hipSuccess) {
-    p->counter = nullptr;
-    return fail(set_error(WH_ERR_NOMEM, "batch: queue allocation failed"));
-  }
-  if (hipMalloc(reinterpret_cast<void**>(&p->thresh), sizeof(double) * size_t(count)) !=
-      hipSuccess) {
-    p->thresh = nullptr;
-    return fail(set_error(WH_ERR_NOMEM, "batch: threshold allocation failed"));
-  }
-  p->tile_bytes = size_t(tscr) * esz;
-  if (!tiles.empty()) {
-    if (hipMalloc(reinterpret_cast<void**>(&p->tiles), sizeof(BatchTile) * tiles.size()) !=
-        hipSuccess) {
-      p->tiles = nullptr;
-      return fail(set_error(WH_ERR_NOMEM, "batch: tile table allocation failed"));
-    }
-    if (hipMalloc(&p->tscratch, p->tile_bytes) != hipSuccess) {
-      p->tscratch = nullptr;
-      return fail(set_error(WH_ERR_NOMEM, "batch: workspace allocation failed"));
-    }
-    if (hipMemcpy(p->tiles, tiles.data(), sizeof(BatchTile) * tiles.size(),
-                  hipMemcpyHostToDevice) != hipSuccess)
-      return fail(set_hip_error(hipGetLastError(), "batch: table upload"));
-  }
-  if (hipMemcpy(p->items, items.data(), sizeof(BatchItem) * size_t(count),
-                hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemset(p->counter, 0, 2 * sizeof(int)) != hipSuccess)
+  unsigned char* at = static_cast<unsigned char*>(p->tables);
+  p->items = reinterpret_cast<BatchItem*>(at);
+  p->counter = reinterpret_cast<int*>(at + item_bytes);
+  p->thresh = reinterpret_cast<double*>(at + head_bytes);
+  p->tiles = reinterpret_cast<BatchTile*>(at + list_at);
+  if (hipMemcpy(at, up.data(), up.size(), hipMemcpyHostToDevice) != hipSuccess ||
+      (!one && list_bytes &&
+       hipMemcpy(at + list_at, tiles.data(), list_bytes, hipMemcpyHostToDevice) != hipSuccess))
     return fail(set_hip_error(hipGetLastError(), "batch: table upload"));
+  p->tile_bytes = size_t(tscr) * esz;
+  if (p->tile_bytes && hipMalloc(&p->tscratch, p->tile_bytes) != hipSuccess) {
+    p->tscratch = nullptr;
+    return fail(set_error(WH_ERR_NOMEM, "batch: workspace allocation failed"));
+  }
 
   // the persistent kernel's shape: a tuned one for this composition, or
   {
@@ -411,11 +413,8 @@ void wh_batch_destroy(wh_batch* p) {
   if (!p) return;
   (void)hipDeviceSynchronize();
   drop_graph(p);
-  if (p->items) (void)hipFree(p->items);
-  if (p->counter) (void)hipFree(p->counter);
-  if (p->tiles) (void)hipFree(p->tiles);
+  if (p->tables) (void)hipFree(p->tables);
   if (p->tscratch) (void)hipFree(p->tscratch);
-  if (p->thresh) (void)hipFree(p->thresh);
   if (p->scratch) (void)hipFree(p->scratch);
   delete p;
 }
