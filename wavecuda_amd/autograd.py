@@ -332,7 +332,8 @@ def fit_level_thresholds(x, clean, nlevels, filter="LA8", lam0=None, steps=300, 
     opt = torch.optim.Adam([lam], lr=lr)
     xd = x.detach()
     if (ttype == W.MODWT and clean.shape == x.shape and clean.dtype == x.dtype
-            and clean.device == x.device and not clean.requires_grad and lam.numel() == J):
+            and clean.device == x.device and not clean.requires_grad and lam.shape == (J,)
+            and torch.is_grad_enabled()):
         losses = _fit_modwt(xd, clean, lam, opt, J, f, steps)
     else:  # shapes and types that torch broadcasts and promotes
         losses = []  # kept on the device: no host round trip per step
