@@ -176,7 +176,8 @@ class ThresholdInverseFn(torch.autograd.Function):
     """y = inverse MODWT of the coefficients with per-level thresholds applied
     as the inverse reads them (one pass; the same operations as thresholding
     first, so the same y bit for bit).  Backward: the inverse's adjoint, then
-    the threshold's gradient."""
+    the threshold's gradient; where only the thresholds' gradient is asked for, one
+    pass that writes no cotangent of the coefficients."""
 
     @staticmethod
     def forward(ctx, c, lam, n, J, filt, hardness, minlevel, maxlevel):
@@ -201,6 +202,13 @@ class ThresholdInverseFn(torch.autograd.Function):
         n, J, filt, hardness, minlevel, maxlevel, squeeze, lam_dtype = ctx.meta
         B = c2.shape[0]
         g2 = g.contiguous().view(B, n)
+        if ctx.needs_input_grad[1] and not ctx.needs_input_grad[0]:
+            glam = torch.empty(J, dtype=torch.float64, device=c2.device)
+            thr = W.make_thresh(True, hardness, minlevel, maxlevel, 0.0, lam64.data_ptr())
+            W.check(W.lib().wh_modwt_thresh_inv_adj(
+                _vp(g2), _vp(c2), None, 1, _vp(glam), n, B, J, filt, _dtype(g2), C.byref(thr),
+                _stream()), "wh_modwt_thresh_inv_adj")
+            return None, glam.to(lam_dtype), None, None, None, None, None, None
         gw = torch.empty(B, 2 * n * J, dtype=g.dtype, device=g.device)
         W.check(W.lib().wh_modwt_inv_adj(_vp(g2), _vp(gw), n, B, J, filt, _dtype(g2), _stream()),
                 "wh_modwt_inv_adj")
@@ -210,6 +218,17 @@ class ThresholdInverseFn(torch.autograd.Function):
             gc = gc[0]
         return (gc, None if glam is None else glam.to(lam_dtype), None, None, None, None, None,
                 None)
+
+
+def _details(x, J, filt):
+    """MODWT coefficients (B, 2 n J) of the signals x, details and S_J only (the
+    other S_j slots are undefined)."""
+    x2, _ = _rows(x.contiguous())
+    B, n = x2.shape
+    w = torch.empty(B, 2 * n * J, dtype=x.dtype, device=x.device)
+    W.check(W.lib().wh_modwt_fwd_details(_vp(x2), _vp(w), n, B, J, filt, _dtype(x), _stream()),
+            "wh_modwt_fwd_details")
+    return w
 
 
 class SmoothLevelsFn(torch.autograd.Function):
@@ -222,11 +241,9 @@ class SmoothLevelsFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, lam, J, filt, hardness):
-        x2, squeeze = _rows(x.contiguous())
-        B, n = x2.shape
-        w = torch.empty(B, 2 * n * J, dtype=x.dtype, device=x.device)
-        W.check(W.lib().wh_modwt_fwd_details(_vp(x2), _vp(w), n, B, J, filt, _dtype(x), _stream()),
-                "wh_modwt_fwd_details")
+        squeeze = x.dim() == 1
+        w = _details(x, J, filt)
+        B, n = w.shape[0], x.shape[-1]
         lam64 = lam.detach().to(device=x.device, dtype=torch.float64).contiguous()
         if lam64.numel() != J:
             raise W.WaveHipError("one threshold per level expected")
@@ -335,18 +352,27 @@ def fit_level_thresholds(x, clean, nlevels, filter="LA8", lam0=None, steps=300, 
             and clean.device == x.device and not clean.requires_grad and lam.shape == (J,)
             and torch.is_grad_enabled()):
         losses = _fit_modwt(xd, clean, lam, opt, J, f, steps)
-    else:  # shapes and types that torch broadcasts and promotes
-        losses = []  # kept on the device: no host round trip per step
-        for _ in range(steps):
-            opt.zero_grad(set_to_none=True)
-            loss = torch.mean((smooth_levels(xd, lam, J, f, ttype) - clean) ** 2)
-            loss.backward()
-            opt.step()
-            losses.append(loss.detach())
-        with torch.no_grad():
-            losses.append(torch.mean((smooth_levels(xd, lam, J, f, ttype) - clean) ** 2))
-        losses = torch.stack(losses)
-    return lam.detach(), losses.double().cpu().tolist()
+        return lam.detach(), losses.double().cpu().tolist()
+    # shapes and types that torch broadcasts and promotes
+    if ttype == W.MODWT:
+        w = _details(xd, J, f)  # the signals do not change
+
+        def smooth():
+            y = ThresholdInverseFn.apply(w, lam, n, J, f, W.SOFT, 0, J - 1)
+            return y.view(x.shape)
+    else:
+        def smooth():
+            return smooth_levels(xd, lam, J, f, ttype)
+    losses = []  # kept on the device: no host round trip per step
+    for _ in range(steps):
+        opt.zero_grad(set_to_none=True)
+        loss = torch.mean((smooth() - clean) ** 2)
+        loss.backward()
+        opt.step()
+        losses.append(loss.detach())
+    with torch.no_grad():
+        losses.append(torch.mean((smooth() - clean) ** 2))
+    return lam.detach(), torch.stack(losses).double().cpu().tolist()
 
 
 def _fit_modwt(x, clean, lam, opt, J, filt, steps):
@@ -356,16 +382,13 @@ def _fit_modwt(x, clean, lam, opt, J, filt, steps):
     adjoint, which sums the thresholds' gradients as it reads the
     coefficients and writes no cotangent of them.  Returns the losses (device
     tensor, in x's type as torch.mean would give them)."""
-    x2, _ = _rows(x.contiguous())
-    B, n = x2.shape
+    w = _details(x, J, filt)
+    B, n = w.shape[0], x.shape[-1]
     ref = clean.contiguous()
-    w = torch.empty(B, 2 * n * J, dtype=x.dtype, device=x.device)
     y = torch.empty(B, n, dtype=x.dtype, device=x.device)
     steps = max(steps, 0)
     losses = torch.empty(steps + 1, dtype=torch.float64, device=x.device)
     dt, L = _dtype(x), W.lib()
-    W.check(L.wh_modwt_fwd_details(_vp(x2), _vp(w), n, B, J, filt, dt, _stream()),
-            "wh_modwt_fwd_details")
     lam.grad = torch.empty_like(lam)
     thr = W.make_thresh(True, W.SOFT, 0, J - 1, 0.0, lam.data_ptr())
     for i in range(steps + 1):
