@@ -31,10 +31,13 @@ namespace {
 // two steps costs 33 us of kernels at n = 2^18 (LA8 MODWT, J = 10) where
 // two rounds of one took 40 and four more launches; at n = 2^16 (D4 DWT) 18
 // against 29.  A round of three needs half again the memory traffic of two
-// steps, so where the halves fill the chip (3 n samples of MODWT beyond the
-// tiles' best range) one point a round stays.
-constexpr int64_t kCvRoundMaxModwt = int64_t(1) << 18;
-constexpr int64_t kCvRoundMaxDwt = int64_t(1) << 20;
+// steps, so where the halves fill the chip one point a round stays.  Whole calls,
+// us, one point -> three: LA8 MODWT J = 10 FP64 2^18 428 -> 377, 2^19 569 -> 523,
+// 2^20 816 -> 1122 (FP32 410 -> 364, 493 -> 468, 675 -> 905; Haar FP32 2^19 level at
+// 424); LA8 DWT FP64 2^20 496 -> 426, 2^21 619 -> 538, 2^22 815 -> 790 but Haar 630
+// -> 672, 2^23 1261 -> 1475.
+constexpr int64_t kCvRoundMaxModwt = int64_t(1) << 19;
+constexpr int64_t kCvRoundMaxDwt = int64_t(1) << 21;
 
 struct StatsBuf {
   SelState sel;
