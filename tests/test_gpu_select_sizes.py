@@ -1,5 +1,5 @@
-"""The selection where its gathered bucket may outgrow the buffer (2^22 values
-and more): equal to sorting, and no input of plain noise falls to the last
+"""The selection where its gathered bucket may outgrow the buffer (beyond 2^23
+values): equal to sorting, and no input of plain noise falls to the last
 resort, one workgroup reading every value (3 ms a median at 2^24 values, where a
 call takes 0.2 ms)."""
 import pytest
@@ -21,7 +21,7 @@ def middle(s):
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
-@pytest.mark.parametrize("n", [1 << 22, (1 << 22) + 1, 1 << 24])
+@pytest.mark.parametrize("n", [1 << 22, 1 << 23, (1 << 23) + 1, 1 << 24, (1 << 24) + 3])
 def test_equals_sorting(n, dtype):
     for seed in range(4):
         x = noise(n, dtype, seed)

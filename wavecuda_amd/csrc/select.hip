@@ -44,7 +44,9 @@ constexpr int kNTB = 1024;  // threads of the one-workgroup steps
 constexpr int kFly = 4;     // loads in flight per thread of the passes
 constexpr int kHold = 8;    // values a thread of the one-workgroup kernel holds
 constexpr int kOneMax = kHold * kNTB;
-constexpr int64_t kRefineMin = int64_t(1) << 22;  // a third pass beyond, if need be: see sel_refine_k
+// a third pass beyond: where the open bucket is too full, and always (sel_refines)
+constexpr int64_t kRefineMin = int64_t(1) << 23, kRefineAll = int64_t(1) << 24;
+constexpr int kRefineFull = 1, kRefineAlways = 2;
 constexpr int kBits = 11;
 constexpr int kBins = 1 << kBits;
 constexpr int kDirect = 256;  // keys ranked by counting
@@ -579,25 +581,28 @@ __global__ __launch_bounds__(kNT) void sel_count_k(SelSrc s, SelState* st, int r
 
 // The open bucket that holds the middle ranks is 2 count / kSelSample values
 // on average (a rank falls in a bucket in proportion to its size) and x times
-// count / kSelSample with probability (1 + x) e^-x.  Up to kRefineMin values it
-// outgrows half of the candidate buffer (x = 16) in two of a million calls;
-// at 2^24 (x = 4) in one of eleven, and a workgroup alone then reads every value:
-// cross-validated smoothing of 2^21 FP32 samples, eight levels of details, 7.0
-// ms instead of 1.0.  So beyond kRefineMin, where the bucket is that full, one
-// more pass counts the leading 11 bits of its keys' offsets.  (Half of the
-// buffer, for the regions fill unevenly.)
+// count / kSelSample or more with probability (1 + x) e^-x.  Up to kRefineMin values
+// it outgrows half of the candidate buffer (x = 16) in two of a million calls, which
+// is left to the last resort, a workgroup alone that reads every value; when the
+// buffer held 2^17 keys that was the lot of one median in eleven at 2^24 values
+// (cross-validated smoothing of 2^21 FP32 samples, eight levels of details: 7.0 ms
+// instead of 1.0).  So beyond kRefineMin, where the bucket is that full, one more
+// pass counts the leading 11 bits of its keys' offsets (half of the buffer, for the
+// regions fill unevenly); beyond kRefineAll it always does, since ranking the
+// bucket's 2^16 keys and more costs one workgroup longer (MAD of 3e7 sorted FP32
+// values 240 us, 337 without).
 __device__ __forceinline__ bool sel_refines(int refine, const Pick& p) {
-  return refine && p.inside > u64(kSelCandCap) / 2;
+  return refine == kRefineAlways || (refine == kRefineFull && p.inside > u64(kSelCandCap) / 2);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kNT) void sel_refine_k(SelSrc s, SelState* st, int round) {
+__global__ __launch_bounds__(kNT) void sel_refine_k(SelSrc s, SelState* st, int round, int refine) {
   __shared__ unsigned hist[kBins];
   __shared__ u64 wsum[kNT / 64];
   __shared__ Pick p;
   const int tid = threadIdx.x;
   block_pick<kNT, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
-  if ((p.found[0] && p.found[1]) || !sel_refines(1, p)) return;
+  if ((p.found[0] && p.found[1]) || !sel_refines(refine, p)) return;
   for (int i = tid; i < kBins; i += kNT) hist[i] = 0;
   __syncthreads();
   const T med = round ? T(st->med) : T(0);
@@ -627,7 +632,7 @@ __global__ __launch_bounds__(kNT) void sel_gather_k(SelSrc s, SelState* st, int 
   if (tid == 0) nlist = 0;
   block_pick<kNT, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
   if (p.found[0] && p.found[1]) return;
-  if (sel_refines(refine, p)) (void)block_narrow<kNT>(st->hist[round], &p, wsum);
+  if (refine && sel_refines(refine, p)) (void)block_narrow<kNT>(st->hist[round], &p, wsum);
   if (p.inside > u64(kSelCandCap)) return;  // the last step reads the values
   const T med = round ? T(st->med) : T(0);
   const uint64_t base = p.base, width = p.width;
@@ -667,7 +672,7 @@ __global__ __launch_bounds__(kNTB) void sel_finish_k(SelSrc s, SelState* st, int
   const int tid = threadIdx.x;
   if (next && tid < kSelSample) smp[tid] = st->sample[tid];
   block_pick<kNTB, kReplicas>(st->bins[round], st->edges[round], s.count, &p, wsum);
-  if (!(p.found[0] && p.found[1]) && sel_refines(refine, p))
+  if (refine && !(p.found[0] && p.found[1]) && sel_refines(refine, p))
     (void)block_narrow<kNTB>(st->hist[round], &p, wsum);
   const T med = round ? T(st->med) : T(0);
   // gathered unless there were too many in all, or for one region
@@ -712,12 +717,12 @@ int select_t(SelSrc s, SelState* st, const SelOut& o, hipStream_t stream) {
   }
   const int64_t E = s.mode == 2 ? s.n : s.count;
   const unsigned blocks = unsigned(std::min<int64_t>((E + kFly * kNT - 1) / (kFly * kNT), 1024));
-  const int refine = s.count > kRefineMin ? 1 : 0;
+  const int refine = s.count > kRefineAll ? kRefineAlways : s.count > kRefineMin ? kRefineFull : 0;
   hipLaunchKernelGGL(sel_sample_k<T>, dim3(1), dim3(kSelSample), 0, stream, s, st);
   for (int round = 0; round < (o.mad ? 2 : 1); ++round) {
     hipLaunchKernelGGL(sel_count_k<T>, dim3(blocks), dim3(kNT), 0, stream, s, st, round);
     if (refine)
-      hipLaunchKernelGGL(sel_refine_k<T>, dim3(blocks), dim3(kNT), 0, stream, s, st, round);
+      hipLaunchKernelGGL(sel_refine_k<T>, dim3(blocks), dim3(kNT), 0, stream, s, st, round, refine);
     hipLaunchKernelGGL(sel_gather_k<T>, dim3(blocks), dim3(kNT), 0, stream, s, st, round, refine);
     hipLaunchKernelGGL(sel_finish_k<T>, dim3(1), dim3(kNTB), 0, stream, s, st, round, refine,
                        (o.mad && round == 0) ? 1 : 0, o);

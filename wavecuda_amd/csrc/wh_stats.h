@@ -33,7 +33,7 @@ struct SelSrc {
 };
 
 // device-resident selection state (select.hip); [2]: values, deviations
-constexpr int kSelCandCap = 1 << 18;  // gathered keys it keeps
+constexpr int kSelCandCap = 1 << 19;  // gathered keys it keeps
 constexpr int kSelSample = 512;
 constexpr int kSelEdges = 104;        // +- 4.6 standard deviations of the sample's middle
 constexpr int kSelReplicas = 8;       // copies of the counters
