@@ -3,7 +3,7 @@
 //
 // A sliding-window workgroup walks its segment chunk by chunk, and every
 // chunk is a chain of memory latency and G barriers; that pays when each
-// workgroup has many chunks.  For a launch of up to 2^20 samples the grid
+// workgroup has many chunks.  For a launch of up to 2^21 samples the grid
 // runs out first: the planner then cut the group depth instead (five fused
 // levels and one launch for each further one), and the time was the launches
 // and chains, not bytes.  Here a workgroup computes one tile and ends: all
